@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include <map>
+#include <utility>
 #include <vector>
 
 #include "bp_internal.h"
@@ -26,6 +27,34 @@ extern "C" void bp_set_error(const char *fmt, ...);
     } while (0)
 
 struct bp_tree_plan;
+
+/* What a resident run (bp_resident.hip) leaves in host memory: the head of
+ * the handle's pinned staging buffer. */
+struct bp_resident_status {
+    unsigned run;      /* the last run that went through */
+    unsigned ran;      /* its iterations */
+    unsigned stopped;  /* the stop test ended it */
+    double last, before; /* with the stop test: the last two deltas */
+    double deltas[256];
+};
+
+/* The plan of a network whose iterations run resident (bp_resident.hip). */
+struct bp_resident {
+    bool on = false;
+    bool single = false;       /* one workgroup */
+    std::vector<std::pair<unsigned, unsigned>> pending; /* runs not waited for yet, with their iterations */
+    unsigned ns = 0, G = 0;    /* slots per thread, workgroups */
+    unsigned limit = 0;        /* iterations per launch */
+    unsigned run = 0, met = 0; /* launches, barriers met */
+    char *memory = nullptr;    /* holds all of the following */
+    unsigned *wg_node = nullptr;
+    unsigned short *wg_slots = nullptr;
+    float *ring = nullptr;
+    size_t ring_stride = 0;
+    double *parts = nullptr;
+    unsigned *counters = nullptr;
+    unsigned long long timeout = 0;
+};
 
 struct bp_dev {
     int device = 0;
@@ -48,8 +77,8 @@ struct bp_dev {
     std::vector<unsigned> toff;       /* the same on the host */
     std::vector<unsigned> in_off_h;   /* [V+1] in_off on the host */
     size_t jfloats = 0;               /* floats in J */
-    float *h_stage = nullptr;         /* pinned host staging for uploads and downloads */
-    size_t h_stage_n = 0;             /* its capacity in floats */
+    char *h_stage = nullptr;          /* pinned host memory: a bp_resident_status, then staging for transfers */
+    size_t h_stage_n = 0;             /* the staging's capacity in floats */
     unsigned char *nvars = nullptr;   /* [V] */
     float *states = nullptr;          /* [V][SP] */
     float *buf[2] = {nullptr, nullptr};
@@ -88,6 +117,9 @@ struct bp_dev {
     std::map<unsigned long long, hipGraphExec_t> graphs;
 
     bp_tree_plan *tree = nullptr;
+    bp_resident res;
+
+    bp_resident_status *status() const { return reinterpret_cast<bp_resident_status *>(h_stage); }
 };
 
 inline unsigned stride_of(unsigned S) { return S <= 2 ? S : S <= 4 ? 4 : S <= 8 ? 8 : 10; }
@@ -118,6 +150,18 @@ void bp_cm_order(Graph_t g, std::vector<unsigned> &order);
  * cap in-slots and cap nodes, or one node with more; entry c is chunk c's
  * (first node, first slot), and a sentinel (V, in_off[V]) closes the list. */
 void bp_build_chunks(const std::vector<unsigned> &in_off, unsigned V, unsigned cap, std::vector<uint2> &chunks);
+
+/* resident runs (bp_resident.hip) */
+int bp_resident_plan(bp_dev *d, const std::vector<unsigned> &slot_src, int cus);
+void bp_resident_free(bp_dev *d);
+int bp_resident_launch(bp_dev *d, unsigned n, bool want_delta, bool until, float conv, double previous,
+                       double *partials);
+bool bp_resident_ran(bp_dev *d, bool until = false);
+extern "C" unsigned long long bp_resident_set_timeout(bp_dev *d, unsigned long long ticks);
+extern "C" unsigned bp_resident_shape(const bp_dev *d, unsigned *workgroups);
+int bp_settle(bp_dev *d); /* before a handle's arrays are used otherwise (bp_device.hip) */
+/* deltas[i] = the sum of partials[i * G .. i * G + G), i < n (bp_device.hip) */
+void bp_launch_finish(const double *partials, unsigned G, unsigned n, double *deltas, hipStream_t st);
 
 /* tree BP (bp_tree.hip) */
 int bp_tree_plan_build(bp_dev *d, Graph_t g);

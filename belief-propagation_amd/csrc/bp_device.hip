@@ -82,10 +82,10 @@ __global__ void k_copy_floats(const float *__restrict__ src, float *__restrict__
         dst[i] = src[i];
 }
 
-__global__ void k_until_reset(double *last, unsigned *stop)
+__global__ void k_until_reset(double *last, unsigned *stop, double before)
 {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
-        *last = -1.0;
+        *last = before;
         *stop = 0;
     }
 }
@@ -125,6 +125,7 @@ extern "C" void bp_free(bp_dev *d)
     for (auto &kv : d->graphs)
         (void)hipGraphExecDestroy(kv.second);
     bp_tree_plan_free(d->tree);
+    bp_resident_free(d);
     free_dev_arrays(d);
     if (d->h_stage)
         (void)hipHostFree(d->h_stage);
@@ -483,7 +484,8 @@ static int check_graph(Graph_t g)
     return 0;
 }
 
-/* the handle's pinned staging buffer, at least n floats */
+/* the handle's pinned staging buffer, at least n floats (called with no
+ * resident run outstanding: its status lies in the same memory) */
 static float *stage_buf(bp_dev *d, size_t n)
 {
     if (n > d->h_stage_n) {
@@ -491,15 +493,18 @@ static float *stage_buf(bp_dev *d, size_t n)
             (void)hipHostFree(d->h_stage);
         d->h_stage = nullptr;
         d->h_stage_n = 0;
-        if (hipHostMalloc((void **)&d->h_stage, std::max<size_t>(n, 1) * sizeof(float), hipHostMallocDefault) !=
-            hipSuccess) {
+        if (hipHostMalloc((void **)&d->h_stage, sizeof(bp_resident_status) + std::max<size_t>(n, 1) * sizeof(float),
+                          hipHostMallocDefault) != hipSuccess) {
             d->h_stage = nullptr;
             bp_set_error("pinned staging buffer of %zu floats: allocation failed", n);
             return nullptr;
         }
         d->h_stage_n = n;
+        d->status()->run = 0;
     }
-    return d->h_stage;
+    if (!d->h_stage)
+        return nullptr;
+    return reinterpret_cast<float *>(d->h_stage + sizeof(bp_resident_status));
 }
 
 /* Host rows (MAX_STATES stride, first n valid) -> device rows (SP stride,
@@ -906,6 +911,13 @@ static int upload_impl(Graph_t g, int device, bp_dev **out, bool plan)
         bp_free(d);
         return -1;
     }
+    /* a network that fits runs its iterations resident; without the memory
+     * for that it runs them one launch each */
+    if (bp_resident_plan(d, slot_src, prop.multiProcessorCount) != 0) {
+        bp_resident_free(d);
+        (void)hipGetLastError();
+        bp_clear_error();
+    }
     /* the tree schedule needs levels; without them bp_tree() reports it */
     if (plan && g->num_levels > 0 && bp_tree_plan_build(d, g) != 0)
         bp_clear_error();
@@ -926,6 +938,8 @@ extern "C" int bp_upload_state(bp_dev *d, Graph_t g)
         return -1;
     }
     HIP_TRY(hipSetDevice(d->device));
+    if (bp_settle(d))
+        return -1;
     return upload_state(d, g, true);
 }
 
@@ -1078,6 +1092,8 @@ extern "C" int bp_loopy_init(bp_dev *d)
         return -1;
     }
     HIP_TRY(hipSetDevice(d->device));
+    if (bp_settle(d))
+        return -1;
     LoopyArgs a = bp_make_args(d);
     a.msg_out = d->msg[d->latest]; /* the previous-message array, graph.c:734 */
     a.buf_out = d->buf[d->bcur];
@@ -1105,6 +1121,81 @@ static void enqueue_iterations(bp_dev *d, unsigned n, int latest, int bcur)
                        d->stop, 0.0f, 0, 0u);
 }
 
+void bp_launch_finish(const double *partials, unsigned G, unsigned n, double *deltas, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_finish, dim3(n), dim3(BLOCK), 0, st, partials, G, n, deltas, nullptr, nullptr, 0.0f, 0, 0u);
+}
+
+/* Fewest iterations for which workgroups that wait for each other are
+ * started: the first one's loads of tables and messages, the last one's
+ * stores and the extra barrier cost about as much as two launches. */
+static constexpr unsigned RESIDENT_LEAST = 3;
+
+static bool use_resident(const bp_dev *d, unsigned n)
+{
+    return d->res.on && (d->res.single || n >= RESIDENT_LEAST);
+}
+
+/* n resident iterations in as many launches as their exchange buffers ask
+ * for.  With deltas the run is waited for; without them it may be left to
+ * bp_settle.  *done: iterations that went through or may still; fewer than n
+ * when a run was given up (res.on is then off). */
+static int run_resident(bp_dev *d, unsigned n, double *deltas, double *partials, unsigned *done)
+{
+    *done = 0;
+    while (*done < n && d->res.on) {
+        unsigned batch = std::min(n - *done, d->res.limit);
+        if (bp_resident_launch(d, batch, deltas != nullptr, false, 0.0f, 0.0, partials))
+            return -1;
+        if (deltas) {
+            HIP_TRY(hipStreamSynchronize(d->stream));
+            if (!bp_resident_ran(d)) {
+                d->res.on = false;
+                return 0;
+            }
+            d->res.pending.clear(); /* the runs before it went through too */
+            std::copy(d->status()->deltas, d->status()->deltas + batch, deltas + *done);
+        } else if (!d->res.single) {
+            d->res.pending.emplace_back(d->res.run, batch);
+        }
+        if (batch & 1u)
+            d->latest ^= 1;
+        d->bcur ^= 1;
+        d->swaps += batch;
+        *done += batch;
+    }
+    return 0;
+}
+
+static int iterate_launches(bp_dev *d, unsigned n, double *deltas);
+
+/* Waits for the resident runs that were not waited for and makes up for the
+ * ones that were given up (each run checks that the one before it went
+ * through, so they are the last ones): their iterations run with a launch
+ * each. */
+int bp_settle(bp_dev *d)
+{
+    bp_resident &r = d->res;
+    if (r.pending.empty())
+        return 0;
+    HIP_TRY(hipStreamSynchronize(d->stream));
+    unsigned missing = 0;
+    if (!bp_resident_ran(d)) {
+        for (size_t i = r.pending.size(); i-- > 0 && r.pending[i].first != d->status()->run;) {
+            missing += r.pending[i].second;
+            d->bcur ^= 1;
+        }
+        r.on = false;
+    }
+    r.pending.clear();
+    if (!missing)
+        return 0;
+    if (missing & 1u)
+        d->latest ^= 1;
+    d->swaps -= missing;
+    return iterate_launches(d, missing, nullptr);
+}
+
 extern "C" int bp_loopy_iterate(bp_dev *d, unsigned int n, double *deltas)
 {
     bp_clear_error();
@@ -1113,8 +1204,20 @@ extern "C" int bp_loopy_iterate(bp_dev *d, unsigned int n, double *deltas)
         return -1;
     }
     HIP_TRY(hipSetDevice(d->device));
-    if (ensure_buffer(d))
+    unsigned done = 0;
+    if (use_resident(d, n)) {
+        if (ensure_buffer(d) || run_resident(d, n, deltas, d->partials, &done))
+            return -1;
+        if (done == n)
+            return 0;
+    }
+    if (bp_settle(d) || ensure_buffer(d))
         return -1;
+    return iterate_launches(d, n - done, deltas ? deltas + done : nullptr);
+}
+
+static int iterate_launches(bp_dev *d, unsigned n, double *deltas)
+{
     unsigned done = 0;
     while (done < n) {
         unsigned batch = std::min(n - done, d->part_cap);
@@ -1205,7 +1308,17 @@ extern "C" int bp_loopy_iterate_noalloc(bp_dev *d, unsigned int n, double *delta
     if (noalloc_scratch(d->device, &sc))
         return -1;
     double *partials = sc, *ds = sc + d->NP;
-    if (ensure_buffer(d))
+    unsigned done = 0;
+    if (use_resident(d, n)) {
+        if (ensure_buffer(d) || run_resident(d, n, deltas, d->partials, &done))
+            return -1;
+        if (done == n)
+            return 0;
+        n -= done;
+        if (deltas)
+            deltas += done;
+    }
+    if (bp_settle(d) || ensure_buffer(d))
         return -1;
     for (unsigned i = 0; i < n; ++i) {
         LoopyArgs a = bp_make_args(d);
@@ -1282,13 +1395,42 @@ static int commit_roles(bp_dev *d, int mode, const Roles &r, unsigned ran)
 static int run_until(bp_dev *d, int mode, float convergence, unsigned max_iterations, unsigned *result,
                      double *tail /* [2]: the last two deltas, nullable */)
 {
-    if (mode == ITER && ensure_buffer(d))
+    if (bp_settle(d) || (mode == ITER && ensure_buffer(d)))
         return -1;
-    hipLaunchKernelGGL(k_until_reset, dim3(1), dim3(64), 0, d->stream, d->last, d->stop);
+    double hist[2] = {-1.0, 0.0}, last = -1.0;
+    unsigned done = 0;
+    bool stopped = false;
+    while (mode == ITER && d->res.on && done < max_iterations && !stopped) {
+        const bp_resident_status *s = d->status();
+        if (bp_resident_launch(d, std::min(max_iterations - done, d->res.limit), false, true, convergence, last,
+                               nullptr))
+            return -1;
+        HIP_TRY(hipStreamSynchronize(d->stream));
+        if (!bp_resident_ran(d, true)) {
+            d->res.on = false;
+            break;
+        }
+        hist[0] = s->ran > 1 ? s->before : hist[1];
+        hist[1] = last = s->last;
+        if (s->ran & 1u)
+            d->latest ^= 1;
+        d->bcur ^= 1;
+        d->swaps += s->ran;
+        done += s->ran;
+        stopped = s->stopped != 0;
+    }
+    if (mode == ITER && (stopped || (done && done == max_iterations))) {
+        *result = stopped ? done - 1 : max_iterations;
+        if (tail) {
+            tail[0] = hist[0];
+            tail[1] = hist[1];
+        }
+        return 0;
+    }
+    hipLaunchKernelGGL(k_until_reset, dim3(1), dim3(64), 0, d->stream, d->last, d->stop, last);
     HIP_TRY(hipGetLastError());
     const unsigned batch = 16;
-    unsigned done = 0, stop = 0;
-    double hist[2] = {-1.0, 0.0};
+    unsigned stop = 0;
     std::vector<double> ds(batch);
     Roles r = {d->latest, d->bcur, false};
     while (done < max_iterations) {
@@ -1320,7 +1462,7 @@ static int run_until(bp_dev *d, int mode, float convergence, unsigned max_iterat
         if (stop)
             break;
     }
-    hipLaunchKernelGGL(k_until_reset, dim3(1), dim3(64), 0, d->stream, d->last, d->stop);
+    hipLaunchKernelGGL(k_until_reset, dim3(1), dim3(64), 0, d->stream, d->last, d->stop, -1.0);
     HIP_TRY(hipStreamSynchronize(d->stream));
     *result = stop ? done - 1 : max_iterations;
     if (tail) {
@@ -1335,7 +1477,7 @@ static int run_until(bp_dev *d, int mode, float convergence, unsigned max_iterat
  * iterations of the batches before the converged one. */
 static int run_batched(bp_dev *d, int mode, float convergence, unsigned max_iterations, unsigned *result)
 {
-    if (mode == ITER && ensure_buffer(d))
+    if (bp_settle(d) || (mode == ITER && ensure_buffer(d)))
         return -1;
     double previous = -1.0, delta = 0.0;
     unsigned num_iter = 0, i;
@@ -1373,7 +1515,7 @@ static int run_batched(bp_dev *d, int mode, float convergence, unsigned max_iter
 /* n iterations of `mode` with no stop test (deltas still reduced). */
 static int run_fixed(bp_dev *d, int mode, unsigned n)
 {
-    if (mode == ITER && ensure_buffer(d))
+    if (bp_settle(d) || (mode == ITER && ensure_buffer(d)))
         return -1;
     Roles r = {d->latest, d->bcur, false};
     for (unsigned i = 0; i < n; ++i) {
@@ -1426,6 +1568,8 @@ extern "C" int bp_restore_states(bp_dev *d)
         return -1;
     }
     HIP_TRY(hipSetDevice(d->device));
+    if (bp_settle(d))
+        return -1;
     size_t n = (size_t)d->V * d->SP;
     if (n) {
         hipLaunchKernelGGL(k_copy_floats, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, d->stream, d->states0,
@@ -1444,6 +1588,8 @@ extern "C" int bp_sync(bp_dev *d)
         return -1;
     }
     HIP_TRY(hipSetDevice(d->device));
+    if (bp_settle(d))
+        return -1;
     HIP_TRY(hipStreamSynchronize(d->stream));
     return 0;
 }
@@ -1456,7 +1602,7 @@ extern "C" int bp_profile_loopy(bp_dev *d, unsigned int n, float *ms)
         return -1;
     }
     HIP_TRY(hipSetDevice(d->device));
-    if (ensure_buffer(d))
+    if (bp_settle(d) || ensure_buffer(d))
         return -1;
     std::vector<hipEvent_t> ev(2 * (size_t)n);
     for (auto &e : ev)
@@ -1491,6 +1637,8 @@ extern "C" int bp_download_states(bp_dev *d, float *out)
 {
     bp_clear_error();
     HIP_TRY(hipSetDevice(d->device));
+    if (bp_settle(d))
+        return -1;
     std::vector<float> st((size_t)d->V * d->SP);
     HIP_TRY(hipMemcpyAsync(st.data(), d->states, st.size() * sizeof(float), hipMemcpyDeviceToHost, d->stream));
     HIP_TRY(hipStreamSynchronize(d->stream));
@@ -1519,6 +1667,8 @@ extern "C" int bp_download(bp_dev *d, Graph_t g)
         return -1;
     }
     HIP_TRY(hipSetDevice(d->device));
+    if (bp_settle(d))
+        return -1;
     size_t VS = (size_t)d->V * d->SP;
     float *st = stage_buf(d, VS);
     if (!st)

@@ -269,9 +269,10 @@ __device__ __forceinline__ double wave_sum(double v)
  * Entries past x are +0, the zero extension a node's products read past
  * the message's own entries, also when the sum is NaN (an infinite table
  * entry): 0 / NaN would be NaN, which the products skip instead of
- * multiplying by 0. */
+ * multiplying by 0.  Returns the sum of the rows: where it is finite every
+ * row's sum is, and no entry of the message is NaN. */
 template <int S, bool MIXED>
-__device__ __forceinline__ void send(const float *__restrict__ Jrow, const float *b, unsigned x, unsigned y, float *m)
+__device__ __forceinline__ float send(const float *__restrict__ Jrow, const float *b, unsigned x, unsigned y, float *m)
 {
     float sum = 0.0f;
 #pragma unroll
@@ -286,11 +287,13 @@ __device__ __forceinline__ void send(const float *__restrict__ Jrow, const float
         }
         m[i] = acc;
     }
+    const float raw = sum;
     if (sum <= 0.0f)
         sum = 1.0f;
 #pragma unroll
     for (int i = 0; i < S; ++i)
         m[i] = (!MIXED || (unsigned)i < x) ? m[i] / sum : 0.0f;
+    return raw;
 }
 
 /* send() for a table whose entries past y are +0 in every row i < x (the
@@ -301,8 +304,8 @@ __device__ __forceinline__ void send(const float *__restrict__ Jrow, const float
  * never -0), so the results are send()'s bit for bit with one select per
  * entry of the row instead of one per product. */
 template <int S>
-__device__ __forceinline__ void send_padded(const float *__restrict__ Jrow, const float *b, unsigned x, unsigned y,
-                                            float *m)
+__device__ __forceinline__ float send_padded(const float *__restrict__ Jrow, const float *b, unsigned x, unsigned y,
+                                             float *m)
 {
     float bb[S];
 #pragma unroll
@@ -318,11 +321,13 @@ __device__ __forceinline__ void send_padded(const float *__restrict__ Jrow, cons
         m[i] = (unsigned)i < x ? acc : 0.0f;
         sum = sum + m[i];
     }
+    const float raw = sum;
     if (sum <= 0.0f)
         sum = 1.0f;
 #pragma unroll
     for (int i = 0; i < S; ++i)
         m[i] = (unsigned)i < x ? m[i] / sum : 0.0f;
+    return raw;
 }
 
 /* Row i of a pooled table (rows of y entries padded to a multiple of four)

@@ -1,0 +1,842 @@
+/*
+ * bp_resident.hip -- loopy iterations of networks that fit on the chip.
+ *
+ * k_resident runs many iterations of src/graph/graph.c:1121-1183 in one
+ * launch.  Each workgroup (one per CU, 1024 threads) owns a contiguous range
+ * of device nodes with their in-slots and keeps what does not change between
+ * iterations -- tables, source indices, slot ranges -- in registers, the
+ * nodes' beliefs in registers and the last two iterations' messages in LDS.
+ * Only the combine buffers travel: 8 or 16 bytes per node and iteration.
+ *
+ * What bounds a launch per iteration is not the arithmetic: a small network
+ * spends its time on launches (5.5 us for 2,600 message edges that take
+ * under 1 us of work, and twice that with the stop test's own launch), and a
+ * million-arc binary one re-reads its tables, indices and messages from the
+ * Infinity Cache every iteration.  The register files hold 128 MB in all,
+ * enough for the tables of 2M binary or 0.75M four-state message edges.
+ *
+ * Exchange between workgroups.  An iteration writes its combine buffers to a
+ * place of its own (`ring`, one per iteration of the launch) with
+ * agent-scope stores, which go through to memory, waits for them, and meets
+ * the other workgroups at a grid barrier.  The next iteration gathers with
+ * ordinary loads: no L2 can hold a stale copy of those lines, because the
+ * launch reads no ring address before the barrier that follows its writes,
+ * and because workgroup ranges are cut at 128-byte lines, so no line has two
+ * writers.  No cache is flushed or invalidated.  (Reading two alternating
+ * buffers past the L2s instead was slower.)
+ *
+ * Gathers.  A lane that gathers alone costs the L2 a request of its own, and
+ * a 500k-node iteration made 1.8M of them: 5.8 of its 14.5 us.  Which thread
+ * takes which slot is free -- the messages meet in LDS -- so each workgroup's
+ * slots are dealt out in order of their source, and lanes that share a line
+ * share the request (half as many on random DAGs).
+ *
+ * The barrier: workgroup w adds 1 to counter w mod 16 (one per 256 bytes) and
+ * the first wave polls all 16.  200 barriers of 256 workgroups, per barrier:
+ * 1.4 us; one flag per workgroup and 64 bytes 2.5 us, flags in a row 3.8, one
+ * counter 3.8.  Up to 64 workgroups every form takes about 1.25 us.
+ *
+ * Workgroups wait for each other, so all must be on the chip at once.  The
+ * grid is at most one workgroup per CU, and the host lets one such launch
+ * run on a device at a time (take_turn).  If other work keeps part of the
+ * chip nevertheless, waits end after `timeout` and the run gives up: nothing
+ * has been written that a later step reads, the first workgroup to give up
+ * (or, past the last barrier, to go on) settles it for all in one word, and
+ * the host then runs the same iterations with a launch each.
+ *
+ * A network whose slots fit one workgroup needs none of this: its combine
+ * buffers stay in LDS as well and it can always run (SINGLE).
+ *
+ * Every float operation is the one k_loopy performs, in its order, so
+ * beliefs and messages are bit-identical to it; the FP64 deltas add the same
+ * terms grouped by workgroup.
+ */
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cstring>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+#include "bp_dev.h"
+
+using namespace bpk;
+
+namespace {
+
+constexpr int RB = 1024;            /* threads per workgroup */
+constexpr int RW = RB / WAVE;
+constexpr unsigned MAX_G = 256;
+constexpr unsigned COUNTERS = 16, COUNTER_STRIDE = 64; /* unsigneds between two counters */
+constexpr int PAD = 8; /* rows past the messages that a node's first read may touch */
+
+struct ResArgs {
+    const unsigned *in_off, *slot_src;
+    const unsigned char *slot_xy, *nvars;
+    const float *J;
+    const unsigned *slot_tab;
+    const unsigned *wg_node;        /* [G + 1] first node of each workgroup */
+    const unsigned short *wg_slots; /* [G][NS * 1024] the slot (within the workgroup's) of each thread and turn */
+    float *states;
+    const float *buf_in; /* combine buffers of the first iteration */
+    float *buf_out;      /* ... of the iteration after the last */
+    float *msg0, *msg1;  /* messages before the run; the other array */
+    float *ring;         /* iteration t's combine buffers at ring + t * ring_stride */
+    size_t ring_stride;
+    unsigned n;       /* iterations, at most */
+    int until;        /* stop test of graph.c:1313 after each */
+    float conv;
+    double previous;  /* the delta before the run, for the test */
+    double *partials; /* DELTA: [n][G] delta partials */
+    double *parts;    /* [2][MAX_G] the running iteration's, for the test */
+    unsigned *counters;
+    unsigned met;     /* barriers that the counters have counted */
+    unsigned *decision;
+    unsigned run;
+    unsigned after;   /* the run that this one goes on from, 0: none outstanding */
+    unsigned long long timeout;
+    bp_resident_status *status; /* host memory */
+};
+
+enum { GO_ON = 0, COMMIT = 1 };
+
+/* Settles the run for all workgroups: the first word wins. */
+__device__ __forceinline__ bool settle(unsigned *decision, unsigned run, unsigned commit)
+{
+    const unsigned mine = run << 1 | commit;
+    unsigned cur = __hip_atomic_load(decision, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    while (cur >> 1 != run)
+        if (__hip_atomic_compare_exchange_strong(decision, &cur, mine, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT))
+            return commit;
+    return cur & 1u;
+}
+
+/* Waits until every workgroup has been at barrier number `number` (from 1).
+ * False: this run has been given up.  All threads of the workgroup call it;
+ * `ok` is shared. */
+__device__ __forceinline__ bool grid_step(const ResArgs &a, unsigned wg, unsigned G, unsigned number, unsigned *ok)
+{
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); /* this wave's combine buffers are in memory */
+    __syncthreads();
+    if (threadIdx.x < WAVE) {
+        const unsigned lane = threadIdx.x;
+        if (lane == 0)
+            __hip_atomic_fetch_add(a.counters + (wg % COUNTERS) * COUNTER_STRIDE, 1u, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+        const unsigned members = lane < COUNTERS ? (G - lane + COUNTERS - 1) / COUNTERS : 0u;
+        const unsigned want = (a.met + number) * members;
+        const unsigned long long t0 = wall_clock64();
+        bool there = false;
+        while (!there) {
+            bool all = true;
+            if (members)
+                all = (int)(__hip_atomic_load(a.counters + lane * COUNTER_STRIDE, __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_AGENT) - want) >= 0;
+            there = __ballot(!all) == 0;
+            if (!there && wall_clock64() - t0 > a.timeout) {
+                /* given up, unless another workgroup is already past the
+                 * last barrier: then all have been here */
+                unsigned c = lane == 0 ? (unsigned)settle(a.decision, a.run, GO_ON) : 0u;
+                there = __builtin_amdgcn_readfirstlane(c) != 0;
+                break;
+            }
+        }
+        if (lane == 0)
+            *ok = there;
+    }
+    __syncthreads();
+    asm volatile("" ::: "memory"); /* no gather moves above the barrier */
+    return *ok != 0;
+}
+
+template <int N> __device__ __forceinline__ void store_row_agent(float *p, const float *v)
+{
+    static_assert(N % 2 == 0, "rows are float pairs");
+#pragma unroll
+    for (int i = 0; i < N / 2; ++i) {
+        const unsigned long long lo = __float_as_uint(v[2 * i]), hi = __float_as_uint(v[2 * i + 1]);
+        __hip_atomic_store(reinterpret_cast<unsigned long long *>(p) + i, lo | hi << 32, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
+/* rows of S floats in LDS */
+template <int S> __device__ __forceinline__ void put_row(float *p, const float *v)
+{
+    if constexpr (S == 2)
+        *reinterpret_cast<float2 *>(p) = make_float2(v[0], v[1]);
+    else if constexpr (S == 4)
+        *reinterpret_cast<float4 *>(p) = make_float4(v[0], v[1], v[2], v[3]);
+    else
+#pragma unroll
+        for (int i = 0; i < S; ++i)
+            p[i] = v[i];
+}
+
+template <int S> __device__ __forceinline__ void get_row(const float *p, float *v) { load_row<S>(p, v); }
+
+/* Nodes per thread: a message edge belongs to one node, and the networks'
+ * nodes have two to four of them. */
+template <int NS> struct NodesPerThread {
+    static constexpr int value = (NS + 1) / 2;
+};
+
+/* N in-messages from p on as factors: those past the node's last one are 1,
+ * and so are NaN entries (CLEAN: there may be some), which the products
+ * skip.  All reads are issued before the first product: a read at a time
+ * made the node phase a chain of LDS latencies as long as the largest
+ * in-degree of the wave's nodes (1.5 of 2.3 us on a 700-node network). */
+template <int S, int N, bool CLEAN>
+__device__ __forceinline__ void factors(const float *p, unsigned cnt, float (&f)[N][S])
+{
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+        get_row<S>(p + j * S, f[j]);
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+#pragma unroll
+        for (int i = 0; i < S; ++i)
+            f[j][i] = (unsigned)j < cnt ? f[j][i] : 1.0f;
+        if (CLEAN)
+            nan_to_one<S>(f[j]);
+    }
+}
+
+/* The node phase of k_loopy: st = N(st * t), t = the product of the
+ * in-messages in slot order, and the combine buffer b = st * the same
+ * factors one by one (graph.c:985-1024, 851-882). */
+template <int S, bool MIXED, int NS, bool CLEAN>
+__device__ __forceinline__ void resident_node(const float *msgs, unsigned cnt, unsigned n, float *st, float *b)
+{
+    /* K messages are kept for both products and the rest read D at a time:
+     * as many as the tables leave registers for */
+    constexpr int HELD = S * S * NS;
+    constexpr int K = HELD > 36 ? 2 : HELD > 16 ? 4 : S == 2 ? 8 : 4, D = HELD > 32 ? 2 : 4;
+    float f[K][S], t[S];
+    factors<S, K, CLEAN>(msgs, cnt, f);
+#pragma unroll
+    for (int i = 0; i < S; ++i)
+        t[i] = 1.0f;
+#pragma unroll
+    for (int j = 0; j < K; ++j)
+        mul_all<S>(t, f[j]);
+    for (unsigned q = K; q < cnt; q += D) {
+        float g[D][S];
+        factors<S, D, CLEAN>(msgs + q * S, cnt - q, g);
+#pragma unroll
+        for (int j = 0; j < D; ++j)
+            mul_all<S>(t, g[j]);
+    }
+    mul_all<S>(st, t);
+    normalise<S, MIXED>(st, n);
+#pragma unroll
+    for (int i = 0; i < S; ++i)
+        b[i] = st[i];
+#pragma unroll
+    for (int j = 0; j < K; ++j)
+        mul_all<S>(b, f[j]);
+    for (unsigned q = K; q < cnt; q += D) {
+        float g[D][S];
+        factors<S, D, CLEAN>(msgs + q * S, cnt - q, g);
+#pragma unroll
+        for (int j = 0; j < D; ++j)
+            mul_all<S>(b, g[j]);
+    }
+}
+
+/* NS slots per thread. */
+template <int S, bool MIXED, int NS, bool SINGLE, bool DELTA>
+__global__ __launch_bounds__(RB) void k_resident(ResArgs a)
+{
+    constexpr int SP = Stride<S>::value;
+    constexpr int NN = NodesPerThread<NS>::value;
+    constexpr int W = RB * NS;
+    /* messages by slot: iteration t's in lm[t & 1] (while the tables are
+     * loaded, a staging area) */
+    __shared__ __align__(16) float lm[2][S * (W + PAD)];
+    __shared__ __align__(16) float lbuf[SINGLE ? SP * RB * NN : 4];
+    __shared__ double red[2][RW];
+    __shared__ double total;
+    __shared__ unsigned ok, committed, suspect;
+    const unsigned tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    const unsigned G = gridDim.x, wg = SINGLE ? 0u : xcd_block(blockIdx.x, G);
+    if (!SINGLE && a.after &&
+        __hip_atomic_load(a.decision, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != (a.after << 1 | COMMIT))
+        return; /* the run before this one was given up */
+    const unsigned n0 = a.wg_node[wg], n1 = a.wg_node[wg + 1];
+    const unsigned s0 = a.in_off[n0], ns = a.in_off[n1] - s0;
+    if (tid == 0)
+        suspect = 0;
+
+    /* what stays: tables, sources (with the state counts in the top byte:
+     * node numbers are at most 2^20 here), places in LDS.  Threads past the
+     * last slot repeat it and put its message into the padding. */
+    float J[NS][S * S];
+    unsigned src[NS], at[(NS + 1) / 2]; /* two places to a register */
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+        src[k] = n0;
+        if (k % 2 == 0)
+            at[k / 2] = 0;
+        if (k * RB + wave * WAVE >= ns)
+            continue; /* the wave has no slot in this turn */
+        const unsigned l = k * RB + tid, q = a.wg_slots[(size_t)wg * W + (l < ns ? l : ns - 1)];
+        const unsigned s = s0 + q;
+        at[k / 2] = k % 2 ? (at[k / 2] & 0xffffu) | q << 16 : q;
+        src[k] = a.slot_src[s];
+        if constexpr (MIXED)
+            src[k] |= (unsigned)a.slot_xy[s] << 24;
+    }
+    /* tables by way of LDS, a row (S = 2: both rows) of all slots at a time:
+     * read in slot order, handed out in source order */
+    constexpr int CH = S == 2 ? 4 : S; /* floats of a slot's table at a time */
+#pragma unroll
+    for (int c = 0; c < S * S / CH; ++c) {
+        float *stage = lm[0];
+        for (unsigned l = tid; l < ns; l += RB) {
+            const unsigned s = s0 + l;
+            float t[CH];
+            load_row<CH>(MIXED ? a.J + a.slot_tab[s] + c * (int)mixed_row_stride(S) : a.J + (size_t)s * S * S + c * CH,
+                         t);
+            put_row<CH>(stage + l * CH, t);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < NS; ++k)
+            if (k * RB + wave * WAVE < ns)
+                get_row<CH>(stage + (k % 2 ? at[k / 2] >> 16 : at[k / 2] & 0xffffu) * CH, J[k] + c * CH);
+        __syncthreads();
+    }
+#pragma unroll
+    for (int k = 0; k < NS; ++k) /* threads past the last slot */
+        if (k * RB + tid >= ns)
+            at[k / 2] = k % 2 ? (at[k / 2] & 0xffffu) | (unsigned)W << 16 : (at[k / 2] & 0xffff0000u) | W;
+    if (DELTA) /* the old messages, to their own slots' places */
+        for (unsigned l = tid; l < ns; l += RB) {
+            float old[S];
+            load_rowp<S, SP>(a.msg0 + (size_t)(s0 + l) * SP, old);
+            put_row<S>(lm[0] + l * S, old);
+        }
+    float st[NN][S];
+    unsigned slots[NN], nn[NN]; /* first in-slot | in-degree << 16 (both below 2^16) */
+#pragma unroll
+    for (int r = 0; r < NN; ++r) {
+        const unsigned v = n0 + r * RB + tid;
+        slots[r] = 0;
+        nn[r] = S;
+#pragma unroll
+        for (int i = 0; i < S; ++i)
+            st[r][i] = 1.0f;
+        if (v < n1) {
+            const unsigned b = a.in_off[v], e = a.in_off[v + 1];
+            slots[r] = (b - s0) | (e - b) << 16;
+            if (MIXED)
+                nn[r] = a.nvars[v];
+            load_rowp<S, SP>(a.states + (size_t)v * SP, st[r]);
+            if constexpr (SINGLE) {
+                float b0[S];
+                load_rowp<S, SP>(a.buf_in + (size_t)v * SP, b0);
+#pragma unroll
+                for (int i = 0; i < S; ++i)
+                    lbuf[v * SP + i] = b0[i];
+            }
+        }
+    }
+    if constexpr (SINGLE) {
+        __syncthreads();
+    } else {
+        if (!grid_step(a, wg, G, 1, &ok)) /* everybody is here */
+            return;
+    }
+
+    double previous = a.previous, before = a.previous;
+    unsigned ran = 0, stopped = 0;
+    for (;;) {
+        const float *in = SINGLE ? lbuf : ran == 0 ? a.buf_in : a.ring + (size_t)(ran - 1) * a.ring_stride;
+        float bsrc[NS][S];
+        if (ran < a.n) {
+#pragma unroll
+            for (int k = 0; k < NS; ++k)
+                load_rowp<S, SP>(in + (size_t)(MIXED ? src[k] & 0xffffffu : src[k]) * SP, bsrc[k]);
+        }
+        if (DELTA && a.until && ran > 0) {
+            /* the stop test on the iteration just done, while the gathers
+             * are under way; every workgroup adds the same partials in the
+             * same order */
+            double sum = 0.0;
+            if constexpr (SINGLE) {
+#pragma unroll
+                for (int w = 0; w < RW; ++w)
+                    sum += red[(ran - 1) & 1][w];
+            } else {
+                if (wave == 0) {
+                    for (unsigned i = lane; i < G; i += WAVE)
+                        sum += __hip_atomic_load(a.parts + ((ran - 1) & 1) * MAX_G + i, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT);
+                    sum = wave_sum(sum);
+                    if (lane == 0)
+                        total = sum;
+                }
+                __syncthreads();
+                sum = total;
+            }
+            before = previous;
+            previous = sum;
+            double change = sum - before;
+            if (change < 0.0)
+                change = -change;
+            if (sum < (double)a.conv || change < (double)a.conv) {
+                stopped = 1;
+                break;
+            }
+        }
+        if (ran == a.n)
+            break;
+        const float *lold = lm[ran & 1];
+        float *lnew = lm[(ran & 1) ^ 1];
+        double dacc = 0.0;
+        bool odd = false; /* a message that may hold NaN */
+#pragma unroll
+        for (int k = 0; k < NS; ++k) {
+            if (k * RB + wave * WAVE >= ns)
+                continue;
+            const unsigned x = MIXED ? src[k] >> 24 & 15u : (unsigned)S, y = MIXED ? src[k] >> 28 : (unsigned)S;
+            const unsigned place = k % 2 ? at[k / 2] >> 16 : at[k / 2] & 0xffffu;
+            float m[S], sum;
+            if constexpr (MIXED)
+                sum = send_padded<S>(J[k], bsrc[k], x, y, m);
+            else
+                sum = send<S, false>(J[k], bsrc[k], S, S, m);
+            odd = odd || !(fabsf(sum) < INFINITY);
+            if (DELTA) {
+                float old[S];
+                get_row<S>(lold + place * S, old);
+                double d = 0.0;
+#pragma unroll
+                for (int i = 0; i < S; ++i)
+                    if (!MIXED || (unsigned)i < x) {
+                        float q = old[i] - m[i];
+                        if (q != q)
+                            q = 0.0f;
+                        d += (double)fabsf(q);
+                    }
+                dacc += k * RB + tid < ns ? d : 0.0;
+            }
+            put_row<S>(lnew + place * S, m);
+        }
+        if (__ballot(odd) != 0 && lane == 0)
+            suspect = ran + 1;
+        if (DELTA) {
+            dacc = wave_sum(dacc);
+            if (lane == 0)
+                red[ran & 1][wave] = dacc;
+        }
+        __syncthreads();
+        const bool clean = __builtin_amdgcn_readfirstlane(suspect) == ran + 1;
+        if (DELTA && wave == RW - 1 && (!SINGLE || !a.until)) {
+            /* the wave with the fewest nodes adds up the workgroup's delta */
+            double sum = red[ran & 1][lane % RW];
+#pragma unroll
+            for (int off = RW / 2; off > 0; off >>= 1)
+                sum += __shfl_xor(sum, off, WAVE);
+            if (lane == 0) {
+                if (!a.until)
+                    a.partials[(size_t)ran * G + wg] = sum;
+                else
+                    __hip_atomic_store(a.parts + (ran & 1) * MAX_G + wg, sum, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < NN; ++r) {
+            if (r * RB + wave * WAVE >= n1 - n0)
+                continue;
+            const unsigned v = n0 + r * RB + tid;
+            if (v < n1) {
+                const float *msgs = lnew + (slots[r] & 0xffffu) * S;
+                const unsigned cnt = slots[r] >> 16, n = nn[r];
+                float b[S];
+                if (clean)
+                    resident_node<S, MIXED, NS, true>(msgs, cnt, n, st[r], b);
+                else
+                    resident_node<S, MIXED, NS, false>(msgs, cnt, n, st[r], b);
+                float row[SP];
+#pragma unroll
+                for (int i = 0; i < SP; ++i)
+                    row[i] = (i < S && (!MIXED || (unsigned)i < n)) ? b[i] : 0.0f;
+                if constexpr (SINGLE) {
+#pragma unroll
+                    for (int i = 0; i < S; ++i)
+                        lbuf[v * SP + i] = row[i];
+                } else {
+                    store_row_agent<SP>(a.ring + (size_t)ran * a.ring_stride + (size_t)v * SP, row);
+                }
+            }
+        }
+        ++ran;
+        if constexpr (SINGLE) {
+            __syncthreads();
+        } else {
+            if (!grid_step(a, wg, G, ran + 1, &ok))
+                return;
+        }
+    }
+
+    if constexpr (!SINGLE) {
+        if (tid == 0)
+            committed = settle(a.decision, a.run, COMMIT);
+        __syncthreads();
+        if (!committed)
+            return;
+    }
+    /* results: beliefs, the combine buffers of the next iteration, the last
+     * two iterations' messages */
+    float *newest = ran & 1 ? a.msg1 : a.msg0, *older = ran & 1 ? a.msg0 : a.msg1;
+    for (unsigned l = tid; l < ns; l += RB) {
+        float m[S], row[SP];
+        get_row<S>(lm[ran & 1] + l * S, m);
+#pragma unroll
+        for (int i = 0; i < SP; ++i)
+            row[i] = i < S ? m[i] : 0.0f;
+        store_row_nt<SP>(newest + (size_t)(s0 + l) * SP, row);
+        if (ran > 1) { /* after one iteration they are in place */
+            get_row<S>(lm[(ran & 1) ^ 1] + l * S, m);
+#pragma unroll
+            for (int i = 0; i < SP; ++i)
+                row[i] = i < S ? m[i] : 0.0f;
+            store_row_nt<SP>(older + (size_t)(s0 + l) * SP, row);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < NN; ++r) {
+        const unsigned v = n0 + r * RB + tid;
+        if (v < n1) {
+            float row[SP];
+#pragma unroll
+            for (int i = 0; i < SP; ++i)
+                row[i] = (i < S && (!MIXED || (unsigned)i < nn[r])) ? st[r][i] : 0.0f;
+            store_row_nt<SP>(a.states + (size_t)v * SP, row);
+            if constexpr (SINGLE) {
+#pragma unroll
+                for (int i = 0; i < SP; ++i)
+                    row[i] = i < S ? lbuf[v * SP + i] : 0.0f;
+            } else {
+                load_row<SP>(a.ring + (size_t)(ran - 1) * a.ring_stride + (size_t)v * SP, row);
+            }
+            store_row_nt<SP>(a.buf_out + (size_t)v * SP, row);
+        }
+    }
+    if (tid == 0 && wg == 0) {
+        a.status->ran = ran;
+        a.status->stopped = stopped;
+        a.status->last = previous;
+        a.status->before = before;
+        __hip_atomic_store(&a.status->run, a.run, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+} // namespace
+
+/* ------------------------------------------------------------------------ */
+/* host side                                                                 */
+
+namespace {
+
+/* Most workgroups of a plan with ns slots per thread: the grid is kept small
+ * where it can be -- a barrier among 64 workgroups costs 1.3 us, among 256
+ * 2.5 us.  `most` slots per thread are what the registers (128 per thread)
+ * and LDS (two iterations' messages) hold. */
+unsigned most_slots(unsigned S) { return S == 2 ? 8 : S == 3 ? 4 : 3; }
+
+/* slots per thread go 1, 2, 4, 8; for four states 1, 2, 3 */
+unsigned next_slots(unsigned ns, unsigned S) { return S == 4 && ns == 2 ? 3 : 2 * ns; }
+
+unsigned most_groups(unsigned ns, unsigned S, unsigned cus)
+{
+    const unsigned full = std::min(cus, MAX_G);
+    return ns == most_slots(S) ? full : std::min(full, 64 * ns);
+}
+
+/* Largest network of one workgroup, in slots per thread: messages and
+ * combine buffers share 160 KB of LDS. */
+unsigned single_slots(unsigned S) { return S == 2 ? 4 : 2; }
+
+unsigned nodes_per_thread(unsigned ns) { return (ns + 1) / 2; }
+
+/* Workgroup ranges: consecutive nodes with at most `slots` in-slots and
+ * `nodes` nodes, cut at multiples of `align` nodes.  Empty when a node group
+ * does not fit. */
+bool cut_ranges(const std::vector<unsigned> &in_off, unsigned V, unsigned slots, unsigned nodes, unsigned align,
+                std::vector<unsigned> &first)
+{
+    first.assign(1, 0);
+    unsigned v = 0;
+    while (v < V) {
+        unsigned b = v;
+        while (v < V) {
+            unsigned e = std::min(V, (v / align + 1) * align);
+            if (in_off[e] - in_off[b] > slots || e - b > nodes)
+                break;
+            v = e;
+        }
+        if (v == b)
+            return false;
+        first.push_back(v);
+    }
+    return first.size() > 1;
+}
+
+/* Each workgroup's slots in order of their source, `per` places for each
+ * workgroup (host threads over the workgroups). */
+void deal_slots(const std::vector<unsigned> &in_off, const std::vector<unsigned> &slot_src,
+                const std::vector<unsigned> &first, unsigned per, std::vector<unsigned short> &order)
+{
+    const unsigned G = (unsigned)first.size() - 1;
+    order.assign((size_t)G * per, 0);
+    auto deal = [&](unsigned w0, unsigned w1) {
+        std::vector<uint64_t> key;
+        for (unsigned w = w0; w < w1; ++w) {
+            const unsigned s0 = in_off[first[w]], s1 = in_off[first[w + 1]];
+            key.clear();
+            for (unsigned s = s0; s < s1; ++s)
+                key.push_back((uint64_t)slot_src[s] << 16 | (s - s0));
+            std::sort(key.begin(), key.end());
+            for (unsigned i = 0; i < key.size(); ++i)
+                order[(size_t)w * per + i] = (unsigned short)key[i];
+        }
+    };
+    const unsigned T = slot_src.size() < (1u << 16) ? 1u
+                                                     : std::min(16u, std::max(1u, std::thread::hardware_concurrency()));
+    std::vector<std::thread> th;
+    for (unsigned t = 1; t < T; ++t)
+        th.emplace_back(deal, (unsigned)((uint64_t)G * t / T), (unsigned)((uint64_t)G * (t + 1) / T));
+    deal(0, G / T);
+    for (auto &x : th)
+        x.join();
+}
+
+/* One resident launch at a time per device: the launches of two streams,
+ * each partly on the chip, would wait for each other.  A launch on another
+ * stream than the last one waits for that stream. */
+constexpr int MAX_DEVICES = 64;
+std::mutex turn_mu;
+struct {
+    hipStream_t last;
+    hipEvent_t ev;
+} turn[MAX_DEVICES];
+
+int take_turn(int device, hipStream_t stream)
+{
+    auto &t = turn[device];
+    if (t.last && t.last != stream) {
+        if (!t.ev)
+            HIP_TRY(hipEventCreateWithFlags(&t.ev, hipEventDisableTiming));
+        HIP_TRY(hipEventRecord(t.ev, t.last));
+        HIP_TRY(hipStreamWaitEvent(stream, t.ev, 0));
+    }
+    t.last = stream;
+    return 0;
+}
+
+template <int S, bool MIXED, int NS, bool SINGLE>
+void launch_d(const ResArgs &a, unsigned G, bool delta, hipStream_t st)
+{
+    if (delta)
+        hipLaunchKernelGGL((k_resident<S, MIXED, NS, SINGLE, true>), dim3(G), dim3(RB), 0, st, a);
+    else
+        hipLaunchKernelGGL((k_resident<S, MIXED, NS, SINGLE, false>), dim3(G), dim3(RB), 0, st, a);
+}
+
+template <int S, bool MIXED>
+void launch_s(const ResArgs &a, unsigned ns, unsigned G, bool single, bool delta, hipStream_t st)
+{
+    if (single) {
+        if (ns == 1)
+            launch_d<S, MIXED, 1, true>(a, 1, delta, st);
+        else if (ns == 2)
+            launch_d<S, MIXED, 2, true>(a, 1, delta, st);
+        else if constexpr (S == 2)
+            launch_d<S, MIXED, 4, true>(a, 1, delta, st);
+        return;
+    }
+    if (ns == 1)
+        launch_d<S, MIXED, 1, false>(a, G, delta, st);
+    else if (ns == 2)
+        launch_d<S, MIXED, 2, false>(a, G, delta, st);
+    else if constexpr (S == 4)
+        launch_d<S, MIXED, 3, false>(a, G, delta, st);
+    else if (ns == 4)
+        launch_d<S, MIXED, 4, false>(a, G, delta, st);
+    else if constexpr (S == 2)
+        launch_d<S, MIXED, 8, false>(a, G, delta, st);
+}
+
+void launch(unsigned S, bool mixed, const ResArgs &a, unsigned ns, unsigned G, bool single, bool delta,
+            hipStream_t st)
+{
+    if (S == 2)
+        launch_s<2, false>(a, ns, G, single, delta, st);
+    else if (S == 3)
+        mixed ? launch_s<3, true>(a, ns, G, single, delta, st) : launch_s<3, false>(a, ns, G, single, delta, st);
+    else
+        mixed ? launch_s<4, true>(a, ns, G, single, delta, st) : launch_s<4, false>(a, ns, G, single, delta, st);
+}
+
+} // namespace
+
+/* Decides whether the graph runs resident and lays out its ranges:
+ * uniform state counts of 2 to 4, or mixed ones up to 3 or 4. */
+int bp_resident_plan(bp_dev *d, const std::vector<unsigned> &slot_src, int cus)
+{
+    bp_resident &r = d->res;
+    if (d->E == 0 || d->S < 2 || d->S > 4 || (d->mixed && d->S == 2) || d->device >= MAX_DEVICES)
+        return 0;
+    std::vector<unsigned> first;
+    const unsigned align = 32 / d->SP; /* nodes per 128-byte line */
+    for (unsigned ns = 1; ns <= single_slots(d->S) && !r.ns; ns *= 2)
+        if (d->E <= ns * RB && d->V <= nodes_per_thread(ns) * RB) {
+            r.ns = ns;
+            r.single = true;
+            first = {0, d->V};
+        }
+    for (unsigned ns = 1; ns <= most_slots(d->S) && !r.ns; ns = next_slots(ns, d->S)) {
+        /* even ranges: the slots spread over as many workgroups as the cap
+         * asks for, a few per cent more where node groups do not fit */
+        const unsigned cap = ns * RB, full = cap * 31 / 32, groups = most_groups(ns, d->S, (unsigned)cus);
+        const unsigned want = (d->E + full - 1) / full;
+        const unsigned even = std::min(cap, (d->E + want - 1) / want + cap / 32);
+        if (want <= groups && cut_ranges(d->in_off_h, d->V, even, nodes_per_thread(ns) * RB, align, first) &&
+            first.size() - 1 <= groups)
+            r.ns = ns;
+    }
+    if (!r.ns)
+        return 0;
+    r.G = (unsigned)first.size() - 1;
+    r.limit = d->part_cap;
+    /* one device allocation, the parts that are copied there first:
+     * counters and decision (zero), ranges, dealt slots; then the delta
+     * partials of the stop test and the ring */
+    std::vector<unsigned short> order;
+    deal_slots(d->in_off_h, slot_src, first, r.ns * RB, order);
+    const size_t words = COUNTERS * COUNTER_STRIDE + COUNTER_STRIDE;
+    std::vector<unsigned> head(words + first.size() + (order.size() + 1) / 2, 0u);
+    std::copy(first.begin(), first.end(), head.begin() + words);
+    std::memcpy(head.data() + words + first.size(), order.data(), order.size() * sizeof(unsigned short));
+    const size_t parts_at = (head.size() * 4 + 127) / 128 * 128, ring_at = parts_at + 2 * MAX_G * sizeof(double);
+    size_t bytes = ring_at;
+    if (!r.single) {
+        /* a place per iteration of a launch: 8 MB of them, 32 at least */
+        r.ring_stride = ((size_t)d->V * d->SP + 31) / 32 * 32;
+        r.limit = std::min<size_t>(r.limit, std::min<size_t>(256, std::max<size_t>(32, (8u << 20) / (4 * r.ring_stride))));
+        bytes += r.ring_stride * r.limit * sizeof(float);
+        int khz = 0;
+        HIP_TRY(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, d->device));
+        r.timeout = (unsigned long long)khz * 1000; /* a second */
+    }
+    HIP_TRY(hipMalloc((void **)&r.memory, bytes));
+    HIP_TRY(hipMemcpy(r.memory, head.data(), head.size() * sizeof(unsigned), hipMemcpyHostToDevice));
+    r.counters = (unsigned *)r.memory;
+    r.wg_node = r.counters + words;
+    r.wg_slots = (unsigned short *)(r.wg_node + first.size());
+    r.parts = (double *)(r.memory + parts_at);
+    r.ring = (float *)(r.memory + ring_at);
+    r.on = true;
+    return 0;
+}
+
+void bp_resident_free(bp_dev *d)
+{
+    bp_resident &r = d->res;
+    {
+        std::lock_guard<std::mutex> lock(turn_mu);
+        if (d->stream && d->device < MAX_DEVICES && turn[d->device].last == d->stream)
+            turn[d->device].last = nullptr;
+    }
+    if (r.memory)
+        (void)hipFree(r.memory);
+    r = bp_resident();
+}
+
+/* Enqueues up to n (<= res.limit) iterations: with want_delta their deltas
+ * go to the status's deltas, and with `until` the stop test ends the run. */
+int bp_resident_launch(bp_dev *d, unsigned n, bool want_delta, bool until, float conv, double previous,
+                       double *partials)
+{
+    bp_resident &r = d->res;
+    ResArgs a;
+    a.in_off = d->in_off;
+    a.slot_src = d->slot_src;
+    a.slot_xy = d->slot_xy;
+    a.nvars = d->nvars;
+    a.J = d->J;
+    a.slot_tab = d->mixed ? d->slot_toff : nullptr;
+    a.wg_node = r.wg_node;
+    a.wg_slots = r.wg_slots;
+    a.states = d->states;
+    a.buf_in = d->buf[d->bcur];
+    a.buf_out = d->buf[d->bcur ^ 1];
+    a.msg0 = d->msg[d->latest];
+    a.msg1 = d->msg[d->latest ^ 1];
+    a.ring = r.ring;
+    a.ring_stride = r.ring_stride;
+    a.n = n;
+    a.until = until;
+    a.conv = conv;
+    a.previous = previous;
+    /* one workgroup: its partial is the delta */
+    a.partials = r.single ? d->status()->deltas : partials;
+    a.parts = r.parts;
+    a.counters = r.counters;
+    a.met = r.met;
+    a.decision = r.counters + COUNTERS * COUNTER_STRIDE;
+    r.run = (r.run + 1) & 0x7fffffffu;
+    a.run = r.run;
+    a.after = r.pending.empty() ? 0u : r.pending.back().first;
+    a.timeout = r.timeout;
+    a.status = d->status();
+    if (!until)
+        r.met += n + 1; /* else bp_resident_ran says how many */
+    if (r.single) {
+        launch(d->S, d->mixed, a, r.ns, 1, true, want_delta || until, d->stream);
+    } else {
+        std::lock_guard<std::mutex> lock(turn_mu);
+        if (take_turn(d->device, d->stream))
+            return -1;
+        launch(d->S, d->mixed, a, r.ns, r.G, false, want_delta || until, d->stream);
+    }
+    if (want_delta && !until && !r.single)
+        bp_launch_finish(partials, r.G, n, d->status()->deltas, d->stream);
+    HIP_TRY(hipGetLastError());
+    return 0;
+}
+
+/* After the stream has been waited for: whether the last launch went
+ * through. */
+bool bp_resident_ran(bp_dev *d, bool until)
+{
+    bp_resident &r = d->res;
+    const bool ran = r.single || d->status()->run == r.run;
+    if (ran && until)
+        r.met += d->status()->ran + 1;
+    return ran;
+}
+
+/* Ticks of the wall clock that the workgroups of a resident run wait for
+ * each other; returns the previous setting.  With 0 a run is given up at its
+ * first wait and its iterations run with a launch each. */
+extern "C" unsigned long long bp_resident_set_timeout(bp_dev *d, unsigned long long ticks)
+{
+    unsigned long long before = d->res.timeout;
+    d->res.timeout = ticks;
+    return before;
+}
+
+/* Slots per thread of the handle's resident runs (0: it runs a launch per
+ * iteration) and their workgroups. */
+extern "C" unsigned bp_resident_shape(const bp_dev *d, unsigned *workgroups)
+{
+    *workgroups = d->res.on ? d->res.G : 0;
+    return d->res.on ? d->res.ns : 0;
+}

@@ -526,6 +526,8 @@ extern "C" int bp_tree(bp_dev *d)
         return -1;
     }
     HIP_TRY(hipSetDevice(d->device));
+    if (bp_settle(d))
+        return -1;
     /* tree BP works on the buffer mirroring the host's edges_messages */
     hipGraphExec_t &exec = d->tree->graph[a_index(d)];
     if (!exec) {

@@ -1,0 +1,187 @@
+"""Resident runs (bp_resident.hip): networks whose tables stay in registers
+through all iterations of a launch.  Beliefs and both message arrays are the
+oracle's, bit for bit, and the FP64 deltas its sums, at the sizes where the
+plan changes: one workgroup or several, 1 to 8 slots per thread, uniform and
+mixed state counts, runs longer than a launch's exchange buffers."""
+from __future__ import annotations
+
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import bp_ctypes as B
+from conftest import bits_report, same_bits
+
+pytestmark = pytest.mark.gpu
+
+
+def networks(lib, **kw):
+    bn = B.generate("c2", **kw)
+    g, h = B.bn_to_graph(bn), B.bn_to_graph(bn)
+    lib.bp_bn_free(bn)
+    return g, h
+
+
+def shape(dev):
+    dev.lib.bp_resident_shape.argtypes = [C.c_void_p, C.POINTER(C.c_uint)]
+    groups = C.c_uint()
+    return dev.lib.bp_resident_shape(dev.h, C.byref(groups)), groups.value
+
+
+def give_up(dev):
+    """Every run ends at its first wait."""
+    dev.lib.bp_resident_set_timeout.argtypes = [C.c_void_p, C.c_ulonglong]
+    dev.lib.bp_resident_set_timeout.restype = C.c_ulonglong
+    dev.lib.bp_resident_set_timeout(dev.h, 0)
+
+
+def oracle_run(orc, h, n):
+    deltas = []
+    orc.init_previous_edge(h)
+    for _ in range(n):
+        orc.loopy_iteration(h, threads=8)
+        deltas.append(orc.delta64(h))
+    return np.array(deltas)
+
+
+def check(g, h):
+    assert same_bits(B.states(g), B.states(h)), bits_report(B.states(g), B.states(h))
+    for which in ("cur", "prev"):
+        assert same_bits(B.messages(g, which), B.messages(h, which)), which
+
+
+# (nodes, states lo, hi, slots per thread, more than one workgroup): about 3.7
+# message edges per node
+CASES = [
+    (2, 2, 2, 1, False),
+    (250, 2, 2, 1, False),
+    (290, 2, 2, 2, False),
+    (1000, 2, 2, 4, False),
+    (1200, 2, 2, 1, True),
+    (250, 3, 3, 1, False),
+    (480, 4, 4, 2, False),
+    (500, 2, 4, 2, False),
+    (700, 2, 3, 1, True),
+    (3001, 2, 4, 1, True),
+    (17500, 2, 2, 2, True),
+    (40000, 3, 3, 2, True),
+    (70001, 2, 4, 3, True),
+    (71000, 3, 3, 4, True),
+    (75000, 2, 2, 4, True),
+    (290000, 2, 2, 8, True),
+]
+
+
+@pytest.mark.parametrize("nodes,lo,hi,per_thread,several", CASES)
+def test_iterations_and_deltas_match_oracle(lib, orc, nodes, lo, hi, per_thread, several):
+    print(f"resident {nodes} nodes, {lo}-{hi} states", flush=True)
+    g, h = networks(lib, num_nodes=nodes, states_lo=lo, states_hi=hi, seed=900 + nodes)
+    n = 12 if nodes < 100000 else 5
+    dev = B.Device(g)
+    ns, groups = shape(dev)
+    assert (ns, groups > 1) == (per_thread, several)
+    dev.init()
+    first = dev.iterate(n - 1, want_deltas=True)
+    last = dev.iterate(1, want_deltas=True)  # on from there, with the other buffers
+    dev.download(g)
+    want = oracle_run(orc, h, n)
+    check(g, h)
+    assert np.allclose(np.append(first, last), want, rtol=1e-12, atol=0)
+    # the same without deltas, from the start, in two runs that are not waited for
+    dev.restore()
+    dev.init()
+    dev.iterate(n - 4)
+    dev.iterate(4)
+    dev.download(g)
+    check(g, h)
+    dev.free()
+    for x in (g, h):
+        lib.graph_destroy(x)
+
+
+@pytest.mark.parametrize("nodes,hi,conv,most", [(300, 2, 1e-3, 200), (900, 2, 1e-30, 300), (5000, 2, 1e-3, 200),
+                                                (3000, 4, 1e-30, 300), (3000, 4, 1e9, 10), (5000, 2, 1e-30, 1)])
+def test_until_matches_oracle(lib, orc, nodes, hi, conv, most):
+    print(f"resident until {nodes} nodes", flush=True)
+    g, h = networks(lib, num_nodes=nodes, states_hi=hi, seed=77 + nodes)
+    dev = B.Device(g)
+    assert shape(dev)[0] > 0
+    dev.init()
+    got = dev.until(conv, most)
+    dev.download(g)
+    orc.init_previous_edge(h)
+    previous, want = -1.0, most
+    for i in range(most):
+        orc.loopy_iteration(h, threads=8)
+        d = orc.delta64(h)
+        if d < np.float32(conv) or abs(d - previous) < np.float32(conv):
+            want = i
+            break
+        previous = d
+    assert got == want
+    check(g, h)
+    dev.free()
+    for x in (g, h):
+        lib.graph_destroy(x)
+
+
+@pytest.mark.parametrize("nodes", [5000, 60000])
+def test_a_run_that_is_given_up_is_made_up_for(lib, orc, nodes):
+    """Workgroups that do not wait at all: the iterations run with a launch
+    each, from the state before the run, whether it was waited for or not."""
+    print(f"given up {nodes} nodes", flush=True)
+    g, h = networks(lib, num_nodes=nodes, states_hi=2, seed=5 + nodes)
+    want = oracle_run(orc, h, 11)
+    for deltas in (False, True):
+        dev = B.Device(g)
+        assert shape(dev)[1] > 1
+        dev.init()
+        dev.iterate(3)  # goes through, or is still under way
+        give_up(dev)
+        dev.iterate(5)
+        got = dev.iterate(3, want_deltas=deltas)
+        dev.download(g)
+        check(g, h)
+        assert not deltas or np.allclose(got, want[-3:], rtol=1e-12, atol=0)
+        dev.restore()
+        dev.free()
+        lib.graph_destroy(g)
+        bn = B.generate("c2", num_nodes=nodes, states_hi=2, seed=5 + nodes)
+        g = B.bn_to_graph(bn)
+        lib.bp_bn_free(bn)
+    dev = B.Device(g)
+    give_up(dev)
+    dev.init()
+    got = dev.until(1e-30, 11)
+    dev.download(g)
+    assert got == 11
+    check(g, h)
+    dev.free()
+    for x in (g, h):
+        lib.graph_destroy(x)
+
+
+def test_runs_on_two_handles_from_two_threads(lib, orc):
+    """Resident runs of different handles take turns on a device."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    print("two handles", flush=True)
+    pairs = [networks(lib, num_nodes=20000 + 64 * k, states_hi=2, seed=40 + k) for k in range(2)]
+
+    def work(g):
+        dev = B.Device(g)
+        for _ in range(10):
+            dev.restore()
+            dev.init()
+            dev.iterate(9)
+        dev.download(g)
+        dev.free()
+
+    with ThreadPoolExecutor(2) as pool:
+        list(pool.map(work, [g for g, _ in pairs]))
+    for g, h in pairs:
+        oracle_run(orc, h, 9)
+        check(g, h)
+        lib.graph_destroy(g)
+        lib.graph_destroy(h)

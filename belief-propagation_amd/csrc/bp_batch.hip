@@ -39,6 +39,7 @@
 #include <vector>
 
 #include "bp_dev.h"
+#include "bp_parallel.h"
 #include "../../include/bp_batch.h"
 
 using namespace bpk;
@@ -50,6 +51,20 @@ __global__ void k_copy_batch(const float *__restrict__ src, float *__restrict__ 
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n)
         dst[i] = src[i];
+}
+
+/* an instance's belief rows (n pairs) and both message arrays (m pairs each;
+ * rows hold an even number of floats), back to back */
+__global__ void k_rows_to_host(const float2 *__restrict__ states, size_t n, const float2 *__restrict__ newest,
+                               const float2 *__restrict__ older, size_t m, float2 *__restrict__ dst)
+{
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n)
+        dst[i] = states[i];
+    else if (i < n + m)
+        dst[i] = newest[i - n];
+    else if (i < n + 2 * m)
+        dst[i] = older[i - n - m];
 }
 
 __global__ void k_zero_counter(unsigned *q)
@@ -165,6 +180,7 @@ struct bp_batch {
     float *d_msg[2] = {nullptr, nullptr};
     double *d_partials = nullptr;
     double *d_deltas = nullptr;
+    float *h_stage = nullptr; /* pinned: one instance's rows, for downloads */
     unsigned deltas_cap = 0;
     Shape shapes[2];
 
@@ -211,6 +227,8 @@ extern "C" void bp_batch_free(bp_batch *b)
         for (void *p : ps)
             if (p)
                 (void)hipFree(p);
+        if (b->h_stage)
+            (void)hipHostFree(b->h_stage);
         if (b->stream)
             (void)hipStreamDestroy(b->stream);
     }
@@ -551,6 +569,11 @@ extern "C" int bp_batch_upload(bp_batch *b, int device)
             up(&sh.d_wide, sh.wide.data(), sh.wide.size()))
             return -1;
     }
+    size_t most = 1;
+    for (unsigned i = 0; i < b->n_inst; ++i)
+        most = std::max<size_t>(most, b->node_row_off[i + 1] - b->node_row_off[i] +
+                                          2 * (b->msg_row_off[i + 1] - b->msg_row_off[i]));
+    HIP_TRY(hipHostMalloc((void **)&b->h_stage, most * sizeof(float), hipHostMallocDefault));
     HIP_TRY(hipMemcpy(b->d_states, b->d_states0, VS * sizeof(float), hipMemcpyDeviceToDevice));
     HIP_TRY(hipMemset(b->d_buf[0], 0, VS * sizeof(float)));
     HIP_TRY(hipMemset(b->d_buf[1], 0, VS * sizeof(float)));
@@ -857,34 +880,59 @@ extern "C" int bp_batch_download(bp_batch *b, unsigned int index, Graph_t g)
     HIP_TRY(hipSetDevice(b->device));
     size_t r0 = b->node_row_off[index], rn = b->node_row_off[index + 1] - r0;
     size_t q0 = b->msg_row_off[index], qn = b->msg_row_off[index + 1] - q0;
-    std::vector<float> st(rn), m0(qn), m1(qn);
-    if (rn)
-        HIP_TRY(hipMemcpyAsync(st.data(), b->d_states + r0, rn * 4, hipMemcpyDeviceToHost, b->stream));
-    if (qn) {
-        HIP_TRY(hipMemcpyAsync(m0.data(), b->d_msg[b->latest] + q0, qn * 4, hipMemcpyDeviceToHost, b->stream));
-        HIP_TRY(hipMemcpyAsync(m1.data(), b->d_msg[b->latest ^ 1] + q0, qn * 4, hipMemcpyDeviceToHost, b->stream));
+    float *st = b->h_stage, *m0 = st + rn, *m1 = m0 + qn;
+    /* one launch that writes pinned memory: three copies took 30 us more,
+     * most of a small instance's download */
+    if (rn + qn) {
+        hipLaunchKernelGGL(k_rows_to_host, dim3(nblocks(rn / 2 + qn)), dim3(256), 0, b->stream,
+                           reinterpret_cast<const float2 *>(b->d_states + r0), rn / 2,
+                           reinterpret_cast<const float2 *>(b->d_msg[b->latest] + q0),
+                           reinterpret_cast<const float2 *>(b->d_msg[b->latest ^ 1] + q0), qn / 2,
+                           reinterpret_cast<float2 *>(st));
+        HIP_TRY(hipGetLastError());
+    }
+    /* where the parts of the two walks below begin, while the copies run */
+    constexpr unsigned PARTS = 16;
+    const size_t grain = 4096;
+    const unsigned parts = (unsigned)std::max<size_t>(1, std::min<size_t>(PARTS, ((size_t)V + E) / grain));
+    size_t node_at[PARTS + 1] = {0}, msg_at[PARTS + 1] = {0};
+    auto node_of = [&](unsigned p) { return (size_t)V * p / parts; };
+    auto slot_of = [&](unsigned p) { return (size_t)E * p / parts; };
+    for (unsigned p = 0; p + 1 < parts; ++p) {
+        size_t r = 0;
+        for (size_t i = node_of(p); i < node_of(p + 1); ++i)
+            r += (b->nvars[n0 + i] + 1u) & ~1u;
+        node_at[p + 1] = node_at[p] + r;
+        r = 0;
+        for (size_t k = slot_of(p); k < slot_of(p + 1); ++k)
+            r += (b->edge_x[s0 + k] + 1u) & ~1u;
+        msg_at[p + 1] = msg_at[p] + r;
     }
     HIP_TRY(hipStreamSynchronize(b->stream));
-    for (size_t i = 0, r = 0; i < V; ++i) {
-        unsigned v = b->node_inv[n0 + i], n = b->nvars[n0 + i];
-        for (unsigned k = 0; k < n; ++k)
-            g->node_states[(size_t)v * MAX_STATES + k] = st[r + k];
-        r += (n + 1u) & ~1u;
-    }
     if (b->swaps & 1u) {
         float **t = g->previous_edge_messages;
         g->previous_edge_messages = g->current_edge_messages;
         g->current_edge_messages = t;
     }
     float *prev = *g->previous_edge_messages, *cur = *g->current_edge_messages;
-    for (size_t k = 0, r = 0; k < E; ++k) {
-        unsigned e = b->slot_edge[s0 + k], x = b->edge_x[s0 + k];
-        for (unsigned i = 0; i < x; ++i) {
-            prev[(size_t)e * MAX_STATES + i] = m0[r + i];
-            cur[(size_t)e * MAX_STATES + i] = m1[r + i];
+    bp_parallel(parts, [&](unsigned p) {
+        size_t r = node_at[p];
+        for (size_t i = node_of(p); i < node_of(p + 1); ++i) {
+            unsigned v = b->node_inv[n0 + i], n = b->nvars[n0 + i];
+            for (unsigned k = 0; k < n; ++k)
+                g->node_states[(size_t)v * MAX_STATES + k] = st[r + k];
+            r += (n + 1u) & ~1u;
         }
-        r += (x + 1u) & ~1u;
-    }
+        r = msg_at[p];
+        for (size_t k = slot_of(p); k < slot_of(p + 1); ++k) {
+            unsigned e = b->slot_edge[s0 + k], x = b->edge_x[s0 + k];
+            for (unsigned i = 0; i < x; ++i) {
+                prev[(size_t)e * MAX_STATES + i] = m0[r + i];
+                cur[(size_t)e * MAX_STATES + i] = m1[r + i];
+            }
+            r += (x + 1u) & ~1u;
+        }
+    });
     return 0;
 }
 

@@ -62,6 +62,7 @@ struct bp_dev {
     unsigned V = 0, E = 0, S = 0, SP = 0;
     bool mixed = false;
 
+    char *memory = nullptr;           /* the device allocation that holds every array below */
     unsigned *in_off = nullptr;       /* [V+1] slot range per node */
     unsigned *slot_src = nullptr;     /* [E] */
     unsigned char *slot_xy = nullptr; /* [E] */
@@ -79,6 +80,10 @@ struct bp_dev {
     size_t jfloats = 0;               /* floats in J */
     char *h_stage = nullptr;          /* pinned host memory: a bp_resident_status, then staging for transfers */
     size_t h_stage_n = 0;             /* the staging's capacity in floats */
+    static constexpr unsigned SLICES = 8;
+    hipEvent_t slice_ev[SLICES] = {};  /* slices of a download, created on first use */
+    unsigned *perm_d = nullptr;        /* [V] node -> device node */
+    unsigned *edge_slot_d = nullptr;   /* [E] reference edge -> slot */
     unsigned char *nvars = nullptr;   /* [V] */
     float *states = nullptr;          /* [V][SP] */
     float *buf[2] = {nullptr, nullptr};

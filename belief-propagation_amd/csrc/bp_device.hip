@@ -14,6 +14,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -24,6 +25,7 @@
 #include <vector>
 
 #include "bp_dev.h"
+#include "bp_parallel.h"
 #include "../../include/bp_hip.h"
 
 using namespace bpk;
@@ -104,15 +106,6 @@ __global__ void k_send_one(const float *J, const float *b, unsigned x, unsigned 
 
 
 
-static void free_dev_arrays(bp_dev *d)
-{
-    void *ptrs[] = {d->Jp, d->slot_pool, d->slot_toff, d->in_off, d->slot_src, d->slot_xy, d->J, d->nvars, d->states, d->buf[0], d->buf[1],
-                    d->msg[0], d->msg[1], d->states0, d->chunk, d->partials, d->deltas, d->last, d->stop};
-    for (void *p : ptrs)
-        if (p)
-            (void)hipFree(p);
-}
-
 extern "C" void bp_free(bp_dev *d)
 {
     if (!d)
@@ -126,10 +119,14 @@ extern "C" void bp_free(bp_dev *d)
         (void)hipGraphExecDestroy(kv.second);
     bp_tree_plan_free(d->tree);
     bp_resident_free(d);
-    free_dev_arrays(d);
+    if (d->memory)
+        (void)hipFree(d->memory);
     if (d->h_stage)
         (void)hipHostFree(d->h_stage);
     d->h_stage = nullptr;
+    for (hipEvent_t ev : d->slice_ev)
+        if (ev)
+            (void)hipEventDestroy(ev);
     if (d->stream)
         (void)hipStreamDestroy(d->stream);
     (void)hipSetDevice(prev);
@@ -142,27 +139,6 @@ extern "C" int bp_device_count(void)
     if (hipGetDeviceCount(&n) != hipSuccess)
         return 0;
     return n;
-}
-
-/* f(begin, end) over [0, n) split across up to 16 host threads (the
- * graph's host arrays are MAX_STATES-strided: the repacking is bound by
- * memory latency, not arithmetic) */
-template <typename F> static void par_for(size_t n, F f)
-{
-    unsigned T = std::min(16u, std::max(1u, std::thread::hardware_concurrency()));
-    if (n < (1u << 16) || T == 1) {
-        f((size_t)0, n);
-        return;
-    }
-    size_t step = (n + T - 1) / T;
-    std::vector<std::thread> th;
-    for (unsigned t = 0; t < T; ++t) {
-        size_t a = t * step, b = std::min(n, a + step);
-        if (a < b)
-            th.emplace_back(f, a, b);
-    }
-    for (auto &x : th)
-        x.join();
 }
 
 /* Chunks: consecutive nodes with at most cap in-slots and cap nodes (cap =
@@ -370,7 +346,7 @@ static void xcd_ranges(Graph_t g, const std::vector<unsigned> &inv, unsigned cap
 static void inverse_of(const std::vector<unsigned> &inv, std::vector<unsigned> &perm)
 {
     perm.resize(inv.size());
-    par_for(inv.size(), [&](size_t a, size_t b) {
+    par_for(inv.size(), 8192, [&](size_t a, size_t b) {
         for (size_t i = a; i < b; ++i)
             perm[inv[i]] = (unsigned)i;
     });
@@ -403,7 +379,7 @@ static void xcd_group(Graph_t g, std::vector<unsigned> &inv, unsigned cap, unsig
         for (auto &t : th)
             t.join();
     }
-    par_for(V, [&](size_t a, size_t b) {
+    par_for(V, 8192, [&](size_t a, size_t b) {
         for (size_t h = a; h < b; ++h) {
             unsigned m = 0;
             for (unsigned x = 0; x < 8; ++x)
@@ -450,6 +426,10 @@ static int check_graph(Graph_t g)
         return -1;
     }
     unsigned V = g->current_num_vertices, E = g->current_num_edges;
+    if (V == 0) {
+        bp_set_error("graph has no nodes");
+        return -1;
+    }
     /* the destination CSR must describe the edges (set_up_dest_nodes_to_edges) */
     for (unsigned v = 0; v < V; ++v) {
         unsigned b = g->dest_nodes_to_edges_node_list[v], e = bp_csr_end(g, g->dest_nodes_to_edges_node_list, v);
@@ -507,53 +487,157 @@ static float *stage_buf(bp_dev *d, size_t n)
     return reinterpret_cast<float *>(d->h_stage + sizeof(bp_resident_status));
 }
 
-/* Host rows (MAX_STATES stride, first n valid) -> device rows (SP stride,
- * zero padded): host row h goes to device row to[h], walked in host order so
- * the large host array streams. */
-static void pack_rows(const float *src, const unsigned *valid, size_t count, unsigned SP, float *out,
-                      const unsigned *to)
+/* ---- transfers -----------------------------------------------------------
+ * The host's rows are in the graph's order, MAX_STATES floats apart; the
+ * device's in its own order, SP apart.  The host packs and unpacks rows in
+ * the graph's order, so both of its sides stream, into pinned memory that
+ * the kernels below read and write over PCIe; the reordering, random access
+ * that took the host about 3 ns a row and thread, happens on the device.
+ * (Downloading 500k binary beliefs: 0.92 ms with a copy to pageable memory
+ * and a host gather.) */
+
+/* rows h0 .. of `src` in the graph's order, row h from device row at[h], one
+ * piece of U floats a thread */
+template <int U>
+__global__ void k_rows_out(const float *__restrict__ src, const unsigned *__restrict__ at, float *__restrict__ dst,
+                           unsigned h0, unsigned pieces, unsigned per_row)
 {
-    par_for(count, [=](size_t a, size_t b) {
-        for (size_t h = a; h < b; ++h) {
-            float *row = out + (size_t)to[h] * SP;
-            unsigned n = valid[h];
-            for (unsigned k = 0; k < SP; ++k)
-                row[k] = (k < n) ? src[h * MAX_STATES + k] : 0.0f;
+    typedef float V __attribute__((ext_vector_type(U)));
+    const unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= pieces)
+        return;
+    const unsigned h = t / per_row, c = t - h * per_row;
+    const size_t row = at[h0 + h];
+    reinterpret_cast<V *>(dst)[(size_t)h0 * per_row + t] = reinterpret_cast<const V *>(src)[row * per_row + c];
+}
+
+/* the other way; dst2 (nullable) gets a copy */
+template <int U>
+__global__ void k_rows_in(const float *__restrict__ src, const unsigned *__restrict__ at, float *__restrict__ dst,
+                          float *__restrict__ dst2, unsigned h0, unsigned pieces, unsigned per_row)
+{
+    typedef float V __attribute__((ext_vector_type(U)));
+    const unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= pieces)
+        return;
+    const unsigned h = t / per_row, c = t - h * per_row;
+    const size_t to = (size_t)at[h0 + h] * per_row + c;
+    const V v = reinterpret_cast<const V *>(src)[(size_t)h0 * per_row + t];
+    reinterpret_cast<V *>(dst)[to] = v;
+    if (dst2)
+        reinterpret_cast<V *>(dst2)[to] = v;
+}
+
+/* mixed state counts: edge e's table, `floats[e + 1] - floats[e]` of them,
+ * to its slot's place */
+__global__ void k_tables_in(const float *__restrict__ src, const unsigned *__restrict__ floats,
+                            const unsigned *__restrict__ slot, const unsigned *__restrict__ place,
+                            float *__restrict__ J, unsigned E)
+{
+    const unsigned e = blockIdx.x * (blockDim.x / 4) + threadIdx.x / 4, q = threadIdx.x % 4;
+    if (e >= E)
+        return;
+    const unsigned b = floats[e] / 4, n = floats[e + 1] / 4 - b;
+    const float4 *from = reinterpret_cast<const float4 *>(src) + b;
+    float4 *to = reinterpret_cast<float4 *>(J + place[slot[e]]);
+    for (unsigned i = q; i < n; i += 4)
+        to[i] = from[i];
+}
+
+/* floats of a thread's piece for rows of `width` floats */
+static unsigned piece_of(unsigned width) { return width % 4 == 0 ? 4 : width % 2 == 0 ? 2 : 1; }
+
+/* rows [h0, h1) of `width` floats in the graph's order into pinned memory */
+static void rows_out(bp_dev *d, const float *src, const unsigned *at, float *pinned, unsigned h0, unsigned h1,
+                     unsigned width)
+{
+    const unsigned u = piece_of(width), per = width / u, most = (1u << 30) / per;
+    for (; h0 < h1; h0 += std::min(most, h1 - h0)) {
+        const unsigned pieces = std::min(most, h1 - h0) * per;
+        const dim3 grid((pieces + 255) / 256), block(256);
+        if (u == 4)
+            hipLaunchKernelGGL(k_rows_out<4>, grid, block, 0, d->stream, src, at, pinned, h0, pieces, per);
+        else if (u == 2)
+            hipLaunchKernelGGL(k_rows_out<2>, grid, block, 0, d->stream, src, at, pinned, h0, pieces, per);
+        else
+            hipLaunchKernelGGL(k_rows_out<1>, grid, block, 0, d->stream, src, at, pinned, h0, pieces, per);
+    }
+}
+
+static void rows_in(bp_dev *d, const float *pinned, const unsigned *at, float *dst, float *dst2, unsigned rows,
+                    unsigned width)
+{
+    const unsigned u = piece_of(width), per = width / u, most = (1u << 30) / per;
+    for (unsigned h0 = 0; h0 < rows; h0 += std::min(most, rows - h0)) {
+        const unsigned pieces = std::min(most, rows - h0) * per;
+        const dim3 grid((pieces + 255) / 256), block(256);
+        if (u == 4)
+            hipLaunchKernelGGL(k_rows_in<4>, grid, block, 0, d->stream, pinned, at, dst, dst2, h0, pieces, per);
+        else if (u == 2)
+            hipLaunchKernelGGL(k_rows_in<2>, grid, block, 0, d->stream, pinned, at, dst, dst2, h0, pieces, per);
+        else
+            hipLaunchKernelGGL(k_rows_in<1>, grid, block, 0, d->stream, pinned, at, dst, dst2, h0, pieces, per);
+    }
+}
+
+/* Rows of the host arrays that one thread packs or unpacks at least. */
+static constexpr size_t ROWS_GRAIN = 8192;
+
+/* host rows [a, b) (MAX_STATES stride, first valid[h] of each) <-> packed
+ * rows (SP stride, zero padded) */
+static void pack_rows(const float *src, const unsigned *valid, size_t a, size_t b, unsigned SP, float *out)
+{
+    for (size_t h = a; h < b; ++h) {
+        const unsigned n = valid[h];
+        for (unsigned k = 0; k < SP; ++k)
+            out[h * SP + k] = (k < n) ? src[h * MAX_STATES + k] : 0.0f;
+    }
+}
+
+static void unpack_rows(const float *in, const unsigned *valid, size_t a, size_t b, unsigned SP, float *dst)
+{
+    for (size_t h = a; h < b; ++h) {
+        const unsigned n = valid[h];
+        for (unsigned k = 0; k < n; ++k)
+            dst[h * MAX_STATES + k] = in[h * SP + k];
+    }
+}
+
+/* f(array, begin, end) over the rows of several arrays as one range */
+template <typename F> static void rows_of_all(const size_t *rows, unsigned arrays, F f)
+{
+    size_t total = 0;
+    for (unsigned i = 0; i < arrays; ++i)
+        total += rows[i];
+    par_for(total, ROWS_GRAIN, [&](size_t a, size_t b) {
+        size_t at = 0;
+        for (unsigned i = 0; i < arrays; at += rows[i++]) {
+            const size_t lo = std::max(a, at), hi = std::min(b, at + rows[i]);
+            if (lo < hi)
+                f(i, lo - at, hi - at);
         }
     });
 }
 
-/* device rows -> host rows (first n of each), in host order */
-static void unpack_rows(const float *in, const unsigned *valid, size_t count, unsigned SP, float *dst,
-                        const unsigned *from)
-{
-    par_for(count, [=](size_t a, size_t b) {
-        for (size_t h = a; h < b; ++h) {
-            const float *row = in + (size_t)from[h] * SP;
-            unsigned n = valid[h];
-            for (unsigned k = 0; k < n; ++k)
-                dst[h * MAX_STATES + k] = row[k];
-        }
-    });
-}
-
-/* The shared table pool.  tables holds the per-slot tables [s][S*S]; the
+/* The shared table pool.  tables holds the tables by edge, [e][S*S], and
+ * slot s reads edge slot_edge[s]'s; the
  * pool holds each table once, in the order of the first slot that reads
  * it, and tab[s] is slot s's pool index, with bit 31 set where s is the
  * later slot of a pair (partner[s] < s) whose table is exactly the
  * transpose of its partner's, which it then reads transposed.  The earlier
  * slot of a pair never reuses, so every slot's choice is independent. */
-static void build_table_pool(const std::vector<unsigned> &partner, const float *tables, unsigned E, unsigned S,
-                             std::vector<unsigned> &tab, std::vector<float> &pool)
+static void build_table_pool(const std::vector<unsigned> &partner, const std::vector<unsigned> &slot_edge,
+                             const float *tables, unsigned E, unsigned S, std::vector<unsigned> &tab,
+                             std::vector<float> &pool)
 {
     const size_t T = (size_t)S * S;
     std::vector<unsigned char> reuse(E, 0);
-    par_for(E, [&](size_t a, size_t b) {
+    par_for(E, 8192, [&](size_t a, size_t b) {
         for (size_t s = a; s < b; ++s) {
             unsigned f = partner[s];
             if (f == ~0u || f >= s)
                 continue;
-            const float *A = tables + s * T, *Bt = tables + (size_t)f * T;
+            const float *A = tables + slot_edge[s] * T, *Bt = tables + slot_edge[f] * T;
             bool t = true;
             for (unsigned i = 0; i < S && t; ++i)
                 for (unsigned j = 0; j < S && t; ++j)
@@ -570,66 +654,77 @@ static void build_table_pool(const std::vector<unsigned> &partner, const float *
         if (reuse[s])
             tab[s] = tab[partner[s]] | 0x80000000u;
     pool.resize((size_t)n * T);
-    par_for(E, [&](size_t a, size_t b) {
+    par_for(E, 8192, [&](size_t a, size_t b) {
         for (size_t s = a; s < b; ++s)
             if (!reuse[s])
-                memcpy(pool.data() + (size_t)tab[s] * T, tables + s * T, T * sizeof(float));
+                memcpy(pool.data() + (size_t)tab[s] * T, tables + slot_edge[s] * T, T * sizeof(float));
     });
+}
+
+/* Floats that upload_state stages: beliefs and both message arrays, then the
+ * tables: [e][S*S], or with mixed state counts each edge's x rows back to
+ * back and behind them where each edge's begin. */
+static size_t state_floats(const bp_dev *d)
+{
+    return std::max(((size_t)d->V + 2 * (size_t)d->E) * d->SP, d->jfloats + (d->mixed ? (size_t)d->E + 1 : 0));
 }
 
 static int upload_state(bp_dev *d, Graph_t g, bool tables)
 {
-    size_t VS = (size_t)d->V * d->SP, ES = (size_t)d->E * d->SP;
-    float *tmp = stage_buf(d, std::max(std::max(VS, ES), tables ? d->jfloats : (size_t)0));
+    const size_t V = d->V, E = d->E, VS = V * d->SP, ES = E * d->SP;
+    const unsigned S = d->S, RS = mixed_row_stride(S);
+    float *tmp = stage_buf(d, state_floats(d));
     if (!tmp)
         return -1;
-    /* node states, in device order */
-    std::vector<unsigned> node_n(d->V);
-    for (unsigned v = 0; v < d->V; ++v)
-        node_n[v] = g->node_num_vars[v];
-    pack_rows(g->node_states, node_n.data(), d->V, d->SP, tmp, d->perm.data());
-    HIP_TRY(hipMemcpyAsync(d->states, tmp, VS * sizeof(float), hipMemcpyHostToDevice, d->stream));
-    HIP_TRY(hipMemcpyAsync(d->states0, tmp, VS * sizeof(float), hipMemcpyHostToDevice, d->stream));
-    HIP_TRY(hipStreamSynchronize(d->stream));
-    /* messages in slot order: msg[0] = previous, msg[1] = current */
-    pack_rows(*g->previous_edge_messages, d->edge_x.data(), d->E, d->SP, tmp, d->edge_slot.data());
-    HIP_TRY(hipMemcpyAsync(d->msg[0], tmp, ES * sizeof(float), hipMemcpyHostToDevice, d->stream));
-    HIP_TRY(hipStreamSynchronize(d->stream));
-    pack_rows(*g->current_edge_messages, d->edge_x.data(), d->E, d->SP, tmp, d->edge_slot.data());
-    HIP_TRY(hipMemcpyAsync(d->msg[1], tmp, ES * sizeof(float), hipMemcpyHostToDevice, d->stream));
+    /* beliefs, previous and current messages */
+    float *prev = tmp + VS, *cur = prev + ES;
+    const float *hp = *g->previous_edge_messages, *hc = *g->current_edge_messages;
+    const size_t rows[3] = {V, E, E};
+    rows_of_all(rows, 3, [&](unsigned which, size_t a, size_t b) {
+        if (which == 0)
+            pack_rows(g->node_states, g->node_num_vars, a, b, d->SP, tmp);
+        else
+            pack_rows(which == 1 ? hp : hc, d->edge_x.data(), a, b, d->SP, which == 1 ? prev : cur);
+    });
+    rows_in(d, tmp, d->perm_d, d->states, d->states0, d->V, d->SP);
+    rows_in(d, prev, d->edge_slot_d, d->msg[0], nullptr, d->E, d->SP);
+    rows_in(d, cur, d->edge_slot_d, d->msg[1], nullptr, d->E, d->SP);
+    HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(d->stream));
     d->cur_is_a = (g->current_edge_messages == &g->edges_messages);
-    if (tables) {
-        unsigned S = d->S;
-        /* mixed: x rows at toff[s], row stride mixed_row_stride(S), zeros
-         * beyond y; uniform: [s][S*S], zeros beyond x rows and y columns */
-        const unsigned RS = mixed_row_stride(S);
-        if (d->mixed)
-            memset(tmp + d->jfloats - (size_t)S * RS, 0, (size_t)S * RS * sizeof(float));
-        par_for(d->E, [&](size_t a, size_t b) {
+    if (tables && E) {
+        unsigned *begin = reinterpret_cast<unsigned *>(tmp + d->jfloats);
+        if (d->mixed) {
+            /* x rows at stride RS, zeros beyond y */
+            unsigned at = 0;
+            for (size_t e = 0; e < E; ++e) {
+                begin[e] = at;
+                at += g->edges_x_dim[e] * RS;
+            }
+            begin[E] = at;
+        }
+        par_for(E, ROWS_GRAIN / 2, [&](size_t a, size_t b) {
             for (size_t e = a; e < b; ++e) {
-                unsigned s = d->edge_slot[e];
-                unsigned x = g->edges_x_dim[e], y = g->edges_y_dim[e];
+                const unsigned x = g->edges_x_dim[e], y = g->edges_y_dim[e];
                 const float *J = g->edges_joint_probabilities + e * MAX_STATES * MAX_STATES;
-                if (d->mixed) {
-                    float *T = tmp + d->toff[s];
-                    for (unsigned i = 0; i < x; ++i)
-                        for (unsigned j = 0; j < RS; ++j)
-                            T[i * RS + j] = (j < y) ? J[i * MAX_STATES + j] : 0.0f;
-                } else {
-                    float *T = tmp + (size_t)s * S * S;
-                    for (unsigned i = 0; i < S; ++i)
-                        for (unsigned j = 0; j < S; ++j)
-                            T[i * S + j] = (i < x && j < y) ? J[i * MAX_STATES + j] : 0.0f;
-                }
+                float *T = tmp + (d->mixed ? begin[e] : e * S * S);
+                const unsigned nr = d->mixed ? x : S, nc = d->mixed ? RS : S;
+                for (unsigned i = 0; i < nr; ++i)
+                    for (unsigned j = 0; j < nc; ++j)
+                        T[i * nc + j] = (i < x && j < y) ? J[i * MAX_STATES + j] : 0.0f;
             }
         });
-        HIP_TRY(hipMemcpyAsync(d->J, tmp, d->jfloats * sizeof(float), hipMemcpyHostToDevice, d->stream));
+        if (d->mixed)
+            hipLaunchKernelGGL(k_tables_in, dim3((unsigned)((E + 63) / 64)), dim3(256), 0, d->stream, tmp, begin,
+                               d->edge_slot_d, d->slot_toff, d->J, d->E);
+        else
+            rows_in(d, tmp, d->edge_slot_d, d->J, nullptr, d->E, S * S);
+        HIP_TRY(hipGetLastError());
         HIP_TRY(hipStreamSynchronize(d->stream));
         if (d->shared) {
             std::vector<unsigned> tab;
             std::vector<float> pool;
-            build_table_pool(d->partner, tmp, d->E, S, tab, pool);
+            build_table_pool(d->partner, d->slot_edge, tmp, d->E, S, tab, pool);
             HIP_TRY(hipMemcpy(d->Jp, pool.data(), pool.size() * sizeof(float), hipMemcpyHostToDevice));
             HIP_TRY(hipMemcpy(d->slot_pool, tab.data(), (size_t)d->E * 4, hipMemcpyHostToDevice));
         }
@@ -651,7 +746,7 @@ static double algorithmic_bytes(Graph_t g)
      * edge: rev[e] says edge e + 1 is e's reverse with the transposed table
      * (tested on all host threads: the tables are 400 bytes apart) */
     std::vector<unsigned char> rev(E, 0), paired(E, 0);
-    par_for(E ? E - 1 : 0, [&](size_t a, size_t b) {
+    par_for(E ? E - 1 : 0, 8192, [&](size_t a, size_t b) {
         for (size_t e = a; e < b; ++e) {
             size_t f = e + 1;
             if (g->edges_src_index[f] != g->edges_dest_index[e] || g->edges_dest_index[f] != g->edges_src_index[e])
@@ -696,7 +791,7 @@ static void plan_table_sharing(bp_dev *d, Graph_t g, const std::vector<uint2> &c
     /* rev[e]: the lowest-numbered edge dest(e) -> src(e), found among the
      * in-edges of src(e) (all host threads) */
     std::vector<unsigned> rev(E, ~0u);
-    par_for(E, [&](size_t a, size_t b) {
+    par_for(E, 8192, [&](size_t a, size_t b) {
         for (size_t e = a; e < b; ++e) {
             unsigned from = g->edges_src_index[e], to = g->edges_dest_index[e];
             if (from == to)
@@ -739,6 +834,36 @@ static void plan_table_sharing(bp_dev *d, Graph_t g, const std::vector<uint2> &c
     if (!d->shared)
         d->partner.clear();
 }
+
+/* The arrays of one device allocation, each at a multiple of 256 bytes. */
+struct Layout {
+    struct Array {
+        void **pointer;
+        const void *from; /* host data, or none */
+        size_t at, bytes;
+    };
+    std::vector<Array> arrays;
+    size_t bytes = 0, end_of_last = 0;
+
+    template <typename T, typename U> void add(T *&pointer, const U *from, size_t count)
+    {
+        arrays.push_back({(void **)&pointer, from, bytes, count * sizeof(T)});
+        end_of_last = bytes + count * sizeof(T);
+        bytes = (end_of_last + 255) / 256 * 256 + (count == 0 ? 256 : 0);
+    }
+    template <typename T> void add(T *&pointer, std::nullptr_t, size_t count) { add(pointer, (const T *)nullptr, count); }
+    void place(char *base) const
+    {
+        for (const Array &a : arrays)
+            *a.pointer = base + a.at;
+    }
+    void gather(char *to) const
+    {
+        for (const Array &a : arrays)
+            if (a.from)
+                std::memcpy(to + a.at, a.from, a.bytes);
+    }
+};
 
 static int upload_impl(Graph_t g, int device, bp_dev **out, bool plan)
 {
@@ -870,38 +995,59 @@ static int upload_impl(Graph_t g, int device, bp_dev **out, bool plan)
             return -1;
         }
         d->jfloats = tot;
-        if (dmalloc(&d->slot_toff, E) ||
-            (E && hipMemcpy(d->slot_toff, d->toff.data(), (size_t)E * 4, hipMemcpyHostToDevice) != hipSuccess)) {
-            bp_set_error("upload of the table offsets failed");
-            bp_free(d);
-            return -1;
-        }
     } else {
         d->jfloats = (size_t)E * S * S;
-    }
-    if (d->shared && (dmalloc(&d->Jp, (size_t)E * S * S) || dmalloc(&d->slot_pool, E))) {
-        bp_free(d);
-        return -1;
-    }
-    if (dmalloc(&d->in_off, V + 1) || dmalloc(&d->slot_src, E) || dmalloc(&d->slot_xy, E) ||
-        dmalloc(&d->J, d->jfloats) || dmalloc(&d->nvars, V) || dmalloc(&d->states, V * SP) ||
-        dmalloc(&d->buf[0], V * SP) || dmalloc(&d->buf[1], V * SP) || dmalloc(&d->msg[0], (size_t)E * SP) ||
-        dmalloc(&d->msg[1], (size_t)E * SP) || dmalloc(&d->states0, V * SP) ||
-        dmalloc(&d->chunk, chunks.size()) || dmalloc(&d->partials, (size_t)d->part_cap * d->NP) ||
-        dmalloc(&d->deltas, std::max(d->part_cap, 16u)) || dmalloc(&d->last, 1) || dmalloc(&d->stop, 1)) {
-        bp_free(d);
-        return -1;
     }
     std::vector<unsigned char> nv(V);
     for (unsigned v = 0; v < V; ++v)
         nv[v] = (unsigned char)d->node_n[v];
-    bool ok = hipMemcpy(d->in_off, in_off.data(), (V + 1) * 4, hipMemcpyHostToDevice) == hipSuccess &&
-              hipMemcpy(d->slot_src, slot_src.data(), (size_t)E * 4, hipMemcpyHostToDevice) == hipSuccess &&
-              hipMemcpy(d->slot_xy, slot_xy.data(), E, hipMemcpyHostToDevice) == hipSuccess &&
-              hipMemcpy(d->nvars, nv.data(), V, hipMemcpyHostToDevice) == hipSuccess &&
-              hipMemcpy(d->chunk, chunks.data(), chunks.size() * sizeof(uint2), hipMemcpyHostToDevice) == hipSuccess &&
-              hipMemset(d->buf[0], 0, V * SP * 4) == hipSuccess && hipMemset(d->buf[1], 0, V * SP * 4) == hipSuccess &&
-              hipMemset(d->stop, 0, 4) == hipSuccess;
+    /* One device allocation for all arrays (17 of them took most of a small
+     * network's upload): first those that come from the host, in one copy,
+     * then those that start as zeros, in one memset (J last before them: its
+     * slack is zero too), then the rest. */
+    Layout at;
+    at.add(d->in_off, in_off.data(), V + 1);
+    at.add(d->slot_src, slot_src.data(), E);
+    at.add(d->slot_xy, slot_xy.data(), E);
+    at.add(d->nvars, nv.data(), V);
+    at.add(d->chunk, chunks.data(), chunks.size());
+    at.add(d->perm_d, d->perm.data(), V);
+    at.add(d->edge_slot_d, d->edge_slot.data(), E);
+    if (d->mixed)
+        at.add(d->slot_toff, d->toff.data(), E);
+    const size_t copied = at.bytes;
+    at.add(d->J, nullptr, d->jfloats);
+    const size_t slack = d->mixed ? (size_t)S * mixed_row_stride(S) : 0, zero = at.end_of_last - slack * sizeof(float);
+    at.add(d->stop, nullptr, 1);
+    at.add(d->buf[0], nullptr, V * SP);
+    at.add(d->buf[1], nullptr, V * SP);
+    const size_t zeroed = at.bytes;
+    at.add(d->states, nullptr, V * SP);
+    at.add(d->states0, nullptr, V * SP);
+    at.add(d->msg[0], nullptr, (size_t)E * SP);
+    at.add(d->msg[1], nullptr, (size_t)E * SP);
+    at.add(d->partials, nullptr, (size_t)d->part_cap * d->NP);
+    at.add(d->deltas, nullptr, std::max(d->part_cap, 16u));
+    at.add(d->last, nullptr, 1);
+    if (d->shared) {
+        at.add(d->Jp, nullptr, (size_t)E * S * S);
+        at.add(d->slot_pool, nullptr, E);
+    }
+    if (hipMalloc((void **)&d->memory, at.bytes) != hipSuccess) {
+        bp_set_error("upload: no %zu bytes of device memory", at.bytes);
+        d->memory = nullptr;
+        bp_free(d);
+        return -1;
+    }
+    at.place(d->memory);
+    char *head = reinterpret_cast<char *>(stage_buf(d, std::max(copied / sizeof(float), state_floats(d))));
+    bool ok = head != nullptr;
+    if (ok) {
+        at.gather(head);
+        ok = hipMemcpyAsync(d->memory, head, copied, hipMemcpyHostToDevice, d->stream) == hipSuccess &&
+             hipMemsetAsync(d->memory + zero, 0, zeroed - zero, d->stream) == hipSuccess &&
+             hipStreamSynchronize(d->stream) == hipSuccess;
+    }
     if (!ok) {
         bp_set_error("upload of the graph structure failed");
         bp_free(d);
@@ -1633,29 +1779,56 @@ extern "C" int bp_profile_loopy(bp_dev *d, unsigned int n, float *ms)
 /* ------------------------------------------------------------------------ */
 /* download                                                                  */
 
+/* Bytes of beliefs that one host thread copies out at least (1.6 MB: 79 us
+ * in slices of 256 KB, 112 us in one; 4 MB: 131 us, with 1 MB slices 165),
+ * and the most slices. */
+static constexpr size_t SLICE_BYTES = 1u << 18;
+static constexpr unsigned MAX_SLICES = bp_dev::SLICES;
+
 extern "C" int bp_download_states(bp_dev *d, float *out)
 {
     bp_clear_error();
     HIP_TRY(hipSetDevice(d->device));
     if (bp_settle(d))
         return -1;
-    std::vector<float> st((size_t)d->V * d->SP);
-    HIP_TRY(hipMemcpyAsync(st.data(), d->states, st.size() * sizeof(float), hipMemcpyDeviceToHost, d->stream));
-    HIP_TRY(hipStreamSynchronize(d->stream));
-    for (unsigned i = 0; i < d->V; ++i)
-        std::memcpy(out + (size_t)d->inv[i] * d->SP, st.data() + (size_t)i * d->SP, d->SP * sizeof(float));
-    return 0;
-}
-
-static int download_msgs(bp_dev *d, const float *dev, float *host)
-{
-    size_t ES = (size_t)d->E * d->SP;
-    float *tmp = stage_buf(d, ES);
+    if (d->V == 0)
+        return 0;
+    const size_t n = (size_t)d->V * d->SP;
+    float *tmp = stage_buf(d, n);
     if (!tmp)
         return -1;
-    HIP_TRY(hipMemcpyAsync(tmp, dev, ES * sizeof(float), hipMemcpyDeviceToHost, d->stream));
-    HIP_TRY(hipStreamSynchronize(d->stream));
-    unpack_rows(tmp, d->edge_x.data(), d->E, d->SP, host, d->edge_slot.data());
+    /* slice by slice: the copy to the caller's memory of one overlaps the
+     * transfer of the next */
+    const unsigned slices = (unsigned)std::max<size_t>(1, std::min<size_t>(MAX_SLICES, n * 4 / SLICE_BYTES));
+    auto first = [&](unsigned i) { return (unsigned)((uint64_t)d->V * i / slices); };
+    for (unsigned i = 0; i < slices; ++i) {
+        rows_out(d, d->states, d->perm_d, tmp, first(i), first(i + 1), d->SP);
+        HIP_TRY(hipGetLastError());
+        if (slices > 1) {
+            if (!d->slice_ev[i])
+                HIP_TRY(hipEventCreateWithFlags(&d->slice_ev[i], hipEventDisableTiming));
+            HIP_TRY(hipEventRecord(d->slice_ev[i], d->stream));
+        }
+    }
+    if (slices == 1) {
+        HIP_TRY(hipStreamSynchronize(d->stream));
+        std::memcpy(out, tmp, n * sizeof(float));
+        return 0;
+    }
+    HIP_TRY(hipEventSynchronize(d->slice_ev[0]));
+    std::atomic<int> bad{0};
+    bp_parallel(slices, [&](unsigned i) {
+        if (hipSetDevice(d->device) != hipSuccess || hipEventSynchronize(d->slice_ev[i]) != hipSuccess) {
+            bad = 1;
+            return;
+        }
+        const size_t a = (size_t)first(i) * d->SP, b = (size_t)first(i + 1) * d->SP;
+        std::memcpy(out + a, tmp + a, (b - a) * sizeof(float));
+    });
+    if (bad) {
+        bp_set_error("bp_download_states: the transfer failed");
+        return -1;
+    }
     return 0;
 }
 
@@ -1669,18 +1842,16 @@ extern "C" int bp_download(bp_dev *d, Graph_t g)
     HIP_TRY(hipSetDevice(d->device));
     if (bp_settle(d))
         return -1;
-    size_t VS = (size_t)d->V * d->SP;
-    float *st = stage_buf(d, VS);
+    const size_t V = d->V, E = d->E, VS = V * d->SP, ES = E * d->SP;
+    float *st = stage_buf(d, VS + 2 * ES);
     if (!st)
         return -1;
-    HIP_TRY(hipMemcpyAsync(st, d->states, VS * sizeof(float), hipMemcpyDeviceToHost, d->stream));
+    float *newest = st + VS, *older = newest + ES;
+    rows_out(d, d->states, d->perm_d, st, 0, d->V, d->SP);
+    rows_out(d, d->msg[d->latest], d->edge_slot_d, newest, 0, d->E, d->SP);
+    rows_out(d, d->msg[d->latest ^ 1], d->edge_slot_d, older, 0, d->E, d->SP);
+    HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(d->stream));
-    {
-        std::vector<unsigned> node_n(d->V);
-        for (unsigned v = 0; v < d->V; ++v)
-            node_n[v] = g->node_num_vars[v];
-        unpack_rows(st, node_n.data(), d->V, d->SP, g->node_states, d->perm.data());
-    }
     /* one pointer swap per iteration run on the device (graph.c:1179-1182) */
     if (d->swaps & 1u) {
         float **t = g->previous_edge_messages;
@@ -1691,9 +1862,14 @@ extern "C" int bp_download(bp_dev *d, Graph_t g)
     d->cur_is_a = (g->current_edge_messages == &g->edges_messages);
     /* the device buffers keep their roles (cached HIP graphs hold their
      * addresses); msg[latest] is the newest, i.e. the host's previous array */
-    if (download_msgs(d, d->msg[d->latest], *g->previous_edge_messages) ||
-        download_msgs(d, d->msg[d->latest ^ 1], *g->current_edge_messages))
-        return -1;
+    float *hp = *g->previous_edge_messages, *hc = *g->current_edge_messages;
+    const size_t rows[3] = {V, E, E};
+    rows_of_all(rows, 3, [&](unsigned which, size_t a, size_t b) {
+        if (which == 0)
+            unpack_rows(st, g->node_num_vars, a, b, d->SP, g->node_states);
+        else
+            unpack_rows(which == 1 ? newest : older, d->edge_x.data(), a, b, d->SP, which == 1 ? hp : hc);
+    });
     return 0;
 }
 

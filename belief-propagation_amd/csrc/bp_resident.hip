@@ -56,10 +56,10 @@
 #include <algorithm>
 #include <cstring>
 #include <mutex>
-#include <thread>
 #include <vector>
 
 #include "bp_dev.h"
+#include "bp_parallel.h"
 
 using namespace bpk;
 
@@ -589,7 +589,7 @@ bool cut_ranges(const std::vector<unsigned> &in_off, unsigned V, unsigned slots,
 }
 
 /* Each workgroup's slots in order of their source, `per` places for each
- * workgroup (host threads over the workgroups). */
+ * workgroup. */
 void deal_slots(const std::vector<unsigned> &in_off, const std::vector<unsigned> &slot_src,
                 const std::vector<unsigned> &first, unsigned per, std::vector<unsigned short> &order)
 {
@@ -607,14 +607,8 @@ void deal_slots(const std::vector<unsigned> &in_off, const std::vector<unsigned>
                 order[(size_t)w * per + i] = (unsigned short)key[i];
         }
     };
-    const unsigned T = slot_src.size() < (1u << 16) ? 1u
-                                                     : std::min(16u, std::max(1u, std::thread::hardware_concurrency()));
-    std::vector<std::thread> th;
-    for (unsigned t = 1; t < T; ++t)
-        th.emplace_back(deal, (unsigned)((uint64_t)G * t / T), (unsigned)((uint64_t)G * (t + 1) / T));
-    deal(0, G / T);
-    for (auto &x : th)
-        x.join();
+    par_for(G, std::max<size_t>(1, 8192 / (slot_src.size() / G + 1)),
+            [&](size_t a, size_t b) { deal((unsigned)a, (unsigned)b); });
 }
 
 /* One resident launch at a time per device: the launches of two streams,

@@ -35,6 +35,7 @@
 #include <cstring>
 #include <map>
 #include <string>
+#include <type_traits>
 #include <unordered_map>
 #include <vector>
 
@@ -678,18 +679,23 @@ static void launch_batch_srl(int mode, const LoopyArgs &a, unsigned G, hipStream
 {
     dim3 grid(G), block(BLOCK);
     unsigned nw = (unsigned)sh.wide.size(), gw = (nw + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
-    if (mode == ITER) {
+    auto go = [&](auto m) {
+        constexpr int MODE = decltype(m)::value;
         if (ev)
-            hipExtLaunchKernelGGL((k_loopy<S, true, ITER, R, true, L>), grid, block, 0, st, ev[0], ev[1], 0, a);
+            hipExtLaunchKernelGGL((k_loopy<S, true, MODE, R, true, L>), grid, block, 0, st, ev[0], ev[1], 0, a);
         else
-            hipLaunchKernelGGL((k_loopy<S, true, ITER, R, true, L>), grid, block, 0, st, a);
+            hipLaunchKernelGGL((k_loopy<S, true, MODE, R, true, L>), grid, block, 0, st, a);
         if (nw)
-            hipLaunchKernelGGL((k_loopy_wide<S, true, ITER>), dim3(gw), block, 0, st, a, sh.d_wide, nw);
-    } else {
-        hipLaunchKernelGGL((k_loopy<S, true, INIT, R, true, L>), grid, block, 0, st, a);
-        if (nw)
-            hipLaunchKernelGGL((k_loopy_wide<S, true, INIT>), dim3(gw), block, 0, st, a, sh.d_wide, nw);
-    }
+            hipLaunchKernelGGL((k_loopy_wide<S, true, MODE>), dim3(gw), block, 0, st, a, sh.d_wide, nw);
+    };
+    if (mode == ITER)
+        go(std::integral_constant<int, ITER>());
+    else if (mode == FWD)
+        go(std::integral_constant<int, FWD>());
+    else if (mode == STEP)
+        go(std::integral_constant<int, STEP>());
+    else
+        go(std::integral_constant<int, INIT>());
 }
 
 /* 1: batches of 5 to 7 states run the two-lane shape on the 8-state kernel
@@ -802,10 +808,10 @@ extern "C" int bp_batch_iterate(bp_batch *b, unsigned int n, double *deltas)
     if (n == 0)
         return 0;
     HIP_TRY(hipSetDevice(b->device));
-    if (ensure_deltas(b, n))
+    if (deltas && ensure_deltas(b, n))
         return -1;
     char key[96];
-    snprintf(key, sizeof(key), "%u/%u/%u/%u/%d/%d", n, b->R, b->L, b->qblock, b->latest, b->bcur);
+    snprintf(key, sizeof(key), "%u/%u/%u/%u/%d/%d/%d", n, b->R, b->L, b->qblock, b->latest, b->bcur, deltas != nullptr);
     auto it = b->graphs.find(key);
     if (it == b->graphs.end()) {
         HIP_TRY(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
@@ -817,9 +823,11 @@ extern "C" int bp_batch_iterate(bp_batch *b, unsigned int n, double *deltas)
             a.buf_out = b->d_buf[bc ^ 1];
             a.msg_in = b->d_msg[lat];
             a.msg_out = b->d_msg[lat ^ 1];
-            launch_batch(b, ITER, a, b->stream);
-            hipLaunchKernelGGL(k_batch_finish, dim3(nblocks(b->n_inst, WAVES_PER_BLOCK)), dim3(256), 0, b->stream,
-                               b->d_partials, sh.d_inst_chunk, b->n_inst, b->d_deltas + (size_t)i * b->n_inst);
+            /* without deltas only the last two iterations store messages */
+            launch_batch(b, deltas ? ITER : i + 2 < n ? FWD : STEP, a, b->stream);
+            if (deltas)
+                hipLaunchKernelGGL(k_batch_finish, dim3(nblocks(b->n_inst, WAVES_PER_BLOCK)), dim3(256), 0, b->stream,
+                                   b->d_partials, sh.d_inst_chunk, b->n_inst, b->d_deltas + (size_t)i * b->n_inst);
             lat ^= 1;
             bc ^= 1;
         }

@@ -901,7 +901,7 @@ static int upload_impl(Graph_t g, int device, bp_dev **out, bool plan)
     unsigned S_all = 1;
     for (unsigned v = 0; v < V; ++v)
         S_all = std::max(S_all, g->node_num_vars[v]);
-    const unsigned cap = WAVE * ((S_all <= 4 && !(S_all >= 4 && BP_PLAIN_L > 1)) ? (unsigned)BP_SLOTS_SMALL : 1u);
+    const unsigned cap = WAVE * (S_all <= 4 ? (unsigned)BP_SLOTS_SMALL : 1u);
     if (g_node_order && V > 1) {
         bp_cm_order(g, d->inv);
         if (g_node_order == 1)
@@ -977,8 +977,8 @@ static int upload_impl(Graph_t g, int device, bp_dev **out, bool plan)
     /* mixed state counts: each slot's table is its own x rows, each row
      * padded to mixed_row_stride(S) floats (16-byte aligned rows, so a row
      * is whole vector loads), behind a per-slot offset; the kernels read
-     * every row up to S unconditionally, so the array carries S rows of
-     * slack past the last table */
+     * every row up to S unconditionally, so the array carries rows of slack
+     * past the last table */
     if (d->mixed) {
         const size_t RS = mixed_row_stride(S);
         d->toff.resize(E);
@@ -988,7 +988,7 @@ static int upload_impl(Graph_t g, int device, bp_dev **out, bool plan)
             d->toff[s] = (unsigned)tot;
             tot += (size_t)g->edges_x_dim[e] * RS;
         }
-        tot += (size_t)S * RS;
+        tot += (size_t)mixed_slack_rows(S) * RS;
         if (tot >= 0xffffffffull) {
             bp_set_error("upload: more than 2^32 table entries");
             bp_free(d);
@@ -1017,7 +1017,7 @@ static int upload_impl(Graph_t g, int device, bp_dev **out, bool plan)
         at.add(d->slot_toff, d->toff.data(), E);
     const size_t copied = at.bytes;
     at.add(d->J, nullptr, d->jfloats);
-    const size_t slack = d->mixed ? (size_t)S * mixed_row_stride(S) : 0, zero = at.end_of_last - slack * sizeof(float);
+    const size_t slack = d->mixed ? (size_t)mixed_slack_rows(S) * mixed_row_stride(S) : 0, zero = at.end_of_last - slack * sizeof(float);
     at.add(d->stop, nullptr, 1);
     at.add(d->buf[0], nullptr, V * SP);
     at.add(d->buf[1], nullptr, V * SP);
@@ -1122,19 +1122,25 @@ LoopyArgs bp_make_args(bp_dev *d)
     return a;
 }
 
+/* Lanes per slot: two for mixed state counts from six on, where one lane
+ * reads a whole table alone.  Iterations without deltas of 50k-node DAGs,
+ * one and two lanes: 2-8 states 20.1 and 11.4 us, 2-9 26.8 and 19.5, 2-6
+ * 14.5 and 11.3, 2-5 10.1 and 10.5 (300k nodes of 2-8: 79 and 44 us; four
+ * lanes 46).  One state count: 8 17.5 and 16.4, 9 15.1 and 15.3, 5 8.9 and
+ * 9.9. */
+template <int S, bool MIXED> struct PlainLanes {
+    static constexpr int value = MIXED && S >= 6 ? 2 : 1;
+};
+
 /* ev (nullable) = {start, stop}: the launch is bracketed by events taken at
  * the kernel's own begin and end (hipExtLaunchKernelGGL), so their elapsed
  * time is the kernel's duration alone, without the gap between launches. */
-template <int S> struct PlainLanes {
-    static constexpr int value = (S >= 4) ? BP_PLAIN_L : 1;
-};
-
 template <int S, bool MIXED, int MODE, bool POOLED>
 static void launch_k(const LoopyArgs &a, unsigned G, hipStream_t st, const hipEvent_t *ev)
 {
     dim3 grid(G), block(BLOCK);
-    if constexpr (PlainLanes<S>::value > 1) {
-        constexpr int L = PlainLanes<S>::value;
+    if constexpr (PlainLanes<S, MIXED>::value > 1) {
+        constexpr int L = PlainLanes<S, MIXED>::value;
         if (ev)
             hipExtLaunchKernelGGL((k_loopy<S, MIXED, MODE, 1, false, L, POOLED>), grid, block, 0, st, ev[0], ev[1], 0,
                                   a);
@@ -1163,6 +1169,8 @@ static void launch_s(int mode, const LoopyArgs &a, unsigned G, hipStream_t st, c
         launch_k<S, MIXED, FWD, POOLED>(a, G, st, ev);
     else if (mode == FINIT)
         launch_k<S, MIXED, FINIT, POOLED>(a, G, st, ev);
+    else if (mode == STEP)
+        launch_k<S, MIXED, STEP, POOLED>(a, G, st, ev);
     else
         launch_k<S, MIXED, PREP, POOLED>(a, G, st, ev);
 }
@@ -1249,8 +1257,9 @@ extern "C" int bp_loopy_init(bp_dev *d)
     return 0;
 }
 
-/* Records n iterations (+ the batch's delta reduction) on the stream. */
-static void enqueue_iterations(bp_dev *d, unsigned n, int latest, int bcur)
+/* Records n iterations on the stream, with the reduction of their deltas if
+ * anybody reads those; otherwise only the last two store their messages. */
+static void enqueue_iterations(bp_dev *d, unsigned n, int latest, int bcur, bool want_deltas)
 {
     for (unsigned i = 0; i < n; ++i) {
         LoopyArgs a = bp_make_args(d);
@@ -1259,12 +1268,12 @@ static void enqueue_iterations(bp_dev *d, unsigned n, int latest, int bcur)
         a.buf_in = d->buf[bcur];
         a.buf_out = d->buf[bcur ^ 1];
         a.partials = d->partials + (size_t)i * d->NP;
-        launch(d, ITER, a);
+        launch(d, want_deltas ? ITER : i + 2 < n ? FWD : STEP, a);
         latest ^= 1;
         bcur ^= 1;
     }
-    hipLaunchKernelGGL(k_finish, dim3(n), dim3(BLOCK), 0, d->stream, d->partials, d->NP, n, d->deltas, d->last,
-                       d->stop, 0.0f, 0, 0u);
+    if (want_deltas)
+        bp_launch_finish(d->partials, d->NP, n, d->deltas, d->stream);
 }
 
 void bp_launch_finish(const double *partials, unsigned G, unsigned n, double *deltas, hipStream_t st)
@@ -1367,12 +1376,13 @@ static int iterate_launches(bp_dev *d, unsigned n, double *deltas)
     unsigned done = 0;
     while (done < n) {
         unsigned batch = std::min(n - done, d->part_cap);
-        unsigned long long key = ((unsigned long long)batch << 2) | ((unsigned)d->latest << 1) | (unsigned)d->bcur;
+        unsigned long long key = ((unsigned long long)batch << 3) | ((deltas ? 1u : 0u) << 2) |
+                                 ((unsigned)d->latest << 1) | (unsigned)d->bcur;
         auto it = d->graphs.find(key);
         if (it == d->graphs.end()) {
             hipGraph_t graph;
             HIP_TRY(hipStreamBeginCapture(d->stream, hipStreamCaptureModeThreadLocal));
-            enqueue_iterations(d, batch, d->latest, d->bcur);
+            enqueue_iterations(d, batch, d->latest, d->bcur, deltas != nullptr);
             HIP_TRY(hipStreamEndCapture(d->stream, &graph));
             hipGraphExec_t exec;
             hipError_t e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);

@@ -71,11 +71,6 @@ namespace bpk {
 #ifndef BP_BLOCK
 #define BP_BLOCK 256
 #endif
-/* Lanes per slot of the plain path (bp_upload handles) for four or more
- * states: 1, 2, 4 or 8 (one for fewer states). */
-#ifndef BP_PLAIN_L
-#define BP_PLAIN_L 1
-#endif
 /* Lanes-per-slot path: 1 writes each new message as one whole row from its
  * LDS copy, one lane per slot, after the passes; 0 lets every lane store
  * the entries it formed. */
@@ -111,8 +106,18 @@ constexpr int WAVES_PER_BLOCK = BLOCK / WAVE;
  * FWD   the beliefs and combine buffer of ITER without storing messages or
  *       the delta, reading states and writing states_out (the unrolled
  *       forward of the adjoint, which keeps every iterate it needs)
- * FINIT the combine buffer of INIT without storing messages */
-enum Mode { ITER = 0, INIT = 1, PREP = 2, EDGE = 3, FWD = 4, FINIT = 5 };
+ * FINIT the combine buffer of INIT without storing messages
+ * STEP  ITER without the delta (and so without the old messages)
+ * A run whose deltas nobody asked for is FWD in place, with STEP for the last
+ * two iterations, whose messages the graph's two arrays hold: the messages in
+ * between are overwritten before anything reads them.  Without them and
+ * their deltas an iteration of the 1M-node 4-state lattice moves 240 MB
+ * instead of 375. */
+enum Mode { ITER = 0, INIT = 1, PREP = 2, EDGE = 3, FWD = 4, FINIT = 5, STEP = 6 };
+
+constexpr bool has_delta(int mode) { return mode == ITER || mode == EDGE; }
+constexpr bool stores_messages(int mode) { return mode == ITER || mode == INIT || mode == EDGE || mode == STEP; }
+constexpr bool updates_beliefs(int mode) { return mode == ITER || mode == FWD || mode == STEP; }
 
 struct LoopyArgs {
     const unsigned *in_off;      /* [V+1] */
@@ -120,8 +125,8 @@ struct LoopyArgs {
     const unsigned char *slot_xy;/* [E] x | y << 4 (mixed networks only) */
     const float *J;              /* [E][S*S] */
     const unsigned char *nvars;  /* [V] (mixed networks only) */
-    float *states;               /* [V][SP] (EDGE, FWD: the beliefs before the iteration) */
-    float *states_out;           /* [V][SP] EDGE, FWD: the beliefs after it */
+    float *states;               /* [V][SP] the beliefs before the iteration */
+    float *states_out;           /* [V][SP] the beliefs after it (ITER, STEP: states) */
     const float *buf_in;         /* [V][SP] gather source (ITER) */
     float *buf_out;              /* [V][SP] */
     const float *msg_in;         /* [E][SP] old messages (ITER) / messages (PREP) */
@@ -169,6 +174,11 @@ template <int S> struct Stride {
  * every row starts 16-byte aligned and is read as whole vector loads. */
 __host__ __device__ constexpr unsigned mixed_row_stride(unsigned S) { return (S + 3u) & ~3u; }
 
+/* Rows of slack after the last mixed table: rows are read whatever the
+ * table's row count, up to S, with several lanes per slot (five or more
+ * states) up to a multiple of the lanes. */
+__host__ __device__ constexpr unsigned mixed_slack_rows(unsigned S) { return S > 4 ? 16u : S; }
+
 /* The batch kernel for up to 8 states with 2 lanes per slot needs 90
  * registers, which leaves room for 5 waves per SIMD; held to 80 (6 waves,
  * no spills once the belief is loaded after the passes) its iteration on
@@ -177,7 +187,7 @@ __host__ __device__ constexpr unsigned mixed_row_stride(unsigned S) { return (S 
 template <bool PACKED, int S, int L> struct MinWaves {
     static constexpr int value = (PACKED && BP_BATCH_MIN_WAVES > 0) ? BP_BATCH_MIN_WAVES
                                  : (BP_MIN_WAVES > 0)                ? BP_MIN_WAVES
-                                 : (PACKED && S == 8 && L == 2)      ? 6
+                                 : (S == 8 && L == 2)                ? 6
                                                                      : 1;
 };
 
@@ -610,9 +620,9 @@ __device__ __forceinline__ void slot_message(const LoopyArgs &a, unsigned s, flo
     constexpr int SP = Stride<S>::value;
     unsigned x;
     compute_message<S, MIXED, MODE, PACKED, POOLED>(a, s, m, x, mrow);
-    if (MODE == PREP || MODE == FWD || MODE == FINIT)
+    if (!stores_messages(MODE))
         return;
-    if (MODE == ITER || MODE == EDGE) {
+    if (has_delta(MODE)) {
         const float *old = PACKED ? a.msg_in + mrow : a.msg_in + (size_t)s * SP;
 #pragma unroll
         for (int i = 0; i < S; ++i) {
@@ -716,10 +726,8 @@ __device__ __forceinline__ void write_node(const LoopyArgs &a, size_t row, const
             store_crow<S>(a.states_out + row, n, b);
             return;
         }
-        if (MODE == FWD)
+        if (updates_beliefs(MODE))
             store_crow<S>(a.states_out + row, n, st);
-        if (MODE == ITER)
-            store_crow<S>(a.states + row, n, st);
         store_crow<S>(a.buf_out + row, n, b);
         return;
     }
@@ -729,19 +737,14 @@ __device__ __forceinline__ void write_node(const LoopyArgs &a, size_t row, const
             a.states_out[row + k] = (k < S && (!MIXED || (unsigned)k < n)) ? b[k] : 0.0f;
         return;
     }
-    if (MODE == FWD) {
-#pragma unroll
-        for (int k = 0; k < SP; ++k)
-            a.states_out[row + k] = (k < S && (!MIXED || (unsigned)k < n)) ? st[k] : 0.0f;
-    }
     /* whole padded rows (zeros beyond the node's state count): a partly
      * written row costs more than the zeros (measured on mixed networks) */
-    if (MODE == ITER) {
+    if (updates_beliefs(MODE)) {
         float r[SP];
 #pragma unroll
         for (int k = 0; k < SP; ++k)
             r[k] = (k < S && (!MIXED || (unsigned)k < n)) ? st[k] : 0.0f;
-        store_row_nt<SP>(a.states + row, r);
+        store_row_nt<SP>(a.states_out + row, r);
     }
     float r[SP];
 #pragma unroll
@@ -825,7 +828,7 @@ __device__ __forceinline__ void node_update(const LoopyArgs &a, size_t row, unsi
             if (CLEAN)
                 nan_to_one<S>(mk[j]);
         }
-    if (MODE == ITER || MODE == FWD) {
+    if (updates_beliefs(MODE)) {
         float t[S];
 #pragma unroll
         for (int k = 0; k < S; ++k)
@@ -881,7 +884,7 @@ __device__ __forceinline__ float pair_swap(float v)
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, false));
 }
 
-/* The node phase of node_update (ITER, INIT; compact rows) with two lanes
+/* The node phase of node_update (not EDGE or PREP) with two lanes
  * per node, for a chunk of at most 32 nodes: lanes 2m and 2m + 1 hold
  * node m's entries [0, H) and [H, 2H), H = S / 2, so each lane does half
  * the products and divisions.  The node's fields come from lane m (which
@@ -891,14 +894,16 @@ __device__ __forceinline__ float pair_swap(float v)
  * As in node_update, each message's NaN entries are replaced by 1 once for
  * both products.  Entries past the node's count n are never summed or
  * stored. */
-template <int S, int MODE>
-__device__ __forceinline__ void node_update_pair(const LoopyArgs &a, unsigned nrow, unsigned q0, unsigned q1, unsigned n,
-                                                 bool ok, const float *lds, unsigned lane)
+template <int S, int MODE, bool PACKED>
+__device__ __forceinline__ void node_update_pair(const LoopyArgs &a, unsigned nb, unsigned nrow, unsigned q0,
+                                                 unsigned q1, unsigned n, bool ok, const float *lds, unsigned lane)
 {
     constexpr int H = S / 2, K = 4;
     const int src = (int)(lane >> 1);
     const unsigned h = lane & 1u, k0 = h * H;
-    const unsigned row = (unsigned)__shfl((int)nrow, src, WAVE) + k0;
+    /* (padded rows: entries past the pair that ends n's stay zero) */
+    const size_t row = (PACKED ? (size_t)(unsigned)__shfl((int)nrow, src, WAVE)
+                               : (size_t)(nb + (unsigned)src) * Stride<S>::value) + k0;
     const unsigned a0 = (unsigned)__shfl((int)q0, src, WAVE), a1 = (unsigned)__shfl((int)q1, src, WAVE);
     const unsigned nn = (unsigned)__shfl((int)n, src, WAVE);
     if (!ok)
@@ -916,7 +921,7 @@ __device__ __forceinline__ void node_update_pair(const LoopyArgs &a, unsigned nr
         if ((unsigned)j < cnt)
             nan_to_one<H>(mk[j]);
     load_crow<H>(a.states + row, st);
-    if (MODE == ITER) {
+    if (updates_beliefs(MODE)) {
         float t[H];
 #pragma unroll
         for (int k = 0; k < H; ++k)
@@ -972,8 +977,8 @@ __device__ __forceinline__ void node_update_pair(const LoopyArgs &a, unsigned nr
         mul_all<H>(b, m);
     }
     const unsigned own = nn > k0 ? nn - k0 : 0u;
-    if (MODE == ITER)
-        store_crow<H>(a.states + row, own, st);
+    if (updates_beliefs(MODE))
+        store_crow<H>(a.states_out + row, own, st);
     store_crow<H>(a.buf_out + row, own, b);
 }
 
@@ -1044,7 +1049,7 @@ __device__ __forceinline__ void chunk_narrow(const LoopyArgs &a, unsigned nb, un
         q1[r] = (BP_NT_LOADS ? __builtin_nontemporal_load(a.in_off + v + 1) : a.in_off[v + 1]) - sb;
         /* INIT and EDGE gather beliefs: keep them cached there */
         if constexpr (!PACKED) {
-            if (MODE == ITER || MODE == PREP || MODE == FWD)
+            if (updates_beliefs(MODE) || MODE == PREP)
                 load_rowp_nt<S, SP>(a.states + (size_t)v * SP, st[r]);
             else
                 load_rowp<S, SP>(a.states + (size_t)v * SP, st[r]);
@@ -1069,7 +1074,7 @@ __device__ __forceinline__ void chunk_narrow(const LoopyArgs &a, unsigned nb, un
             } else if constexpr (PACKED) {
                 xy[r] = a.slot_xy[s];
             }
-            if (!PACKED && (MODE == ITER || MODE == EDGE || MODE == PREP))
+            if (!PACKED && (has_delta(MODE) || MODE == PREP))
                 load_rowp_nt<S, SP>(a.msg_in + (size_t)s * SP, old[r]);
         }
     }
@@ -1087,7 +1092,7 @@ __device__ __forceinline__ void chunk_narrow(const LoopyArgs &a, unsigned nb, un
             unsigned wn = even_width(nv), exn = wave_excl_scan(wn, lane);
             nrow[r] = vb + exn;
             vb += wave_total(exn, wn);
-            if (MODE == ITER || MODE == EDGE || MODE == PREP)
+            if (has_delta(MODE) || MODE == PREP)
                 load_crow<S>(a.msg_in + mrow[r], old[r]);
             load_crow<S>(a.states + nrow[r], st[r]);
         }
@@ -1133,7 +1138,7 @@ __device__ __forceinline__ void chunk_narrow(const LoopyArgs &a, unsigned nb, un
                     send<S, MIXED>(J[r], bsrc[r], x, y, m);
                 else
                     send_from_memory<S, MIXED, PACKED, POOLED>(a, s, xy[r], bsrc[r], m);
-                if (MODE == ITER || MODE == EDGE) {
+                if (has_delta(MODE)) {
 #pragma unroll
                     for (int i = 0; i < S; ++i) {
                         if (!MIXED || (unsigned)i < x) {
@@ -1144,7 +1149,7 @@ __device__ __forceinline__ void chunk_narrow(const LoopyArgs &a, unsigned nb, un
                         }
                     }
                 }
-                if (MODE == ITER || MODE == INIT || MODE == EDGE) {
+                if (stores_messages(MODE)) {
                     if constexpr (PACKED) {
                         store_crow<S>(a.msg_out + mrow[r], x, m);
                     } else {
@@ -1187,6 +1192,8 @@ __device__ __forceinline__ void chunk_rows(const LoopyArgs &a, unsigned nb, unsi
     constexpr int W = WAVE;
     constexpr int G = WAVE / L;
     constexpr int NR = (SP + L - 1) / L; /* rows per lane, pad rows included */
+    /* tables whose rows start 16-byte aligned and end in zeros */
+    constexpr bool PADDED = PACKED || MIXED;
     const unsigned k = lane % L, g = lane / L, base = lane - k;
     unsigned v = nb + lane, q0 = 0, q1 = 0, n = S;
     float st[S];
@@ -1232,8 +1239,12 @@ __device__ __forceinline__ void chunk_rows(const LoopyArgs &a, unsigned nb, unsi
                 load_crow_z<S>(src + u, min(xy & 15u, xy >> 4), b);
             else
                 load_rowp<S, SP>(src + (size_t)u * SP, b);
+            if constexpr (MIXED && !PACKED)
+#pragma unroll
+                for (int j = 0; j < S; ++j)
+                    b[j] = (unsigned)j < (xy >> 4) ? b[j] : 0.0f;
         }
-        if (MODE == ITER || MODE == EDGE) {
+        if (has_delta(MODE)) {
             if constexpr (PACKED)
                 load_crow<S>(a.msg_in + mrow, old);
             else
@@ -1242,7 +1253,7 @@ __device__ __forceinline__ void chunk_rows(const LoopyArgs &a, unsigned nb, unsi
 #pragma unroll
         for (int j = 0; j < S; ++j) {
             stage_f[j * W + lane] = b[j];
-            if (MODE == ITER || MODE == EDGE)
+            if (has_delta(MODE))
                 stage_f[(S + j) * W + lane] = old[j];
         }
         stage_u[lane] = xy;
@@ -1253,7 +1264,7 @@ __device__ __forceinline__ void chunk_rows(const LoopyArgs &a, unsigned nb, unsi
             if constexpr (PACKED) {
                 load_crow<S>(a.states + nrow, st);
             } else {
-                if (MODE == ITER || MODE == PREP || MODE == FWD)
+                if (updates_beliefs(MODE) || MODE == PREP)
                     load_rowp_nt<S, SP>(a.states + (size_t)v * SP, st);
                 else
                     load_rowp<S, SP>(a.states + (size_t)v * SP, st);
@@ -1273,23 +1284,30 @@ __device__ __forceinline__ void chunk_rows(const LoopyArgs &a, unsigned nb, unsi
      * costing occupancy). */
     auto load_pass = [&](int p, float (&tv)[NR][S]) {
         unsigned q = p * G + g, s = sb + q;
-        if constexpr (PACKED && MODE != PREP) {
+        if constexpr (PADDED && MODE != PREP) {
             /* Every row this lane multiplies, read unconditionally as
              * aligned four-float vectors: row i of the pooled table starts
              * at i * st, st = y rounded up to four, and the pool ends with
              * slack for the rows and vectors past a table's last one.
              * Columns y..st-1 are the pool's zero padding; a vector wholly
              * past st belongs to the next row and is replaced by zeros, so
-             * every entry j >= y is +0.  Rows i >= x hold whatever lies
+             * every entry j >= y is +0.  (Mixed tables of a plain handle:
+             * the same with st = mixed_row_stride(S).)  Rows i >= x hold whatever lies
              * there and are never used (run_pass drops them).  A slot past
              * the chunk reads from the pool's start. */
             const bool act = s < se;
             const unsigned xy = stage_u[q], tq = stage_u[W + q]; /* stale past the chunk */
             const unsigned y = act ? (xy >> 4) : 1u;
-            const unsigned st = (y + 3u) & ~3u;
-            const float *T = a.tabs + (act ? tq : 0u) + k * st;
+            const unsigned st = PACKED ? (y + 3u) & ~3u : mixed_row_stride(S);
+            const float *T = (PACKED ? a.tabs : a.J) + (act ? tq : 0u) + k * st;
 #pragma unroll
             for (int r = 0; r < NR; ++r) {
+                if (!PACKED && r * L >= S) {
+#pragma unroll
+                    for (int j = 0; j < S; ++j)
+                        tv[r][j] = 0.0f;
+                    continue;
+                }
                 const float *row = T + (size_t)(r * L) * st;
 #pragma unroll
                 for (int qv = 0; qv < (S + 3) / 4; ++qv) {
@@ -1297,7 +1315,7 @@ __device__ __forceinline__ void chunk_rows(const LoopyArgs &a, unsigned nb, unsi
 #pragma unroll
                     for (int c = 0; c < 4; ++c)
                         if (4 * qv + c < S)
-                            tv[r][4 * qv + c] = (qv == 0 || (unsigned)(4 * qv) < y) ? w[c] : 0.0f;
+                            tv[r][4 * qv + c] = (!PACKED || qv == 0 || (unsigned)(4 * qv) < y) ? w[c] : 0.0f;
                 }
             }
             return;
@@ -1309,34 +1327,19 @@ __device__ __forceinline__ void chunk_rows(const LoopyArgs &a, unsigned nb, unsi
                 tv[r][j] = 0.0f;
         if (MODE == PREP || s >= se)
             return;
-        unsigned x = S, y = S;
-        if (MIXED) {
-            unsigned xy = stage_u[q];
-            x = xy & 15u;
-            y = xy >> 4;
-        }
-        const float *T = PACKED ? a.tabs + stage_u[W + q]
-                         : MIXED ? a.J + stage_u[W + q]
-                         : POOLED ? a.J + (size_t)(stage_u[W + q] & 0x7fffffffu) * S * S
+        const float *T = POOLED ? a.J + (size_t)(stage_u[W + q] & 0x7fffffffu) * S * S
                                   : a.J + (size_t)s * S * S;
 #pragma unroll
         for (int r = 0; r < NR; ++r) {
             unsigned i = k + r * L;
-            if (i < (unsigned)S && (!MIXED || i < x)) {
-                if constexpr (PACKED) {
-                    load_pooled_row<S>(T, i, y, tv[r]);
-                } else if constexpr (POOLED) {
+            if (i < (unsigned)S) {
+                if constexpr (POOLED) {
                     /* row i of the slot's table: row i of the stored one,
                      * or its column i when the slot reads it transposed */
                     const bool tr = (stage_u[W + q] >> 31) != 0;
 #pragma unroll
                     for (int j = 0; j < S; ++j)
                         tv[r][j] = T[tr ? j * S + i : i * S + j];
-                } else if constexpr (MIXED) {
-                    constexpr int RS = (int)mixed_row_stride(S);
-#pragma unroll
-                    for (int j = 0; j < S; ++j)
-                        tv[r][j] = (unsigned)j < y ? T[(size_t)i * RS + j] : 0.0f;
                 } else {
 #pragma unroll
                     for (int j = 0; j < S; ++j)
@@ -1348,17 +1351,14 @@ __device__ __forceinline__ void chunk_rows(const LoopyArgs &a, unsigned nb, unsi
     auto run_pass = [&](int p, const float (&tv)[NR][S]) {
         unsigned q = p * G + g, s = sb + q;
         bool act = s < se;
-        unsigned x = S, y = S;
+        unsigned x = S;
         float acc[NR];
 #pragma unroll
         for (int r = 0; r < NR; ++r)
             acc[r] = 0.0f;
         if (act) {
-            if (MIXED) {
-                unsigned xy = stage_u[q];
-                x = xy & 15u;
-                y = xy >> 4;
-            }
+            if (MIXED)
+                x = stage_u[q] & 15u;
             if (MODE == PREP) {
 #pragma unroll
                 for (int r = 0; r < NR; ++r) {
@@ -1366,7 +1366,7 @@ __device__ __forceinline__ void chunk_rows(const LoopyArgs &a, unsigned nb, unsi
                     if (i < (unsigned)S)
                         acc[r] = stage_f[i * W + q];
                 }
-            } else if constexpr (PACKED) {
+            } else if constexpr (PADDED) {
                 /* The staged row holds +0 from y on (staging), and so does
                  * every table entry j >= y (load_pass): each such product
                  * is +0 and adding it leaves the sum unchanged (a sum that
@@ -1394,11 +1394,10 @@ __device__ __forceinline__ void chunk_rows(const LoopyArgs &a, unsigned nb, unsi
                 for (int r = 0; r < NR; ++r) {
                     unsigned i = k + r * L;
                     float sacc = 0.0f;
-                    if (i < (unsigned)S && (!MIXED || i < x)) {
+                    if (i < (unsigned)S) {
 #pragma unroll
                         for (int j = 0; j < S; ++j)
-                            if (!MIXED || (unsigned)j < y)
-                                sacc = sacc + tv[r][j] * b[j];
+                            sacc = sacc + tv[r][j] * b[j];
                     }
                     acc[r] = sacc;
                 }
@@ -1412,7 +1411,7 @@ __device__ __forceinline__ void chunk_rows(const LoopyArgs &a, unsigned nb, unsi
         } else {
             /* the row sums in row order, from the lanes that hold them */
             float sum = 0.0f;
-            if constexpr (PACKED && L == 2) {
+            if constexpr (PADDED && L == 2) {
                 /* rows 2r and 2r + 1 sit in acc[r] of the pair's low and
                  * high lane: the low lane adds them in row order, taking
                  * each odd row from its neighbour by one DPP swap, and the
@@ -1447,7 +1446,7 @@ __device__ __forceinline__ void chunk_rows(const LoopyArgs &a, unsigned nb, unsi
                 if (i >= (unsigned)SP)
                     continue;
                 if (i < (unsigned)S) {
-                    if ((MODE == ITER || MODE == EDGE) && (!MIXED || i < x)) {
+                    if (has_delta(MODE) && (!MIXED || i < x)) {
                         float qd = stage_f[(S + i) * W + q] - m[r];
                         if (qd != qd)
                             qd = 0.0f;
@@ -1455,7 +1454,7 @@ __device__ __forceinline__ void chunk_rows(const LoopyArgs &a, unsigned nb, unsi
                     }
                     lds[i * W + q] = m[r];
                 }
-                if ((MODE == ITER || MODE == INIT || MODE == EDGE) && !BP_ROWS_MSG_FROM_LDS && !PACKED)
+                if (stores_messages(MODE) && !BP_ROWS_MSG_FROM_LDS && !PACKED)
                     a.msg_out[(size_t)s * SP + i] = (i < (unsigned)S) ? m[r] : 0.0f;
             }
         }
@@ -1466,12 +1465,12 @@ __device__ __forceinline__ void chunk_rows(const LoopyArgs &a, unsigned nb, unsi
             break; /* the chunk's slots are all done */
         float tv[NR][S];
         load_pass(p, tv);
-        if constexpr (PACKED)
+        if constexpr (PADDED)
             __builtin_amdgcn_sched_barrier(0); /* every table load issued before the first product */
         run_pass(p, tv);
     }
     wave_sync();
-    if ((MODE == ITER || MODE == INIT || MODE == EDGE) && (BP_ROWS_MSG_FROM_LDS || PACKED)) {
+    if (stores_messages(MODE) && (BP_ROWS_MSG_FROM_LDS || PACKED)) {
         /* the new messages, one whole row per slot (zeros beyond the
          * message's entries are in LDS already) */
         unsigned s = sb + lane;
@@ -1486,9 +1485,9 @@ __device__ __forceinline__ void chunk_rows(const LoopyArgs &a, unsigned nb, unsi
                 store_row_nt<SP>(a.msg_out + (size_t)s * SP, row);
         }
     }
-    if constexpr (PACKED && L == 2 && S == 8 && late_states && (MODE == ITER || MODE == INIT)) {
+    if constexpr (PADDED && L == 2 && S == 8 && late_states && MODE != EDGE && MODE != PREP) {
         if (ne - nb <= (unsigned)(W / 2)) {
-            node_update_pair<S, MODE>(a, nrow, q0, q1, n, nb + (lane >> 1) < ne, lds, lane);
+            node_update_pair<S, MODE, PACKED>(a, nb, nrow, q0, q1, n, nb + (lane >> 1) < ne, lds, lane);
             return;
         }
     }
@@ -1564,9 +1563,9 @@ __device__ void chunk_wide(const LoopyArgs &a, unsigned v, unsigned sb, unsigned
     }
 #pragma unroll
     for (int k = 0; k < S; ++k)
-        acc[k] = (MODE == ITER || MODE == FWD) ? 1.0f : st[k];
+        acc[k] = updates_beliefs(MODE) ? 1.0f : st[k];
     walk_wide<S, MIXED, MODE, PACKED, POOLED>(a, sb, se, lds, lane, dacc, true, acc, n, cbase.y);
-    if (MODE == ITER || MODE == FWD) {
+    if (updates_beliefs(MODE)) {
 #pragma unroll
         for (int k = 0; k < S; ++k)
             if (!MIXED || (unsigned)k < n)
@@ -1630,7 +1629,7 @@ __global__ __launch_bounds__(BLOCK, (MinWaves<PACKED, S, L>::value)) void k_loop
     if (a.stop && *a.stop)
         return;
     /* lanes-per-slot path: staged slot operands (rows b and old, state counts, tables) */
-    __shared__ float stage_f[WAVES_PER_BLOCK][L > 1 ? 2 * S * WAVE : 1];
+    __shared__ float stage_f[WAVES_PER_BLOCK][L > 1 ? (has_delta(MODE) ? 2 : 1) * S * WAVE : 1];
     __shared__ unsigned stage_u[WAVES_PER_BLOCK][L > 1 ? 2 * WAVE : 1];
     /* the new messages.  With L > 1 they take the place of the staged rows
      * b (the first S * WAVE floats of stage_f): a slot's message is written
@@ -1641,7 +1640,7 @@ __global__ __launch_bounds__(BLOCK, (MinWaves<PACKED, S, L>::value)) void k_loop
     unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
     float *lds_w = (L > 1) ? stage_f[wave] : lds_own[wave];
     double dacc = 0.0;
-    const bool per_chunk = (MODE == ITER || MODE == EDGE) && a.chunk_partials != nullptr;
+    const bool per_chunk = has_delta(MODE) && a.chunk_partials != nullptr;
     if (a.queue) {
         /* work queue: each wave takes blocks of qblock consecutive positions
          * of the chunk order */
@@ -1677,7 +1676,7 @@ __global__ __launch_bounds__(BLOCK, (MinWaves<PACKED, S, L>::value)) void k_loop
     }
     /* one FP64 partial per wave, no workgroup barrier: a wave that is done
      * leaves at once instead of waiting for the slowest of its group */
-    if ((MODE == ITER || MODE == EDGE) && !per_chunk) {
+    if (has_delta(MODE) && !per_chunk) {
         double d = wave_sum(dacc);
         if (lane == 0)
             a.partials[blockIdx.x * WAVES_PER_BLOCK + wave] = d;
@@ -1700,7 +1699,7 @@ __global__ __launch_bounds__(BLOCK) void k_loopy_wide(LoopyArgs a, const unsigne
     double dacc = 0.0;
     chunk_wide<S, MIXED, MODE, true, false>(a, lo.x, lo.y, hi.y, lds[wave], lane, dacc, a.chunk_base[c]);
     wave_sync();
-    if (MODE == ITER || MODE == EDGE)
+    if (has_delta(MODE))
         flush_chunk_partial(a, c, lane, dacc);
 }
 

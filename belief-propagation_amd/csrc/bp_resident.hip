@@ -13,7 +13,8 @@
  * under 1 us of work, and twice that with the stop test's own launch), and a
  * million-arc binary one re-reads its tables, indices and messages from the
  * Infinity Cache every iteration.  The register files hold 128 MB in all,
- * enough for the tables of 2M binary or 0.75M four-state message edges.
+ * enough for the tables of 2M binary, 0.75M four-state or 0.25M eight-state
+ * message edges.
  *
  * Exchange between workgroups.  An iteration writes its combine buffers to a
  * place of its own (`ring`, one per iteration of the launch) with
@@ -84,6 +85,7 @@ struct ResArgs {
     float *msg0, *msg1;  /* messages before the run; the other array */
     float *ring;         /* iteration t's combine buffers at ring + t * ring_stride */
     size_t ring_stride;
+    unsigned S;       /* the network's largest state count */
     unsigned n;       /* iterations, at most */
     int until;        /* stop test of graph.c:1313 after each */
     float conv;
@@ -167,8 +169,10 @@ template <int S> __device__ __forceinline__ void put_row(float *p, const float *
 {
     if constexpr (S == 2)
         *reinterpret_cast<float2 *>(p) = make_float2(v[0], v[1]);
-    else if constexpr (S == 4)
-        *reinterpret_cast<float4 *>(p) = make_float4(v[0], v[1], v[2], v[3]);
+    else if constexpr (S % 4 == 0)
+#pragma unroll
+        for (int i = 0; i < S; i += 4)
+            *reinterpret_cast<float4 *>(p + i) = make_float4(v[i], v[i + 1], v[i + 2], v[i + 3]);
     else
 #pragma unroll
         for (int i = 0; i < S; ++i)
@@ -298,8 +302,17 @@ __global__ __launch_bounds__(RB) void k_resident(ResArgs a)
         for (unsigned l = tid; l < ns; l += RB) {
             const unsigned s = s0 + l;
             float t[CH];
-            load_row<CH>(MIXED ? a.J + a.slot_tab[s] + c * (int)mixed_row_stride(S) : a.J + (size_t)s * S * S + c * CH,
-                         t);
+            if (MIXED && (S < 8 || a.slot_tab)) {
+                load_row<CH>(a.J + a.slot_tab[s] + c * (int)mixed_row_stride(S), t);
+            } else if (MIXED) { /* one state count of 5 to 8 on the 8-state kernel */
+                const unsigned n = a.S;
+                const float *T = a.J + ((size_t)s * n + c) * n;
+#pragma unroll
+                for (int j = 0; j < CH; ++j)
+                    t[j] = (unsigned)c < n && (unsigned)j < n ? T[j] : 0.0f;
+            } else {
+                load_row<CH>(a.J + (size_t)s * S * S + c * CH, t);
+            }
             put_row<CH>(stage + l * CH, t);
         }
         __syncthreads();
@@ -548,7 +561,7 @@ namespace {
  * where it can be -- a barrier among 64 workgroups costs 1.3 us, among 256
  * 2.5 us.  `most` slots per thread are what the registers (128 per thread)
  * and LDS (two iterations' messages) hold. */
-unsigned most_slots(unsigned S) { return S == 2 ? 8 : S == 3 ? 4 : 3; }
+unsigned most_slots(unsigned S) { return S == 2 ? 8 : S == 3 ? 4 : S == 4 ? 3 : 1; }
 
 /* slots per thread go 1, 2, 4, 8; for four states 1, 2, 3 */
 unsigned next_slots(unsigned ns, unsigned S) { return S == 4 && ns == 2 ? 3 : 2 * ns; }
@@ -561,7 +574,7 @@ unsigned most_groups(unsigned ns, unsigned S, unsigned cus)
 
 /* Largest network of one workgroup, in slots per thread: messages and
  * combine buffers share 160 KB of LDS. */
-unsigned single_slots(unsigned S) { return S == 2 ? 4 : 2; }
+unsigned single_slots(unsigned S) { return S == 2 ? 4 : S <= 4 ? 2 : 1; }
 
 unsigned nodes_per_thread(unsigned ns) { return (ns + 1) / 2; }
 
@@ -670,7 +683,9 @@ void launch_s(const ResArgs &a, unsigned ns, unsigned G, bool single, bool delta
 void launch(unsigned S, bool mixed, const ResArgs &a, unsigned ns, unsigned G, bool single, bool delta,
             hipStream_t st)
 {
-    if (S == 2)
+    if (S > 4) /* 5 to 8 states: rows are 8 floats apart in every case */
+        single ? launch_d<8, true, 1, true>(a, 1, delta, st) : launch_d<8, true, 1, false>(a, G, delta, st);
+    else if (S == 2)
         launch_s<2, false>(a, ns, G, single, delta, st);
     else if (S == 3)
         mixed ? launch_s<3, true>(a, ns, G, single, delta, st) : launch_s<3, false>(a, ns, G, single, delta, st);
@@ -681,11 +696,11 @@ void launch(unsigned S, bool mixed, const ResArgs &a, unsigned ns, unsigned G, b
 } // namespace
 
 /* Decides whether the graph runs resident and lays out its ranges:
- * uniform state counts of 2 to 4, or mixed ones up to 3 or 4. */
+ * uniform state counts of 2 to 8, or mixed ones up to 3 to 8. */
 int bp_resident_plan(bp_dev *d, const std::vector<unsigned> &slot_src, int cus)
 {
     bp_resident &r = d->res;
-    if (d->E == 0 || d->S < 2 || d->S > 4 || (d->mixed && d->S == 2) || d->device >= MAX_DEVICES)
+    if (d->E == 0 || d->S < 2 || d->S > 8 || (d->mixed && d->S == 2) || d->device >= MAX_DEVICES)
         return 0;
     std::vector<unsigned> first;
     const unsigned align = 32 / d->SP; /* nodes per 128-byte line */
@@ -766,6 +781,7 @@ int bp_resident_launch(bp_dev *d, unsigned n, bool want_delta, bool until, float
     a.nvars = d->nvars;
     a.J = d->J;
     a.slot_tab = d->mixed ? d->slot_toff : nullptr;
+    a.S = d->S;
     a.wg_node = r.wg_node;
     a.wg_slots = r.wg_slots;
     a.states = d->states;

@@ -205,7 +205,7 @@ def bench_configs(presets=("c2", "c3"), steps: int = 20, warmup: int = 3) -> dic
         def step():
             dev.restore()
             dev.init()
-            dev.iterate(ITERATIONS)
+            dev.iterate(ITERATIONS, want_deltas=True)
 
         for _ in range(warmup):
             step()
@@ -410,7 +410,7 @@ def main():
         # every step starts again from the uploaded states (device to device)
         dev.restore()
         dev.init()
-        dev.iterate(ITERATIONS)
+        dev.iterate(ITERATIONS, want_deltas=True)  # deltas nobody reads are not formed
 
     for _ in range(args.warmup):
         step()

@@ -17,7 +17,7 @@ pytestmark = pytest.mark.gpu
 
 
 def networks(lib, **kw):
-    bn = B.generate("c2", **kw)
+    bn = B.generate("c4net" if kw["states_hi"] > 4 else "c2", **kw)
     g, h = B.bn_to_graph(bn), B.bn_to_graph(bn)
     lib.bp_bn_free(bn)
     return g, h
@@ -70,6 +70,14 @@ CASES = [
     (71000, 3, 3, 4, True),
     (75000, 2, 2, 4, True),
     (290000, 2, 2, 8, True),
+    (250, 2, 8, 1, False),
+    (200, 5, 5, 1, False),
+    (270, 5, 5, 1, True),
+    (320, 2, 6, 1, True),
+    (1500, 7, 7, 1, True),
+    (2001, 2, 7, 1, True),
+    (60000, 2, 8, 1, True),
+    (9000, 8, 8, 1, True),
 ]
 
 
@@ -101,10 +109,10 @@ def test_iterations_and_deltas_match_oracle(lib, orc, nodes, lo, hi, per_thread,
 
 
 @pytest.mark.parametrize("nodes,hi,conv,most", [(300, 2, 1e-3, 200), (900, 2, 1e-30, 300), (5000, 2, 1e-3, 200),
-                                                (3000, 4, 1e-30, 300), (3000, 4, 1e9, 10), (5000, 2, 1e-30, 1)])
+                                                (3000, 4, 1e-30, 300), (3000, 4, 1e9, 10), (5000, 2, 1e-30, 1), (1000, 8, 1e-3, 200)])
 def test_until_matches_oracle(lib, orc, nodes, hi, conv, most):
     print(f"resident until {nodes} nodes", flush=True)
-    g, h = networks(lib, num_nodes=nodes, states_hi=hi, seed=77 + nodes)
+    g, h = networks(lib, num_nodes=nodes, states_lo=2, states_hi=hi, seed=77 + nodes)
     dev = B.Device(g)
     assert shape(dev)[0] > 0
     dev.init()

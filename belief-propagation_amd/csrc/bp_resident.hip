@@ -181,72 +181,113 @@ template <int S> __device__ __forceinline__ void put_row(float *p, const float *
 
 template <int S> __device__ __forceinline__ void get_row(const float *p, float *v) { load_row<S>(p, v); }
 
-/* Nodes per thread: a message edge belongs to one node, and the networks'
- * nodes have two to four of them. */
-template <int NS> struct NodesPerThread {
-    static constexpr int value = (NS + 1) / 2;
+/* Lanes per node in the node phase, and rounds of the workgroup over its
+ * nodes: a message edge belongs to one node, and the networks' nodes have
+ * two to four of them.  Eight states take four lanes of two: a workgroup of
+ * 1,024 slots has some 290 nodes, work for five of its 16 waves otherwise. */
+template <int S> struct LanesPerNode {
+    static constexpr int value = S == 8 ? 4 : 1;
+};
+template <int S, int NS> struct NodeRounds {
+    static constexpr int value = S == 8 ? 2 : (NS + 1) / 2;
 };
 
-/* N in-messages from p on as factors: those past the node's last one are 1,
- * and so are NaN entries (CLEAN: there may be some), which the products
- * skip.  All reads are issued before the first product: a read at a time
- * made the node phase a chain of LDS latencies as long as the largest
- * in-degree of the wave's nodes (1.5 of 2.3 us on a 700-node network). */
-template <int S, int N, bool CLEAN>
-__device__ __forceinline__ void factors(const float *p, unsigned cnt, float (&f)[N][S])
+/* N in-messages from p on, S floats apart, as factors, H entries of each:
+ * those past the node's last one are 1, and so are NaN entries (CLEAN: there
+ * may be some), which the products skip.  All reads are issued before the
+ * first product: a read at a time made the node phase a chain of LDS
+ * latencies as long as the largest in-degree of the wave's nodes (1.5 of
+ * 2.3 us on a 700-node network). */
+template <int S, int H, int N, bool CLEAN>
+__device__ __forceinline__ void factors(const float *p, unsigned cnt, float (&f)[N][H])
 {
 #pragma unroll
     for (int j = 0; j < N; ++j)
-        get_row<S>(p + j * S, f[j]);
+        get_row<H>(p + j * S, f[j]);
 #pragma unroll
     for (int j = 0; j < N; ++j) {
 #pragma unroll
-        for (int i = 0; i < S; ++i)
+        for (int i = 0; i < H; ++i)
             f[j][i] = (unsigned)j < cnt ? f[j][i] : 1.0f;
         if (CLEAN)
-            nan_to_one<S>(f[j]);
+            nan_to_one<H>(f[j]);
     }
+}
+
+/* normalise() over four lanes of two entries each: the sum runs through the
+ * lanes in entry order, from 0.0 left to right as with one lane. */
+__device__ __forceinline__ void normalise_quad(float *v, unsigned h, unsigned n)
+{
+    float sum = 0.0f;
+#pragma unroll
+    for (unsigned step = 0; step < 4; ++step) {
+        if (step > 0) {
+            /* quad_perm (0, 0, 1, 2): each lane gets its left neighbour's */
+            const float left = __int_as_float(
+                __builtin_amdgcn_update_dpp(0, __float_as_int(sum), 0x90, 0xF, 0xF, false));
+            sum = h == step ? left : sum;
+        }
+        if (h == step) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                if (2 * h + i < n)
+                    sum = sum + v[i];
+        }
+    }
+    /* quad_perm (3, 3, 3, 3) */
+    sum = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(sum), 0xFF, 0xF, 0xF, false));
+    if (sum <= 0.0f)
+        sum = 1.0f;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+        if (2 * h + i < n)
+            v[i] = v[i] / sum;
 }
 
 /* The node phase of k_loopy: st = N(st * t), t = the product of the
  * in-messages in slot order, and the combine buffer b = st * the same
- * factors one by one (graph.c:985-1024, 851-882). */
-template <int S, bool MIXED, int NS, bool CLEAN>
-__device__ __forceinline__ void resident_node(const float *msgs, unsigned cnt, unsigned n, float *st, float *b)
+ * factors one by one (graph.c:985-1024, 851-882).  H entries of the node,
+ * from h * H on. */
+template <int S, bool MIXED, int NS, bool CLEAN, int H>
+__device__ __forceinline__ void resident_node(const float *msgs, unsigned cnt, unsigned n, unsigned h, float *st,
+                                              float *b)
 {
     /* K messages are kept for both products and the rest read D at a time:
      * as many as the tables leave registers for */
     constexpr int HELD = S * S * NS;
-    constexpr int K = HELD > 36 ? 2 : HELD > 16 ? 4 : S == 2 ? 8 : 4, D = HELD > 32 ? 2 : 4;
-    float f[K][S], t[S];
-    factors<S, K, CLEAN>(msgs, cnt, f);
+    constexpr int K = H == 2 && HELD <= 16 ? 8 : HELD > 36 && S < 8 ? 2 : 4, D = HELD > 32 && S < 8 ? 2 : 4;
+    float f[K][H], t[H];
+    factors<S, H, K, CLEAN>(msgs, cnt, f);
 #pragma unroll
-    for (int i = 0; i < S; ++i)
+    for (int i = 0; i < H; ++i)
         t[i] = 1.0f;
 #pragma unroll
     for (int j = 0; j < K; ++j)
-        mul_all<S>(t, f[j]);
+        mul_all<H>(t, f[j]);
     for (unsigned q = K; q < cnt; q += D) {
-        float g[D][S];
-        factors<S, D, CLEAN>(msgs + q * S, cnt - q, g);
+        float g[D][H];
+        factors<S, H, D, CLEAN>(msgs + q * S, cnt - q, g);
 #pragma unroll
         for (int j = 0; j < D; ++j)
-            mul_all<S>(t, g[j]);
+            mul_all<H>(t, g[j]);
     }
-    mul_all<S>(st, t);
-    normalise<S, MIXED>(st, n);
+    mul_all<H>(st, t);
+    if constexpr (H < S)
+        normalise_quad(st, h, n);
+    else
+        normalise<S, MIXED>(st, n);
 #pragma unroll
-    for (int i = 0; i < S; ++i)
+    for (int i = 0; i < H; ++i)
         b[i] = st[i];
 #pragma unroll
     for (int j = 0; j < K; ++j)
-        mul_all<S>(b, f[j]);
+        mul_all<H>(b, f[j]);
     for (unsigned q = K; q < cnt; q += D) {
-        float g[D][S];
-        factors<S, D, CLEAN>(msgs + q * S, cnt - q, g);
+        float g[D][H];
+        factors<S, H, D, CLEAN>(msgs + q * S, cnt - q, g);
 #pragma unroll
         for (int j = 0; j < D; ++j)
-            mul_all<S>(b, g[j]);
+            mul_all<H>(b, g[j]);
     }
 }
 
@@ -255,12 +296,14 @@ template <int S, bool MIXED, int NS, bool SINGLE, bool DELTA>
 __global__ __launch_bounds__(RB) void k_resident(ResArgs a)
 {
     constexpr int SP = Stride<S>::value;
-    constexpr int NN = NodesPerThread<NS>::value;
+    constexpr int LN = LanesPerNode<S>::value, NN = NodeRounds<S, NS>::value;
+    constexpr int H = S / LN, HP = LN > 1 ? H : SP; /* a lane's entries of a node, and of its row */
+    constexpr int RN = RB / LN;                     /* nodes of a round */
     constexpr int W = RB * NS;
     /* messages by slot: iteration t's in lm[t & 1] (while the tables are
      * loaded, a staging area) */
     __shared__ __align__(16) float lm[2][S * (W + PAD)];
-    __shared__ __align__(16) float lbuf[SINGLE ? SP * RB * NN : 4];
+    __shared__ __align__(16) float lbuf[SINGLE ? SP * RN * NN : 4];
     __shared__ double red[2][RW];
     __shared__ double total;
     __shared__ unsigned ok, committed, suspect;
@@ -332,28 +375,29 @@ __global__ __launch_bounds__(RB) void k_resident(ResArgs a)
             load_rowp<S, SP>(a.msg0 + (size_t)(s0 + l) * SP, old);
             put_row<S>(lm[0] + l * S, old);
         }
-    float st[NN][S];
+    const unsigned h = tid % LN; /* which entries of its nodes the lane has: from h * H on */
+    float st[NN][H];
     unsigned slots[NN], nn[NN]; /* first in-slot | in-degree << 16 (both below 2^16) */
 #pragma unroll
     for (int r = 0; r < NN; ++r) {
-        const unsigned v = n0 + r * RB + tid;
+        const unsigned v = n0 + r * RN + tid / LN;
         slots[r] = 0;
         nn[r] = S;
 #pragma unroll
-        for (int i = 0; i < S; ++i)
+        for (int i = 0; i < H; ++i)
             st[r][i] = 1.0f;
         if (v < n1) {
             const unsigned b = a.in_off[v], e = a.in_off[v + 1];
             slots[r] = (b - s0) | (e - b) << 16;
             if (MIXED)
                 nn[r] = a.nvars[v];
-            load_rowp<S, SP>(a.states + (size_t)v * SP, st[r]);
+            load_rowp<H, HP>(a.states + (size_t)v * SP + h * H, st[r]);
             if constexpr (SINGLE) {
-                float b0[S];
-                load_rowp<S, SP>(a.buf_in + (size_t)v * SP, b0);
+                float b0[H];
+                load_rowp<H, HP>(a.buf_in + (size_t)v * SP + h * H, b0);
 #pragma unroll
-                for (int i = 0; i < S; ++i)
-                    lbuf[v * SP + i] = b0[i];
+                for (int i = 0; i < H; ++i)
+                    lbuf[v * SP + h * H + i] = b0[i];
             }
         }
     }
@@ -464,27 +508,27 @@ __global__ __launch_bounds__(RB) void k_resident(ResArgs a)
         }
 #pragma unroll
         for (int r = 0; r < NN; ++r) {
-            if (r * RB + wave * WAVE >= n1 - n0)
+            if (r * RN + wave * (WAVE / LN) >= n1 - n0)
                 continue;
-            const unsigned v = n0 + r * RB + tid;
-            if (v < n1) {
-                const float *msgs = lnew + (slots[r] & 0xffffu) * S;
+            const unsigned v = n0 + r * RN + tid / LN;
+            if (v < n1) { /* all lanes of a node or none */
+                const float *msgs = lnew + (slots[r] & 0xffffu) * S + h * H;
                 const unsigned cnt = slots[r] >> 16, n = nn[r];
-                float b[S];
+                float b[H];
                 if (clean)
-                    resident_node<S, MIXED, NS, true>(msgs, cnt, n, st[r], b);
+                    resident_node<S, MIXED, NS, true, H>(msgs, cnt, n, h, st[r], b);
                 else
-                    resident_node<S, MIXED, NS, false>(msgs, cnt, n, st[r], b);
-                float row[SP];
+                    resident_node<S, MIXED, NS, false, H>(msgs, cnt, n, h, st[r], b);
+                float row[HP];
 #pragma unroll
-                for (int i = 0; i < SP; ++i)
-                    row[i] = (i < S && (!MIXED || (unsigned)i < n)) ? b[i] : 0.0f;
+                for (int i = 0; i < HP; ++i)
+                    row[i] = (i < H && (!MIXED || h * H + i < n)) ? b[i] : 0.0f;
                 if constexpr (SINGLE) {
 #pragma unroll
-                    for (int i = 0; i < S; ++i)
-                        lbuf[v * SP + i] = row[i];
+                    for (int i = 0; i < H; ++i)
+                        lbuf[v * SP + h * H + i] = row[i];
                 } else {
-                    store_row_agent<SP>(a.ring + (size_t)ran * a.ring_stride + (size_t)v * SP, row);
+                    store_row_agent<HP>(a.ring + (size_t)ran * a.ring_stride + (size_t)v * SP + h * H, row);
                 }
             }
         }
@@ -524,21 +568,22 @@ __global__ __launch_bounds__(RB) void k_resident(ResArgs a)
     }
 #pragma unroll
     for (int r = 0; r < NN; ++r) {
-        const unsigned v = n0 + r * RB + tid;
+        const unsigned v = n0 + r * RN + tid / LN;
         if (v < n1) {
-            float row[SP];
+            const size_t at_row = (size_t)v * SP + h * H;
+            float row[HP];
 #pragma unroll
-            for (int i = 0; i < SP; ++i)
-                row[i] = (i < S && (!MIXED || (unsigned)i < nn[r])) ? st[r][i] : 0.0f;
-            store_row_nt<SP>(a.states + (size_t)v * SP, row);
+            for (int i = 0; i < HP; ++i)
+                row[i] = (i < H && (!MIXED || h * H + i < nn[r])) ? st[r][i] : 0.0f;
+            store_row_nt<HP>(a.states + at_row, row);
             if constexpr (SINGLE) {
 #pragma unroll
-                for (int i = 0; i < SP; ++i)
-                    row[i] = i < S ? lbuf[v * SP + i] : 0.0f;
+                for (int i = 0; i < HP; ++i)
+                    row[i] = i < H ? lbuf[at_row + i] : 0.0f;
             } else {
-                load_row<SP>(a.ring + (size_t)(ran - 1) * a.ring_stride + (size_t)v * SP, row);
+                load_row<HP>(a.ring + (size_t)(ran - 1) * a.ring_stride + at_row, row);
             }
-            store_row_nt<SP>(a.buf_out + (size_t)v * SP, row);
+            store_row_nt<HP>(a.buf_out + at_row, row);
         }
     }
     if (tid == 0 && wg == 0) {
@@ -576,7 +621,7 @@ unsigned most_groups(unsigned ns, unsigned S, unsigned cus)
  * combine buffers share 160 KB of LDS. */
 unsigned single_slots(unsigned S) { return S == 2 ? 4 : S <= 4 ? 2 : 1; }
 
-unsigned nodes_per_thread(unsigned ns) { return (ns + 1) / 2; }
+unsigned most_nodes(unsigned ns, unsigned S) { return S > 4 ? RB / 2 : (ns + 1) / 2 * RB; }
 
 /* Workgroup ranges: consecutive nodes with at most `slots` in-slots and
  * `nodes` nodes, cut at multiples of `align` nodes.  Empty when a node group
@@ -705,7 +750,7 @@ int bp_resident_plan(bp_dev *d, const std::vector<unsigned> &slot_src, int cus)
     std::vector<unsigned> first;
     const unsigned align = 32 / d->SP; /* nodes per 128-byte line */
     for (unsigned ns = 1; ns <= single_slots(d->S) && !r.ns; ns *= 2)
-        if (d->E <= ns * RB && d->V <= nodes_per_thread(ns) * RB) {
+        if (d->E <= ns * RB && d->V <= most_nodes(ns, d->S)) {
             r.ns = ns;
             r.single = true;
             first = {0, d->V};
@@ -716,7 +761,7 @@ int bp_resident_plan(bp_dev *d, const std::vector<unsigned> &slot_src, int cus)
         const unsigned cap = ns * RB, full = cap * 31 / 32, groups = most_groups(ns, d->S, (unsigned)cus);
         const unsigned want = (d->E + full - 1) / full;
         const unsigned even = std::min(cap, (d->E + want - 1) / want + cap / 32);
-        if (want <= groups && cut_ranges(d->in_off_h, d->V, even, nodes_per_thread(ns) * RB, align, first) &&
+        if (want <= groups && cut_ranges(d->in_off_h, d->V, even, most_nodes(ns, d->S), align, first) &&
             first.size() - 1 <= groups)
             r.ns = ns;
     }

@@ -34,6 +34,7 @@ struct bp_resident_status {
     unsigned run;      /* the last run that went through */
     unsigned ran;      /* its iterations */
     unsigned stopped;  /* the stop test ended it */
+    unsigned gave_up;  /* a run on a caller's stream was given up */
     double last, before; /* with the stop test: the last two deltas */
     double deltas[256];
 };
@@ -46,6 +47,7 @@ struct bp_resident {
     unsigned ns = 0, G = 0;    /* slots per thread, workgroups */
     unsigned limit = 0;        /* iterations per launch */
     unsigned run = 0, met = 0; /* launches, barriers met */
+    unsigned settled = 0;      /* the last run on a caller's stream that settles (one workgroup's need not) */
     char *memory = nullptr;    /* holds all of the following */
     unsigned *wg_node = nullptr;
     unsigned short *wg_slots = nullptr;

@@ -481,6 +481,7 @@ static float *stage_buf(bp_dev *d, size_t n)
         }
         d->h_stage_n = n;
         d->status()->run = 0;
+        d->status()->gave_up = 0;
     }
     if (!d->h_stage)
         return nullptr;

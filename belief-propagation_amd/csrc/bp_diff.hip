@@ -41,21 +41,11 @@
 #include <map>
 #include <vector>
 
-#include "bp_dev.h"
+#include "bp_adjoint.h"
+#include "bp_resident.h"
 #include "../../include/bp_diff.h"
 
 using namespace bpk;
-
-/* Slots per lane of the adjoint for four or fewer states (one above). */
-#ifndef BP_ADJ_SLOTS_SMALL
-#define BP_ADJ_SLOTS_SMALL 2
-#endif
-/* 1: each slot's w is written at the slot's position in the source-grouped
- * list, so a node reads its out-edges' w contiguously; 0: w in slot order,
- * gathered through the list */
-#ifndef BP_ADJ_W_SRC
-#define BP_ADJ_W_SRC 1
-#endif
 
 namespace {
 
@@ -63,23 +53,6 @@ constexpr unsigned NONE = 0xffffffffu;
 
 struct ParentRec {
     unsigned offset, n_par, slot_f, slot_r;
-};
-
-struct AdjArgs {
-    const unsigned *in_off, *slot_src, *out_off, *out_slot;
-    const unsigned *slot_pos; /* position of each slot in the source-grouped list (out_slot's inverse) */
-    const float *J;
-    const uint2 *chunk;
-    unsigned nchunks;
-    const float *st_prev; /* st_{t-1} */
-    const float *st_cur;  /* st_t (step 0: st_0) */
-    const float *bsrc;    /* buf_{t-1} (step 0: st_0) */
-    const float *gst_in;  /* dL/dst_t along paths through later iterates and the loss */
-    float *gst_out;       /* dL/dst_{t-1} through st_t (step 0: dL/dst_0 without w_0) */
-    const float *w_in;    /* w_{t+1} or NULL */
-    float *w_out;         /* w_t */
-    float *jbar;          /* [E][S*S] */
-    int jbar_first;       /* write instead of accumulate */
 };
 
 __global__ void k_copy(const float *__restrict__ src, float *__restrict__ dst, size_t n)
@@ -147,68 +120,9 @@ __global__ void k_initial(const float *__restrict__ P, const unsigned *__restric
     st0[t] = (tb != NONE && k < S) ? P[tb + k] : base[t];
 }
 
-/* acc += rows[o] for o in [o0, o1), in order; four rows loaded before any
- * is added */
-template <int S, int SP>
-__device__ __forceinline__ void sum_rows_contig(const float *__restrict__ rows, unsigned o0, unsigned o1, float *acc)
-{
-    for (unsigned o = o0; o < o1; o += 4) {
-        float x[4][S];
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            load_rowp<S, SP>(rows + (size_t)((o + u < o1) ? o + u : o) * SP, x[u]);
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            if (o + u < o1)
-#pragma unroll
-                for (int k = 0; k < S; ++k)
-                    acc[k] = acc[k] + x[u][k];
-    }
-}
-
-/* the node's sum of its out-edges' w (BP_ADJ_W_SRC: stored in list order) */
-template <int S, int SP>
-__device__ __forceinline__ void sum_out_w(const float *__restrict__ w, const unsigned *__restrict__ out_slot,
-                                          unsigned o0, unsigned o1, float *acc);
-
-/* acc += rows[out_slot[o]] for o in [o0, o1), in order; four index loads,
- * then four row loads, are issued before any is added */
-template <int S, int SP>
-__device__ __forceinline__ void sum_out_rows(const float *__restrict__ rows, const unsigned *__restrict__ out_slot,
-                                             unsigned o0, unsigned o1, float *acc)
-{
-    for (unsigned o = o0; o < o1; o += 4) {
-        unsigned idx[4];
-        float x[4][S];
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            idx[u] = out_slot[(o + u < o1) ? o + u : o];
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            load_rowp<S, SP>(rows + (size_t)idx[u] * SP, x[u]);
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            if (o + u < o1)
-#pragma unroll
-                for (int k = 0; k < S; ++k)
-                    acc[k] = acc[k] + x[u][k];
-    }
-}
-
-template <int S, int SP>
-__device__ __forceinline__ void sum_out_w(const float *__restrict__ w, const unsigned *__restrict__ out_slot,
-                                          unsigned o0, unsigned o1, float *acc)
-{
-    if constexpr (BP_ADJ_W_SRC)
-        sum_rows_contig<S, SP>(w, o0, o1, acc);
-    else
-        sum_out_rows<S, SP>(w, out_slot, o0, o1, acc);
-}
-
 template <int S, int STEP0, int R>
 __global__ __launch_bounds__(BLOCK) void k_adjoint(AdjArgs a)
 {
-    constexpr int SP = Stride<S>::value;
     constexpr int W = WAVE * R;
     __shared__ float lm[WAVES_PER_BLOCK][S * W];
     __shared__ float ldt[WAVES_PER_BLOCK][S * W];
@@ -219,186 +133,8 @@ __global__ __launch_bounds__(BLOCK) void k_adjoint(AdjArgs a)
     unsigned w = xcd_block(blockIdx.x, gridDim.x) * WAVES_PER_BLOCK + wave;
     unsigned c0 = (unsigned)(((unsigned long long)w * a.nchunks) / Wt);
     unsigned c1 = (unsigned)(((unsigned long long)(w + 1) * a.nchunks) / Wt);
-    float *LM = lm[wave], *LDT = ldt[wave];
-    unsigned short *LN = lnode[wave], *LQ = lq[wave];
-    for (unsigned c = c0; c < c1; ++c) {
-        uint2 lo = bpk::uniform_load(a.chunk + c), hi = bpk::uniform_load(a.chunk + c + 1);
-        unsigned nb = lo.x, sb = lo.y, ne = hi.x, se = hi.y;
-        /* slot phase 1: the message of every slot, kept with its operands */
-        float Jr[R][S * S], b[R][S], m[R][S], sig[R];
-        bool pos[R];
-        unsigned u[R];
-        /* lanes past the chunk's end load a valid neighbour (results
-         * dropped): branch-free loads, all in flight before the gathers */
-        const bool any_slots = se > sb; /* uniform: no stand-in slot otherwise */
-        const unsigned s_last = se - 1;
-        if (any_slots) {
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                unsigned s = sb + r * WAVE + lane;
-                if (s >= se)
-                    s = s_last;
-                u[r] = a.slot_src[s];
-                load_row<S * S>(a.J + (size_t)s * S * S, Jr[r]);
-            }
-#pragma unroll
-            for (int r = 0; r < R; ++r)
-                load_rowp<S, SP>(a.bsrc + (size_t)u[r] * SP, b[r]);
-        }
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            unsigned s = sb + r * WAVE + lane;
-            if (s < se) {
-                float sum = 0.0f;
-#pragma unroll
-                for (int i = 0; i < S; ++i) {
-                    float acc = 0.0f;
-#pragma unroll
-                    for (int j = 0; j < S; ++j)
-                        acc = acc + Jr[r][i * S + j] * b[r][j];
-                    m[r][i] = acc;
-                    sum = sum + acc;
-                }
-                pos[r] = sum > 0.0f;
-                if (!pos[r])
-                    sum = 1.0f;
-                sig[r] = sum;
-#pragma unroll
-                for (int i = 0; i < S; ++i) {
-                    m[r][i] = m[r][i] / sum;
-                    LM[i * W + r * WAVE + lane] = m[r][i];
-                }
-            }
-        }
-        wave_sync();
-        /* node phase: dT, dst_{t-1} */
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            unsigned v = nb + r * WAVE + lane;
-            if (v < ne) {
-                unsigned q0 = a.in_off[v] - sb, q1 = a.in_off[v + 1] - sb;
-                unsigned o0 = a.out_off[v], o1 = a.out_off[v + 1];
-                float st[S], g[S], T[S], gb[S], dT[S];
-                load_rowp<S, SP>(a.st_cur + (size_t)v * SP, st);
-                load_rowp<S, SP>(a.gst_in + (size_t)v * SP, g);
-#pragma unroll
-                for (int k = 0; k < S; ++k) {
-                    T[k] = 1.0f;
-                    gb[k] = 0.0f;
-                }
-                for (unsigned q = q0; q < q1; ++q) {
-#pragma unroll
-                    for (int k = 0; k < S; ++k) {
-                        float mk = LM[k * W + q];
-                        if (mk == mk)
-                            T[k] = T[k] * mk;
-                    }
-                }
-                if (a.w_in)
-                    sum_out_w<S, SP>(a.w_in, a.out_slot, o0, o1, gb);
-                float out[S];
-                if (STEP0) {
-#pragma unroll
-                    for (int k = 0; k < S; ++k) {
-                        dT[k] = gb[k] * st[k];
-                        out[k] = g[k] + gb[k] * T[k];
-                    }
-                } else {
-                    float sp[S], ds[S], av[S];
-                    load_rowp<S, SP>(a.st_prev + (size_t)v * SP, sp);
-                    bool indeg = q1 > q0;
-                    float sa = 0.0f, dot = 0.0f;
-#pragma unroll
-                    for (int k = 0; k < S; ++k) {
-                        ds[k] = g[k] + gb[k] * T[k];
-                        dT[k] = gb[k] * st[k];
-                        av[k] = indeg ? sp[k] * T[k] : sp[k];
-                        sa = sa + av[k];
-                        dot = dot + ds[k] * st[k];
-                    }
-#pragma unroll
-                    for (int k = 0; k < S; ++k) {
-                        float da = (sa > 0.0f) ? (ds[k] - dot) / sa : ds[k];
-                        out[k] = indeg ? da * T[k] : da;
-                        if (indeg)
-                            dT[k] = dT[k] + da * sp[k];
-                    }
-                }
-#pragma unroll
-                for (int k = 0; k < SP; ++k)
-                    a.gst_out[(size_t)v * SP + k] = (k < S) ? out[k] : 0.0f;
-                unsigned l = r * WAVE + lane;
-#pragma unroll
-                for (int k = 0; k < S; ++k)
-                    LDT[k * W + l] = dT[k];
-                LQ[2 * l] = (unsigned short)q0;
-                LQ[2 * l + 1] = (unsigned short)q1;
-                for (unsigned q = q0; q < q1; ++q)
-                    LN[q] = (unsigned short)l;
-            }
-        }
-        wave_sync();
-        /* slot phase 2: dm, dz, dJ, w */
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            unsigned s = sb + r * WAVE + lane;
-            if (s < se) {
-                unsigned q = r * WAVE + lane;
-                unsigned l = LN[q], q0 = LQ[2 * l], q1 = LQ[2 * l + 1];
-                float P[S];
-#pragma unroll
-                for (int k = 0; k < S; ++k)
-                    P[k] = 1.0f;
-                for (unsigned p = q0; p < q1; ++p) {
-                    if (p == q)
-                        continue;
-#pragma unroll
-                    for (int k = 0; k < S; ++k) {
-                        float mk = LM[k * W + p];
-                        if (mk == mk)
-                            P[k] = P[k] * mk;
-                    }
-                }
-                float dm[S], dz[S], dot = 0.0f;
-#pragma unroll
-                for (int k = 0; k < S; ++k) {
-                    dm[k] = (m[r][k] == m[r][k]) ? LDT[k * W + l] * P[k] : 0.0f;
-                    dot = dot + dm[k] * m[r][k];
-                }
-#pragma unroll
-                for (int k = 0; k < S; ++k)
-                    dz[k] = pos[r] ? (dm[k] - dot) / sig[r] : dm[k];
-                float *jb = a.jbar + (size_t)s * S * S;
-                float gJ[S * S];
-                if (!a.jbar_first)
-                    load_row<S * S>(jb, gJ);
-#pragma unroll
-                for (int i = 0; i < S; ++i)
-#pragma unroll
-                    for (int j = 0; j < S; ++j)
-                        gJ[i * S + j] = a.jbar_first ? dz[i] * b[r][j] : gJ[i * S + j] + dz[i] * b[r][j];
-#pragma unroll
-                for (int i = 0; i < S * S; ++i)
-                    jb[i] = gJ[i];
-                float wv[SP];
-#pragma unroll
-                for (int j = 0; j < SP; ++j) {
-                    float acc = 0.0f;
-                    if (j < S) {
-#pragma unroll
-                        for (int i = 0; i < S; ++i)
-                            acc = acc + Jr[r][i * S + j] * dz[i];
-                    }
-                    wv[j] = acc;
-                }
-                size_t wrow = BP_ADJ_W_SRC ? (size_t)a.slot_pos[s] : (size_t)s;
-#pragma unroll
-                for (int j = 0; j < SP; ++j)
-                    a.w_out[wrow * SP + j] = wv[j];
-            }
-        }
-        wave_sync();
-    }
+    for (unsigned c = c0; c < c1; ++c)
+        adjoint_chunk<S, STEP0, R>(a, c, lm[wave], ldt[wave], lnode[wave], lq[wave], lane);
 }
 
 /* dL/dst_0 = the step-0 partial + sum of w_0 over the node's out-slots */
@@ -626,22 +362,33 @@ struct bp_diff {
     /* iterates: checkpoints t = 0, c, 2c, ...; a segment's recomputed ones;
      * the forward's scratch; the last beliefs */
     unsigned K = 0, c = 0, nck = 0;
+    /* Iterates (beliefs and combine buffers) up to this many bytes are all
+     * kept: recomputing the ones between checkpoints of every fifth took 24
+     * launches of a 30-iteration backward, 290 of its 1460 us on 200k nodes,
+     * to save 150 of the card's 288,000 MB. */
+    size_t keep_bytes = 512u << 20;
+    size_t stride = 0;          /* floats between two iterates: whole 128-byte lines */
+    unsigned max_in = 0;        /* largest in-degree */
     bool have_forward = false, have_params = false;
+    bool kept = false;          /* the last forward's iterates are all in ck_st, ck_buf */
     float *ck_st = nullptr, *ck_buf = nullptr;
     float *seg_st = nullptr, *seg_buf = nullptr;
     float *fw_st[2] = {nullptr, nullptr}, *fw_buf[2] = {nullptr, nullptr};
     float *final_st = nullptr;
+    /* resident backward: the rows of w of every step, and where each is */
+    float *rows = nullptr;
+    unsigned *out_at = nullptr;
     std::map<std::pair<unsigned, unsigned>, hipGraphExec_t> fwd_graphs, bwd_graphs;
 };
 
 static void diff_release_storage(bp_diff *x)
 {
     float *ps[] = {x->ck_st, x->ck_buf, x->seg_st, x->seg_buf, x->fw_st[0], x->fw_st[1], x->fw_buf[0], x->fw_buf[1],
-                   x->final_st};
+                   x->final_st, x->rows};
     for (float *p : ps)
         if (p)
             (void)hipFree(p);
-    x->ck_st = x->ck_buf = x->seg_st = x->seg_buf = x->final_st = nullptr;
+    x->ck_st = x->ck_buf = x->seg_st = x->seg_buf = x->final_st = x->rows = nullptr;
     x->fw_st[0] = x->fw_st[1] = x->fw_buf[0] = x->fw_buf[1] = nullptr;
     for (auto &kv : x->fwd_graphs)
         (void)hipGraphExecDestroy(kv.second);
@@ -661,7 +408,7 @@ extern "C" void bp_diff_free(bp_diff *x)
         (void)hipDeviceSynchronize();
     }
     diff_release_storage(x);
-    void *ps[] = {x->adj_chunk, x->defs, x->G, x->perm_d, x->inv_d, x->row_first_d, x->row_stride_d, x->row_def_d, x->par_def, x->prior_tb, x->out_off, x->out_slot, x->slot_pos, x->slot_edge, x->def_of, x->def_tb, x->def_slice,
+    void *ps[] = {x->out_at, x->adj_chunk, x->defs, x->G, x->perm_d, x->inv_d, x->row_first_d, x->row_stride_d, x->row_def_d, x->par_def, x->prior_tb, x->out_off, x->out_slot, x->slot_pos, x->slot_edge, x->def_of, x->def_tb, x->def_slice,
                   x->def_pbegin, x->def_prior, x->parents, x->P, x->st0, x->gin, x->gst[0], x->gst[1],
                   x->w[0], x->w[1], x->jbar, x->dst0p, x->dst0};
     for (void *p : ps)
@@ -901,7 +648,13 @@ extern "C" int bp_diff_create(const bp_bn *bn, unsigned int num_param_defs, int 
         x->E = x->d->E;
         x->S = x->d->S;
         x->SP = x->d->SP;
+        x->stride = ((size_t)x->V * x->SP + 31) / 32 * 32;
+        for (unsigned v = 0; v < x->V; ++v)
+            x->max_in = std::max(x->max_in, x->d->in_off_h[v + 1] - x->d->in_off_h[v]);
         rc = diff_build(x, bn, num_param_defs, g);
+        if (rc == 0 && bp_resident_diff_fits(x->d, x->max_in) &&
+            (dmalloc(&x->out_at, x->E) || bp_resident_diff_places(x->d, x->slot_pos, x->out_at)))
+            rc = -1;
     }
     graph_destroy(g);
     if (rc) {
@@ -996,13 +749,21 @@ static int diff_storage(bp_diff *x, unsigned K, unsigned c)
     if (x->K == K && x->c == c && x->final_st)
         return 0;
     diff_release_storage(x);
-    size_t VS = (size_t)x->V * x->SP;
+    size_t VS = x->stride;
     unsigned nck = K / c + 1;
     if (dmalloc(&x->ck_st, nck * VS) || dmalloc(&x->ck_buf, nck * VS) || dmalloc(&x->seg_st, (size_t)c * VS) ||
         dmalloc(&x->seg_buf, (size_t)c * VS) || dmalloc(&x->fw_st[0], VS) || dmalloc(&x->fw_st[1], VS) ||
         dmalloc(&x->fw_buf[0], VS) || dmalloc(&x->fw_buf[1], VS) || dmalloc(&x->final_st, VS)) {
         diff_release_storage(x);
         return -1;
+    }
+    /* (without the memory for it the backward runs its launches) */
+    if (c == 1 && x->out_at) {
+        const size_t rows = ((size_t)K + 1) * bp_resident_diff_rows(x->d);
+        if (rows * sizeof(float) <= x->keep_bytes && hipMalloc((void **)&x->rows, rows * sizeof(float)) != hipSuccess) {
+            x->rows = nullptr;
+            (void)hipGetLastError();
+        }
     }
     x->K = K;
     x->c = c;
@@ -1047,7 +808,7 @@ static int capture_end(bp_diff *x, hipGraphExec_t *exec)
 
 static void enqueue_forward(bp_diff *x, hipStream_t st)
 {
-    size_t VS = (size_t)x->V * x->SP;
+    const size_t VS = x->stride;
     unsigned K = x->K, c = x->c;
     fwd_step(x, FINIT, x->st0, nullptr, nullptr, x->ck_buf, st);
     const float *sp = x->st0, *bp = x->ck_buf;
@@ -1064,7 +825,18 @@ static void enqueue_forward(bp_diff *x, hipStream_t st)
         sp = so;
         bp = bo;
     }
-    hipLaunchKernelGGL(k_copy, dim3(blocks_for(VS)), dim3(256), 0, st, sp, x->final_st, VS);
+    const size_t n = (size_t)x->V * x->SP;
+    hipLaunchKernelGGL(k_copy, dim3(blocks_for(n)), dim3(256), 0, st, sp, x->final_st, n);
+}
+
+/* Whether the iterates, all kept, are run resident (not into a graph that is
+ * being captured: a run counts its barriers once). */
+static bool use_resident(bp_diff *x, hipStream_t st)
+{
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (st && hipStreamIsCapturing(st, &capturing) != hipSuccess)
+        (void)hipGetLastError();
+    return x->c == 1 && capturing == hipStreamCaptureStatusNone && bp_resident_diff_fits(x->d, x->max_in);
 }
 
 extern "C" int bp_diff_forward(bp_diff *x, unsigned int K, unsigned int c, float *beliefs, void *stream)
@@ -1079,12 +851,30 @@ extern "C" int bp_diff_forward(bp_diff *x, unsigned int K, unsigned int c, float
         return -1;
     }
     HIP_TRY(hipSetDevice(x->d->device));
-    if (diff_storage(x, K, c))
-        return -1;
-    /* the ck_st[0] slot is the initial beliefs themselves */
     size_t VS = (size_t)x->V * x->SP;
+    const unsigned every = 2 * ((size_t)K + 1) * x->stride * sizeof(float) <= x->keep_bytes ? 1 : c;
+    if (diff_storage(x, K, every)) {
+        if (every == c)
+            return -1;
+        (void)hipGetLastError(); /* not the memory for all of them */
+        bp_clear_error();
+        if (diff_storage(x, K, c))
+            return -1;
+    }
+    c = x->c;
     hipStream_t st = (hipStream_t)stream;
+    /* the ck_st[0] slot is the initial beliefs themselves */
     hipLaunchKernelGGL(k_copy, dim3(blocks_for(VS)), dim3(256), 0, st, x->st0, x->ck_st, VS);
+    if (K && use_resident(x, st)) {
+        fwd_step(x, FINIT, x->st0, nullptr, nullptr, x->ck_buf, st);
+        if (bp_resident_diff_forward(x->d, K, x->ck_st, x->ck_buf, x->stride, st))
+            return -1;
+        hipLaunchKernelGGL(k_gather_rows, dim3(blocks_for(VS)), dim3(256), 0, st, x->ck_st + K * x->stride, x->perm_d,
+                           beliefs, x->V, x->SP);
+        HIP_TRY(hipGetLastError());
+        x->have_forward = x->kept = true;
+        return 0;
+    }
     auto key = std::make_pair(K, c);
     auto it = x->fwd_graphs.find(key);
     if (it == x->fwd_graphs.end()) {
@@ -1101,6 +891,7 @@ extern "C" int bp_diff_forward(bp_diff *x, unsigned int K, unsigned int c, float
                        x->SP);
     HIP_TRY(hipGetLastError());
     x->have_forward = true;
+    x->kept = false;
     return 0;
 }
 
@@ -1150,9 +941,12 @@ static void adj_step(bp_diff *x, int step0, const float *st_prev, const float *s
 #undef BP_ADJ_CASE
 }
 
+static void enqueue_backward_tail(bp_diff *x, const float *w0, hipStream_t st);
+static void enqueue_parent_grad(bp_diff *x, hipStream_t st);
+
 static void enqueue_backward(bp_diff *x, hipStream_t st)
 {
-    size_t VS = (size_t)x->V * x->SP;
+    const size_t VS = x->stride;
     unsigned K = x->K, c = x->c;
     unsigned nseg = (K + c - 1) / c;
     const float *gin = x->gin; /* dL/dst_K */
@@ -1181,7 +975,12 @@ static void enqueue_backward(bp_diff *x, hipStream_t st)
     }
     /* step 0: init */
     adj_step(x, 1, nullptr, x->st0, x->st0, gin, x->dst0p, w_in, x->w[0] == w_in ? x->w[1] : x->w[0], first, st);
-    const float *w0 = (x->w[0] == w_in) ? x->w[1] : x->w[0];
+    enqueue_backward_tail(x, (x->w[0] == w_in) ? x->w[1] : x->w[0], st);
+}
+
+/* dL/d(initial beliefs) and the per-parent sums */
+static void enqueue_backward_tail(bp_diff *x, const float *w0, hipStream_t st)
+{
     dim3 gv(blocks_for(x->V)), b256(256);
 #define BP_IG_CASE(SS)                                                                                     \
     case SS:                                                                                               \
@@ -1201,6 +1000,11 @@ static void enqueue_backward(bp_diff *x, hipStream_t st)
         BP_IG_CASE(10)
     }
 #undef BP_IG_CASE
+    enqueue_parent_grad(x, st);
+}
+
+static void enqueue_parent_grad(bp_diff *x, hipStream_t st)
+{
     size_t nG = (size_t)x->nrec * x->S * x->S;
     if (nG)
         hipLaunchKernelGGL(k_parent_grad, dim3(blocks_for(nG)), dim3(256), 0, st, x->jbar, x->parents, x->G, x->nrec,
@@ -1270,18 +1074,30 @@ extern "C" int bp_diff_backward_ex(bp_diff *x, const float *grad_beliefs, float 
     size_t VS = (size_t)x->V * x->SP;
     hipLaunchKernelGGL(k_gather_rows, dim3(blocks_for(VS)), dim3(256), 0, st, grad_beliefs, x->inv_d, x->gin, x->V,
                        x->SP);
-    auto key = std::make_pair(x->K, x->c);
-    auto it = x->bwd_graphs.find(key);
-    if (it == x->bwd_graphs.end()) {
-        hipGraphExec_t exec = nullptr;
-        if (capture_begin(x))
+    if (x->kept && x->rows && use_resident(x, st)) {
+        bp_adjoint_arrays arrays = {x->out_off, x->out_slot, x->slot_pos, x->adj_chunk, x->adj_nchunks, x->st0, x->gin,
+                                    {x->gst[0], x->gst[1]}, {x->w[0], x->w[1]}, x->jbar, x->dst0p, x->dst0,
+                                    x->out_at, x->rows};
+        if (bp_resident_diff_backward(x->d, x->K, x->ck_st, x->ck_buf, x->stride, arrays, st))
             return -1;
-        enqueue_backward(x, x->d->stream);
-        if (capture_end(x, &exec))
-            return -1;
-        it = x->bwd_graphs.emplace(key, exec).first;
+        enqueue_parent_grad(x, st);
+    } else {
+        if (x->kept) /* the launches look for the last beliefs here */
+            hipLaunchKernelGGL(k_copy, dim3(blocks_for(VS)), dim3(256), 0, st, x->ck_st + x->K * x->stride,
+                               x->final_st, VS);
+        auto key = std::make_pair(x->K, x->c);
+        auto it = x->bwd_graphs.find(key);
+        if (it == x->bwd_graphs.end()) {
+            hipGraphExec_t exec = nullptr;
+            if (capture_begin(x))
+                return -1;
+            enqueue_backward(x, x->d->stream);
+            if (capture_end(x, &exec))
+                return -1;
+            it = x->bwd_graphs.emplace(key, exec).first;
+        }
+        HIP_TRY(hipGraphLaunch(it->second, st));
     }
-    HIP_TRY(hipGraphLaunch(it->second, st));
     if (grad_params)
         launch_param_grad(x, 0, grad_params, st);
     size_t SS = (size_t)x->S * x->S;
@@ -1330,3 +1146,8 @@ extern "C" int bp_diff_tables(bp_diff *x, float *out)
         std::memcpy(out + (size_t)x->d->slot_edge[s] * SS, tmp.data() + (size_t)s * SS, SS * sizeof(float));
     return 0;
 }
+
+/* For checks: the handle a network's runs use, and the bytes of iterates that
+ * are kept whatever the checkpoint interval. */
+extern "C" bp_dev *bp_diff_device(bp_diff *x) { return x->d; }
+extern "C" void bp_diff_set_keep(bp_diff *x, unsigned long long bytes) { x->keep_bytes = bytes; }

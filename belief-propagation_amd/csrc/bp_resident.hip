@@ -59,18 +59,12 @@
 #include <mutex>
 #include <vector>
 
-#include "bp_dev.h"
 #include "bp_parallel.h"
+#include "bp_resident.h"
 
 using namespace bpk;
 
 namespace {
-
-constexpr int RB = 1024;            /* threads per workgroup */
-constexpr int RW = RB / WAVE;
-constexpr unsigned MAX_G = 256;
-constexpr unsigned COUNTERS = 16, COUNTER_STRIDE = 64; /* unsigneds between two counters */
-constexpr int PAD = 8; /* rows past the messages that a node's first read may touch */
 
 struct ResArgs {
     const unsigned *in_off, *slot_src;
@@ -85,6 +79,7 @@ struct ResArgs {
     float *msg0, *msg1;  /* messages before the run; the other array */
     float *ring;         /* iteration t's combine buffers at ring + t * ring_stride */
     size_t ring_stride;
+    float *keep;      /* non-null: every iteration's beliefs go to keep + t * ring_stride, and nothing else is left */
     unsigned S;       /* the network's largest state count */
     unsigned n;       /* iterations, at most */
     int until;        /* stop test of graph.c:1313 after each */
@@ -92,94 +87,9 @@ struct ResArgs {
     double previous;  /* the delta before the run, for the test */
     double *partials; /* DELTA: [n][G] delta partials */
     double *parts;    /* [2][MAX_G] the running iteration's, for the test */
-    unsigned *counters;
-    unsigned met;     /* barriers that the counters have counted */
-    unsigned *decision;
-    unsigned run;
-    unsigned after;   /* the run that this one goes on from, 0: none outstanding */
-    unsigned long long timeout;
+    Meeting meeting;
     bp_resident_status *status; /* host memory */
 };
-
-enum { GO_ON = 0, COMMIT = 1 };
-
-/* Settles the run for all workgroups: the first word wins. */
-__device__ __forceinline__ bool settle(unsigned *decision, unsigned run, unsigned commit)
-{
-    const unsigned mine = run << 1 | commit;
-    unsigned cur = __hip_atomic_load(decision, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    while (cur >> 1 != run)
-        if (__hip_atomic_compare_exchange_strong(decision, &cur, mine, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                 __HIP_MEMORY_SCOPE_AGENT))
-            return commit;
-    return cur & 1u;
-}
-
-/* Waits until every workgroup has been at barrier number `number` (from 1).
- * False: this run has been given up.  All threads of the workgroup call it;
- * `ok` is shared. */
-__device__ __forceinline__ bool grid_step(const ResArgs &a, unsigned wg, unsigned G, unsigned number, unsigned *ok)
-{
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); /* this wave's combine buffers are in memory */
-    __syncthreads();
-    if (threadIdx.x < WAVE) {
-        const unsigned lane = threadIdx.x;
-        if (lane == 0)
-            __hip_atomic_fetch_add(a.counters + (wg % COUNTERS) * COUNTER_STRIDE, 1u, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-        const unsigned members = lane < COUNTERS ? (G - lane + COUNTERS - 1) / COUNTERS : 0u;
-        const unsigned want = (a.met + number) * members;
-        const unsigned long long t0 = wall_clock64();
-        bool there = false;
-        while (!there) {
-            bool all = true;
-            if (members)
-                all = (int)(__hip_atomic_load(a.counters + lane * COUNTER_STRIDE, __ATOMIC_RELAXED,
-                                              __HIP_MEMORY_SCOPE_AGENT) - want) >= 0;
-            there = __ballot(!all) == 0;
-            if (!there && wall_clock64() - t0 > a.timeout) {
-                /* given up, unless another workgroup is already past the
-                 * last barrier: then all have been here */
-                unsigned c = lane == 0 ? (unsigned)settle(a.decision, a.run, GO_ON) : 0u;
-                there = __builtin_amdgcn_readfirstlane(c) != 0;
-                break;
-            }
-        }
-        if (lane == 0)
-            *ok = there;
-    }
-    __syncthreads();
-    asm volatile("" ::: "memory"); /* no gather moves above the barrier */
-    return *ok != 0;
-}
-
-template <int N> __device__ __forceinline__ void store_row_agent(float *p, const float *v)
-{
-    static_assert(N % 2 == 0, "rows are float pairs");
-#pragma unroll
-    for (int i = 0; i < N / 2; ++i) {
-        const unsigned long long lo = __float_as_uint(v[2 * i]), hi = __float_as_uint(v[2 * i + 1]);
-        __hip_atomic_store(reinterpret_cast<unsigned long long *>(p) + i, lo | hi << 32, __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-    }
-}
-
-/* rows of S floats in LDS */
-template <int S> __device__ __forceinline__ void put_row(float *p, const float *v)
-{
-    if constexpr (S == 2)
-        *reinterpret_cast<float2 *>(p) = make_float2(v[0], v[1]);
-    else if constexpr (S % 4 == 0)
-#pragma unroll
-        for (int i = 0; i < S; i += 4)
-            *reinterpret_cast<float4 *>(p + i) = make_float4(v[i], v[i + 1], v[i + 2], v[i + 3]);
-    else
-#pragma unroll
-        for (int i = 0; i < S; ++i)
-            p[i] = v[i];
-}
-
-template <int S> __device__ __forceinline__ void get_row(const float *p, float *v) { load_row<S>(p, v); }
 
 /* Lanes per node in the node phase, and rounds of the workgroup over its
  * nodes: a message edge belongs to one node, and the networks' nodes have
@@ -191,28 +101,6 @@ template <int S> struct LanesPerNode {
 template <int S, int NS> struct NodeRounds {
     static constexpr int value = S == 8 ? 2 : (NS + 1) / 2;
 };
-
-/* N in-messages from p on, S floats apart, as factors, H entries of each:
- * those past the node's last one are 1, and so are NaN entries (CLEAN: there
- * may be some), which the products skip.  All reads are issued before the
- * first product: a read at a time made the node phase a chain of LDS
- * latencies as long as the largest in-degree of the wave's nodes (1.5 of
- * 2.3 us on a 700-node network). */
-template <int S, int H, int N, bool CLEAN>
-__device__ __forceinline__ void factors(const float *p, unsigned cnt, float (&f)[N][H])
-{
-#pragma unroll
-    for (int j = 0; j < N; ++j)
-        get_row<H>(p + j * S, f[j]);
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-#pragma unroll
-        for (int i = 0; i < H; ++i)
-            f[j][i] = (unsigned)j < cnt ? f[j][i] : 1.0f;
-        if (CLEAN)
-            nan_to_one<H>(f[j]);
-    }
-}
 
 /* normalise() over four lanes of two entries each: the sum runs through the
  * lanes in entry order, from 0.0 left to right as with one lane. */
@@ -309,9 +197,8 @@ __global__ __launch_bounds__(RB) void k_resident(ResArgs a)
     __shared__ unsigned ok, committed, suspect;
     const unsigned tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const unsigned G = gridDim.x, wg = SINGLE ? 0u : xcd_block(blockIdx.x, G);
-    if (!SINGLE && a.after &&
-        __hip_atomic_load(a.decision, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != (a.after << 1 | COMMIT))
-        return; /* the run before this one was given up */
+    if (!SINGLE && called_off(a.meeting))
+        return;
     const unsigned n0 = a.wg_node[wg], n1 = a.wg_node[wg + 1];
     const unsigned s0 = a.in_off[n0], ns = a.in_off[n1] - s0;
     if (tid == 0)
@@ -404,13 +291,17 @@ __global__ __launch_bounds__(RB) void k_resident(ResArgs a)
     if constexpr (SINGLE) {
         __syncthreads();
     } else {
-        if (!grid_step(a, wg, G, 1, &ok)) /* everybody is here */
+        if (!grid_step(a.meeting, wg, G, 1, &ok)) /* everybody is here */
             return;
     }
 
     double previous = a.previous, before = a.previous;
     unsigned ran = 0, stopped = 0;
     for (;;) {
+        hold(at);
+        hold(slots);
+        if (MIXED)
+            hold(src);
         const float *in = SINGLE ? lbuf : ran == 0 ? a.buf_in : a.ring + (size_t)(ran - 1) * a.ring_stride;
         float bsrc[NS][S];
         if (ran < a.n) {
@@ -523,12 +414,21 @@ __global__ __launch_bounds__(RB) void k_resident(ResArgs a)
 #pragma unroll
                 for (int i = 0; i < HP; ++i)
                     row[i] = (i < H && (!MIXED || h * H + i < n)) ? b[i] : 0.0f;
+                const size_t to = (size_t)ran * a.ring_stride + (size_t)v * SP + h * H;
                 if constexpr (SINGLE) {
 #pragma unroll
                     for (int i = 0; i < H; ++i)
                         lbuf[v * SP + h * H + i] = row[i];
+                    if (a.keep)
+                        store_row_nt<HP>(a.ring + to, row);
                 } else {
-                    store_row_agent<HP>(a.ring + (size_t)ran * a.ring_stride + (size_t)v * SP + h * H, row);
+                    store_row_agent<HP>(a.ring + to, row);
+                }
+                if (a.keep) {
+#pragma unroll
+                    for (int i = 0; i < HP; ++i)
+                        row[i] = (i < H && (!MIXED || h * H + i < n)) ? st[r][i] : 0.0f;
+                    store_row_nt<HP>(a.keep + to, row);
                 }
             }
         }
@@ -536,18 +436,20 @@ __global__ __launch_bounds__(RB) void k_resident(ResArgs a)
         if constexpr (SINGLE) {
             __syncthreads();
         } else {
-            if (!grid_step(a, wg, G, ran + 1, &ok))
+            if (!grid_step(a.meeting, wg, G, ran + 1, &ok))
                 return;
         }
     }
 
     if constexpr (!SINGLE) {
         if (tid == 0)
-            committed = settle(a.decision, a.run, COMMIT);
+            committed = settle(a.meeting.decision, a.meeting.run, COMMIT);
         __syncthreads();
         if (!committed)
             return;
     }
+    if (a.keep)
+        return;
     /* results: beliefs, the combine buffers of the next iteration, the last
      * two iterations' messages */
     float *newest = ran & 1 ? a.msg1 : a.msg0, *older = ran & 1 ? a.msg0 : a.msg1;
@@ -591,7 +493,7 @@ __global__ __launch_bounds__(RB) void k_resident(ResArgs a)
         a.status->stopped = stopped;
         a.status->last = previous;
         a.status->before = before;
-        __hip_atomic_store(&a.status->run, a.run, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(&a.status->run, a.meeting.run, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -608,13 +510,13 @@ namespace {
  * and LDS (two iterations' messages) hold. */
 unsigned most_slots(unsigned S) { return S == 2 ? 8 : S == 3 ? 4 : S == 4 ? 3 : 1; }
 
-/* slots per thread go 1, 2, 4, 8; for four states 1, 2, 3 */
-unsigned next_slots(unsigned ns, unsigned S) { return S == 4 && ns == 2 ? 3 : 2 * ns; }
+/* slots per thread go 1, 2, 4, 8; for three and four states 1, 2, 3, 4 */
+unsigned next_slots(unsigned ns, unsigned S) { return S > 2 && ns >= 2 ? ns + 1 : 2 * ns; }
 
 unsigned most_groups(unsigned ns, unsigned S, unsigned cus)
 {
     const unsigned full = std::min(cus, MAX_G);
-    return ns == most_slots(S) ? full : std::min(full, 64 * ns);
+    return ns == most_slots(S) || ns > 2 ? full : std::min(full, 64 * ns);
 }
 
 /* Largest network of one workgroup, in slots per thread: messages and
@@ -671,26 +573,16 @@ void deal_slots(const std::vector<unsigned> &in_off, const std::vector<unsigned>
 
 /* One resident launch at a time per device: the launches of two streams,
  * each partly on the chip, would wait for each other.  A launch on another
- * stream than the last one waits for that stream. */
+ * stream than the last one waits for that one: by an event recorded now if
+ * the last stream is a handle's, which lives until bp_resident_free, or when
+ * it was launched if it is a caller's. */
 constexpr int MAX_DEVICES = 64;
 std::mutex turn_mu;
 struct {
+    bool any, foreign;
     hipStream_t last;
     hipEvent_t ev;
 } turn[MAX_DEVICES];
-
-int take_turn(int device, hipStream_t stream)
-{
-    auto &t = turn[device];
-    if (t.last && t.last != stream) {
-        if (!t.ev)
-            HIP_TRY(hipEventCreateWithFlags(&t.ev, hipEventDisableTiming));
-        HIP_TRY(hipEventRecord(t.ev, t.last));
-        HIP_TRY(hipStreamWaitEvent(stream, t.ev, 0));
-    }
-    t.last = stream;
-    return 0;
-}
 
 template <int S, bool MIXED, int NS, bool SINGLE>
 void launch_d(const ResArgs &a, unsigned G, bool delta, hipStream_t st)
@@ -717,12 +609,15 @@ void launch_s(const ResArgs &a, unsigned ns, unsigned G, bool single, bool delta
         launch_d<S, MIXED, 1, false>(a, G, delta, st);
     else if (ns == 2)
         launch_d<S, MIXED, 2, false>(a, G, delta, st);
-    else if constexpr (S == 4)
-        launch_d<S, MIXED, 3, false>(a, G, delta, st);
-    else if (ns == 4)
-        launch_d<S, MIXED, 4, false>(a, G, delta, st);
-    else if constexpr (S == 2)
-        launch_d<S, MIXED, 8, false>(a, G, delta, st);
+    if constexpr (S > 2)
+        if (ns == 3)
+            launch_d<S, MIXED, 3, false>(a, G, delta, st);
+    if constexpr (S < 4)
+        if (ns == 4)
+            launch_d<S, MIXED, 4, false>(a, G, delta, st);
+    if constexpr (S == 2)
+        if (ns == 8)
+            launch_d<S, MIXED, 8, false>(a, G, delta, st);
 }
 
 void launch(unsigned S, bool mixed, const ResArgs &a, unsigned ns, unsigned G, bool single, bool delta,
@@ -739,6 +634,47 @@ void launch(unsigned S, bool mixed, const ResArgs &a, unsigned ns, unsigned G, b
 }
 
 } // namespace
+
+std::mutex &bp_resident_mutex() { return turn_mu; }
+
+int bp_resident_turn(int device, hipStream_t stream)
+{
+    auto &t = turn[device];
+    if (!t.ev)
+        HIP_TRY(hipEventCreateWithFlags(&t.ev, hipEventDisableTiming));
+    if (t.any && t.last != stream) {
+        if (!t.foreign)
+            HIP_TRY(hipEventRecord(t.ev, t.last));
+        HIP_TRY(hipStreamWaitEvent(stream, t.ev, 0));
+    }
+    return 0;
+}
+
+int bp_resident_turn_taken(int device, hipStream_t stream, bool foreign)
+{
+    auto &t = turn[device];
+    t.any = true;
+    t.last = stream;
+    t.foreign = foreign;
+    if (foreign)
+        HIP_TRY(hipEventRecord(t.ev, stream));
+    return 0;
+}
+
+Meeting bp_resident_meeting(bp_dev *d, unsigned barriers, unsigned after)
+{
+    bp_resident &r = d->res;
+    Meeting m;
+    m.counters = r.counters;
+    m.met = r.met;
+    m.decision = r.counters + COUNTERS * COUNTER_STRIDE;
+    m.after = after;
+    r.run = (r.run + 1) & 0x7fffffffu;
+    m.run = r.run;
+    m.timeout = r.timeout;
+    r.met += barriers;
+    return m;
+}
 
 /* Decides whether the graph runs resident and lays out its ranges:
  * uniform state counts of 2 to 8, or mixed ones up to 3 to 8. */
@@ -785,10 +721,10 @@ int bp_resident_plan(bp_dev *d, const std::vector<unsigned> &slot_src, int cus)
         r.ring_stride = ((size_t)d->V * d->SP + 31) / 32 * 32;
         r.limit = std::min<size_t>(r.limit, std::min<size_t>(256, std::max<size_t>(32, (8u << 20) / (4 * r.ring_stride))));
         bytes += r.ring_stride * r.limit * sizeof(float);
-        int khz = 0;
-        HIP_TRY(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, d->device));
-        r.timeout = (unsigned long long)khz * 1000; /* a second */
     }
+    int khz = 0;
+    HIP_TRY(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, d->device));
+    r.timeout = (unsigned long long)khz * 1000; /* a second */
     HIP_TRY(hipMalloc((void **)&r.memory, bytes));
     HIP_TRY(hipMemcpy(r.memory, head.data(), head.size() * sizeof(unsigned), hipMemcpyHostToDevice));
     r.counters = (unsigned *)r.memory;
@@ -806,7 +742,7 @@ void bp_resident_free(bp_dev *d)
     {
         std::lock_guard<std::mutex> lock(turn_mu);
         if (d->stream && d->device < MAX_DEVICES && turn[d->device].last == d->stream)
-            turn[d->device].last = nullptr;
+            turn[d->device].any = false; /* the stream has been waited for */
     }
     if (r.memory)
         (void)hipFree(r.memory);
@@ -827,6 +763,7 @@ int bp_resident_launch(bp_dev *d, unsigned n, bool want_delta, bool until, float
     a.J = d->J;
     a.slot_tab = d->mixed ? d->slot_toff : nullptr;
     a.S = d->S;
+    a.keep = nullptr;
     a.wg_node = r.wg_node;
     a.wg_slots = r.wg_slots;
     a.states = d->states;
@@ -843,26 +780,55 @@ int bp_resident_launch(bp_dev *d, unsigned n, bool want_delta, bool until, float
     /* one workgroup: its partial is the delta */
     a.partials = r.single ? d->status()->deltas : partials;
     a.parts = r.parts;
-    a.counters = r.counters;
-    a.met = r.met;
-    a.decision = r.counters + COUNTERS * COUNTER_STRIDE;
-    r.run = (r.run + 1) & 0x7fffffffu;
-    a.run = r.run;
-    a.after = r.pending.empty() ? 0u : r.pending.back().first;
-    a.timeout = r.timeout;
+    /* with the stop test bp_resident_ran says how many barriers there were */
+    a.meeting = bp_resident_meeting(d, until || r.single ? 0 : n + 1, r.pending.empty() ? 0u : r.pending.back().first);
     a.status = d->status();
-    if (!until)
-        r.met += n + 1; /* else bp_resident_ran says how many */
     if (r.single) {
         launch(d->S, d->mixed, a, r.ns, 1, true, want_delta || until, d->stream);
     } else {
         std::lock_guard<std::mutex> lock(turn_mu);
-        if (take_turn(d->device, d->stream))
+        if (bp_resident_turn(d->device, d->stream))
             return -1;
         launch(d->S, d->mixed, a, r.ns, r.G, false, want_delta || until, d->stream);
+        if (bp_resident_turn_taken(d->device, d->stream, false))
+            return -1;
     }
     if (want_delta && !until && !r.single)
         bp_launch_finish(partials, r.G, n, d->status()->deltas, d->stream);
+    HIP_TRY(hipGetLastError());
+    return 0;
+}
+
+/* The unrolled forward of the adjoint: K iterations from the beliefs st[0]
+ * and combine buffers buf[0] to st[1..K] and buf[1..K], rows of a `stride`
+ * each, on a caller's stream.  A run that is given up leaves them to
+ * k_forward_rescue (bp_resident_diff.hip). */
+int bp_resident_forward(bp_dev *d, unsigned K, float *st, float *buf, size_t stride, hipStream_t stream,
+                        Meeting *meeting)
+{
+    bp_resident &r = d->res;
+    ResArgs a = {};
+    a.in_off = d->in_off;
+    a.slot_src = d->slot_src;
+    a.slot_xy = d->slot_xy;
+    a.nvars = d->nvars;
+    a.J = d->J;
+    a.wg_node = r.wg_node;
+    a.wg_slots = r.wg_slots;
+    a.S = d->S;
+    a.states = st;
+    a.buf_in = buf;
+    a.ring = buf + stride;
+    a.keep = st + stride;
+    a.ring_stride = stride;
+    a.n = K;
+    a.parts = r.parts;
+    a.meeting = bp_resident_meeting(d, r.single ? 0 : K + 1, r.single ? 0 : r.settled);
+    if (!r.single)
+        r.settled = r.run;
+    a.status = d->status();
+    *meeting = a.meeting;
+    launch(d->S, d->mixed, a, r.ns, r.G, r.single, false, stream);
     HIP_TRY(hipGetLastError());
     return 0;
 }
@@ -873,7 +839,7 @@ bool bp_resident_ran(bp_dev *d, bool until)
 {
     bp_resident &r = d->res;
     const bool ran = r.single || d->status()->run == r.run;
-    if (ran && until)
+    if (ran && until && !r.single)
         r.met += d->status()->ran + 1;
     return ran;
 }

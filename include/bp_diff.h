@@ -18,7 +18,8 @@
  *
  * Forward.  init_previous_edge + K iterations of the node-centric schedule
  * (bit-identical beliefs to bp_loopy_iterate on the same tables), keeping
- * the beliefs and combine buffers of every c-th iteration.
+ * the beliefs and combine buffers of every iteration where they take at
+ * most 512 MB, and otherwise of every c-th.
  *
  * Backward.  Reverse-mode adjoint of the same recursion, in exact
  * arithmetic terms:
@@ -26,7 +27,10 @@
  *   st_t[v] = N(st_{t-1}[v] (.) T_t[v]),  buf_t[v] = st_t[v] (.) T_t[v],
  * with m_0 and buf_0 from st_0 (init).  Iterates between checkpoints are
  * recomputed by the forward kernel, segment by segment.  Returns dL/dTABLE
- * for every parameter entry given dL/dbeliefs after iteration K.
+ * for every parameter entry given dL/dbeliefs after iteration K.  Networks
+ * whose tables, and their gradients, fit on the chip go through all
+ * iterations in one launch, forward and backward; under stream capture each
+ * iteration is a launch of its own.
  *
  * Limits: every node has the same state count, and no node has more than
  * 128 in-edges (64 for more than 4 states); bp_diff_create reports others.

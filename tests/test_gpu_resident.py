@@ -9,6 +9,7 @@ import ctypes as C
 
 import numpy as np
 import pytest
+import torch
 
 import bp_ctypes as B
 from conftest import bits_report, same_bits
@@ -67,7 +68,8 @@ CASES = [
     (17500, 2, 2, 2, True),
     (40000, 3, 3, 2, True),
     (70001, 2, 4, 3, True),
-    (71000, 3, 3, 4, True),
+    (71000, 3, 3, 3, True),
+    (215000, 3, 3, 4, True),
     (75000, 2, 2, 4, True),
     (290000, 2, 2, 8, True),
     (250, 2, 8, 1, False),
@@ -193,3 +195,69 @@ def test_runs_on_two_handles_from_two_threads(lib, orc):
         check(g, h)
         lib.graph_destroy(g)
         lib.graph_destroy(h)
+
+
+# (nodes, states, workgroups): 1, 2 and the most slots per thread of the
+# adjoint; the last of each state count is too large for it
+DIFF_CASES = [(200, 2), (5000, 2), (30000, 2), (150000, 2), (300000, 2), (300, 3), (3000, 3), (40000, 3), (200000, 3),
+              (250, 4), (8000, 4), (60000, 4)]
+
+
+def gradient(net, K, every, log, seed):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    theta = torch.randn(net.num_params, generator=gen, device="cuda")
+    if not log:
+        theta = net.softmax_tables(theta).contiguous()
+    theta.requires_grad_(True)
+    weight = torch.rand(net.V, net.S, generator=gen, device="cuda")
+    out = []
+    for _ in range(2):
+        theta.grad = None
+        b = (net.beliefs_from_log if log else net.beliefs)(theta, K, every)
+        (b * weight).sum().backward()
+        out += [b.detach().cpu().numpy(), theta.grad.cpu().numpy()]
+    return out
+
+
+@pytest.mark.parametrize("nodes,states", DIFF_CASES)
+def test_gradient_is_that_of_the_launches(lib, nodes, states):
+    """Forward and adjoint with everything kept on the chip, against launches
+    that keep every third iterate and recompute the others; twice, so that a
+    second run goes on from the first."""
+    from belief_network_wrapper import DifferentiableNetwork
+
+    print(f"gradient {nodes} nodes {states} states", flush=True)
+    lib.bp_diff_set_keep.argtypes = [C.c_void_p, C.c_ulonglong]
+    family = "c5" if states < 4 else "c1"
+    got = []
+    for keep in (True, False):
+        net = DifferentiableNetwork.generate(family, num_nodes=nodes, states_lo=states, states_hi=states, seed=3)
+        if not keep:
+            lib.bp_diff_set_keep(net.h, 0)
+        got.append([gradient(net, 7, 3, log, 5) for log in (True, False)])
+        got[-1].append(gradient(net, 1, 3, True, 6))
+        net.close()
+    for a, b in zip(*got):
+        for x, y in zip(a, b):
+            assert same_bits(x, y)
+
+
+@pytest.mark.parametrize("nodes", [300, 5000])
+def test_a_gradient_that_is_given_up_is_made_up_for(lib, nodes):
+    from belief_network_wrapper import DifferentiableNetwork
+
+    print(f"gradient given up, {nodes} nodes", flush=True)
+    lib.bp_diff_set_keep.argtypes = [C.c_void_p, C.c_ulonglong]
+    lib.bp_diff_device.argtypes = [C.c_void_p]
+    lib.bp_diff_device.restype = C.c_void_p
+    lib.bp_resident_set_timeout.argtypes = [C.c_void_p, C.c_ulonglong]
+    net = DifferentiableNetwork.generate("c5", num_nodes=nodes)
+    lib.bp_diff_set_keep(net.h, 0)
+    want = gradient(net, 5, 2, True, 9)
+    net.close()
+    net = DifferentiableNetwork.generate("c5", num_nodes=nodes)
+    lib.bp_resident_set_timeout(lib.bp_diff_device(net.h), 0)
+    for _ in range(2):  # made up for on the device, then by launches
+        for x, y in zip(gradient(net, 5, 2, True, 9), want):
+            assert same_bits(x, y)
+    net.close()

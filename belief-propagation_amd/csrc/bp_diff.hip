@@ -2,12 +2,12 @@
  * bp_diff.hip -- differentiable loopy BP: the parameter -> table map, the
  * unrolled forward with checkpoints, and the hand-written adjoint.
  *
- * Parameters are the TABLEs of a network's CPT definitions.  k_tables
+ * Parameters are the TABLEs of a network's CPT definitions.  k_set_params
  * rebuilds every slot's pairwise table from them with the XMLBIF reader's
  * loop (src/bnf-xml-parser/xml-expression.c:384-400, restated in
  * bp_model.c): for parent state j and child state k, the sequential f32 sum
  * of the TABLE entries in the blocks of that parent's state, so the tables
- * are bit-identical to the reader's.  k_initial puts root priors into the
+ * are bit-identical to the reader's.  It also puts root priors into the
  * initial beliefs, as graph_set_node_state does (xml-expression.c:290-317).
  *
  * The forward is the loopy kernel in its FWD/FINIT modes: the node-centric
@@ -62,62 +62,182 @@ __global__ void k_copy(const float *__restrict__ src, float *__restrict__ dst, s
         dst[i] = src[i];
 }
 
-/* One thread per (parent record, child state k, parent state j):
- * J_fwd[j][k] = the sequential f32 sum of TABLE[k * slice + idx] over the
- * configurations idx in which the parent is in state j, in ascending idx
- * order -- the blocks of the reader's loop, in its order -- written to the
- * forward slot and, transposed, to the reverse slot.  Loads are issued eight
- * at a time ahead of the adds, which stay in order; no division per entry. */
-__global__ void k_tables(const float *__restrict__ P, const ParentRec *__restrict__ parents,
-                         const unsigned *__restrict__ par_def, const unsigned *__restrict__ def_tb,
-                         const unsigned *__restrict__ def_slice, float *__restrict__ J, unsigned nrec, unsigned S)
+/* The parameter kernels' share of work: whole definitions, whose tables fit
+ * in LDS together, or (BIG) some rows of one that is larger. */
+struct Piece {
+    unsigned def0, ndefs, row0, row1;
+};
+constexpr unsigned BIG = 0x80000000u;       /* in ndefs */
+constexpr unsigned PIECE_FLOATS = 4608;     /* table entries of a piece, or its parents' gradient entries */
+constexpr unsigned PIECE_DEFS = 128;
+constexpr int PIECE_THREADS = 256;
+
+struct DefInfo {
+    unsigned tb, slice, pbegin, pend, prior, rbegin; /* rbegin: the definition's first softmax row */
+    unsigned at;                                     /* its table's place in LDS; rows of slice | 1 floats */
+    unsigned pad;
+};
+
+/* A pairwise table entry: the sequential f32 sum of the TABLE entries of one
+ * child state whose configurations have the parent in one state, in
+ * ascending order -- the blocks of the reader's loop, in its order.  p is the
+ * first of them; `count` (a power of S, as every node has S states) lie in
+ * runs of `o`, one run in every o * S.  They are taken S at a time, which
+ * are S apart for o = 1 and adjacent otherwise, so that the place is carried
+ * along once per S entries; U times S loads are issued ahead of their adds. */
+template <int S, int U> __device__ __forceinline__ float table_sum(const float *p, unsigned count, unsigned o)
 {
-    size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (size_t)nrec * S * S)
-        return;
-    unsigned pr = (unsigned)(t / ((size_t)S * S)), kj = (unsigned)(t % ((size_t)S * S));
-    unsigned k = kj / S, j = kj % S;
-    ParentRec rec = parents[pr];
-    if (j >= rec.n_par)
-        return;
-    unsigned d = par_def[pr];
-    unsigned slice = def_slice[d], o = rec.offset, n = rec.n_par;
-    const float *T = P + def_tb[d] + (size_t)k * slice + (size_t)j * o;
-    unsigned cnt = slice / n; /* entries with the parent in state j */
     float acc = 0.0f;
-    /* entry m of the sum is T[(m / o) * n * o + m % o]; (hi, lo) = (m / o,
-     * m % o) is carried along instead of divided out */
-    unsigned hi = 0, lo = 0;
-    for (unsigned m0 = 0; m0 < cnt; m0 += 8) {
-        float v[8];
+    if (count < (unsigned)S || S == 1) {
+        acc += *p;
+        return acc;
+    }
+    const unsigned apart = o == 1 ? S : 1, run = o == 1 ? 1 : o / S, step = o == 1 ? 0 : S;
+    const unsigned jump = o == 1 ? S * S : o * (S - 1), groups = count / S;
+    unsigned left = run;
+    for (unsigned g = 0; g < groups; g += U) {
+        float v[U][S];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            v[u] = (m0 + u < cnt) ? T[(size_t)hi * n * o + lo] : 0.0f;
-            if (++lo == o) {
-                lo = 0;
-                ++hi;
+        for (int u = 0; u < U; ++u) {
+#pragma unroll
+            for (int i = 0; i < S; ++i)
+                v[u][i] = p[i * apart];
+            if (g + u + 1 < groups) {
+                p += step;
+                if (--left == 0) {
+                    left = run;
+                    p += jump;
+                }
             }
         }
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
-            if (m0 + u < cnt)
-                acc += v[u];
+        for (int u = 0; u < U; ++u)
+            if (g + u < groups)
+#pragma unroll
+                for (int i = 0; i < S; ++i)
+                    acc += v[u][i];
     }
-    size_t SS = (size_t)S * S;
-    J[rec.slot_f * SS + j * S + k] = acc;
-    if (rec.slot_r != NONE)
-        J[rec.slot_r * SS + k * S + j] = acc;
+    return acc;
 }
 
-__global__ void k_initial(const float *__restrict__ P, const unsigned *__restrict__ prior_tb,
-                          const float *__restrict__ base, float *__restrict__ st0, unsigned V, unsigned S, unsigned SP)
+template <int S>
+__device__ __forceinline__ void put_table_entry(float *J, const ParentRec &rec, unsigned k, unsigned j, float x)
 {
-    size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (size_t)V * SP)
+    J[(size_t)rec.slot_f * (S * S) + j * S + k] = x;
+    if (rec.slot_r != NONE)
+        J[(size_t)rec.slot_r * (S * S) + k * S + j] = x;
+}
+
+/* Parameters to tables and initial beliefs.  P is theta, or (LOG) its
+ * softmax over each row (a definition's child states under one parent
+ * configuration); J_fwd[j][k] of each parent record is table_sum's, written
+ * to the forward slot and, transposed, to the reverse slot; a root's prior
+ * becomes its initial belief.
+ *
+ * Bound by reading theta and writing P once each.  P stays in LDS between
+ * the two halves: sums that read it from memory eight entries at a time were
+ * chains of a dozen and more round trips for a node with six parents (210k
+ * definitions of 3 states, 21.6M parameters: softmax 71 us, sums 129, priors
+ * 4; now 72 in all, 2.6 TB/s of theta, P and tables).  A row per thread, four at a time: consecutive threads read
+ * consecutive floats, in runs of a definition's slice; its rows are an odd
+ * number of floats apart in LDS, or all child states of a table would share
+ * a bank for two and four states. */
+template <int S, bool LOG>
+__global__ __launch_bounds__(PIECE_THREADS) void k_set_params(const float *__restrict__ theta,
+                                                              const Piece *__restrict__ pieces,
+                                                              const DefInfo *__restrict__ defs,
+                                                              const unsigned short *__restrict__ row_def,
+                                                              const ParentRec *__restrict__ parents,
+                                                              const unsigned *__restrict__ par_def,
+                                                              float *__restrict__ P, float *__restrict__ J,
+                                                              float *__restrict__ st0, unsigned SP)
+{
+    constexpr int U = S <= 4 ? 4 : 1;
+    constexpr unsigned SS = (unsigned)S * S;
+    __shared__ float table[PIECE_FLOATS];
+    __shared__ DefInfo def[PIECE_DEFS];
+    const Piece c = pieces[blockIdx.x];
+    const unsigned nd = c.ndefs & ~BIG, tid = threadIdx.x;
+    const bool big = c.ndefs & BIG;
+    for (unsigned d = tid; d < nd; d += PIECE_THREADS)
+        def[d] = defs[c.def0 + d];
+    __syncthreads();
+    for (unsigned r0 = c.row0 + tid; r0 < c.row1; r0 += U * PIECE_THREADS) {
+        float v[U][S];
+        unsigned first[U], slice[U], at[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            unsigned r = r0 + u * PIECE_THREADS;
+            r = r < c.row1 ? r : r0;
+            const DefInfo &di = def[row_def[r]];
+            slice[u] = di.slice;
+            first[u] = di.tb + (r - di.rbegin);
+            at[u] = di.at + (r - di.rbegin);
+#pragma unroll
+            for (int k = 0; k < S; ++k)
+                v[u][k] = theta[first[u] + k * slice[u]];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (r0 + u * PIECE_THREADS >= c.row1)
+                break;
+            if (LOG) {
+                float mx = -INFINITY, sum = 0.0f;
+#pragma unroll
+                for (int k = 0; k < S; ++k)
+                    mx = fmaxf(mx, v[u][k]);
+#pragma unroll
+                for (int k = 0; k < S; ++k) {
+                    v[u][k] = expf(v[u][k] - mx);
+                    sum += v[u][k];
+                }
+#pragma unroll
+                for (int k = 0; k < S; ++k)
+                    v[u][k] = v[u][k] / sum;
+            }
+#pragma unroll
+            for (int k = 0; k < S; ++k) {
+                P[first[u] + k * slice[u]] = v[u][k];
+                if (!big)
+                    table[at[u] + k * (slice[u] | 1)] = v[u][k];
+            }
+        }
+    }
+    if (big)
         return;
-    unsigned v = (unsigned)(t / SP), k = (unsigned)(t % SP);
-    unsigned tb = prior_tb[v];
-    st0[t] = (tb != NONE && k < S) ? P[tb + k] : base[t];
+    __syncthreads();
+    const unsigned pb = def[0].pbegin, n = (def[nd - 1].pend - pb) * SS;
+    for (unsigned t = tid; t < n; t += PIECE_THREADS) {
+        const unsigned pr = pb + t / SS, kj = t % SS, k = kj / S, j = kj % S;
+        const ParentRec rec = parents[pr];
+        const DefInfo &di = def[par_def[pr] - c.def0];
+        const float *p = table + di.at + k * (di.slice | 1) + j * rec.offset;
+        put_table_entry<S>(J, rec, k, j, table_sum<S, S == 2 ? 4 : S == 3 ? 3 : S <= 5 ? 2 : 1>(p, di.slice / S, rec.offset));
+    }
+    for (unsigned d = tid; d < nd; d += PIECE_THREADS)
+        if (def[d].prior != NONE)
+#pragma unroll
+            for (int k = 0; k < S; ++k)
+                st0[(size_t)def[d].prior * SP + k] = table[def[d].at + k];
+}
+
+/* The table entries of definitions too large for a piece, from P in memory:
+ * the time is that of the longest sum's round trips, so 24 and more loads
+ * go out together. */
+template <int S>
+__global__ void k_big_tables(const unsigned *__restrict__ recs, unsigned nrecs, const DefInfo *__restrict__ defs,
+                             const ParentRec *__restrict__ parents, const unsigned *__restrict__ par_def,
+                             const float *__restrict__ P, float *__restrict__ J)
+{
+    constexpr unsigned SS = (unsigned)S * S;
+    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= (size_t)nrecs * SS)
+        return;
+    const unsigned pr = recs[t / SS], kj = (unsigned)(t % SS), k = kj / S, j = kj % S;
+    const ParentRec rec = parents[pr];
+    const DefInfo di = defs[par_def[pr]];
+    const float *p = P + di.tb + (size_t)k * di.slice + (size_t)j * rec.offset;
+    put_table_entry<S>(J, rec, k, j, table_sum<S, (23 + S) / S>(p, di.slice / S, rec.offset));
 }
 
 template <int S, int STEP0, int R>
@@ -155,151 +275,95 @@ __global__ void k_initial_grad(const float *__restrict__ part, const float *__re
         out[(size_t)v * SP + k] = (k < S) ? acc[k] : 0.0f;
 }
 
-/* G[pr][k][j] = dJ of the forward slot at [j][k] + dJ of the reverse slot at
- * [k][j]: everything a parameter entry of the definition gets through
- * parent record pr when that parent is in state j and the child in k */
-__global__ void k_parent_grad(const float *__restrict__ jbar, const ParentRec *__restrict__ parents,
-                              float *__restrict__ G, unsigned nrec, unsigned S)
+/* dL/dparams, or (LOG) dL/dtheta: the transpose of k_set_params.  Parent
+ * record pr of a definition gives each entry with its parent in state j and
+ * the child in k
+ *   G[pr][k][j] = dJ of the forward slot at [j][k] + of the reverse slot at [k][j],
+ * formed in LDS first.  An entry's gradient is the sum over the records, in
+ * order; they run from the definition's last GIVEN (offset 1) to its first,
+ * so j is a base-S digit of the configuration, from the lowest up.  A thread
+ * has a row, whose entries share the configuration, and for LOG sends it
+ * through the softmax's transpose dtheta = P (.) (dP - <P, dP>).
+ *
+ * Bound by reading P and writing the gradient once.  (As two launches with G
+ * in memory: 21 + 61 us for 21.6M parameters; now 55, 3.5 TB/s.) */
+template <int S, bool LOG>
+__global__ __launch_bounds__(PIECE_THREADS) void k_param_grad(const float *__restrict__ jbar,
+                                                              const Piece *__restrict__ pieces,
+                                                              const DefInfo *__restrict__ defs,
+                                                              const unsigned short *__restrict__ row_def,
+                                                              const ParentRec *__restrict__ parents,
+                                                              const float *__restrict__ dst0,
+                                                              const float *__restrict__ P, float *__restrict__ out,
+                                                              unsigned SP)
 {
-    size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    size_t SS = (size_t)S * S;
-    if (t >= (size_t)nrec * SS)
-        return;
-    unsigned pr = (unsigned)(t / SS), kj = (unsigned)(t % SS), k = kj / S, j = kj % S;
-    ParentRec rec = parents[pr];
-    float g = 0.0f;
-    if (j < rec.n_par) {
-        g = jbar[(size_t)rec.slot_f * SS + j * S + k];
+    constexpr int U = S <= 4 ? 2 : 1;
+    constexpr unsigned SS = (unsigned)S * S;
+    __shared__ float G[PIECE_FLOATS];
+    __shared__ DefInfo def[PIECE_DEFS];
+    const Piece c = pieces[blockIdx.x];
+    const unsigned nd = c.ndefs & ~BIG, tid = threadIdx.x;
+    for (unsigned d = tid; d < nd; d += PIECE_THREADS)
+        def[d] = defs[c.def0 + d];
+    const unsigned pb = defs[c.def0].pbegin, n = (defs[c.def0 + nd - 1].pend - pb) * SS;
+    for (unsigned t = tid; t < n; t += PIECE_THREADS) {
+        const unsigned kj = t % SS, k = kj / S, j = kj % S;
+        const ParentRec rec = parents[pb + t / SS];
+        float g = jbar[(size_t)rec.slot_f * SS + j * S + k];
         if (rec.slot_r != NONE)
             g = g + jbar[(size_t)rec.slot_r * SS + k * S + j];
+        G[t] = g;
     }
-    G[t] = g;
-}
-
-/* dL/dparam: the transpose of k_tables and k_initial, from the per-parent
- * sums G: parameter k * slice + idx of a definition gets, for each parent
- * record in order, G[record][k][j] with j that parent's state in
- * configuration idx.  Every node has S states, so a definition's records,
- * which run from its last GIVEN (offset 1) to its first, read the base-S
- * digits of idx from the lowest up: one division by the constant S per
- * record.  The G entries of up to eight records are loaded before any is
- * added. */
-struct DefInfo {
-    unsigned tb, slice, pbegin, pend, prior, rbegin, pad1, pad2; /* rbegin: the definition's first softmax row */
-};
-
-template <int S>
-__global__ void k_param_grad(const float *__restrict__ G, const float *__restrict__ dst0,
-                             const unsigned *__restrict__ def_of, const DefInfo *__restrict__ defs,
-                             float *__restrict__ out, unsigned num_params, unsigned SP)
-{
-    constexpr unsigned SS = (unsigned)S * S;
-    unsigned p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= num_params)
-        return;
-    DefInfo di = defs[def_of[p]];
-    unsigned local = p - di.tb;
-    unsigned k = local / di.slice, x = local - k * di.slice;
-    const float *Gk = G + k * S;
-    float g = 0.0f;
-    for (unsigned base = di.pbegin; base < di.pend; base += 8) {
-        float f[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            f[u] = 0.0f;
-            if (base + u < di.pend) {
-                unsigned q = x / (unsigned)S, j = x - q * (unsigned)S;
-                x = q;
-                f[u] = Gk[(size_t)(base + u) * SS + j];
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-            if (base + u < di.pend)
-                g = g + f[u];
-    }
-    if (di.prior != NONE)
-        g = g + dst0[(size_t)di.prior * SP + k];
-    out[p] = g;
-}
-
-/* dL/dtheta for the log-parameters directly: one thread per softmax row
- * (a definition's child states under one parent configuration cc).  Every
- * entry of the row has the same configuration, so its digits are formed
- * once; each entry's parameter gradient is k_param_grad's sum, in its
- * order, and the row then goes through the softmax's transpose
- * dtheta = P (.) (dP - <P, dP>) -- the same operations as k_param_grad
- * followed by k_softmax_back, without the parameter gradient in memory. */
-template <int S>
-__global__ void k_param_grad_log(const float *__restrict__ G, const float *__restrict__ dst0,
-                                 const unsigned *__restrict__ row_def, const DefInfo *__restrict__ defs,
-                                 const float *__restrict__ P, float *__restrict__ gtheta, unsigned nrows, unsigned SP)
-{
-    constexpr unsigned SS = (unsigned)S * S;
-    constexpr int U = (S <= 4) ? 8 : 4;
-    unsigned r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nrows)
-        return;
-    DefInfo di = defs[row_def[r]];
-    unsigned cc = r - di.rbegin, x = cc;
-    float g[S];
-#pragma unroll
-    for (int k = 0; k < S; ++k)
-        g[k] = 0.0f;
-    for (unsigned base = di.pbegin; base < di.pend; base += U) {
-        float f[U][S];
+    __syncthreads();
+    for (unsigned r0 = c.row0 + tid; r0 < c.row1; r0 += U * PIECE_THREADS) {
+        float pv[U][S], g[U][S];
+        unsigned first[U], slice[U];
+        const DefInfo *di[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            if (base + u < di.pend) {
-                unsigned q = x / (unsigned)S, j = x - q * (unsigned)S;
-                x = q;
-                const float *Gr = G + (size_t)(base + u) * SS + j;
+            unsigned r = r0 + u * PIECE_THREADS;
+            r = r < c.row1 ? r : r0;
+            di[u] = def + row_def[r];
+            slice[u] = di[u]->slice;
+            first[u] = di[u]->tb + (r - di[u]->rbegin);
+            if (LOG)
 #pragma unroll
                 for (int k = 0; k < S; ++k)
-                    f[u][k] = Gr[k * S];
-            }
+                    pv[u][k] = P[first[u] + k * slice[u]];
         }
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-            if (base + u < di.pend)
+        for (int u = 0; u < U; ++u) {
+            unsigned x = first[u] - di[u]->tb;
+            const float *Gd = G + (di[u]->pbegin - pb) * SS;
+#pragma unroll
+            for (int k = 0; k < S; ++k)
+                g[u][k] = 0.0f;
+            for (unsigned m = di[u]->pend - di[u]->pbegin; m; --m, Gd += SS) {
+                const unsigned q = x / (unsigned)S, j = x - q * (unsigned)S;
+                x = q;
 #pragma unroll
                 for (int k = 0; k < S; ++k)
-                    g[k] = g[k] + f[u][k];
-    }
-    if (di.prior != NONE)
+                    g[u][k] = g[u][k] + Gd[k * S + j];
+            }
+            if (di[u]->prior != NONE)
 #pragma unroll
-        for (int k = 0; k < S; ++k)
-            g[k] = g[k] + dst0[(size_t)di.prior * SP + k];
-    float pv[S], dot = 0.0f;
+                for (int k = 0; k < S; ++k)
+                    g[u][k] = g[u][k] + dst0[(size_t)di[u]->prior * SP + k];
+            if (LOG) {
+                float dot = 0.0f;
 #pragma unroll
-    for (int k = 0; k < S; ++k) {
-        pv[k] = P[di.tb + (size_t)k * di.slice + cc];
-        dot += pv[k] * g[k];
-    }
+                for (int k = 0; k < S; ++k)
+                    dot += pv[u][k] * g[u][k];
 #pragma unroll
-    for (int k = 0; k < S; ++k)
-        gtheta[di.tb + (size_t)k * di.slice + cc] = pv[k] * (g[k] - dot);
-}
-
-/* P = softmax of theta over each row (a definition's child states under
- * one parent configuration): entries first[r] + k * stride[r], k < S */
-__global__ void k_softmax(const float *__restrict__ theta, const unsigned *__restrict__ first,
-                          const unsigned *__restrict__ stride, float *__restrict__ P, unsigned nrows, unsigned S)
-{
-    unsigned r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nrows)
-        return;
-    unsigned f = first[r], st = stride[r];
-    float mx = -INFINITY;
-    for (unsigned k = 0; k < S; ++k)
-        mx = fmaxf(mx, theta[f + k * st]);
-    float e[MAX_STATES], sum = 0.0f;
-    for (unsigned k = 0; k < S; ++k) {
-        e[k] = expf(theta[f + k * st] - mx);
-        sum += e[k];
+                for (int k = 0; k < S; ++k)
+                    g[u][k] = pv[u][k] * (g[u][k] - dot);
+            }
+            if (r0 + u * PIECE_THREADS < c.row1)
+#pragma unroll
+                for (int k = 0; k < S; ++k)
+                    out[first[u] + k * slice[u]] = g[u][k];
+        }
     }
-    for (unsigned k = 0; k < S; ++k)
-        P[f + k * st] = e[k] / sum;
 }
 
 /* dst[i] = src[idx[i]] for rows of SP floats (between the caller's node
@@ -325,6 +389,21 @@ __global__ void k_slot_to_edge(const float *__restrict__ src, const unsigned *__
     dst[(size_t)slot_edge[s] * width + i] = src[t];
 }
 
+/* fn<states>(...) */
+#define FOR_STATES(states, fn, ...)                                                                              \
+    switch (states) {                                                                                            \
+    case 1: fn<1>(__VA_ARGS__); break;                                                                           \
+    case 2: fn<2>(__VA_ARGS__); break;                                                                           \
+    case 3: fn<3>(__VA_ARGS__); break;                                                                           \
+    case 4: fn<4>(__VA_ARGS__); break;                                                                           \
+    case 5: fn<5>(__VA_ARGS__); break;                                                                           \
+    case 6: fn<6>(__VA_ARGS__); break;                                                                           \
+    case 7: fn<7>(__VA_ARGS__); break;                                                                           \
+    case 8: fn<8>(__VA_ARGS__); break;                                                                           \
+    case 9: fn<9>(__VA_ARGS__); break;                                                                           \
+    case 10: fn<10>(__VA_ARGS__); break;                                                                         \
+    }
+
 inline unsigned blocks_for(size_t n, unsigned b = 256) { return (unsigned)((n + b - 1) / b); }
 
 } // namespace
@@ -337,18 +416,17 @@ struct bp_diff {
     std::vector<uint32_t> row_stride, row_len;
 
     unsigned *par_def = nullptr; /* definition of each parent record */
-    unsigned nrec = 0;
-    unsigned *prior_tb = nullptr;
     unsigned *out_off = nullptr, *out_slot = nullptr, *slot_pos = nullptr, *slot_edge = nullptr;
-    unsigned *def_of = nullptr, *def_tb = nullptr, *def_slice = nullptr, *def_pbegin = nullptr, *def_prior = nullptr;
-    DefInfo *defs = nullptr; /* the same per definition, packed for k_param_grad */
-    float *G = nullptr;      /* [nrec][S][S] per-parent gradient sums */
+    DefInfo *defs = nullptr;
     ParentRec *parents = nullptr;
+    Piece *pieces = nullptr;
+    unsigned npieces = 0;
+    unsigned short *row_def = nullptr; /* each softmax row's definition, from its piece's first */
+    unsigned *big_recs = nullptr;      /* records of definitions larger than a piece */
+    unsigned nbig = 0;
 
     float *P = nullptr;     /* parameters */
     unsigned *perm_d = nullptr, *inv_d = nullptr; /* node -> device node, device node -> node */
-    unsigned *row_first_d = nullptr, *row_stride_d = nullptr; /* softmax rows */
-    unsigned *row_def_d = nullptr;                            /* each softmax row's definition */
     float *st0 = nullptr;   /* initial beliefs */
     float *gin = nullptr;   /* dL/dbeliefs (copy) */
     float *gst[2] = {nullptr, nullptr};
@@ -408,8 +486,8 @@ extern "C" void bp_diff_free(bp_diff *x)
         (void)hipDeviceSynchronize();
     }
     diff_release_storage(x);
-    void *ps[] = {x->out_at, x->adj_chunk, x->defs, x->G, x->perm_d, x->inv_d, x->row_first_d, x->row_stride_d, x->row_def_d, x->par_def, x->prior_tb, x->out_off, x->out_slot, x->slot_pos, x->slot_edge, x->def_of, x->def_tb, x->def_slice,
-                  x->def_pbegin, x->def_prior, x->parents, x->P, x->st0, x->gin, x->gst[0], x->gst[1],
+    void *ps[] = {x->out_at, x->adj_chunk, x->defs, x->perm_d, x->inv_d, x->row_def, x->par_def, x->pieces, x->big_recs, x->out_off,
+                  x->out_slot, x->slot_pos, x->slot_edge, x->parents, x->P, x->st0, x->gin, x->gst[0], x->gst[1],
                   x->w[0], x->w[1], x->jbar, x->dst0p, x->dst0};
     for (void *p : ps)
         if (p)
@@ -473,6 +551,47 @@ static int diff_validate(const bp_bn *bn, unsigned npd, Graph_t g)
     return 0;
 }
 
+/* cut the definitions into pieces; sets their places in LDS.  Pieces are
+ * four times smaller where that gives the card twice as many as it has
+ * CUs. */
+static int build_pieces(bp_diff *x, std::vector<DefInfo> &defs)
+{
+    const unsigned S = x->S, SS = S * S, npd = (unsigned)defs.size();
+    const unsigned limit = x->num_params < 512 * PIECE_FLOATS ? PIECE_FLOATS / 4 : PIECE_FLOATS;
+    const unsigned big_rows = std::max(1u, limit / S);
+    std::vector<Piece> pieces;
+    std::vector<unsigned short> row_def(x->num_rows);
+    std::vector<unsigned> big_recs;
+    for (unsigned d = 0; d < npd;) {
+        unsigned floats = 0, recs = 0, e = d;
+        while (e < npd && e - d < PIECE_DEFS) {
+            const DefInfo &di = defs[e];
+            const size_t f = (size_t)S * (di.slice | 1), r = (size_t)(di.pend - di.pbegin) * SS;
+            if (f > PIECE_FLOATS || (e > d && (floats + f > limit || recs + r > PIECE_FLOATS)))
+                break;
+            defs[e].at = floats;
+            std::fill_n(row_def.begin() + di.rbegin, di.slice, (unsigned short)(e - d));
+            floats += (unsigned)f;
+            recs += (unsigned)r;
+            ++e;
+        }
+        if (e > d) {
+            pieces.push_back({d, e - d, defs[d].rbegin, defs[e - 1].rbegin + defs[e - 1].slice});
+            d = e;
+            continue;
+        }
+        const DefInfo &di = defs[d];
+        for (unsigned r = 0; r < di.slice; r += big_rows)
+            pieces.push_back({d, 1 | BIG, di.rbegin + r, di.rbegin + std::min(r + big_rows, di.slice)});
+        for (unsigned q = di.pbegin; q < di.pend; ++q)
+            big_recs.push_back(q);
+        ++d;
+    }
+    x->npieces = (unsigned)pieces.size();
+    x->nbig = (unsigned)big_recs.size();
+    return upload_vec(&x->pieces, pieces) || upload_vec(&x->row_def, row_def) || upload_vec(&x->big_recs, big_recs) ? -1 : 0;
+}
+
 static int diff_build(bp_diff *x, const bp_bn *bn, unsigned npd, Graph_t g)
 {
     bp_dev *d = x->d;
@@ -482,7 +601,7 @@ static int diff_build(bp_diff *x, const bp_bn *bn, unsigned npd, Graph_t g)
     /* replay the reader's edge emission: definitions in order, parents last
      * GIVEN first, forward edge then reverse edge unless the parent is
      * observed (bp_graph_add_cpt_edges) */
-    std::vector<unsigned> def_of(x->num_params), def_tb(npd), def_slice(npd), def_pbegin(npd + 1, 0), def_prior(npd, NONE);
+    std::vector<unsigned> def_tb(npd), def_slice(npd), def_pbegin(npd + 1, 0), def_prior(npd, NONE);
     std::vector<ParentRec> prs;
     std::vector<unsigned> par_def;
     unsigned e = 0;
@@ -496,8 +615,6 @@ static int diff_build(bp_diff *x, const bp_bn *bn, unsigned npd, Graph_t g)
         def_tb[dd] = (unsigned)t0;
         unsigned slice = (unsigned)((t1 - t0) / nch);
         def_slice[dd] = slice;
-        for (uint64_t p = t0; p < t1; ++p)
-            def_of[p] = dd;
         unsigned offset = 1;
         for (uint64_t pi = g1; pi-- > g0;) {
             unsigned parent = bn->def_given[pi];
@@ -528,16 +645,14 @@ static int diff_build(bp_diff *x, const bp_bn *bn, unsigned npd, Graph_t g)
         return -1;
     }
     /* initial beliefs: the last GIVEN-less definition of a node sets them */
-    std::vector<unsigned> state_def(V, NONE), prior_tb(V, NONE);
+    std::vector<unsigned> state_def(V, NONE);
     for (unsigned dd = 0; dd < bn->num_defs; ++dd)
         if (bn->def_given_begin[dd + 1] == bn->def_given_begin[dd])
             state_def[bn->def_for[dd]] = dd;
     /* per device node (the handle numbers nodes in its own order) */
     for (unsigned v = 0; v < V; ++v)
-        if (state_def[v] != NONE && state_def[v] < npd) {
-            prior_tb[d->perm[v]] = def_tb[state_def[v]];
+        if (state_def[v] != NONE && state_def[v] < npd)
             def_prior[state_def[v]] = d->perm[v];
-        }
     std::vector<DefInfo> definfo(npd);
     for (unsigned dd = 0; dd < npd; ++dd)
         definfo[dd] = DefInfo{def_tb[dd], def_slice[dd], def_pbegin[dd], def_pbegin[dd + 1], def_prior[dd], 0, 0, 0};
@@ -549,24 +664,17 @@ static int diff_build(bp_diff *x, const bp_bn *bn, unsigned npd, Graph_t g)
     x->row_first.clear();
     x->row_stride.clear();
     x->row_len.clear();
-    std::vector<unsigned> row_def;
     for (unsigned dd = 0; dd < npd; ++dd) {
         unsigned nch = bn->num_states[bn->def_for[dd]];
         for (unsigned cc = 0; cc < def_slice[dd]; ++cc) {
             x->row_first.push_back((uint64_t)def_tb[dd] + cc);
             x->row_stride.push_back(def_slice[dd]);
             x->row_len.push_back(nch);
-            row_def.push_back(dd);
         }
     }
     x->num_rows = (unsigned)x->row_first.size();
-    {
-        std::vector<unsigned> rf(x->row_first.begin(), x->row_first.end());
-        if (upload_vec(&x->row_first_d, rf) || upload_vec(&x->row_stride_d, x->row_stride) ||
-            upload_vec(&x->row_def_d, row_def))
-            return -1;
-    }
-    x->nrec = (unsigned)prs.size();
+    if (build_pieces(x, definfo))
+        return -1;
     /* source-grouped slots */
     std::vector<unsigned> out_off(V + 1, 0), out_slot(E), slot_src(E);
     for (unsigned s = 0; s < E; ++s) {
@@ -599,13 +707,10 @@ static int diff_build(bp_diff *x, const bp_bn *bn, unsigned npd, Graph_t g)
             return -1;
     }
     size_t VS = (size_t)V * d->SP, ES = (size_t)E * d->SP;
-    if (upload_vec(&x->perm_d, d->perm) || upload_vec(&x->inv_d, d->inv) || upload_vec(&x->prior_tb, prior_tb) ||
+    if (upload_vec(&x->perm_d, d->perm) || upload_vec(&x->inv_d, d->inv) ||
         upload_vec(&x->out_off, out_off) ||
         upload_vec(&x->out_slot, out_slot) || upload_vec(&x->slot_pos, slot_pos) || upload_vec(&x->slot_edge, d->slot_edge) ||
-        upload_vec(&x->def_of, def_of) || upload_vec(&x->def_tb, def_tb) || upload_vec(&x->def_slice, def_slice) ||
-        upload_vec(&x->def_pbegin, def_pbegin) || upload_vec(&x->def_prior, def_prior) ||
-        upload_vec(&x->defs, definfo) || dmalloc(&x->G, std::max<size_t>((size_t)prs.size() * S * S, 1)) ||
-        upload_vec(&x->parents, prs) || upload_vec(&x->par_def, par_def) || dmalloc(&x->P, x->num_params) ||
+        upload_vec(&x->defs, definfo) || upload_vec(&x->parents, prs) || upload_vec(&x->par_def, par_def) || dmalloc(&x->P, x->num_params) ||
         dmalloc(&x->st0, VS) || dmalloc(&x->gin, VS) || dmalloc(&x->gst[0], VS) || dmalloc(&x->gst[1], VS) ||
         dmalloc(&x->w[0], ES) || dmalloc(&x->w[1], ES) || dmalloc(&x->jbar, (size_t)E * S * S) ||
         dmalloc(&x->dst0p, VS) || dmalloc(&x->dst0, VS))
@@ -652,6 +757,15 @@ extern "C" int bp_diff_create(const bp_bn *bn, unsigned int num_param_defs, int 
         for (unsigned v = 0; v < x->V; ++v)
             x->max_in = std::max(x->max_in, x->d->in_off_h[v + 1] - x->d->in_off_h[v]);
         rc = diff_build(x, bn, num_param_defs, g);
+        /* nodes without a parameter prior keep their initial beliefs */
+        if (rc == 0 && x->V &&
+            hipMemcpyAsync(x->st0, x->d->states0, (size_t)x->V * x->SP * sizeof(float), hipMemcpyDeviceToDevice,
+                           x->d->stream) != hipSuccess) {
+            bp_set_error("bp_diff_create: copying the initial beliefs failed");
+            rc = -1;
+        }
+        if (rc == 0 && hipStreamSynchronize(x->d->stream) != hipSuccess)
+            rc = -1;
         if (rc == 0 && bp_resident_diff_fits(x->d, x->max_in) &&
             (dmalloc(&x->out_at, x->E) || bp_resident_diff_places(x->d, x->slot_pos, x->out_at)))
             rc = -1;
@@ -692,56 +806,40 @@ extern "C" int bp_diff_rows(const bp_diff *x, uint64_t *row_first, uint32_t *row
     return 0;
 }
 
-extern "C" int bp_diff_set_params(bp_diff *x, const float *params, void *stream)
+template <int S> static void launch_set_params(bp_diff *x, bool log, const float *theta, hipStream_t st)
+{
+    if (x->npieces)
+        hipLaunchKernelGGL((log ? k_set_params<S, true> : k_set_params<S, false>), dim3(x->npieces),
+                           dim3(PIECE_THREADS), 0, st, theta, x->pieces, x->defs, x->row_def, x->parents, x->par_def,
+                           x->P, x->d->J, x->st0, x->SP);
+    if (x->nbig)
+        hipLaunchKernelGGL(k_big_tables<S>, dim3(blocks_for((size_t)x->nbig * S * S, 64)), dim3(64), 0, st,
+                           x->big_recs, x->nbig, x->defs, x->parents, x->par_def, x->P, x->d->J);
+}
+
+static int set_params(bp_diff *x, bool log, const float *theta, const char *who, void *stream)
 {
     bp_clear_error();
-    if (!x || !params) {
-        bp_set_error("bp_diff_set_params: NULL argument");
+    if (!x || !theta) {
+        bp_set_error("%s: NULL argument", who);
         return -1;
     }
-    hipStream_t st = (hipStream_t)stream;
     HIP_TRY(hipSetDevice(x->d->device));
-    if (x->num_params)
-        hipLaunchKernelGGL(k_copy, dim3(blocks_for(x->num_params)), dim3(256), 0, st, params, x->P,
-                           (size_t)x->num_params);
-    size_t nT = (size_t)x->nrec * x->S * x->S;
-    if (nT)
-        hipLaunchKernelGGL(k_tables, dim3(blocks_for(nT)), dim3(256), 0, st, x->P, x->parents, x->par_def, x->def_tb,
-                           x->def_slice, x->d->J, x->nrec, x->S);
-    size_t VS = (size_t)x->V * x->SP;
-    if (VS)
-        hipLaunchKernelGGL(k_initial, dim3(blocks_for(VS)), dim3(256), 0, st, x->P, x->prior_tb, x->d->states0,
-                           x->st0, x->V, x->S, x->SP);
+    FOR_STATES(x->S, launch_set_params, x, log, theta, (hipStream_t)stream);
     HIP_TRY(hipGetLastError());
     x->have_params = true;
     x->have_forward = false;
     return 0;
 }
 
+extern "C" int bp_diff_set_params(bp_diff *x, const float *params, void *stream)
+{
+    return set_params(x, false, params, "bp_diff_set_params", stream);
+}
+
 extern "C" int bp_diff_set_log_params(bp_diff *x, const float *theta, void *stream)
 {
-    bp_clear_error();
-    if (!x || !theta) {
-        bp_set_error("bp_diff_set_log_params: NULL argument");
-        return -1;
-    }
-    hipStream_t st = (hipStream_t)stream;
-    HIP_TRY(hipSetDevice(x->d->device));
-    if (x->num_rows)
-        hipLaunchKernelGGL(k_softmax, dim3(blocks_for(x->num_rows)), dim3(256), 0, st, theta, x->row_first_d,
-                           x->row_stride_d, x->P, x->num_rows, x->S);
-    size_t nT = (size_t)x->nrec * x->S * x->S;
-    if (nT)
-        hipLaunchKernelGGL(k_tables, dim3(blocks_for(nT)), dim3(256), 0, st, x->P, x->parents, x->par_def, x->def_tb,
-                           x->def_slice, x->d->J, x->nrec, x->S);
-    size_t VS = (size_t)x->V * x->SP;
-    if (VS)
-        hipLaunchKernelGGL(k_initial, dim3(blocks_for(VS)), dim3(256), 0, st, x->P, x->prior_tb, x->d->states0,
-                           x->st0, x->V, x->S, x->SP);
-    HIP_TRY(hipGetLastError());
-    x->have_params = true;
-    x->have_forward = false;
-    return 0;
+    return set_params(x, true, theta, "bp_diff_set_log_params", stream);
 }
 
 static int diff_storage(bp_diff *x, unsigned K, unsigned c)
@@ -942,7 +1040,6 @@ static void adj_step(bp_diff *x, int step0, const float *st_prev, const float *s
 }
 
 static void enqueue_backward_tail(bp_diff *x, const float *w0, hipStream_t st);
-static void enqueue_parent_grad(bp_diff *x, hipStream_t st);
 
 static void enqueue_backward(bp_diff *x, hipStream_t st)
 {
@@ -979,82 +1076,25 @@ static void enqueue_backward(bp_diff *x, hipStream_t st)
 }
 
 /* dL/d(initial beliefs) and the per-parent sums */
+template <int S> static void launch_initial_grad(bp_diff *x, const float *w0, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_initial_grad<S>, dim3(blocks_for(x->V)), dim3(256), 0, st, x->dst0p, w0, x->out_off,
+                       x->out_slot, x->dst0, x->V);
+}
+
 static void enqueue_backward_tail(bp_diff *x, const float *w0, hipStream_t st)
 {
-    dim3 gv(blocks_for(x->V)), b256(256);
-#define BP_IG_CASE(SS)                                                                                     \
-    case SS:                                                                                               \
-        hipLaunchKernelGGL(k_initial_grad<SS>, gv, b256, 0, st, x->dst0p, w0, x->out_off, x->out_slot,     \
-                           x->dst0, x->V);                                                                 \
-        break;
-    switch (x->S) {
-        BP_IG_CASE(1)
-        BP_IG_CASE(2)
-        BP_IG_CASE(3)
-        BP_IG_CASE(4)
-        BP_IG_CASE(5)
-        BP_IG_CASE(6)
-        BP_IG_CASE(7)
-        BP_IG_CASE(8)
-        BP_IG_CASE(9)
-        BP_IG_CASE(10)
-    }
-#undef BP_IG_CASE
-    enqueue_parent_grad(x, st);
+    FOR_STATES(x->S, launch_initial_grad, x, w0, st);
 }
 
-static void enqueue_parent_grad(bp_diff *x, hipStream_t st)
+/* The gradient of the parameters or (log) of the log-parameters from the
+ * tables' and initial beliefs' of the last backward. */
+template <int S> static void launch_param_grad(bp_diff *x, bool log, float *out, hipStream_t st)
 {
-    size_t nG = (size_t)x->nrec * x->S * x->S;
-    if (nG)
-        hipLaunchKernelGGL(k_parent_grad, dim3(blocks_for(nG)), dim3(256), 0, st, x->jbar, x->parents, x->G, x->nrec,
-                           x->S);
-}
-
-/* The gradient of the parameters (log = 0: dL/dparams into out) or of the
- * log-parameters (log = 1: dL/dtheta, the softmax's transpose folded in),
- * from the per-parent sums of the last backward. */
-static void launch_param_grad(bp_diff *x, int log, float *out, hipStream_t st)
-{
-    if (log && x->num_rows) {
-        switch (x->S) {
-#define BP_PGL_CASE(SS)                                                                                          \
-    case SS:                                                                                                     \
-        hipLaunchKernelGGL(k_param_grad_log<SS>, dim3(blocks_for(x->num_rows)), dim3(256), 0, st, x->G, x->dst0,  \
-                           x->row_def_d, x->defs, x->P, out, x->num_rows, x->SP);                                \
-        break;
-            BP_PGL_CASE(1)
-            BP_PGL_CASE(2)
-            BP_PGL_CASE(3)
-            BP_PGL_CASE(4)
-            BP_PGL_CASE(5)
-            BP_PGL_CASE(6)
-            BP_PGL_CASE(7)
-            BP_PGL_CASE(8)
-            BP_PGL_CASE(9)
-            BP_PGL_CASE(10)
-#undef BP_PGL_CASE
-        }
-    } else if (!log && x->num_params) {
-        switch (x->S) {
-#define BP_PG_CASE(SS)                                                                                        \
-    case SS:                                                                                                  \
-        hipLaunchKernelGGL(k_param_grad<SS>, dim3(blocks_for(x->num_params)), dim3(256), 0, st, x->G, x->dst0, \
-                           x->def_of, x->defs, out, x->num_params, x->SP);                                     \
-        break;
-            BP_PG_CASE(1)
-            BP_PG_CASE(2)
-            BP_PG_CASE(3)
-            BP_PG_CASE(4)
-            BP_PG_CASE(5)
-            BP_PG_CASE(6)
-            BP_PG_CASE(7)
-            BP_PG_CASE(8)
-            BP_PG_CASE(9)
-            BP_PG_CASE(10)
-#undef BP_PG_CASE
-        }
-    }
+    if (x->npieces)
+        hipLaunchKernelGGL((log ? k_param_grad<S, true> : k_param_grad<S, false>), dim3(x->npieces),
+                           dim3(PIECE_THREADS), 0, st, x->jbar, x->pieces, x->defs, x->row_def, x->parents, x->dst0,
+                           x->P, out, x->SP);
 }
 
 extern "C" int bp_diff_backward_ex(bp_diff *x, const float *grad_beliefs, float *grad_params, float *grad_tables,
@@ -1080,7 +1120,6 @@ extern "C" int bp_diff_backward_ex(bp_diff *x, const float *grad_beliefs, float 
                                     x->out_at, x->rows};
         if (bp_resident_diff_backward(x->d, x->K, x->ck_st, x->ck_buf, x->stride, arrays, st))
             return -1;
-        enqueue_parent_grad(x, st);
     } else {
         if (x->kept) /* the launches look for the last beliefs here */
             hipLaunchKernelGGL(k_copy, dim3(blocks_for(VS)), dim3(256), 0, st, x->ck_st + x->K * x->stride,
@@ -1099,7 +1138,7 @@ extern "C" int bp_diff_backward_ex(bp_diff *x, const float *grad_beliefs, float 
         HIP_TRY(hipGraphLaunch(it->second, st));
     }
     if (grad_params)
-        launch_param_grad(x, 0, grad_params, st);
+        FOR_STATES(x->S, launch_param_grad, x, false, grad_params, st);
     size_t SS = (size_t)x->S * x->S;
     if (grad_tables && x->E)
         hipLaunchKernelGGL(k_slot_to_edge, dim3(blocks_for((size_t)x->E * SS)), dim3(256), 0, st, x->jbar,
@@ -1124,7 +1163,7 @@ extern "C" int bp_diff_backward_log(bp_diff *x, const float *grad_beliefs, float
     }
     if (bp_diff_backward_ex(x, grad_beliefs, nullptr, nullptr, nullptr, stream))
         return -1;
-    launch_param_grad(x, 1, grad_theta, (hipStream_t)stream);
+    FOR_STATES(x->S, launch_param_grad, x, true, grad_theta, (hipStream_t)stream);
     HIP_TRY(hipGetLastError());
     return 0;
 }

@@ -256,3 +256,101 @@ def test_full_scale_c5(lib):
         print(f"directional derivative: fd {fd:.8f}, adjoint {gr @ v.numpy():.8f}", flush=True)
         assert abs(fd - gr @ v.numpy()) <= 5e-3 * max(1.0, abs(fd))
     teardown(lib, bn, g, net)
+
+
+# (states, parents, nodes): tables of every size around what the parameter
+# kernels take in one piece (4,608 entries, 128 definitions), odd remainders,
+# and definitions that are split
+PARAM_CASES = [(1, (0, 4), 300), (2, (0, 0), 1000), (2, (0, 5), 400), (2, (10, 11), 60), (2, (12, 12), 40),
+               (3, (0, 3), 501), (3, (6, 7), 40), (4, (0, 4), 200), (4, (5, 6), 30), (5, (0, 3), 100), (5, (4, 5), 20),
+               (6, (2, 4), 40), (7, (1, 3), 50), (8, (1, 4), 30), (9, (0, 3), 60), (9, (3, 4), 12)]
+
+
+@pytest.mark.parametrize("states,parents,nodes", PARAM_CASES)
+def test_parameter_maps(lib, states, parents, nodes):
+    """Parameters to tables and initial beliefs, and the gradients back,
+    against the same f32 sums in numpy (bit for bit) and, for the softmax, in
+    float64: every operation of a row's n = states + parents + 16 rounds
+    once, so entries agree to n ulp of the sums of magnitudes."""
+    print(f"parameters {states} states {parents} parents {nodes} nodes", flush=True)
+    bn, A, g, G, net = setup("c5", num_nodes=nodes, states_lo=states, states_hi=states, indegree_dist=0,
+                             indeg_lo=parents[0], indeg_hi=parents[1], max_children=40)
+    S, E, npd = net.S, net.E, net.num_param_defs
+    rng = np.random.default_rng(states * 100 + parents[1])
+    P = torch.tensor(A["table"][: net.num_params], device="cuda")
+    K = 2
+    b0 = net.beliefs(P, 0, 1).cpu().numpy()
+    assert np.array_equal(b0.view(np.uint32), B.states(g)[:, :S].copy().view(np.uint32))
+    J = G["edges_J"].reshape(E, 10, 10)[:, :S, :S]
+
+    def back(gt, gi):
+        """the tables' and initial beliefs' gradients, summed per parameter, and the sums of magnitudes"""
+        out, mag, e = np.zeros(net.num_params, np.float32), np.zeros(net.num_params), 0
+        last = {}
+        for d in range(len(A["def_for"])):
+            if A["given_begin"][d + 1] == A["given_begin"][d]:
+                last[A["def_for"][d]] = d
+        for d in range(npd):
+            t0, t1 = int(A["table_begin"][d]), int(A["table_begin"][d + 1])
+            cc, o = np.arange((t1 - t0) // S), 1
+            acc, m = np.zeros((S, len(cc)), np.float32), np.zeros((S, len(cc)))
+            for parent in A["given"][int(A["given_begin"][d]): int(A["given_begin"][d + 1])][::-1]:
+                x = gt[e].reshape(S, S).T.copy()
+                e += 1
+                if not G["observed"][parent]:
+                    x = x + gt[e].reshape(S, S)
+                    e += 1
+                acc = acc + x[:, cc // o % S]
+                m += np.abs(x[:, cc // o % S])
+                o *= S
+            child = A["def_for"][d]
+            if last.get(child) == d:
+                acc = acc + gi[child, :S, None]
+                m += np.abs(gi[child, :S, None])
+            out[t0:t1], mag[t0:t1] = acc.ravel(), m.ravel()
+        assert e == E
+        return out, mag
+
+    for log in (False, True):
+        theta = torch.tensor(rng.standard_normal(net.num_params).astype(np.float32), device="cuda")
+        if log:
+            net._set_log_params(theta)
+        else:
+            net._set_params(P)
+            assert np.array_equal(net.tables_host().view(np.uint32), J.copy().view(np.uint32))
+        net._forward(K, 1)
+        gb = torch.tensor(rng.standard_normal((net.V, net.stride)).astype(np.float32), device="cuda")
+        gb[:, S:] = 0
+        gp, gt, gi = net._backward(gb, True, True)
+        gt, gi = gt.cpu().numpy(), gi.cpu().numpy()
+        want, mag = back(gt, gi)
+        assert np.array_equal(gp.cpu().numpy().view(np.uint32), want.view(np.uint32))
+        if not log:
+            continue
+        got = net._backward_log(gb).cpu().numpy()
+        rows = net._rows.cpu().numpy()
+        th = theta.cpu().numpy().astype(np.float64)[rows]
+        p = np.exp(th - th.max(1, keepdims=True))
+        p /= p.sum(1, keepdims=True)
+        w = want.astype(np.float64)[rows]
+        ref = p * (w - (p * w).sum(1, keepdims=True))
+        n = S + parents[1] + 16
+        bound = n * 2.0**-23 * (p * (mag[rows] + (p * mag[rows]).sum(1, keepdims=True)))
+        assert np.all(np.abs(got[rows] - ref) <= bound + 1e-44)
+        # the tables from the softmax, against sums in float64 of its exact entries
+        flat = np.zeros(net.num_params)
+        flat[rows] = p
+        e, tables = 0, net.tables_host()
+        for d in range(npd):
+            t0, t1 = int(A["table_begin"][d]), int(A["table_begin"][d + 1])
+            T, o = flat[t0:t1].reshape(S, -1), 1
+            for parent in A["given"][int(A["given_begin"][d]): int(A["given_begin"][d + 1])][::-1]:
+                x = T.reshape(S, -1, S, o).sum((1, 3))
+                tol = (T.shape[1] // S + n) * 2.0**-23 * x
+                assert np.all(np.abs(tables[e].T - x) <= tol)
+                e += 1
+                if not G["observed"][parent]:
+                    assert np.all(np.abs(tables[e] - x) <= tol)
+                    e += 1
+                o *= S
+    teardown(lib, bn, g, net)

@@ -43,6 +43,7 @@ using namespace bpk;
 #ifndef BP_TREE_WAVE_BLOCK
 #define BP_TREE_WAVE_BLOCK 64
 #endif
+static_assert(BP_TREE_SMALL_WAVE <= BP_TREE_SMALL_BLOCK, "a thread for each node of a small sub-wave");
 static_assert(BP_TREE_WAVE_BLOCK >= 64 && BP_TREE_WAVE_BLOCK <= 256, "k_tree_wave is bounded to 256 threads");
 constexpr unsigned WAVE_BLOCK = BP_TREE_WAVE_BLOCK;
 constexpr unsigned SMALL_WAVE = BP_TREE_SMALL_WAVE;
@@ -80,62 +81,114 @@ struct TreeArgs {
     const unsigned char *wave_start;  /* [waves] 1: a start wave (sends from the node's own state) */
 };
 
-template <int S, bool MIXED>
-__device__ __forceinline__ void tree_entry(const TreeArgs &a, unsigned entry, int start)
+/* Messages sent together: their slots' numbers, then their tables, are
+ * loaded ahead of the product they wait for.  (One after the other, each
+ * was two dependent reads and a store that the next could not pass: 14
+ * children of a node took 14 times 1 us, and a wave waits for its longest.
+ * A run's kernels: 1M-node tree 240 us, 162 now; 10k-node tree 88 us, 54
+ * now, of which some 2.5 us for each small wave and 4.5 for each launch, two
+ * dependent reads that miss the caches and the stores.) */
+template <int S> struct Sends {
+    static constexpr int value = S <= 2 ? 4 : S <= 3 ? 3 : S <= 4 ? 2 : 1;
+};
+
+template <int S> struct TreeWork {
+    static constexpr int A = Sends<S>::value;
+    uint4 lo, hi;      /* the entry */
+    unsigned slot[A];
+    float J[A][S * S];
+    unsigned xy[A];
+};
+
+template <int S> __device__ __forceinline__ void tree_load(const TreeArgs &a, unsigned entry, TreeWork<S> &w)
 {
-    constexpr int SP = Stride<S>::value;
     const uint4 *e4 = reinterpret_cast<const uint4 *>(a.ent + entry);
-    uint4 lo = e4[0], hi = e4[1];
-    unsigned v = lo.x, in_b = lo.y, in_e = lo.z, act_b = lo.w, act_e = hi.x;
-    unsigned n = MIXED ? hi.y : (unsigned)S;
-    float buf[S], m[S];
-    if (start) {
+    w.lo = e4[0];
+    w.hi = e4[1];
+}
+
+/* the slots of its sends from q on (stand-ins past the last) */
+template <int S> __device__ __forceinline__ void tree_slots(const TreeArgs &a, unsigned q, TreeWork<S> &w)
+{
 #pragma unroll
-        for (int k = 0; k < S; ++k)
-            buf[k] = a.states[(size_t)v * SP + k];
-    } else {
+    for (int u = 0; u < TreeWork<S>::A; ++u)
+        w.slot[u] = a.act_slot[q + u < w.hi.x ? q + u : q];
+}
+
+template <int S, bool MIXED> __device__ __forceinline__ void tree_tables(const TreeArgs &a, TreeWork<S> &w)
+{
+    unsigned at[TreeWork<S>::A];
 #pragma unroll
-        for (int k = 0; k < S; ++k)
-            buf[k] = (!MIXED || (unsigned)k < n) ? 1.0f : 0.0f;
-        unsigned s = in_b;
-        /* four rows loaded before they are combined (in slot order), so a
-         * node's in-messages are fetched together instead of one latency each */
-        for (; s + 4 <= in_e; s += 4) {
-            float m4[4][S];
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-#pragma unroll
-                for (int k = 0; k < S; ++k)
-                    m4[j][k] = a.msg[(size_t)(s + j) * SP + k];
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                combine<S, MIXED>(buf, m4[j], n);
-        }
-        for (; s < in_e; ++s) {
-#pragma unroll
-            for (int k = 0; k < S; ++k)
-                m[k] = a.msg[(size_t)s * SP + k];
-            combine<S, MIXED>(buf, m, n);
+    for (int u = 0; u < TreeWork<S>::A; ++u) {
+        if constexpr (MIXED) {
+            w.xy[u] = a.slot_xy[w.slot[u]];
+            at[u] = a.slot_tab[w.slot[u]];
         }
     }
-    for (unsigned q = act_b; q < act_e; ++q) {
-        unsigned s = a.act_slot[q];
-        unsigned x = S, y = S;
-        if (MIXED) {
-            unsigned xy = a.slot_xy[s];
-            x = xy & 15u;
-            y = xy >> 4;
-        }
-        if constexpr (MIXED) {
-            float Jd[S * S];
-            load_mixed_rows<S>(a.J + a.slot_tab[s], Jd);
-            send_padded<S>(Jd, buf, x, y, m);
-        } else {
-            send<S, MIXED>(a.J + (size_t)s * S * S, buf, x, y, m);
-        }
+#pragma unroll
+    for (int u = 0; u < TreeWork<S>::A; ++u) {
+        if constexpr (MIXED)
+            load_mixed_rows<S>(a.J + at[u], w.J[u]);
+        else
+            load_row<S * S>(a.J + (size_t)w.slot[u] * S * S, w.J[u]);
+    }
+}
+
+/* what an entry sends: its state, or the product of its in-messages in slot
+ * order, eight rows (four of more than four states) loaded before they are
+ * combined */
+template <int S, bool MIXED>
+__device__ __forceinline__ void tree_product(const TreeArgs &a, const TreeWork<S> &w, int start, float *buf)
+{
+    constexpr int SP = Stride<S>::value;
+    constexpr int U = S <= 4 ? 8 : 4;
+    const unsigned v = w.lo.x, in_b = w.lo.y, in_e = w.lo.z, n = MIXED ? w.hi.y : (unsigned)S;
+    if (start) {
+        load_rowp<S, SP>(a.states + (size_t)v * SP, buf);
+        return;
+    }
+#pragma unroll
+    for (int k = 0; k < S; ++k)
+        buf[k] = (!MIXED || (unsigned)k < n) ? 1.0f : 0.0f;
+    for (unsigned s = in_b; s < in_e; s += U) {
+        float m[U][S];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            load_rowp<S, SP>(a.msg + (size_t)(s + u < in_e ? s + u : s) * SP, m[u]);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (s + u < in_e)
+                combine<S, MIXED>(buf, m[u], n);
+    }
+}
+
+template <int S, bool MIXED>
+__device__ __forceinline__ void tree_send(const TreeArgs &a, unsigned q, const TreeWork<S> &w, const float *buf)
+{
+    constexpr int SP = Stride<S>::value;
+#pragma unroll
+    for (int u = 0; u < TreeWork<S>::A; ++u) {
+        if (q + u >= w.hi.x)
+            break;
+        float m[S];
+        if constexpr (MIXED)
+            send_padded<S>(w.J[u], buf, w.xy[u] & 15u, w.xy[u] >> 4, m);
+        else
+            send<S, MIXED>(w.J[u], buf, S, S, m);
 #pragma unroll
         for (int k = 0; k < SP; ++k)
-            a.msg[(size_t)s * SP + k] = (k < S) ? m[k] : 0.0f;
+            a.msg[(size_t)w.slot[u] * SP + k] = (k < S) ? m[k] : 0.0f;
+    }
+}
+
+/* the sends after the first A */
+template <int S, bool MIXED>
+__device__ __forceinline__ void tree_other_sends(const TreeArgs &a, TreeWork<S> w, const float *buf)
+{
+    for (unsigned q = w.lo.w + TreeWork<S>::A; q < w.hi.x; q += TreeWork<S>::A) {
+        tree_slots(a, q, w);
+        tree_tables<S, MIXED>(a, w);
+        tree_send<S, MIXED>(a, q, w, buf);
     }
 }
 
@@ -144,21 +197,62 @@ template <int S, bool MIXED>
 __global__ __launch_bounds__(256) void k_tree_wave(TreeArgs a, unsigned begin, unsigned count, int start)
 {
     unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < count)
-        tree_entry<S, MIXED>(a, begin + i, start);
+    if (i >= count)
+        return;
+    TreeWork<S> w;
+    float buf[S];
+    tree_load(a, begin + i, w);
+    tree_slots(a, w.lo.w, w);
+    tree_tables<S, MIXED>(a, w);
+    tree_product<S, MIXED>(a, w, start, buf);
+    tree_send<S, MIXED>(a, w.lo.w, w, buf);
+    tree_other_sends<S, MIXED>(a, w, buf);
 }
 
-/* consecutive small sub-waves [w0, w1) in one workgroup: each wave's nodes,
- * then a workgroup barrier (which orders the messages one wave writes
- * before the next wave reads them) */
+/* Consecutive small sub-waves [w0, w1) in one workgroup, a thread for each
+ * of a wave's nodes (at most SMALL_WAVE = SMALL_BLOCK); the workgroup
+ * barrier orders the messages one wave writes before the next reads them.
+ * Only messages depend on the waves before: a wave's entries, and for up to
+ * four states its first tables, are read while the one before it runs. */
 template <int S, bool MIXED>
 __global__ __launch_bounds__(SMALL_BLOCK) void k_tree_waves_small(TreeArgs a, unsigned w0, unsigned w1)
 {
+    constexpr bool AHEAD = S <= 4;
+    TreeWork<S> now, next;
+    unsigned b = a.wave_begin[w0], e = a.wave_begin[w0 + 1];
+    bool have = b + threadIdx.x < e;
+    if (have) {
+        tree_load(a, b + threadIdx.x, now);
+        tree_slots(a, now.lo.w, now);
+        if constexpr (AHEAD)
+            tree_tables<S, MIXED>(a, now);
+    }
     for (unsigned w = w0; w < w1; ++w) {
-        unsigned b = a.wave_begin[w], e = a.wave_begin[w + 1];
-        int start = a.wave_start[w];
-        for (unsigned entry = b + threadIdx.x; entry < e; entry += blockDim.x)
-            tree_entry<S, MIXED>(a, entry, start);
+        const int start = a.wave_start[w];
+        const unsigned end = a.wave_begin[w + 1 < w1 ? w + 2 : w + 1];
+        const bool then = e + threadIdx.x < end;
+        float buf[S];
+        if (then)
+            tree_load(a, e + threadIdx.x, next);
+        if (have) {
+            if constexpr (!AHEAD && S < 9)
+                tree_tables<S, MIXED>(a, now);
+            tree_product<S, MIXED>(a, now, start, buf);
+            if constexpr (S >= 9) /* registers for one of the two */
+                tree_tables<S, MIXED>(a, now);
+        }
+        if (then)
+            tree_slots(a, next.lo.w, next);
+        if (have) {
+            tree_send<S, MIXED>(a, now.lo.w, now, buf);
+            tree_other_sends<S, MIXED>(a, now, buf);
+        }
+        if constexpr (AHEAD)
+            if (then)
+                tree_tables<S, MIXED>(a, next);
+        now = next;
+        have = then;
+        e = end;
         __syncthreads();
     }
 }
@@ -173,18 +267,22 @@ __global__ __launch_bounds__(256) void k_tree_marginalize(const unsigned *in_off
     if (v >= V)
         return;
     unsigned n = MIXED ? nvars[v] : S;
-    float t[S], m[S], st[S];
+    constexpr int U = S <= 4 ? 8 : 4; /* rows loaded before they are combined */
+    float t[S], st[S];
+    load_rowp<S, SP>(states + (size_t)v * SP, st);
 #pragma unroll
-    for (int k = 0; k < S; ++k) {
+    for (int k = 0; k < S; ++k)
         t[k] = 1.0f;
-        st[k] = states[(size_t)v * SP + k];
-    }
     unsigned b = in_off[v], e = in_off[v + 1];
-    for (unsigned s = b; s < e; ++s) {
+    for (unsigned s = b; s < e; s += U) {
+        float m[U][S];
 #pragma unroll
-        for (int k = 0; k < S; ++k)
-            m[k] = msg[(size_t)s * SP + k];
-        combine<S, MIXED>(t, m, n);
+        for (int u = 0; u < U; ++u)
+            load_rowp<S, SP>(msg + (size_t)(s + u < e ? s + u : s) * SP, m[u]);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (s + u < e)
+                combine<S, MIXED>(t, m[u], n);
     }
     if (e > b) {
 #pragma unroll
@@ -295,6 +393,13 @@ struct PlanBuilder {
     }
 };
 
+/* A node's sends go to several entries, each with its own copy of the
+ * product: a sub-wave waits for the thread with the most sends.  At most 16
+ * entries, so that the products' reads stay linear in the node's degree;
+ * not where a wave would become too large for one workgroup by it.  (1M-node
+ * tree 430 -> 405 us with its beliefs read back, 10k-node tree 80 -> 71.) */
+unsigned entry_parts(unsigned sends) { return std::min(16u, (sends + 3) / 4); }
+
 int upload_plan(bp_dev *d, PlanBuilder &pb, bp_tree_plan **out)
 {
     /* Entry records in device numbering.  The entries of one sub-wave are
@@ -307,7 +412,7 @@ int upload_plan(bp_dev *d, PlanBuilder &pb, bp_tree_plan **out)
     std::vector<TreeEntry> ent;
     std::vector<unsigned> act, wbeg{0}, idx;
     std::vector<unsigned char> wstart;
-    ent.reserve(pb.entries.size());
+    ent.reserve(pb.entries.size() + pb.act_slot.size() / 4);
     act.reserve(pb.act_slot.size());
     for (size_t w = 0; w + 1 < pb.wave_begin.size(); ++w) {
         idx.clear();
@@ -317,11 +422,18 @@ int upload_plan(bp_dev *d, PlanBuilder &pb, bp_tree_plan **out)
         std::sort(idx.begin(), idx.end(), [&](unsigned x, unsigned y) {
             return pb.act_slot[pb.act_off[x]] < pb.act_slot[pb.act_off[y]];
         });
+        size_t parts = 0;
+        for (unsigned i : idx)
+            parts += entry_parts(pb.act_off[i + 1] - pb.act_off[i]);
+        const bool split = parts <= SMALL_WAVE || idx.size() > SMALL_WAVE;
         for (unsigned i : idx) {
             unsigned v = d->perm[pb.entries[i]];
             unsigned ab = (unsigned)act.size();
             act.insert(act.end(), pb.act_slot.begin() + pb.act_off[i], pb.act_slot.begin() + pb.act_off[i + 1]);
-            ent.push_back(TreeEntry{v, d->in_off_h[v], d->in_off_h[v + 1], ab, (unsigned)act.size(), d->node_n[v], 0, 0});
+            const unsigned end = (unsigned)act.size(), n = end - ab, k = split ? entry_parts(n) : 1;
+            for (unsigned j = 0; j < k; ++j)
+                ent.push_back(TreeEntry{v, d->in_off_h[v], d->in_off_h[v + 1], ab + (unsigned)((uint64_t)n * j / k),
+                                        ab + (unsigned)((uint64_t)n * (j + 1) / k), d->node_n[v], 0, 0});
         }
         if (ent.size() != wbeg.back()) {
             wbeg.push_back((unsigned)ent.size());

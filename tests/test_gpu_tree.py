@@ -2,6 +2,8 @@
 src/c_benchmark/main.c:205-215), bit for bit."""
 from __future__ import annotations
 
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -129,3 +131,39 @@ def test_duplicate_level_entries_are_rejected(lib):
     lib.propagate_using_levels_start(g)
     assert "twice" in B.last_error()
     lib.graph_destroy(g)
+
+
+@pytest.mark.parametrize("nodes,lo,hi", [(60, 1, 1), (60, 2, 2), (6000, 2, 2), (4000, 3, 3), (3000, 4, 4), (500, 5, 5),
+                                         (500, 8, 8), (300, 9, 9), (3000, 1, 3), (3000, 2, 4), (500, 2, 6), (500, 2, 9)])
+def test_tree_nodes_of_every_degree(lib, orc, nodes, lo, hi):
+    """Sub-waves above and below a workgroup's threads, nodes with 1 to 21
+    sends and in-messages (they are taken up to 4 and 8 at a time)."""
+    print(f"degrees, {nodes} nodes of {lo}-{hi} states", flush=True)
+    rng = np.random.default_rng(nodes + hi)
+    parent = [0] + [int(rng.integers(0, v)) for v in range(1, nodes)]
+    for c in range(1, 22):
+        hub = len(parent)
+        parent.append(int(rng.integers(0, nodes)))
+        parent += [hub] * c
+    V = len(parent)
+    n = rng.integers(lo, hi + 1, V)
+    bn = lib.bp_bn_create(V)
+    for v in range(V):
+        assert lib.bp_bn_set_var(bn, v, f"n{v}".encode(), int(n[v])) == 0
+    for v in range(V):
+        t = rng.random((n[v], 1 if v == 0 else n[parent[v]])).astype(np.float32) + np.float32(0.1)
+        t = (t / t.sum(0)).astype(np.float32).ravel()
+        par = (C.c_uint * 1)(parent[v])
+        assert lib.bp_bn_add_def(bn, v, par if v else None, 1 if v else 0, t.ctypes.data_as(B.f32p), t.size) == 0
+    g = B.bn_to_graph(bn, levels=True)
+    h = B.bn_to_graph(bn, levels=True)
+    dev = B.Device(g)
+    dev.tree()
+    dev.download(g)
+    orc.tree_run(h)
+    assert same_bits(B.messages(g, "tree"), B.messages(h, "tree"))
+    assert same_bits(B.states(g), B.states(h))
+    dev.free()
+    lib.graph_destroy(g)
+    lib.graph_destroy(h)
+    lib.bp_bn_free(bn)

@@ -48,18 +48,24 @@ __device__ __forceinline__ bool called_off(const Meeting &a)
            __hip_atomic_load(a.decision, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != (a.after << 1 | COMMIT);
 }
 
-/* Waits until every workgroup has been at barrier number `number` (from 1).
- * False: this run has been given up.  All threads of the workgroup call it;
- * `ok` is shared. */
-__device__ __forceinline__ bool grid_step(const Meeting &a, unsigned wg, unsigned G, unsigned number, unsigned *ok)
+/* The grid barrier in two halves, with work between them that needs nothing
+ * of other workgroups.  All threads of the workgroup call both; arriving is
+ * also a workgroup barrier. */
+__device__ __forceinline__ void grid_arrive(const Meeting &a, unsigned wg)
 {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); /* this wave's combine buffers are in memory */
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); /* this wave's rows are in memory */
     __syncthreads();
+    if (threadIdx.x == 0)
+        __hip_atomic_fetch_add(a.counters + (wg % COUNTERS) * COUNTER_STRIDE, 1u, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+}
+
+/* Waits until every workgroup has been at barrier number `number` (from 1).
+ * False: this run has been given up.  `ok` is shared. */
+__device__ __forceinline__ bool grid_wait(const Meeting &a, unsigned G, unsigned number, unsigned *ok)
+{
     if (threadIdx.x < WAVE) {
         const unsigned lane = threadIdx.x;
-        if (lane == 0)
-            __hip_atomic_fetch_add(a.counters + (wg % COUNTERS) * COUNTER_STRIDE, 1u, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
         const unsigned members = lane < COUNTERS ? (G - lane + COUNTERS - 1) / COUNTERS : 0u;
         const unsigned want = (a.met + number) * members;
         const unsigned long long t0 = wall_clock64();
@@ -84,6 +90,12 @@ __device__ __forceinline__ bool grid_step(const Meeting &a, unsigned wg, unsigne
     __syncthreads();
     asm volatile("" ::: "memory"); /* no gather moves above the barrier */
     return *ok != 0;
+}
+
+__device__ __forceinline__ bool grid_step(const Meeting &a, unsigned wg, unsigned G, unsigned number, unsigned *ok)
+{
+    grid_arrive(a, wg);
+    return grid_wait(a, G, number, ok);
 }
 
 template <int N> __device__ __forceinline__ void store_row_agent(float *p, const float *v)

@@ -19,8 +19,11 @@
  * ordinary loads, as the combine buffers are in bp_resident.hip.  (Rows
  * scattered to their place in the source-grouped list, as the launches have
  * it, are 8-byte stores through to memory and loads past the caches here.)
- * Measured, per step: 200k nodes of 3 states (600k slots) 30 us, against 38
- * with scattered rows and 35 as launches; 2k nodes 9.4 against 17.
+ * What a step needs of the kept iterates alone (messages, their products)
+ * comes between arriving at the grid barrier and waiting there.
+ * Measured, per step: 200k nodes of 3 states (725k slots) 25 us, against 30
+ * with all of it behind the barrier, 38 with scattered rows and 35 as
+ * launches; 2k nodes 8.5, against 9.5 and 17 as launches.
  * Everything else that is read was written by an earlier launch.
  *
  * Both runs are enqueued on the caller's stream and not waited for.  The
@@ -73,6 +76,7 @@ __global__ __launch_bounds__(T) void k_resident_adjoint(ResAdjArgs a)
     constexpr int SP = Stride<S>::value;
     constexpr int NN = T < RB ? (NS / 2 + 1) / 2 * 2 : (NS + 1) / 2; /* nodes per thread */
     constexpr int W = T * NS;
+    constexpr bool EARLY = NS == 1;
     __shared__ __align__(16) float lm[S * (W + PAD)]; /* messages by slot */
     __shared__ __align__(16) float ldt[S * T * NN];  /* the nodes' dT */
     __shared__ unsigned short lnode[W];               /* the slot's node */
@@ -129,6 +133,23 @@ __global__ __launch_bounds__(T) void k_resident_adjoint(ResAdjArgs a)
                         acc[i] = acc[i] + x[u][i];
         }
     };
+    /* the product of the messages that a slot's node gets beside its own */
+    auto siblings = [&](int k, float *P) {
+        const unsigned place = k % 2 ? at[k / 2] >> 16 : at[k / 2] & 0xffffu;
+        const unsigned q0 = sib[k] >> 11 & 0x1fffu, cnt = (sib[k] >> 24) + 1, own = place - q0;
+#pragma unroll
+        for (int i = 0; i < S; ++i)
+            P[i] = 1.0f;
+        for (unsigned q = 0; q < cnt; q += 4) {
+            float f[4][S];
+            factors<S, S, 4, true>(lm + (q0 + q) * S, cnt - q, f);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int i = 0; i < S; ++i)
+                    P[i] = P[i] * (q + j == own ? 1.0f : f[j][i]);
+        }
+    };
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < NS; ++k) {
@@ -160,8 +181,7 @@ __global__ __launch_bounds__(T) void k_resident_adjoint(ResAdjArgs a)
         __syncthreads();
     }
     unsigned number = 1;
-    if (!grid_step(a.meeting, wg, G, number++, &ok)) /* everybody is here */
-        return;
+    grid_arrive(a.meeting, wg);
 
     for (unsigned t = a.K + 1; t-- > 0;) {
         const bool last = t == 0; /* step 0: m_0 from st_0 */
@@ -201,52 +221,67 @@ __global__ __launch_bounds__(T) void k_resident_adjoint(ResAdjArgs a)
             }
         }
         __syncthreads();
+        /* the products of the nodes' in-messages and, with a slot per
+         * thread, of each slot's siblings */
+        float Tm[NN][S], P[EARLY ? NS : 1][S];
+#pragma unroll
+        for (int r = 0; r < NN; ++r) {
+            const unsigned cnt = slots[r] >> 16;
+            const float *msgs = lm + (slots[r] & 0xffffu) * S;
+#pragma unroll
+            for (int i = 0; i < S; ++i)
+                Tm[r][i] = 1.0f;
+            for (unsigned q = 0; q < cnt; q += 4) {
+                float f[4][S];
+                factors<S, S, 4, true>(msgs + q * S, cnt - q, f);
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    mul_all<S>(Tm[r], f[j]);
+            }
+        }
+        if constexpr (EARLY)
+#pragma unroll
+            for (int k = 0; k < NS; ++k)
+                if (k * T + tid < ns)
+                    siblings(k, P[k]);
+        /* the other workgroups' w of the step before (the first time: all are here) */
+        if (!grid_wait(a.meeting, G, number++, &ok))
+            return;
         /* node phase: dT, dL/dst_{t-1} */
 #pragma unroll
         for (int r = 0; r < NN; ++r) {
             const unsigned l = r * T + tid, v = n0 + l;
             if (v < n1) {
-                const unsigned cnt = slots[r] >> 16;
-                const float *msgs = lm + (slots[r] & 0xffffu) * S;
-                float Tm[S], gb[S], dT[S], stp[S], stc[S];
+                float gb[S], dT[S], stp[S], stc[S];
                 load_rowp<S, SP>((last ? a.st0 : a.st + (size_t)t * a.stride) + (size_t)v * SP, stc);
                 if (!last)
                     load_rowp<S, SP>((t > 1 ? a.st + (size_t)(t - 1) * a.stride : a.st0) + (size_t)v * SP, stp);
 #pragma unroll
-                for (int i = 0; i < S; ++i) {
-                    Tm[i] = 1.0f;
+                for (int i = 0; i < S; ++i)
                     gb[i] = 0.0f;
-                }
-                for (unsigned q = 0; q < cnt; q += 4) {
-                    float f[4][S];
-                    factors<S, S, 4, true>(msgs + q * S, cnt - q, f);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        mul_all<S>(Tm, f[j]);
-                }
                 if (t < a.K)
                     add_w(a.w + (size_t)(t + 1) * a.w_stride, o0[r], o1[r], gb);
                 if (last) {
 #pragma unroll
                     for (int i = 0; i < S; ++i) {
                         dT[i] = gb[i] * stc[i];
-                        g[r][i] = g[r][i] + gb[i] * Tm[i];
+                        g[r][i] = g[r][i] + gb[i] * Tm[r][i];
                     }
                 } else {
-                    const bool indeg = cnt > 0;
+                    const bool indeg = slots[r] >> 16;
                     float ds[S], sa = 0.0f, dot = 0.0f;
 #pragma unroll
                     for (int i = 0; i < S; ++i) {
-                        ds[i] = g[r][i] + gb[i] * Tm[i];
+                        ds[i] = g[r][i] + gb[i] * Tm[r][i];
                         dT[i] = gb[i] * stc[i];
-                        const float av = indeg ? stp[i] * Tm[i] : stp[i];
+                        const float av = indeg ? stp[i] * Tm[r][i] : stp[i];
                         sa = sa + av;
                         dot = dot + ds[i] * stc[i];
                     }
 #pragma unroll
                     for (int i = 0; i < S; ++i) {
                         const float da = (sa > 0.0f) ? (ds[i] - dot) / sa : ds[i];
-                        g[r][i] = indeg ? da * Tm[i] : da;
+                        g[r][i] = indeg ? da * Tm[r][i] : da;
                         if (indeg)
                             dT[i] = dT[i] + da * stp[i];
                     }
@@ -262,25 +297,15 @@ __global__ __launch_bounds__(T) void k_resident_adjoint(ResAdjArgs a)
             const unsigned l = k * T + tid;
             if (l < ns) {
                 const unsigned place = k % 2 ? at[k / 2] >> 16 : at[k / 2] & 0xffffu;
-                const unsigned q0 = sib[k] >> 11 & 0x1fffu, cnt = (sib[k] >> 24) + 1, own = place - q0;
-                float P[S], m[S], dT[S], dm[S], dz[S], dot = 0.0f;
-#pragma unroll
-                for (int i = 0; i < S; ++i)
-                    P[i] = 1.0f;
-                for (unsigned q = 0; q < cnt; q += 4) {
-                    float f[4][S];
-                    factors<S, S, 4, true>(lm + (q0 + q) * S, cnt - q, f);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-#pragma unroll
-                        for (int i = 0; i < S; ++i)
-                            P[i] = P[i] * (q + j == own ? 1.0f : f[j][i]);
-                }
+                float (&Pk)[S] = P[EARLY ? k : 0];
+                float m[S], dT[S], dm[S], dz[S], dot = 0.0f;
+                if constexpr (!EARLY)
+                    siblings(k, Pk);
                 get_row<S>(lm + place * S, m);
                 get_row<S>(ldt + (sib[k] & 0x7ffu) * S, dT);
 #pragma unroll
                 for (int i = 0; i < S; ++i) {
-                    dm[i] = (m[i] == m[i]) ? dT[i] * P[i] : 0.0f;
+                    dm[i] = (m[i] == m[i]) ? dT[i] * Pk[i] : 0.0f;
                     dot = dot + dm[i] * m[i];
                 }
 #pragma unroll
@@ -304,9 +329,10 @@ __global__ __launch_bounds__(T) void k_resident_adjoint(ResAdjArgs a)
                 store_row_agent<SP>(wout + l * SP, wv);
             }
         }
-        if (!grid_step(a.meeting, wg, G, number++, &ok))
-            return;
+        grid_arrive(a.meeting, wg);
     }
+    if (!grid_wait(a.meeting, G, number, &ok))
+        return;
     if (tid == 0)
         committed = settle(a.meeting.decision, a.meeting.run, COMMIT);
     __syncthreads();

@@ -145,7 +145,7 @@ template <typename T> static int dmalloc(T **p, size_t count)
  * stream st over the handle's chunks (ev: optional start/stop events). */
 bpk::LoopyArgs bp_make_args(bp_dev *d);
 void bp_launch_loopy(bp_dev *d, int mode, const bpk::LoopyArgs &a, hipStream_t st, const hipEvent_t *ev = nullptr);
-int bp_upload_graph(Graph_t g, int device, bp_dev **out);
+int bp_upload_graph(Graph_t g, int device, bp_dev **out); /* for gradients */
 
 /* Device node numbering: bp_node_order_mode() is what bp_set_node_order
  * chose (1: Cuthill-McKee, 0: the graph's own order); bp_cm_order fills
@@ -159,7 +159,7 @@ void bp_cm_order(Graph_t g, std::vector<unsigned> &order);
 void bp_build_chunks(const std::vector<unsigned> &in_off, unsigned V, unsigned cap, std::vector<uint2> &chunks);
 
 /* resident runs (bp_resident.hip) */
-int bp_resident_plan(bp_dev *d, const std::vector<unsigned> &slot_src, int cus);
+int bp_resident_plan(bp_dev *d, const std::vector<unsigned> &slot_src, bool gradients, int cus);
 void bp_resident_free(bp_dev *d);
 int bp_resident_launch(bp_dev *d, unsigned n, bool want_delta, bool until, float conv, double previous,
                        double *partials);

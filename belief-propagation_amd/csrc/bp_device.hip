@@ -866,7 +866,7 @@ struct Layout {
     }
 };
 
-static int upload_impl(Graph_t g, int device, bp_dev **out, bool plan)
+static int upload_impl(Graph_t g, int device, bp_dev **out, bool plan, bool gradients)
 {
     bp_clear_error();
     *out = nullptr;
@@ -1060,7 +1060,7 @@ static int upload_impl(Graph_t g, int device, bp_dev **out, bool plan)
     }
     /* a network that fits runs its iterations resident; without the memory
      * for that it runs them one launch each */
-    if (bp_resident_plan(d, slot_src, prop.multiProcessorCount) != 0) {
+    if (bp_resident_plan(d, slot_src, gradients, prop.multiProcessorCount) != 0) {
         bp_resident_free(d);
         (void)hipGetLastError();
         bp_clear_error();
@@ -1072,10 +1072,10 @@ static int upload_impl(Graph_t g, int device, bp_dev **out, bool plan)
     return 0;
 }
 
-extern "C" int bp_upload(Graph_t g, int device, bp_dev **out) { return upload_impl(g, device, out, true); }
+extern "C" int bp_upload(Graph_t g, int device, bp_dev **out) { return upload_impl(g, device, out, true, false); }
 
-/* an upload without the tree schedule, for the adjoint and batched handles */
-int bp_upload_graph(Graph_t g, int device, bp_dev **out) { return upload_impl(g, device, out, false); }
+/* an upload without the tree schedule, for the adjoint */
+int bp_upload_graph(Graph_t g, int device, bp_dev **out) { return upload_impl(g, device, out, false, true); }
 
 extern "C" int bp_upload_state(bp_dev *d, Graph_t g)
 {
@@ -1914,7 +1914,7 @@ static bp_dev *dropin_device_status(Graph_t g)
     if (d && impl->dev_cache_generation == impl->generation)
         return bp_upload_state(d, g) == 0 ? d : nullptr;
     bp_dev_cache_release(impl);
-    if (upload_impl(g, -1, &d, false) != 0)
+    if (upload_impl(g, -1, &d, false, false) != 0)
         return nullptr;
     impl->dev_cache = d;
     impl->dev_cache_generation = impl->generation;

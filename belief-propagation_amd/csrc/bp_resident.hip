@@ -504,19 +504,26 @@ __global__ __launch_bounds__(RB) void k_resident(ResArgs a)
 
 namespace {
 
-/* Most workgroups of a plan with ns slots per thread: the grid is kept small
- * where it can be -- a barrier among 64 workgroups costs 1.3 us, among 256
- * 2.5 us.  `most` slots per thread are what the registers (128 per thread)
- * and LDS (two iterations' messages) hold. */
+/* Slots per thread that the registers (128 per thread) and LDS (two
+ * iterations' messages) hold. */
 unsigned most_slots(unsigned S) { return S == 2 ? 8 : S == 3 ? 4 : S == 4 ? 3 : 1; }
 
 /* slots per thread go 1, 2, 4, 8; for three and four states 1, 2, 3, 4 */
 unsigned next_slots(unsigned ns, unsigned S) { return S > 2 && ns >= 2 ? ns + 1 : 2 * ns; }
 
-unsigned most_groups(unsigned ns, unsigned S, unsigned cus)
+/* Most workgroups of a plan with ns slots per thread.  All CUs: fewer slots
+ * per thread are worth more than the barrier among more workgroups costs
+ * (1.25 us among 64, 1.4 among 256).  Per iteration, us, at most 64 ns
+ * workgroups / all: 100k binary nodes 5.47 / 5.00, 20k nodes of 3 states
+ * 4.11 / 3.90, 100k nodes of 2-4 states 7.15 / 6.63; gradients, a backward
+ * of 31 steps: 20k nodes of 3 states 457 / 330, 120k 782 / 602.  Binary
+ * networks with a slot per thread have too little to do: 40k nodes 3.79 /
+ * 3.87 and with the stop test 5.05 / 5.26, 60k 4.29 / 4.50 and 5.59 / 6.05,
+ * so half the CUs there, except for gradients (40k nodes 311 / 233). */
+unsigned most_groups(unsigned ns, unsigned S, bool gradients, unsigned cus)
 {
     const unsigned full = std::min(cus, MAX_G);
-    return ns == most_slots(S) || ns > 2 ? full : std::min(full, 64 * ns);
+    return S == 2 && ns == 1 && !gradients ? (full + 1) / 2 : full;
 }
 
 /* Largest network of one workgroup, in slots per thread: messages and
@@ -678,7 +685,7 @@ Meeting bp_resident_meeting(bp_dev *d, unsigned barriers, unsigned after)
 
 /* Decides whether the graph runs resident and lays out its ranges:
  * uniform state counts of 2 to 8, or mixed ones up to 3 to 8. */
-int bp_resident_plan(bp_dev *d, const std::vector<unsigned> &slot_src, int cus)
+int bp_resident_plan(bp_dev *d, const std::vector<unsigned> &slot_src, bool gradients, int cus)
 {
     bp_resident &r = d->res;
     if (d->E == 0 || d->S < 2 || d->S > 8 || (d->mixed && d->S == 2) || d->device >= MAX_DEVICES)
@@ -694,7 +701,7 @@ int bp_resident_plan(bp_dev *d, const std::vector<unsigned> &slot_src, int cus)
     for (unsigned ns = 1; ns <= most_slots(d->S) && !r.ns; ns = next_slots(ns, d->S)) {
         /* even ranges: the slots spread over as many workgroups as the cap
          * asks for, a few per cent more where node groups do not fit */
-        const unsigned cap = ns * RB, full = cap * 31 / 32, groups = most_groups(ns, d->S, (unsigned)cus);
+        const unsigned cap = ns * RB, full = cap * 31 / 32, groups = most_groups(ns, d->S, gradients, (unsigned)cus);
         const unsigned want = (d->E + full - 1) / full;
         const unsigned even = std::min(cap, (d->E + want - 1) / want + cap / 32);
         if (want <= groups && cut_ranges(d->in_off_h, d->V, even, most_nodes(ns, d->S), align, first) &&

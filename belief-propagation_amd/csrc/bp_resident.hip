@@ -385,10 +385,8 @@ __global__ __launch_bounds__(RB) void k_resident(ResArgs a)
         const bool clean = __builtin_amdgcn_readfirstlane(suspect) == ran + 1;
         if (DELTA && wave == RW - 1 && (!SINGLE || !a.until)) {
             /* the wave with the fewest nodes adds up the workgroup's delta */
-            double sum = red[ran & 1][lane % RW];
-#pragma unroll
-            for (int off = RW / 2; off > 0; off >>= 1)
-                sum += __shfl_xor(sum, off, WAVE);
+            static_assert(RW == 16, "a row of lanes");
+            const double sum = row_sum(red[ran & 1][lane % RW]);
             if (lane == 0) {
                 if (!a.until)
                     a.partials[(size_t)ran * G + wg] = sum;

@@ -99,16 +99,20 @@ int bp_restore_states(bp_dev *d);
 /* init_previous_edge on the device. */
 int bp_loopy_init(bp_dev *d);
 
-/* n loopy iterations; deltas (nullable) receives the FP64 delta of each.
- * The launches are replayed from a cached HIP graph. */
+/* n loopy iterations; deltas (nullable) receives the FP64 delta of each;
+ * without it deltas are not formed.  A network that fits on the chip (up to
+ * 2.1M message edges of 2 states, 262k of 8) runs them in one launch;
+ * otherwise the launches are replayed from a cached HIP graph.  A launch
+ * that was given up (its workgroups wait for each other at most a second) is
+ * made up for by the handle's next call. */
 int bp_loopy_iterate(bp_dev *d, unsigned int n, double *deltas);
 
 /* No counterpart in the reference.  For callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): n loopy iterations with the results of
  * bp_loopy_iterate, bit for bit, that call no hipMalloc, hipFree or other
- * allocating routine and create no HIP graph.  The FP64 delta partials and
- * deltas live in a fixed 4 MiB device array of the library, one per GPU:
+ * allocating routine and create no HIP graph.  Of a handle whose iterations
+ * run a launch each, the FP64 delta partials and deltas live in a fixed 4 MiB device array of the library, one per GPU:
  * the call fails with an error when the handle's delta partials per
  * iteration (one per wave of its grid: about one per 64-128 message edges)
  * plus n exceed 524,288 doubles, i.e. from about 30M message edges on.

@@ -39,7 +39,7 @@
  *
  * Workgroups wait for each other, so all must be on the chip at once.  The
  * grid is at most one workgroup per CU, and the host lets one such launch
- * run on a device at a time (take_turn).  If other work keeps part of the
+ * run on a device at a time (bp_resident_turn).  If other work keeps part of the
  * chip nevertheless, waits end after `timeout` and the run gives up: nothing
  * has been written that a later step reads, the first workgroup to give up
  * (or, past the last barrier, to go on) settles it for all in one word, and
@@ -47,6 +47,11 @@
  *
  * A network whose slots fit one workgroup needs none of this: its combine
  * buffers stay in LDS as well and it can always run (SINGLE).
+ *
+ * Measured, per iteration, us (a launch each / plain / with deltas / with the
+ * stop test): 500k binary nodes 18.8 (with deltas) / 10.6 / 11.6 / 13.3, 5k
+ * - / 2.9 / 3.2 / 3.4, 700 in one workgroup 5.5 / 1.7 / 2.2 / 2.3, 200k of 3
+ * states 12.5 (plain) / 9.2 / 9.6 / 10.9.
  *
  * Every float operation is the one k_loopy performs, in its order, so
  * beliefs and messages are bit-identical to it; the FP64 deltas add the same

@@ -484,13 +484,9 @@ static void build_shape(bp_batch *b, Shape &sh, unsigned R)
     sh.built = true;
 }
 
-template <typename T> static int up(T **dst, const T *src, size_t n)
+template <typename T> static int up(bp_batch *b, T **dst, const T *src, size_t n)
 {
-    if (dmalloc(dst, n))
-        return -1;
-    if (n)
-        HIP_TRY(hipMemcpy(*dst, src, n * sizeof(T), hipMemcpyHostToDevice));
-    return 0;
+    return dmalloc(dst, n) || copy_on(b->stream, *dst, src, n * sizeof(T), hipMemcpyHostToDevice) ? -1 : 0;
 }
 
 extern "C" int bp_batch_upload(bp_batch *b, int device)
@@ -553,10 +549,10 @@ extern "C" int bp_batch_upload(bp_batch *b, int device)
     std::vector<unsigned> in_off(b->in_off);
     in_off.push_back(b->E);
     unsigned maxchunks = std::max(b->shapes[0].nchunks, b->shapes[1].nchunks);
-    if (up(&b->d_in_off, in_off.data(), in_off.size()) || up(&b->d_slot_src, b->slot_src.data(), b->E) ||
-        up(&b->d_slot_tab, b->slot_tab.data(), b->E) || up(&b->d_slot_xy, b->slot_xy.data(), b->E) ||
-        up(&b->d_nvars, b->nvars.data(), b->V) || up(&b->d_tabs, b->tabs.data(), b->tabs.size()) ||
-        up(&b->d_states0, st.data(), VS) || dmalloc(&b->d_states, VS) || dmalloc(&b->d_buf[0], VS) ||
+    if (up(b, &b->d_in_off, in_off.data(), in_off.size()) || up(b, &b->d_slot_src, b->slot_src.data(), b->E) ||
+        up(b, &b->d_slot_tab, b->slot_tab.data(), b->E) || up(b, &b->d_slot_xy, b->slot_xy.data(), b->E) ||
+        up(b, &b->d_nvars, b->nvars.data(), b->V) || up(b, &b->d_tabs, b->tabs.data(), b->tabs.size()) ||
+        up(b, &b->d_states0, st.data(), VS) || dmalloc(&b->d_states, VS) || dmalloc(&b->d_buf[0], VS) ||
         dmalloc(&b->d_buf[1], VS) || dmalloc(&b->d_msg[0], ES) || dmalloc(&b->d_msg[1], ES) ||
         dmalloc(&b->d_partials, std::max(maxchunks, 1u)) || dmalloc(&b->d_queue, 1))
         return -1;
@@ -564,10 +560,10 @@ extern "C" int bp_batch_upload(bp_batch *b, int device)
         Shape &sh = b->shapes[k];
         if (!sh.built)
             continue;
-        if (up(&sh.d_chunk, sh.chunks.data(), sh.chunks.size()) ||
-            up(&sh.d_inst_chunk, sh.inst_chunk.data(), sh.inst_chunk.size()) ||
-            up(&sh.d_order, sh.order.data(), sh.order.size()) || up(&sh.d_base, sh.base.data(), sh.base.size()) ||
-            up(&sh.d_wide, sh.wide.data(), sh.wide.size()))
+        if (up(b, &sh.d_chunk, sh.chunks.data(), sh.chunks.size()) ||
+            up(b, &sh.d_inst_chunk, sh.inst_chunk.data(), sh.inst_chunk.size()) ||
+            up(b, &sh.d_order, sh.order.data(), sh.order.size()) || up(b, &sh.d_base, sh.base.data(), sh.base.size()) ||
+            up(b, &sh.d_wide, sh.wide.data(), sh.wide.size()))
             return -1;
     }
     size_t most = 1;
@@ -575,11 +571,10 @@ extern "C" int bp_batch_upload(bp_batch *b, int device)
         most = std::max<size_t>(most, b->node_row_off[i + 1] - b->node_row_off[i] +
                                           2 * (b->msg_row_off[i + 1] - b->msg_row_off[i]));
     HIP_TRY(hipHostMalloc((void **)&b->h_stage, most * sizeof(float), hipHostMallocDefault));
-    HIP_TRY(hipMemcpy(b->d_states, b->d_states0, VS * sizeof(float), hipMemcpyDeviceToDevice));
-    HIP_TRY(hipMemset(b->d_buf[0], 0, VS * sizeof(float)));
-    HIP_TRY(hipMemset(b->d_buf[1], 0, VS * sizeof(float)));
-    HIP_TRY(hipMemset(b->d_msg[0], 0, ES * sizeof(float)));
-    HIP_TRY(hipMemset(b->d_msg[1], 0, ES * sizeof(float)));
+    if (copy_on(b->stream, b->d_states, b->d_states0, VS * sizeof(float), hipMemcpyDeviceToDevice) ||
+        zero_on(b->stream, b->d_buf[0], VS * sizeof(float)) || zero_on(b->stream, b->d_buf[1], VS * sizeof(float)) ||
+        zero_on(b->stream, b->d_msg[0], ES * sizeof(float)) || zero_on(b->stream, b->d_msg[1], ES * sizeof(float)))
+        return -1;
     /* host staging no longer needed (downloads keep slot_edge, edge_x, offsets, nvars) */
     std::vector<float>().swap(b->st_stage);
     std::vector<unsigned>().swap(b->slot_src);

@@ -140,6 +140,24 @@ template <typename T> static int dmalloc(T **p, size_t count)
     return 0;
 }
 
+/* A copy or fill that has been made on return, by way of a stream of the
+ * library's own.  hipMemcpy and hipMemset use the null stream, which while
+ * another thread captures a graph refuses the call and spoils the capture. */
+inline int copy_on(hipStream_t st, void *dst, const void *src, size_t bytes, hipMemcpyKind kind)
+{
+    if (bytes) {
+        HIP_TRY(hipMemcpyAsync(dst, src, bytes, kind, st));
+        HIP_TRY(hipStreamSynchronize(st));
+    }
+    return 0;
+}
+inline int zero_on(hipStream_t st, void *dst, size_t bytes)
+{
+    HIP_TRY(hipMemsetAsync(dst, 0, bytes, st));
+    HIP_TRY(hipStreamSynchronize(st));
+    return 0;
+}
+
 /* Loopy kernel launch shared with the adjoint (bp_diff.hip): the handle's
  * arrays as kernel arguments, and one launch of k_loopy<S, MIXED, mode> on
  * stream st over the handle's chunks (ev: optional start/stop events). */

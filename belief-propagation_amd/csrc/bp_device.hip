@@ -726,8 +726,9 @@ static int upload_state(bp_dev *d, Graph_t g, bool tables)
             std::vector<unsigned> tab;
             std::vector<float> pool;
             build_table_pool(d->partner, d->slot_edge, tmp, d->E, S, tab, pool);
-            HIP_TRY(hipMemcpy(d->Jp, pool.data(), pool.size() * sizeof(float), hipMemcpyHostToDevice));
-            HIP_TRY(hipMemcpy(d->slot_pool, tab.data(), (size_t)d->E * 4, hipMemcpyHostToDevice));
+            if (copy_on(d->stream, d->Jp, pool.data(), pool.size() * sizeof(float), hipMemcpyHostToDevice) ||
+                copy_on(d->stream, d->slot_pool, tab.data(), (size_t)d->E * 4, hipMemcpyHostToDevice))
+                return -1;
         }
     }
     d->latest = 0;

@@ -481,11 +481,9 @@ extern "C" void bp_diff_free(bp_diff *x)
 {
     if (!x)
         return;
-    if (x->d) {
+    if (x->d)
         (void)hipSetDevice(x->d->device);
-        (void)hipDeviceSynchronize();
-    }
-    diff_release_storage(x);
+    diff_release_storage(x); /* hipFree waits for the device, callers' streams included */
     void *ps[] = {x->out_at, x->adj_chunk, x->defs, x->perm_d, x->inv_d, x->row_def, x->par_def, x->pieces, x->big_recs, x->out_off,
                   x->out_slot, x->slot_pos, x->slot_edge, x->parents, x->P, x->st0, x->gin, x->gst[0], x->gst[1],
                   x->w[0], x->w[1], x->jbar, x->dst0p, x->dst0};
@@ -496,13 +494,10 @@ extern "C" void bp_diff_free(bp_diff *x)
     delete x;
 }
 
-template <typename T> static int upload_vec(T **dst, const std::vector<T> &v)
+template <typename T> static int upload_vec(bp_diff *x, T **dst, const std::vector<T> &v)
 {
-    if (dmalloc(dst, v.size()))
-        return -1;
-    if (!v.empty())
-        HIP_TRY(hipMemcpy(*dst, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
-    return 0;
+    return dmalloc(dst, v.size()) ||
+           copy_on(x->d->stream, *dst, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice) ? -1 : 0;
 }
 
 /* checks that need no device: one state count, in-degrees within a wave's
@@ -589,7 +584,10 @@ static int build_pieces(bp_diff *x, std::vector<DefInfo> &defs)
     }
     x->npieces = (unsigned)pieces.size();
     x->nbig = (unsigned)big_recs.size();
-    return upload_vec(&x->pieces, pieces) || upload_vec(&x->row_def, row_def) || upload_vec(&x->big_recs, big_recs) ? -1 : 0;
+    return upload_vec(x, &x->pieces, pieces) || upload_vec(x, &x->row_def, row_def) ||
+                   upload_vec(x, &x->big_recs, big_recs)
+               ? -1
+               : 0;
 }
 
 static int diff_build(bp_diff *x, const bp_bn *bn, unsigned npd, Graph_t g)
@@ -703,14 +701,14 @@ static int diff_build(bp_diff *x, const bp_bn *bn, unsigned npd, Graph_t g)
         x->adj_nchunks = (unsigned)ch.size() - 1;
         unsigned want = (x->adj_nchunks + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
         x->adj_G = std::max(8u, (want + 7u) & ~7u);
-        if (upload_vec(&x->adj_chunk, ch))
+        if (upload_vec(x, &x->adj_chunk, ch))
             return -1;
     }
     size_t VS = (size_t)V * d->SP, ES = (size_t)E * d->SP;
-    if (upload_vec(&x->perm_d, d->perm) || upload_vec(&x->inv_d, d->inv) ||
-        upload_vec(&x->out_off, out_off) ||
-        upload_vec(&x->out_slot, out_slot) || upload_vec(&x->slot_pos, slot_pos) || upload_vec(&x->slot_edge, d->slot_edge) ||
-        upload_vec(&x->defs, definfo) || upload_vec(&x->parents, prs) || upload_vec(&x->par_def, par_def) || dmalloc(&x->P, x->num_params) ||
+    if (upload_vec(x, &x->perm_d, d->perm) || upload_vec(x, &x->inv_d, d->inv) || upload_vec(x, &x->out_off, out_off) ||
+        upload_vec(x, &x->out_slot, out_slot) || upload_vec(x, &x->slot_pos, slot_pos) ||
+        upload_vec(x, &x->slot_edge, d->slot_edge) || upload_vec(x, &x->defs, definfo) ||
+        upload_vec(x, &x->parents, prs) || upload_vec(x, &x->par_def, par_def) || dmalloc(&x->P, x->num_params) ||
         dmalloc(&x->st0, VS) || dmalloc(&x->gin, VS) || dmalloc(&x->gst[0], VS) || dmalloc(&x->gst[1], VS) ||
         dmalloc(&x->w[0], ES) || dmalloc(&x->w[1], ES) || dmalloc(&x->jbar, (size_t)E * S * S) ||
         dmalloc(&x->dst0p, VS) || dmalloc(&x->dst0, VS))

@@ -757,7 +757,8 @@ int bp_resident_plan(bp_dev *d, const std::vector<unsigned> &slot_src, bool grad
     HIP_TRY(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, d->device));
     r.timeout = (unsigned long long)khz * 1000; /* a second */
     HIP_TRY(hipMalloc((void **)&r.memory, bytes));
-    HIP_TRY(hipMemcpy(r.memory, head.data(), head.size() * sizeof(unsigned), hipMemcpyHostToDevice));
+    if (copy_on(d->stream, r.memory, head.data(), head.size() * sizeof(unsigned), hipMemcpyHostToDevice))
+        return -1;
     r.counters = (unsigned *)r.memory;
     r.wg_node = r.counters + words;
     r.wg_slots = (unsigned short *)(r.wg_node + first.size());

@@ -449,13 +449,10 @@ int upload_plan(bp_dev *d, PlanBuilder &pb, bp_tree_plan **out)
         bp_tree_plan_free(p);
         return -1;
     }
-    bool ok = (ne == 0 || hipMemcpy(p->ent, ent.data(), ne * sizeof(TreeEntry), hipMemcpyHostToDevice) == hipSuccess) &&
-              (act.empty() || hipMemcpy(p->act_slot, act.data(), act.size() * 4, hipMemcpyHostToDevice) == hipSuccess) &&
-              hipMemcpy(p->wave_begin_d, wbeg.data(), wbeg.size() * 4, hipMemcpyHostToDevice) == hipSuccess &&
-              (wstart.empty() ||
-               hipMemcpy(p->wave_start_d, wstart.data(), wstart.size(), hipMemcpyHostToDevice) == hipSuccess);
-    if (!ok) {
-        bp_set_error("upload of the tree schedule failed");
+    if (copy_on(d->stream, p->ent, ent.data(), ne * sizeof(TreeEntry), hipMemcpyHostToDevice) ||
+        copy_on(d->stream, p->act_slot, act.data(), act.size() * 4, hipMemcpyHostToDevice) ||
+        copy_on(d->stream, p->wave_begin_d, wbeg.data(), wbeg.size() * 4, hipMemcpyHostToDevice) ||
+        copy_on(d->stream, p->wave_start_d, wstart.data(), wstart.size(), hipMemcpyHostToDevice)) {
         bp_tree_plan_free(p);
         return -1;
     }

@@ -1,0 +1,123 @@
+"""The library's host side against a HIP runtime on host memory
+(fake_hip.c), where every call is logged and kernels do nothing.  Each test
+runs in a process of its own: the fake must be there before the library."""
+from __future__ import annotations
+
+import ctypes as C
+import os
+import subprocess
+import sys
+from pathlib import Path
+
+import pytest
+
+HERE = Path(__file__).resolve().parent
+
+
+@pytest.fixture(scope="session")
+def fake(tmp_path_factory):
+    so = tmp_path_factory.mktemp("fake") / "fake_hip.so"
+    subprocess.run([os.environ.get("CC", "gcc"), "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__",
+                    "-I/opt/rocm/include", "-o", str(so), str(HERE / "fake_hip.c"), "-lpthread"], check=True)
+    return so
+
+
+@pytest.fixture
+def run(fake, request):
+    """Runs the function child_<name of the test> in a new process."""
+
+    def go(*args):
+        name = request.node.originalname.removeprefix("test_")
+        p = subprocess.run([sys.executable, str(HERE / "test_host_runtime.py"), str(fake), name, *map(str, args)],
+                           capture_output=True, text=True, timeout=120)
+        assert p.returncode == 0, p.stdout[-2000:] + p.stderr[-3000:]
+
+    return go
+
+
+class Fake:
+    """The fake in a child process, and the library on top of it."""
+
+    def __init__(self, so):
+        sys.path[:0] = [str(HERE), str(HERE.parent / "belief-propagation_amd")]
+        self.so = C.CDLL(so, mode=C.RTLD_GLOBAL)
+        self.so.fake_log.restype = C.c_char_p
+        self.so.fake_heap_calls.restype = C.c_ulonglong
+        self.so.fake_most_bytes.argtypes = [C.c_size_t]
+        import bp_ctypes as B
+
+        self.B, self.lib = B, B.load()
+        self.lib.bp_set_abort_on_error(0)
+
+    def log(self):
+        return [x.split() for x in self.so.fake_log().decode().splitlines()]
+
+    def calls(self, *names):
+        return [x for x in self.log() if x[0] in names]
+
+    def clear(self):
+        self.so.fake_clear()
+
+    def when(self, event, f):
+        """f() at the next capture or launch, once."""
+        setter = getattr(self.so, "fake_on_" + event)
+
+        def once():
+            setter(None)
+            f()
+
+        self.hook = C.CFUNCTYPE(None)(once)
+        setter(self.hook)
+
+    def device(self, nodes, states=2, family="c2"):
+        bn = self.B.generate(family, num_nodes=nodes, states_lo=states, states_hi=states, seed=nodes)
+        g = self.B.bn_to_graph(bn, levels=True)
+        self.lib.bp_bn_free(bn)
+        self.lib.bp_resident_shape.argtypes = [C.c_void_p, C.POINTER(C.c_uint)]
+        d, groups = self.B.Device(g), C.c_uint()
+        assert self.lib.bp_resident_shape(d.h, C.byref(groups)) > 0 and groups.value > 1
+        self.lib.graph_destroy(g)
+        return d
+
+
+# ---------------------------------------------------------------------------
+
+@pytest.mark.parametrize("what", ["device", "tree", "batch", "diff"])
+def test_uploads_beside_a_capture(run, what):
+    """Handles may be used from different threads: another handle comes and
+    goes while one captures its iterations."""
+    run(what)
+
+
+def child_uploads_beside_a_capture(fake, what):
+    from concurrent.futures import ThreadPoolExecutor
+
+    B, lib = fake.B, fake.lib
+
+    def other():
+        bn = B.generate("c5" if what == "diff" else "c2", num_nodes=500)
+        g = B.bn_to_graph(bn, levels=what == "tree")
+        if what == "diff":
+            h = C.c_void_p()
+            B.check(lib.bp_diff_create(bn, 500, 0, C.byref(h)), "bp_diff_create")
+            lib.bp_diff_free(h)
+        elif what == "batch":
+            batch = B.Batch()
+            batch.add(g)
+            batch.upload()
+            batch.free()
+        else:
+            B.Device(g).free()
+        lib.graph_destroy(g)
+        lib.bp_bn_free(bn)
+
+    a = fake.device(3000)
+    a.init()
+    with ThreadPoolExecutor(1) as thread:
+        fake.when("capture", lambda: thread.submit(other).result(timeout=60))
+        a.iterate(2)
+    assert len(fake.calls("stream")) == 2 and not fake.calls("memcpy", "memset", "devicesync")
+
+
+if __name__ == "__main__":
+    globals()["child_" + sys.argv[2]](Fake(sys.argv[1]), *sys.argv[3:])

@@ -603,16 +603,16 @@ void deal_slots(const std::vector<unsigned> &in_off, const std::vector<unsigned>
 }
 
 /* One resident launch at a time per device: the launches of two streams,
- * each partly on the chip, would wait for each other.  A launch on another
- * stream than the last one waits for that one: by an event recorded now if
- * the last stream is a handle's, which lives until bp_resident_free, or when
- * it was launched if it is a caller's. */
+ * each partly on the chip, would wait for each other.  Each leaves an event
+ * behind it on its own stream, and a launch on another stream waits for that.
+ * Nothing is put on another launch's stream: its owner may be capturing on it
+ * in another thread, or have queued more work since. */
 constexpr int MAX_DEVICES = 64;
 std::mutex turn_mu;
 struct {
-    bool any, foreign;
+    bool any;
     hipStream_t last;
-    hipEvent_t ev;
+    hipEvent_t ev; /* after the last launch */
 } turn[MAX_DEVICES];
 
 template <int S, bool MIXED, int NS, bool SINGLE>
@@ -673,22 +673,17 @@ int bp_resident_turn(int device, hipStream_t stream)
     auto &t = turn[device];
     if (!t.ev)
         HIP_TRY(hipEventCreateWithFlags(&t.ev, hipEventDisableTiming));
-    if (t.any && t.last != stream) {
-        if (!t.foreign)
-            HIP_TRY(hipEventRecord(t.ev, t.last));
+    if (t.any && t.last != stream)
         HIP_TRY(hipStreamWaitEvent(stream, t.ev, 0));
-    }
     return 0;
 }
 
-int bp_resident_turn_taken(int device, hipStream_t stream, bool foreign)
+int bp_resident_turn_taken(int device, hipStream_t stream)
 {
     auto &t = turn[device];
     t.any = true;
     t.last = stream;
-    t.foreign = foreign;
-    if (foreign)
-        HIP_TRY(hipEventRecord(t.ev, stream));
+    HIP_TRY(hipEventRecord(t.ev, stream));
     return 0;
 }
 
@@ -822,7 +817,7 @@ int bp_resident_launch(bp_dev *d, unsigned n, bool want_delta, bool until, float
         if (bp_resident_turn(d->device, d->stream))
             return -1;
         launch(d->S, d->mixed, a, r.ns, r.G, false, want_delta || until, d->stream);
-        if (bp_resident_turn_taken(d->device, d->stream, false))
+        if (bp_resident_turn_taken(d->device, d->stream))
             return -1;
     }
     if (want_delta && !until && !r.single)

@@ -198,6 +198,61 @@ def test_runs_on_two_handles_from_two_threads(lib, orc):
         lib.graph_destroy(h)
 
 
+def test_runs_beside_first_captures_of_another_handle(lib, orc):
+    """One thread's new handles run resident and then for the first time what
+    is captured into graphs (one and two iterations, the tree schedule), while
+    another thread's runs take their turns."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    print("runs beside captures", flush=True)
+
+    def graph(nodes, seed):
+        bn = B.generate("c2", num_nodes=nodes, states_hi=2, seed=seed)
+        g = B.bn_to_graph(bn, levels=True)
+        lib.bp_bn_free(bn)
+        return g
+
+    seeds = [70 + k for k in range(6)]
+    capturing = [(graph(3000, s), graph(3000, s), graph(3000, s)) for s in seeds]
+    g, h = graph(20000, 7), graph(20000, 7)
+
+    def first_times():
+        for a, t, _ in capturing:
+            dev = B.Device(a)
+            dev.init()
+            for n in (9, 1, 2, 5, 2):  # resident, captured, captured, resident, captured again
+                dev.iterate(n)
+            dev.download(a)
+            dev.tree()
+            dev.download(t)
+            dev.free()
+
+    def runs():
+        dev = B.Device(g)
+        for _ in range(200):
+            dev.restore()
+            dev.init()
+            dev.iterate(9)
+        dev.download(g)
+        assert shape(dev)[0] > 0  # none was given up
+        dev.free()
+
+    with ThreadPoolExecutor(2) as pool:
+        for f in (pool.submit(first_times), pool.submit(runs)):
+            f.result()
+    oracle_run(orc, h, 9)
+    check(g, h)
+    for a, t, want in capturing:
+        oracle_run(orc, want, 19)
+        check(a, want)
+        orc.tree_run(want)
+        assert same_bits(B.states(t), B.states(want)), bits_report(B.states(t), B.states(want))
+        for x in (a, t, want):
+            lib.graph_destroy(x)
+    for x in (g, h):
+        lib.graph_destroy(x)
+
+
 # (nodes, states, workgroups): 1, 2 and the most slots per thread of the
 # adjoint; the last of each state count is too large for it
 DIFF_CASES = [(200, 2), (5000, 2), (100000, 2), (150000, 2), (300000, 2), (300, 3), (3000, 3), (100000, 3),

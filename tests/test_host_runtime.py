@@ -119,5 +119,32 @@ def child_uploads_beside_a_capture(fake, what):
     assert len(fake.calls("stream")) == 2 and not fake.calls("memcpy", "memset", "devicesync")
 
 
+@pytest.mark.parametrize("captures", ["iterate", "tree"])
+def test_a_run_keeps_off_a_stream_in_capture(run, captures):
+    """Handles may be used from different threads: a resident run starts
+    while the handle that ran before it captures on its own stream."""
+    run(captures)
+
+
+def child_a_run_keeps_off_a_stream_in_capture(fake, captures):
+    from concurrent.futures import ThreadPoolExecutor
+
+    a, b = fake.device(3000), fake.device(5000)
+    a.init()
+    b.init()
+    a.iterate(9)
+    fake.clear()
+    with ThreadPoolExecutor(1) as other:
+        fake.when("capture", lambda: other.submit(b.iterate, 9).result(timeout=30))
+        a.iterate(2) if captures == "iterate" else a.tree()
+    begin, end = (fake.log().index(x[0]) for x in (fake.calls("begincapture"), fake.calls("endcapture")))
+    inside = fake.log()[begin:end]
+    own = fake.calls("begincapture")[0][1]
+    # b's run went to its own stream, after a's run, and left a's stream alone
+    assert [x for x in inside if x[0] == "launch" and x[1] != own and "captured" not in x]
+    assert [x for x in inside if x[0] == "wait" and x[1] != own]
+    assert not [x for x in inside if x[0] == "record" and x[2] == own], inside
+
+
 if __name__ == "__main__":
     globals()["child_" + sys.argv[2]](Fake(sys.argv[1]), *sys.argv[3:])

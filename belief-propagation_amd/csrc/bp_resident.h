@@ -161,10 +161,11 @@ __device__ __forceinline__ void factors(const float *p, unsigned cnt, float (&f)
 } // namespace bpk
 
 /* The host's side of a meeting (bp_resident.hip): the next run of the
- * handle, with `barriers` of them, and its turn on the device. */
+ * handle, with `barriers` of them, and its turn on the device; foreign: on a
+ * stream that is not the handle's own. */
 bpk::Meeting bp_resident_meeting(bp_dev *d, unsigned barriers, unsigned after);
 int bp_resident_turn(int device, hipStream_t stream);
-int bp_resident_turn_taken(int device, hipStream_t stream);
+int bp_resident_turn_taken(int device, hipStream_t stream, bool foreign);
 std::mutex &bp_resident_mutex();
 
 /* The unrolled forward and its adjoint (bp_diff.hip) as resident runs on a

@@ -605,12 +605,15 @@ void deal_slots(const std::vector<unsigned> &in_off, const std::vector<unsigned>
 /* One resident launch at a time per device: the launches of two streams,
  * each partly on the chip, would wait for each other.  Each leaves an event
  * behind it on its own stream, and a launch on another stream waits for that.
+ * After a launch on a caller's stream every launch waits: equal values do not
+ * say that it is the same stream (hipStreamPerThread is one value for all
+ * threads, and that of a destroyed stream is given out again).
  * Nothing is put on another launch's stream: its owner may be capturing on it
  * in another thread, or have queued more work since. */
 constexpr int MAX_DEVICES = 64;
 std::mutex turn_mu;
 struct {
-    bool any;
+    bool any, foreign; /* foreign: on a caller's stream */
     hipStream_t last;
     hipEvent_t ev; /* after the last launch */
 } turn[MAX_DEVICES];
@@ -673,15 +676,16 @@ int bp_resident_turn(int device, hipStream_t stream)
     auto &t = turn[device];
     if (!t.ev)
         HIP_TRY(hipEventCreateWithFlags(&t.ev, hipEventDisableTiming));
-    if (t.any && t.last != stream)
+    if (t.any && (t.foreign || t.last != stream))
         HIP_TRY(hipStreamWaitEvent(stream, t.ev, 0));
     return 0;
 }
 
-int bp_resident_turn_taken(int device, hipStream_t stream)
+int bp_resident_turn_taken(int device, hipStream_t stream, bool foreign)
 {
     auto &t = turn[device];
     t.any = true;
+    t.foreign = foreign;
     t.last = stream;
     HIP_TRY(hipEventRecord(t.ev, stream));
     return 0;
@@ -768,7 +772,7 @@ void bp_resident_free(bp_dev *d)
     bp_resident &r = d->res;
     {
         std::lock_guard<std::mutex> lock(turn_mu);
-        if (d->stream && d->device < MAX_DEVICES && turn[d->device].last == d->stream)
+        if (d->stream && d->device < MAX_DEVICES && !turn[d->device].foreign && turn[d->device].last == d->stream)
             turn[d->device].any = false; /* the stream has been waited for */
     }
     if (r.memory)
@@ -817,7 +821,7 @@ int bp_resident_launch(bp_dev *d, unsigned n, bool want_delta, bool until, float
         if (bp_resident_turn(d->device, d->stream))
             return -1;
         launch(d->S, d->mixed, a, r.ns, r.G, false, want_delta || until, d->stream);
-        if (bp_resident_turn_taken(d->device, d->stream))
+        if (bp_resident_turn_taken(d->device, d->stream, false))
             return -1;
     }
     if (want_delta && !until && !r.single)

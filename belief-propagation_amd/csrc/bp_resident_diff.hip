@@ -599,7 +599,7 @@ int bp_resident_diff_forward(bp_dev *d, unsigned K, float *st, float *buf, size_
             hipLaunchKernelGGL(k_forward_rescue<4>, dim3(1), dim3(BLOCK), 0, stream, a, st, buf, stride, K, m, word);
         HIP_TRY(hipGetLastError());
     }
-    return bp_resident_turn_taken(d->device, stream);
+    return bp_resident_turn_taken(d->device, stream, true);
 }
 
 int bp_resident_diff_backward(bp_dev *d, unsigned K, const float *st, const float *buf, size_t stride,
@@ -653,5 +653,5 @@ int bp_resident_diff_backward(bp_dev *d, unsigned K, const float *st, const floa
     else
         go(std::integral_constant<int, 4>());
     HIP_TRY(hipGetLastError());
-    return bp_resident_turn_taken(d->device, stream);
+    return bp_resident_turn_taken(d->device, stream, true);
 }

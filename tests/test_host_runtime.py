@@ -146,5 +146,28 @@ def child_a_run_keeps_off_a_stream_in_capture(fake, captures):
     assert not [x for x in inside if x[0] == "record" and x[2] == own], inside
 
 
+def test_equal_streams_of_two_callers(run):
+    """A caller's stream of the same value may be another one (destroyed and
+    made anew, or hipStreamPerThread of another thread)."""
+    run()
+
+
+def child_equal_streams_of_two_callers(fake):
+    B, lib, stream, passes = fake.B, fake.lib, C.c_void_p(0), []
+    for nodes in (3000, 4000):
+        bn = B.generate("c5", num_nodes=nodes)
+        h = C.c_void_p()
+        B.check(lib.bp_diff_create(bn, nodes, 0, C.byref(h)), "bp_diff_create")
+        info = (C.c_uint64 * 6)()
+        lib.bp_diff_info(h, info)
+        passes.append((h, (C.c_float * info[4])(), (C.c_float * (info[0] * info[3]))()))
+    for h, theta, out in passes:
+        fake.clear()
+        B.check(lib.bp_diff_set_log_params(h, theta, stream), "bp_diff_set_log_params")
+        B.check(lib.bp_diff_forward(h, 5, 2, out, stream), "bp_diff_forward")
+    # the second handle's run, on the stream value of the first's
+    assert len(fake.calls("wait")) == 1 and len(fake.calls("record")) == 1
+
+
 if __name__ == "__main__":
     globals()["child_" + sys.argv[2]](Fake(sys.argv[1]), *sys.argv[3:])

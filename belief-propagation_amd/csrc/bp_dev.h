@@ -7,7 +7,6 @@
 #include <hip/hip_runtime.h>
 
 #include <map>
-#include <utility>
 #include <vector>
 
 #include "bp_internal.h"
@@ -43,7 +42,12 @@ struct bp_resident_status {
 struct bp_resident {
     bool on = false;
     bool single = false;       /* one workgroup */
-    std::vector<std::pair<unsigned, unsigned>> pending; /* runs not waited for yet, with their iterations */
+    /* runs not waited for yet, oldest first, with their iterations */
+    static constexpr unsigned MOST_PENDING = 64;
+    struct {
+        unsigned run, n;
+    } pending[MOST_PENDING];
+    unsigned npending = 0;
     unsigned ns = 0, G = 0;    /* slots per thread, workgroups */
     unsigned limit = 0;        /* iterations per launch */
     unsigned run = 0, met = 0; /* launches, barriers met */

@@ -1293,6 +1293,19 @@ static bool use_resident(const bp_dev *d, unsigned n)
     return d->res.on && (d->res.single || n >= RESIDENT_LEAST);
 }
 
+/* Drops the runs that went through: those up to the last that said so. */
+static void forget_finished(bp_dev *d)
+{
+    bp_resident &r = d->res;
+    const unsigned last = __atomic_load_n(&d->status()->run, __ATOMIC_ACQUIRE);
+    for (unsigned i = r.npending; i-- > 0;)
+        if (r.pending[i].run == last) {
+            std::copy(r.pending + i + 1, r.pending + r.npending, r.pending);
+            r.npending -= i + 1;
+            return;
+        }
+}
+
 /* n resident iterations in as many launches as their exchange buffers ask
  * for.  With deltas the run is waited for; without them it may be left to
  * bp_settle.  *done: iterations that went through or may still; fewer than n
@@ -1302,6 +1315,16 @@ static int run_resident(bp_dev *d, unsigned n, double *deltas, double *partials,
     *done = 0;
     while (*done < n && d->res.on) {
         unsigned batch = std::min(n - *done, d->res.limit);
+        if (!deltas && d->res.npending == bp_resident::MOST_PENDING) {
+            forget_finished(d);
+            if (d->res.npending == bp_resident::MOST_PENDING)
+                HIP_TRY(hipStreamSynchronize(d->stream));
+            forget_finished(d);
+            if (d->res.npending == bp_resident::MOST_PENDING) { /* all given up */
+                d->res.on = false;
+                return 0;
+            }
+        }
         if (bp_resident_launch(d, batch, deltas != nullptr, false, 0.0f, 0.0, partials))
             return -1;
         if (deltas) {
@@ -1310,10 +1333,10 @@ static int run_resident(bp_dev *d, unsigned n, double *deltas, double *partials,
                 d->res.on = false;
                 return 0;
             }
-            d->res.pending.clear(); /* the runs before it went through too */
+            d->res.npending = 0; /* the runs before it went through too */
             std::copy(d->status()->deltas, d->status()->deltas + batch, deltas + *done);
         } else if (!d->res.single) {
-            d->res.pending.emplace_back(d->res.run, batch);
+            d->res.pending[d->res.npending++] = {d->res.run, batch};
         }
         if (batch & 1u)
             d->latest ^= 1;
@@ -1326,31 +1349,37 @@ static int run_resident(bp_dev *d, unsigned n, double *deltas, double *partials,
 
 static int iterate_launches(bp_dev *d, unsigned n, double *deltas);
 
-/* Waits for the resident runs that were not waited for and makes up for the
+/* Waits for the resident runs that were not waited for and takes back the
  * ones that were given up (each run checks that the one before it went
- * through, so they are the last ones): their iterations run with a launch
- * each. */
-int bp_settle(bp_dev *d)
+ * through, so they are the last ones).  *missing: their iterations, to be run
+ * with a launch each. */
+static int take_back(bp_dev *d, unsigned *missing)
 {
     bp_resident &r = d->res;
-    if (r.pending.empty())
+    *missing = 0;
+    if (!r.npending)
         return 0;
     HIP_TRY(hipStreamSynchronize(d->stream));
-    unsigned missing = 0;
-    if (!bp_resident_ran(d)) {
-        for (size_t i = r.pending.size(); i-- > 0 && r.pending[i].first != d->status()->run;) {
-            missing += r.pending[i].second;
-            d->bcur ^= 1;
-        }
+    forget_finished(d);
+    if (!bp_resident_ran(d))
         r.on = false;
+    for (unsigned i = 0; i < r.npending; ++i) {
+        *missing += r.pending[i].n;
+        d->bcur ^= 1;
     }
-    r.pending.clear();
-    if (!missing)
-        return 0;
-    if (missing & 1u)
+    r.npending = 0;
+    if (*missing & 1u)
         d->latest ^= 1;
-    d->swaps -= missing;
-    return iterate_launches(d, missing, nullptr);
+    d->swaps -= *missing;
+    return 0;
+}
+
+int bp_settle(bp_dev *d)
+{
+    unsigned missing;
+    if (take_back(d, &missing))
+        return -1;
+    return missing ? iterate_launches(d, missing, nullptr) : 0;
 }
 
 extern "C" int bp_loopy_iterate(bp_dev *d, unsigned int n, double *deltas)
@@ -1476,14 +1505,16 @@ extern "C" int bp_loopy_iterate_noalloc(bp_dev *d, unsigned int n, double *delta
         if (deltas)
             deltas += done;
     }
-    if (bp_settle(d) || ensure_buffer(d))
+    unsigned missing; /* of earlier runs that were given up */
+    if (take_back(d, &missing) || ensure_buffer(d))
         return -1;
-    for (unsigned i = 0; i < n; ++i) {
+    for (unsigned i = 0; i < missing + n; ++i) {
         LoopyArgs a = bp_make_args(d);
         a.partials = partials;
-        launch(d, ITER, a);
-        hipLaunchKernelGGL(k_finish, dim3(1), dim3(BLOCK), 0, d->stream, partials, d->NP, 1u, ds + i, nullptr,
-                           nullptr, 0.0f, 0, 0u);
+        launch(d, i < missing ? STEP : ITER, a);
+        if (i >= missing)
+            hipLaunchKernelGGL(k_finish, dim3(1), dim3(BLOCK), 0, d->stream, partials, d->NP, 1u, ds + (i - missing),
+                               nullptr, nullptr, 0.0f, 0, 0u);
         d->latest ^= 1;
         d->bcur ^= 1;
         d->swaps += 1;

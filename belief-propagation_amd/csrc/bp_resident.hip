@@ -615,7 +615,7 @@ std::mutex turn_mu;
 struct {
     bool any, foreign; /* foreign: on a caller's stream */
     hipStream_t last;
-    hipEvent_t ev; /* after the last launch */
+    hipEvent_t ev; /* after the last launch; created with the device's first plan */
 } turn[MAX_DEVICES];
 
 template <int S, bool MIXED, int NS, bool SINGLE>
@@ -673,9 +673,7 @@ std::mutex &bp_resident_mutex() { return turn_mu; }
 
 int bp_resident_turn(int device, hipStream_t stream)
 {
-    auto &t = turn[device];
-    if (!t.ev)
-        HIP_TRY(hipEventCreateWithFlags(&t.ev, hipEventDisableTiming));
+    const auto &t = turn[device];
     if (t.any && (t.foreign || t.last != stream))
         HIP_TRY(hipStreamWaitEvent(stream, t.ev, 0));
     return 0;
@@ -752,6 +750,11 @@ int bp_resident_plan(bp_dev *d, const std::vector<unsigned> &slot_src, bool grad
         r.limit = std::min<size_t>(r.limit, std::min<size_t>(256, std::max<size_t>(32, (8u << 20) / (4 * r.ring_stride))));
         bytes += r.ring_stride * r.limit * sizeof(float);
     }
+    {
+        std::lock_guard<std::mutex> lock(turn_mu);
+        if (!turn[d->device].ev)
+            HIP_TRY(hipEventCreateWithFlags(&turn[d->device].ev, hipEventDisableTiming));
+    }
     int khz = 0;
     HIP_TRY(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, d->device));
     r.timeout = (unsigned long long)khz * 1000; /* a second */
@@ -812,7 +815,7 @@ int bp_resident_launch(bp_dev *d, unsigned n, bool want_delta, bool until, float
     a.partials = r.single ? d->status()->deltas : partials;
     a.parts = r.parts;
     /* with the stop test bp_resident_ran says how many barriers there were */
-    a.meeting = bp_resident_meeting(d, until || r.single ? 0 : n + 1, r.pending.empty() ? 0u : r.pending.back().first);
+    a.meeting = bp_resident_meeting(d, until || r.single ? 0 : n + 1, r.npending ? r.pending[r.npending - 1].run : 0u);
     a.status = d->status();
     if (r.single) {
         launch(d->S, d->mixed, a, r.ns, 1, true, want_delta || until, d->stream);

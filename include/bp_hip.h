@@ -118,7 +118,9 @@ int bp_loopy_iterate(bp_dev *d, unsigned int n, double *deltas);
  * plus n exceed 524,288 doubles, i.e. from about 30M message edges on.
  * Calls that overlap on
  * one GPU share that array and race.  deltas (nullable) receives the n FP64
- * deltas; without it the call returns without waiting for the GPU. */
+ * deltas; without it the call returns without waiting for the GPU, unless 64
+ * resident runs of the handle are outstanding, or one of them was given up
+ * and has to be made up for (with launches, not with a graph). */
 int bp_loopy_iterate_noalloc(bp_dev *d, unsigned int n, double *deltas);
 
 /* Like loopy_propagate_until: runs until the stop test fires or

@@ -173,6 +173,30 @@ def test_a_run_that_is_given_up_is_made_up_for(lib, orc, nodes):
         lib.graph_destroy(x)
 
 
+@pytest.mark.parametrize("giving_up", [False, True])
+def test_many_runs_that_are_not_waited_for(lib, orc, giving_up):
+    """More runs outstanding than a handle keeps on record, by the entry point
+    that allocates nothing; given up from the 40th on."""
+    print(f"outstanding, given up {giving_up}", flush=True)
+    g, h = networks(lib, num_nodes=5000, states_hi=2, seed=13)
+    dev = B.Device(g)
+    dev.init()
+    for i in range(70):
+        if giving_up and i == 40:
+            give_up(dev)
+        B.check(lib.bp_loopy_iterate_noalloc(dev.h, 3, None), "bp_loopy_iterate_noalloc")
+    deltas = (C.c_double * 4)()
+    B.check(lib.bp_loopy_iterate_noalloc(dev.h, 4, deltas), "bp_loopy_iterate_noalloc")
+    dev.download(g)
+    assert (shape(dev)[0] == 0) == giving_up
+    want = oracle_run(orc, h, 214)
+    check(g, h)
+    assert np.allclose(deltas[:], want[-4:], rtol=1e-12, atol=0)
+    dev.free()
+    for x in (g, h):
+        lib.graph_destroy(x)
+
+
 def test_runs_on_two_handles_from_two_threads(lib, orc):
     """Resident runs of different handles take turns on a device."""
     from concurrent.futures import ThreadPoolExecutor

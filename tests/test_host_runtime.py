@@ -169,5 +169,34 @@ def child_equal_streams_of_two_callers(fake):
     assert len(fake.calls("wait")) == 1 and len(fake.calls("record")) == 1
 
 
+@pytest.mark.parametrize("deltas", [0, 1])
+def test_noalloc_allocates_nothing(run, deltas):
+    """No device or pinned memory, no events, no graphs, nothing from the
+    heap: from the first run of the process on, however many are outstanding,
+    and when runs are given up (here all of them)."""
+    run(deltas)
+
+
+def child_noalloc_allocates_nothing(fake, deltas):
+    d, lib = fake.device(3000), fake.lib
+    d.init()
+    out = (C.c_double * 20)()
+    lib.bp_loopy_iterate_noalloc(d.h, 0, None)  # (looks the scratch array up)
+    fake.clear()
+    calls = 70  # more than may be outstanding
+    for i in range(calls):
+        last = i == calls - 1
+        fake.B.check(lib.bp_loopy_iterate_noalloc(d.h, 20, out if last and int(deltas) else None), "noalloc")
+    assert fake.so.fake_heap_calls() == 0
+    log = fake.log()
+    assert {x[0] for x in log} <= {"launch", "record", "sync"}, {x[0] for x in log}
+    # 64 runs that were given up, their iterations, and those of the other
+    # calls with a delta for each
+    assert len(fake.calls("launch")) == 64 + 64 * 20 + 6 * 20 * 2
+    groups = C.c_uint()
+    assert lib.bp_resident_shape(d.h, C.byref(groups)) == 0
+    d.free()
+
+
 if __name__ == "__main__":
     globals()["child_" + sys.argv[2]](Fake(sys.argv[1]), *sys.argv[3:])

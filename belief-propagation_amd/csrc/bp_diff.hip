@@ -1184,7 +1184,9 @@ extern "C" int bp_diff_tables(bp_diff *x, float *out)
     return 0;
 }
 
-/* For checks: the handle a network's runs use, and the bytes of iterates that
- * are kept whatever the checkpoint interval. */
+/* For checks: the handle a network's runs use, whether a run of it was given
+ * up (ask after the stream has been waited for), and the bytes of iterates
+ * that are kept whatever the checkpoint interval. */
 extern "C" bp_dev *bp_diff_device(bp_diff *x) { return x->d; }
+extern "C" unsigned bp_diff_gave_up(const bp_diff *x) { return x->d->status()->gave_up; }
 extern "C" void bp_diff_set_keep(bp_diff *x, unsigned long long bytes) { x->keep_bytes = bytes; }

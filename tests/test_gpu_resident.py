@@ -277,6 +277,96 @@ def test_runs_beside_first_captures_of_another_handle(lib, orc):
         lib.graph_destroy(x)
 
 
+@pytest.mark.parametrize("nodes,lo,hi", [(200, 1, 3), (3000, 1, 3), (3000, 1, 4), (40000, 1, 4), (200, 1, 8),
+                                         (9000, 1, 6), (9000, 1, 8)])
+def test_nodes_of_one_state_match_oracle(lib, orc, nodes, lo, hi):
+    print(f"one-state nodes among {nodes}, up to {hi}", flush=True)
+    g, h = networks(lib, num_nodes=nodes, states_lo=lo, states_hi=hi, seed=600 + nodes + hi)
+    assert (B.view_u32(g.contents.node_num_vars, nodes) == 1).any()
+    dev = B.Device(g)
+    assert shape(dev)[0] > 0
+    dev.init()
+    got = dev.iterate(9, want_deltas=True)
+    dev.download(g)
+    want = oracle_run(orc, h, 9)
+    check(g, h)
+    assert np.allclose(got, want, rtol=1e-12, atol=0)
+    dev.free()
+    for x in (g, h):
+        lib.graph_destroy(x)
+
+
+@pytest.mark.parametrize("hi", [2, 4, 8])
+@pytest.mark.parametrize("entry", ["iterate", "deltas", "until", "noalloc"])
+def test_runs_are_given_up_where_no_workgroup_waits(lib, orc, entry, hi):
+    """That runs without patience do give up, by every entry point, and that
+    the results are the oracle's all the same."""
+    print(f"given up: {entry}, up to {hi} states", flush=True)
+    g, h = networks(lib, num_nodes=9000, states_hi=hi, seed=21 + hi)
+    dev = B.Device(g)
+    assert shape(dev)[1] > 1
+    give_up(dev)
+    dev.init()
+    n = 12
+    if entry == "until":
+        assert dev.until(1e-30, n) == n
+    elif entry == "noalloc":
+        B.check(lib.bp_loopy_iterate_noalloc(dev.h, n, None), "bp_loopy_iterate_noalloc")
+    else:
+        dev.iterate(n, want_deltas=entry == "deltas")
+    dev.download(g)
+    assert shape(dev) == (0, 0)  # launches from now on
+    oracle_run(orc, h, n)
+    check(g, h)
+    dev.free()
+    for x in (g, h):
+        lib.graph_destroy(x)
+
+
+@pytest.mark.parametrize("first", ["forward", "adjoint"])
+@pytest.mark.parametrize("nodes,states", [(3000, 2), (40000, 2), (5000, 3), (30000, 3), (8000, 4)])
+def test_gradients_are_given_up_where_no_workgroup_waits(lib, nodes, states, first):
+    """The forward and the adjoint, or the adjoint alone, made up for on the
+    device, and then a pass of launches, against launches throughout."""
+    from belief_network_wrapper import DifferentiableNetwork
+
+    print(f"gradient given up in the {first}, {nodes} nodes {states} states", flush=True)
+    lib.bp_diff_set_keep.argtypes = [C.c_void_p, C.c_ulonglong]
+    for f in (lib.bp_diff_device, lib.bp_diff_gave_up):
+        f.argtypes = [C.c_void_p]
+    lib.bp_diff_device.restype = C.c_void_p
+    lib.bp_resident_set_timeout.argtypes = [C.c_void_p, C.c_ulonglong]
+    lib.bp_resident_shape.argtypes = [C.c_void_p, C.POINTER(C.c_uint)]
+    got = []
+    for patient in (True, False):
+        net = DifferentiableNetwork.generate("c5" if states < 4 else "c1", num_nodes=nodes, states_lo=states,
+                                             states_hi=states, seed=11)
+        gen = torch.Generator(device="cuda").manual_seed(9)
+        theta = torch.randn(net.num_params, generator=gen, device="cuda").requires_grad_(True)
+        weight = torch.rand(net.V, net.S, generator=gen, device="cuda")
+        if patient:
+            lib.bp_diff_set_keep(net.h, 0)
+        else:
+            groups = C.c_uint()
+            assert lib.bp_resident_shape(lib.bp_diff_device(net.h), C.byref(groups)) > 0 and groups.value > 1
+        got.append([])
+        for _ in range(2):
+            theta.grad = None
+            if not patient and first == "forward":
+                lib.bp_resident_set_timeout(lib.bp_diff_device(net.h), 0)
+            b = net.beliefs_from_log(theta, 5, 2)
+            if not patient and first == "adjoint":
+                torch.cuda.synchronize()
+                lib.bp_resident_set_timeout(lib.bp_diff_device(net.h), 0)
+            (b * weight).sum().backward()
+            torch.cuda.synchronize()
+            assert lib.bp_diff_gave_up(net.h) == (0 if patient else 1)
+            got[-1] += [b.detach().cpu().numpy(), theta.grad.cpu().numpy()]
+        net.close()
+    for x, y in zip(*got):
+        assert same_bits(x, y)
+
+
 # (nodes, states, workgroups): 1, 2 and the most slots per thread of the
 # adjoint; the last of each state count is too large for it
 DIFF_CASES = [(200, 2), (5000, 2), (100000, 2), (150000, 2), (300000, 2), (300, 3), (3000, 3), (100000, 3),

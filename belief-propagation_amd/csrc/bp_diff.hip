@@ -842,8 +842,6 @@ extern "C" int bp_diff_set_log_params(bp_diff *x, const float *theta, void *stre
 
 static int diff_storage(bp_diff *x, unsigned K, unsigned c)
 {
-    if (x->K == K && x->c == c && x->final_st)
-        return 0;
     diff_release_storage(x);
     size_t VS = x->stride;
     unsigned nck = K / c + 1;
@@ -949,7 +947,10 @@ extern "C" int bp_diff_forward(bp_diff *x, unsigned int K, unsigned int c, float
     HIP_TRY(hipSetDevice(x->d->device));
     size_t VS = (size_t)x->V * x->SP;
     const unsigned every = 2 * ((size_t)K + 1) * x->stride * sizeof(float) <= x->keep_bytes ? 1 : c;
-    if (diff_storage(x, K, every)) {
+    /* (where the memory for all of them is not to be had, the storage for the
+     * interval stays: trying again each time freed and allocated everything) */
+    const bool stored = x->final_st && x->K == K && (x->c == every || x->c == c);
+    if (!stored && diff_storage(x, K, every)) {
         if (every == c)
             return -1;
         (void)hipGetLastError(); /* not the memory for all of them */

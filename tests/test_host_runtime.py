@@ -198,5 +198,33 @@ def child_noalloc_allocates_nothing(fake, deltas):
     d.free()
 
 
+def test_storage_is_kept_where_not_every_iterate_fits(run):
+    """Passes after the first allocate nothing, with the memory for every
+    iterate and without it."""
+    run()
+
+
+def child_storage_is_kept_where_not_every_iterate_fits(fake):
+    B, lib, nodes, K, every = fake.B, fake.lib, 3000, 30, 5
+    bn = B.generate("c5", num_nodes=nodes)
+    h = C.c_void_p()
+    B.check(lib.bp_diff_create(bn, nodes, 0, C.byref(h)), "bp_diff_create")
+    info = (C.c_uint64 * 6)()
+    lib.bp_diff_info(h, info)
+    row = 4 * info[0] * info[3]
+    theta, out, grad = (C.c_float * info[4])(), (C.c_float * (row // 4))(), (C.c_float * info[4])()
+    for most in (2**62, (K + 1) * row // 2):  # in bytes of one allocation
+        fake.so.fake_most_bytes(most)
+        for i in range(3):
+            fake.clear()
+            B.check(lib.bp_diff_set_log_params(h, theta, None), "bp_diff_set_log_params")
+            B.check(lib.bp_diff_forward(h, K, every, out, None), "bp_diff_forward")
+            B.check(lib.bp_diff_backward_log(h, out, grad, None), "bp_diff_backward_log")
+            B.check(lib.bp_diff_forward(h, K, every, out, None), "bp_diff_forward")
+            used = fake.calls("malloc", "free", "instantiate", "graphdestroy")
+            assert bool(used) == (i == 0), used
+        K += 1  # anew
+
+
 if __name__ == "__main__":
     globals()["child_" + sys.argv[2]](Fake(sys.argv[1]), *sys.argv[3:])

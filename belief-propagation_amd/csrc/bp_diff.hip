@@ -923,14 +923,44 @@ static void enqueue_forward(bp_diff *x, hipStream_t st)
     hipLaunchKernelGGL(k_copy, dim3(blocks_for(n)), dim3(256), 0, st, sp, x->final_st, n);
 }
 
-/* Whether the iterates, all kept, are run resident (not into a graph that is
- * being captured: a run counts its barriers once). */
-static bool use_resident(bp_diff *x, hipStream_t st)
+static bool is_capturing(hipStream_t st)
 {
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     if (st && hipStreamIsCapturing(st, &capturing) != hipSuccess)
         (void)hipGetLastError();
-    return x->c == 1 && capturing == hipStreamCaptureStatusNone && bp_resident_diff_fits(x->d, x->max_in);
+    return capturing != hipStreamCaptureStatusNone;
+}
+
+/* Whether the iterates, all kept, are run resident (not into a graph that is
+ * being captured: a run counts its barriers once). */
+static bool use_resident(bp_diff *x, hipStream_t st)
+{
+    return x->c == 1 && !is_capturing(st) && bp_resident_diff_fits(x->d, x->max_in);
+}
+
+/* enqueue's launches on the caller's stream, by way of a graph that is kept
+ * for this K and c; one by one into a graph of the caller's, which a graph
+ * launched here would not become part of. */
+static int run_launches(bp_diff *x, std::map<std::pair<unsigned, unsigned>, hipGraphExec_t> &graphs,
+                        void (*enqueue)(bp_diff *, hipStream_t), hipStream_t st)
+{
+    if (is_capturing(st)) {
+        enqueue(x, st);
+        return 0;
+    }
+    const auto key = std::make_pair(x->K, x->c);
+    auto it = graphs.find(key);
+    if (it == graphs.end()) {
+        hipGraphExec_t exec = nullptr;
+        if (capture_begin(x))
+            return -1;
+        enqueue(x, x->d->stream);
+        if (capture_end(x, &exec))
+            return -1;
+        it = graphs.emplace(key, exec).first;
+    }
+    HIP_TRY(hipGraphLaunch(it->second, st));
+    return 0;
 }
 
 extern "C" int bp_diff_forward(bp_diff *x, unsigned int K, unsigned int c, float *beliefs, void *stream)
@@ -947,9 +977,15 @@ extern "C" int bp_diff_forward(bp_diff *x, unsigned int K, unsigned int c, float
     HIP_TRY(hipSetDevice(x->d->device));
     size_t VS = (size_t)x->V * x->SP;
     const unsigned every = 2 * ((size_t)K + 1) * x->stride * sizeof(float) <= x->keep_bytes ? 1 : c;
+    hipStream_t st = (hipStream_t)stream;
     /* (where the memory for all of them is not to be had, the storage for the
      * interval stays: trying again each time freed and allocated everything) */
     const bool stored = x->final_st && x->K == K && (x->c == every || x->c == c);
+    if (!stored && is_capturing(st)) {
+        bp_set_error("bp_diff_forward: the first call with %u iterations and interval %u allocates and cannot be captured",
+                     K, c);
+        return -1;
+    }
     if (!stored && diff_storage(x, K, every)) {
         if (every == c)
             return -1;
@@ -959,7 +995,6 @@ extern "C" int bp_diff_forward(bp_diff *x, unsigned int K, unsigned int c, float
             return -1;
     }
     c = x->c;
-    hipStream_t st = (hipStream_t)stream;
     /* the ck_st[0] slot is the initial beliefs themselves */
     hipLaunchKernelGGL(k_copy, dim3(blocks_for(VS)), dim3(256), 0, st, x->st0, x->ck_st, VS);
     if (K && use_resident(x, st)) {
@@ -972,18 +1007,8 @@ extern "C" int bp_diff_forward(bp_diff *x, unsigned int K, unsigned int c, float
         x->have_forward = x->kept = true;
         return 0;
     }
-    auto key = std::make_pair(K, c);
-    auto it = x->fwd_graphs.find(key);
-    if (it == x->fwd_graphs.end()) {
-        hipGraphExec_t exec = nullptr;
-        if (capture_begin(x))
-            return -1;
-        enqueue_forward(x, x->d->stream);
-        if (capture_end(x, &exec))
-            return -1;
-        it = x->fwd_graphs.emplace(key, exec).first;
-    }
-    HIP_TRY(hipGraphLaunch(it->second, st));
+    if (run_launches(x, x->fwd_graphs, enqueue_forward, st))
+        return -1;
     hipLaunchKernelGGL(k_gather_rows, dim3(blocks_for(VS)), dim3(256), 0, st, x->final_st, x->perm_d, beliefs, x->V,
                        x->SP);
     HIP_TRY(hipGetLastError());
@@ -1123,18 +1148,8 @@ extern "C" int bp_diff_backward_ex(bp_diff *x, const float *grad_beliefs, float 
         if (x->kept) /* the launches look for the last beliefs here */
             hipLaunchKernelGGL(k_copy, dim3(blocks_for(VS)), dim3(256), 0, st, x->ck_st + x->K * x->stride,
                                x->final_st, VS);
-        auto key = std::make_pair(x->K, x->c);
-        auto it = x->bwd_graphs.find(key);
-        if (it == x->bwd_graphs.end()) {
-            hipGraphExec_t exec = nullptr;
-            if (capture_begin(x))
-                return -1;
-            enqueue_backward(x, x->d->stream);
-            if (capture_end(x, &exec))
-                return -1;
-            it = x->bwd_graphs.emplace(key, exec).first;
-        }
-        HIP_TRY(hipGraphLaunch(it->second, st));
+        if (run_launches(x, x->bwd_graphs, enqueue_backward, st))
+            return -1;
     }
     if (grad_params)
         FOR_STATES(x->S, launch_param_grad, x, false, grad_params, st);

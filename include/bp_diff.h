@@ -30,7 +30,9 @@
  * for every parameter entry given dL/dbeliefs after iteration K.  Networks
  * whose tables, and their gradients, fit on the chip go through all
  * iterations in one launch, forward and backward; under stream capture each
- * iteration is a launch of its own.
+ * iteration is a launch of its own.  The first call with a K and c allocates
+ * and cannot be captured.  A captured graph uses what is stored for its K and
+ * c: a call with another pair, or bp_diff_free, ends its use.
  *
  * Limits: every node has the same state count, and no node has more than
  * 128 in-edges (64 for more than 4 states); bp_diff_create reports others.

@@ -17,6 +17,8 @@ accumulate multiplicatively every iteration (graph.c:1008-1012), and after
 """
 from __future__ import annotations
 
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
@@ -24,6 +26,7 @@ import torch
 import bp_ctypes as B
 import bp_diff_oracle as D
 from belief_network_wrapper import DifferentiableNetwork
+from conftest import same_bits
 
 pytestmark = pytest.mark.gpu
 
@@ -211,6 +214,55 @@ def test_fused_softmax_matches_torch_softmax(lib):
     print(f"fused softmax: beliefs max |diff| {float((b1 - b2).abs().max()):.2e}, gradient rel l2 {rel:.2e}")
     assert rel < 1e-3
     teardown(lib, bn, g, net)
+
+
+@pytest.mark.parametrize("nodes,every,keep", [(250, 3, True), (2000, 3, True), (2000, 3, False), (2000, 9, False),
+                                              (60000, 2, True)])
+def test_a_captured_step_gives_the_eager_one(lib, nodes, every, keep):
+    """A step captured into a caller's graph and replayed with other
+    parameters, eager steps and waits between the replays: networks of one
+    workgroup, of several, and with checkpoints."""
+    print(f"captured step, {nodes} nodes, every {every}, keep {keep}", flush=True)
+    K = 7
+    net = DifferentiableNetwork.generate("c5", num_nodes=nodes, seed=12)
+    if not keep:
+        lib.bp_diff_set_keep.argtypes = [C.c_void_p, C.c_ulonglong]
+        lib.bp_diff_set_keep(net.h, 0)
+    gen = torch.Generator(device="cuda").manual_seed(12)
+    thetas = [torch.randn(net.num_params, generator=gen, device="cuda") for _ in range(4)]
+    gin = torch.rand(net.V, net.stride, generator=gen, device="cuda")
+    theta, out, grad = thetas[0].clone(), torch.empty_like(gin), torch.empty_like(thetas[0])
+
+    def step():
+        stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+        ptr = [C.c_void_p(x.data_ptr()) for x in (theta, out, gin, grad)]
+        B.check(lib.bp_diff_set_log_params(net.h, ptr[0], stream), "bp_diff_set_log_params")
+        B.check(lib.bp_diff_forward(net.h, K, every, ptr[1], stream), "bp_diff_forward")
+        B.check(lib.bp_diff_backward_log(net.h, ptr[2], ptr[3], stream), "bp_diff_backward_log")
+
+    def results(run, t):
+        theta.copy_(t)
+        out.fill_(-1)
+        grad.fill_(-1)
+        torch.cuda.synchronize()
+        run()
+        torch.cuda.synchronize()
+        return out.cpu().numpy(), grad.cpu().numpy()
+
+    first, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with pytest.raises(RuntimeError, match="cannot be captured"):
+        with torch.cuda.graph(first, stream=stream):
+            step()
+    want = [results(step, t) for t in thetas]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        step()
+    for i, t in enumerate(thetas):
+        for x, y in zip(results(graph.replay, t), want[i]):
+            assert same_bits(x, y)
+        for x, y in zip(results(step, thetas[i - 1]), want[i - 1]):
+            assert same_bits(x, y)
+    net.close()
 
 
 def test_full_scale_c5(lib):

@@ -34,6 +34,7 @@
 #include <cstdio>
 #include <cstring>
 #include <map>
+#include <mutex>
 #include <string>
 #include <type_traits>
 #include <unordered_map>
@@ -182,6 +183,7 @@ struct bp_batch {
     double *d_partials = nullptr;
     double *d_deltas = nullptr;
     float *h_stage = nullptr; /* pinned: one instance's rows, for downloads */
+    std::mutex download_mu;   /* several threads may read different instances */
     unsigned deltas_cap = 0;
     Shape shapes[2];
 
@@ -883,6 +885,7 @@ extern "C" int bp_batch_download(bp_batch *b, unsigned int index, Graph_t g)
     HIP_TRY(hipSetDevice(b->device));
     size_t r0 = b->node_row_off[index], rn = b->node_row_off[index + 1] - r0;
     size_t q0 = b->msg_row_off[index], qn = b->msg_row_off[index + 1] - q0;
+    std::lock_guard<std::mutex> lock(b->download_mu);
     float *st = b->h_stage, *m0 = st + rn, *m1 = m0 + qn;
     /* one launch that writes pinned memory: three copies took 30 us more,
      * most of a small instance's download */

@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include <map>
+#include <mutex>
 #include <vector>
 
 #include "bp_internal.h"
@@ -86,6 +87,7 @@ struct bp_dev {
     size_t jfloats = 0;               /* floats in J */
     char *h_stage = nullptr;          /* pinned host memory: a bp_resident_status, then staging for transfers */
     size_t h_stage_n = 0;             /* the staging's capacity in floats */
+    std::mutex download_mu;           /* results may be read by several threads; they share the staging */
     static constexpr unsigned SLICES = 8;
     hipEvent_t slice_ev[SLICES] = {};  /* slices of a download, created on first use */
     unsigned *perm_d = nullptr;        /* [V] node -> device node */

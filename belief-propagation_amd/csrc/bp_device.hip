@@ -1832,6 +1832,7 @@ extern "C" int bp_download_states(bp_dev *d, float *out)
 {
     bp_clear_error();
     HIP_TRY(hipSetDevice(d->device));
+    std::lock_guard<std::mutex> lock(d->download_mu);
     if (bp_settle(d))
         return -1;
     if (d->V == 0)
@@ -1883,6 +1884,7 @@ extern "C" int bp_download(bp_dev *d, Graph_t g)
         return -1;
     }
     HIP_TRY(hipSetDevice(d->device));
+    std::lock_guard<std::mutex> lock(d->download_mu);
     if (bp_settle(d))
         return -1;
     const size_t V = d->V, E = d->E, VS = V * d->SP, ES = E * d->SP;

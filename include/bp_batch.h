@@ -80,7 +80,8 @@ int bp_batch_iterate(bp_batch *b, unsigned int n, double *deltas);
 /* Writes instance `index`'s beliefs and both message arrays into g (the
  * network that was added, or one with the same structure), as if
  * init_previous_edge and the iterations since had run on g itself,
- * message pointer swaps included. */
+ * message pointer swaps included.  Several threads may read different
+ * instances of one batch; their transfers are made one after the other. */
 int bp_batch_download(bp_batch *b, unsigned int index, Graph_t g);
 
 int bp_batch_sync(bp_batch *b);

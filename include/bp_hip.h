@@ -12,7 +12,8 @@
  *  2. A device-resident handle (bp_dev) for callers that keep the graph on
  *     the GPU across calls: upload once, iterate, download when needed.  A
  *     handle owns one HIP stream; calls on different handles may run from
- *     different threads.
+ *     different threads, and so may several threads' bp_download and
+ *     bp_download_states of one handle (one after the other).
  *
  * Reference interfaces replaced:
  *   loopy_propagate_until_hip       <- loopy_propagate_until_cuda

@@ -226,5 +226,46 @@ def child_storage_is_kept_where_not_every_iterate_fits(fake):
         K += 1  # anew
 
 
+@pytest.mark.parametrize("what", ["batch", "states"])
+def test_downloads_of_one_handle_from_two_threads(run, what):
+    """They share the handle's staging memory, so the second transfer starts
+    when the first one's rows have been read."""
+    run(what)
+
+
+def child_downloads_of_one_handle_from_two_threads(fake, what):
+    import time
+    from concurrent.futures import ThreadPoolExecutor
+
+    B, lib = fake.B, fake.lib
+    if what == "batch":
+        bn = B.generate("c4net", num_nodes=300, states_hi=4)
+        graphs = [B.bn_to_graph(bn) for _ in range(2)]
+        b = B.Batch()
+        for g in graphs:
+            b.add(g)
+        b.upload()
+        b.init()
+        download = lambda i: b.download(i, graphs[i])  # noqa: E731
+    else:
+        d = fake.device(3000)
+        info = d.info()
+        rows = [(C.c_float * (info["V"] * info["stride"]))() for _ in range(2)]
+        download = lambda i: B.check(lib.bp_download_states(d.h, rows[i]), "bp_download_states")  # noqa: E731
+    seen = []
+
+    def meanwhile():
+        seen.append(thread.submit(download, 1))
+        time.sleep(0.3)
+        seen.append(len(fake.calls("launch")))
+
+    with ThreadPoolExecutor(1) as thread:
+        fake.clear()
+        fake.when("launch", meanwhile)
+        download(0)
+        seen[0].result(timeout=30)
+    assert seen[1] == 1 and len(fake.calls("launch")) == 2
+
+
 if __name__ == "__main__":
     globals()["child_" + sys.argv[2]](Fake(sys.argv[1]), *sys.argv[3:])

@@ -183,6 +183,7 @@ _SIGNATURES = {
     "bp_dev_info": (C.c_int, [C.c_void_p, C.POINTER(C.c_uint64)]),
     "bp_loopy_algorithmic_bytes": (C.c_double, [C.c_void_p]),
     "bp_profile_loopy": (C.c_int, [C.c_void_p, C.c_uint, f32p]),
+    "bp_profile_run": (C.c_int, [C.c_void_p, C.c_uint, f32p]),
     # bp_model.h
     "bp_gen_preset": (C.c_int, [C.c_char_p, C.POINTER(GenParams)]),
     "bp_bn_generate": (C.c_void_p, [C.POINTER(GenParams)]),
@@ -496,6 +497,11 @@ class Device:
         ms = (C.c_float * n)()
         check(self.lib.bp_profile_loopy(self.h, n, ms), "bp_profile_loopy")
         return np.array(ms[:n], dtype=np.float64)
+
+    def profile_run(self, n: int) -> float | None:
+        """ms of the launch that runs n iterations; None where each is a launch of its own"""
+        ms = C.c_float()
+        return ms.value if self.lib.bp_profile_run(self.h, n, C.byref(ms)) == 0 else None
 
     def free(self):
         if self.h:

@@ -186,7 +186,7 @@ void bp_build_chunks(const std::vector<unsigned> &in_off, unsigned V, unsigned c
 int bp_resident_plan(bp_dev *d, const std::vector<unsigned> &slot_src, bool gradients, int cus);
 void bp_resident_free(bp_dev *d);
 int bp_resident_launch(bp_dev *d, unsigned n, bool want_delta, bool until, float conv, double previous,
-                       double *partials);
+                       double *partials, const hipEvent_t *ev = nullptr);
 bool bp_resident_ran(bp_dev *d, bool until = false);
 extern "C" unsigned long long bp_resident_set_timeout(bp_dev *d, unsigned long long ticks);
 extern "C" unsigned bp_resident_shape(const bp_dev *d, unsigned *workgroups);

@@ -1310,7 +1310,8 @@ static void forget_finished(bp_dev *d)
  * for.  With deltas the run is waited for; without them it may be left to
  * bp_settle.  *done: iterations that went through or may still; fewer than n
  * when a run was given up (res.on is then off). */
-static int run_resident(bp_dev *d, unsigned n, double *deltas, double *partials, unsigned *done)
+static int run_resident(bp_dev *d, unsigned n, double *deltas, double *partials, unsigned *done,
+                        const hipEvent_t *ev = nullptr)
 {
     *done = 0;
     while (*done < n && d->res.on) {
@@ -1325,7 +1326,7 @@ static int run_resident(bp_dev *d, unsigned n, double *deltas, double *partials,
                 return 0;
             }
         }
-        if (bp_resident_launch(d, batch, deltas != nullptr, false, 0.0f, 0.0, partials))
+        if (bp_resident_launch(d, batch, deltas != nullptr, false, 0.0f, 0.0, partials, ev))
             return -1;
         if (deltas) {
             HIP_TRY(hipStreamSynchronize(d->stream));
@@ -1817,6 +1818,37 @@ extern "C" int bp_profile_loopy(bp_dev *d, unsigned int n, float *ms)
     for (auto &e : ev)
         (void)hipEventDestroy(e);
     return 0;
+}
+
+extern "C" int bp_profile_run(bp_dev *d, unsigned int n, float *ms)
+{
+    bp_clear_error();
+    if (!d || !ms) {
+        bp_set_error("bp_profile_run: NULL argument");
+        return -1;
+    }
+    HIP_TRY(hipSetDevice(d->device));
+    if (bp_settle(d) || ensure_buffer(d))
+        return -1;
+    if (!use_resident(d, n) || n == 0 || n > d->res.limit) {
+        bp_set_error("bp_profile_run: %u iterations of this handle are not one launch", n);
+        return -1;
+    }
+    hipEvent_t ev[2];
+    HIP_TRY(hipEventCreate(&ev[0]));
+    HIP_TRY(hipEventCreate(&ev[1]));
+    std::vector<double> deltas(n);
+    unsigned done = 0;
+    int rc = run_resident(d, n, deltas.data(), d->partials, &done, ev);
+    if (rc == 0 && done != n) {
+        bp_set_error("bp_profile_run: the run was given up");
+        rc = -1;
+    }
+    if (rc == 0)
+        HIP_TRY(hipEventElapsedTime(ms, ev[0], ev[1]));
+    (void)hipEventDestroy(ev[0]);
+    (void)hipEventDestroy(ev[1]);
+    return rc;
 }
 
 /* ------------------------------------------------------------------------ */

@@ -784,9 +784,10 @@ void bp_resident_free(bp_dev *d)
 }
 
 /* Enqueues up to n (<= res.limit) iterations: with want_delta their deltas
- * go to the status's deltas, and with `until` the stop test ends the run. */
+ * go to the status's deltas, and with `until` the stop test ends the run.  ev
+ * (nullable): events before and after the kernel. */
 int bp_resident_launch(bp_dev *d, unsigned n, bool want_delta, bool until, float conv, double previous,
-                       double *partials)
+                       double *partials, const hipEvent_t *ev)
 {
     bp_resident &r = d->res;
     ResArgs a;
@@ -818,12 +819,20 @@ int bp_resident_launch(bp_dev *d, unsigned n, bool want_delta, bool until, float
     a.meeting = bp_resident_meeting(d, until || r.single ? 0 : n + 1, r.npending ? r.pending[r.npending - 1].run : 0u);
     a.status = d->status();
     if (r.single) {
+        if (ev)
+            HIP_TRY(hipEventRecord(ev[0], d->stream));
         launch(d->S, d->mixed, a, r.ns, 1, true, want_delta || until, d->stream);
+        if (ev)
+            HIP_TRY(hipEventRecord(ev[1], d->stream));
     } else {
         std::lock_guard<std::mutex> lock(turn_mu);
         if (bp_resident_turn(d->device, d->stream))
             return -1;
+        if (ev)
+            HIP_TRY(hipEventRecord(ev[0], d->stream));
         launch(d->S, d->mixed, a, r.ns, r.G, false, want_delta || until, d->stream);
+        if (ev)
+            HIP_TRY(hipEventRecord(ev[1], d->stream));
         if (bp_resident_turn_taken(d->device, d->stream, false))
             return -1;
     }

@@ -162,6 +162,13 @@ double bp_loopy_algorithmic_bytes(const bp_dev *d);
  * ms[i] gets iteration i. */
 int bp_profile_loopy(bp_dev *d, unsigned int n, float *ms);
 
+/* Times the launch that bp_loopy_iterate makes for n iterations with deltas,
+ * by HIP events before and after it; *ms gets its duration.  An error where
+ * they are not one launch: the network does not fit on the chip, a run was
+ * given up, or n is 0 or beyond what a launch holds (32 iterations at least;
+ * fewer than three iterations only if the network fits one workgroup). */
+int bp_profile_run(bp_dev *d, unsigned int n, float *ms);
+
 #ifdef __cplusplus
 }
 #endif

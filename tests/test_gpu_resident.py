@@ -296,6 +296,27 @@ def test_nodes_of_one_state_match_oracle(lib, orc, nodes, lo, hi):
         lib.graph_destroy(x)
 
 
+@pytest.mark.parametrize("nodes", [900, 9000])
+def test_the_timed_launch_is_the_run(lib, orc, nodes):
+    """bp_profile_run leaves what bp_loopy_iterate would, and refuses what is
+    not one launch."""
+    g, h = networks(lib, num_nodes=nodes, states_hi=2, seed=31)
+    dev = B.Device(g)
+    dev.init()
+    assert dev.profile_run(20) > 0
+    assert dev.profile_run(0) is None and dev.profile_run(257) is None
+    dev.download(g)
+    oracle_run(orc, h, 20)
+    check(g, h)
+    if shape(dev)[1] > 1:
+        give_up(dev)
+        assert dev.profile_run(20) is None and "given up" in B.last_error()
+        assert dev.profile_run(20) is None and "not one launch" in B.last_error()
+    dev.free()
+    for x in (g, h):
+        lib.graph_destroy(x)
+
+
 @pytest.mark.parametrize("hi", [2, 4, 8])
 @pytest.mark.parametrize("entry", ["iterate", "deltas", "until", "noalloc"])
 def test_runs_are_given_up_where_no_workgroup_waits(lib, orc, entry, hi):

@@ -188,6 +188,7 @@ void bp_resident_free(bp_dev *d);
 int bp_resident_launch(bp_dev *d, unsigned n, bool want_delta, bool until, float conv, double previous,
                        double *partials, const hipEvent_t *ev = nullptr);
 bool bp_resident_ran(bp_dev *d, bool until = false);
+std::mutex &bp_resident_mutex(); /* held while a handle's stream is in capture */
 extern "C" unsigned long long bp_resident_set_timeout(bp_dev *d, unsigned long long ticks);
 extern "C" unsigned bp_resident_shape(const bp_dev *d, unsigned *workgroups);
 int bp_settle(bp_dev *d); /* before a handle's arrays are used otherwise (bp_device.hip) */

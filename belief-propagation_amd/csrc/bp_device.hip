@@ -1413,9 +1413,12 @@ static int iterate_launches(bp_dev *d, unsigned n, double *deltas)
         auto it = d->graphs.find(key);
         if (it == d->graphs.end()) {
             hipGraph_t graph;
-            HIP_TRY(hipStreamBeginCapture(d->stream, hipStreamCaptureModeThreadLocal));
-            enqueue_iterations(d, batch, d->latest, d->bcur, deltas != nullptr);
-            HIP_TRY(hipStreamEndCapture(d->stream, &graph));
+            {
+                std::lock_guard<std::mutex> lock(bp_resident_mutex());
+                HIP_TRY(hipStreamBeginCapture(d->stream, hipStreamCaptureModeThreadLocal));
+                enqueue_iterations(d, batch, d->latest, d->bcur, deltas != nullptr);
+                HIP_TRY(hipStreamEndCapture(d->stream, &graph));
+            }
             hipGraphExec_t exec;
             hipError_t e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
             (void)hipGraphDestroy(graph);

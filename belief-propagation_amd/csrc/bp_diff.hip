@@ -952,11 +952,14 @@ static int run_launches(bp_diff *x, std::map<std::pair<unsigned, unsigned>, hipG
     auto it = graphs.find(key);
     if (it == graphs.end()) {
         hipGraphExec_t exec = nullptr;
-        if (capture_begin(x))
-            return -1;
-        enqueue(x, x->d->stream);
-        if (capture_end(x, &exec))
-            return -1;
+        {
+            std::lock_guard<std::mutex> lock(bp_resident_mutex());
+            if (capture_begin(x))
+                return -1;
+            enqueue(x, x->d->stream);
+            if (capture_end(x, &exec))
+                return -1;
+        }
         it = graphs.emplace(key, exec).first;
     }
     HIP_TRY(hipGraphLaunch(it->second, st));

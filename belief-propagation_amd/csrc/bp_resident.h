@@ -5,8 +5,6 @@
  */
 #pragma once
 
-#include <mutex>
-
 #include "bp_dev.h"
 
 namespace bpk {
@@ -166,7 +164,6 @@ __device__ __forceinline__ void factors(const float *p, unsigned cnt, float (&f)
 bpk::Meeting bp_resident_meeting(bp_dev *d, unsigned barriers, unsigned after);
 int bp_resident_turn(int device, hipStream_t stream);
 int bp_resident_turn_taken(int device, hipStream_t stream, bool foreign);
-std::mutex &bp_resident_mutex();
 
 /* The unrolled forward and its adjoint (bp_diff.hip) as resident runs on a
  * caller's stream.  st, buf: the iterates' beliefs and combine buffers, K + 1

@@ -603,19 +603,27 @@ void deal_slots(const std::vector<unsigned> &in_off, const std::vector<unsigned>
 }
 
 /* One resident launch at a time per device: the launches of two streams,
- * each partly on the chip, would wait for each other.  Each leaves an event
- * behind it on its own stream, and a launch on another stream waits for that.
- * After a launch on a caller's stream every launch waits: equal values do not
+ * each partly on the chip, would wait for each other.  A launch on another
+ * stream than the last one waits for an event behind that one.
+ *
+ * If the last stream is a handle's, which lives until bp_resident_free, the
+ * event is recorded by the launch that needs it: recorded behind every launch
+ * it took 1 to 5 us of each call (10 iterations of 5,000 nodes with deltas
+ * and beliefs read back 73 / 78 us, 500k nodes 321 / 326).  The stream's
+ * owner may be another thread, so captures on a handle's stream are made
+ * under the same lock: an event recorded in one would become part of it, and
+ * so would the launch that waits for it.
+ *
+ * A caller's stream may be in capture or gone by then: its event is recorded
+ * with the launch, and every launch waits for it, since equal values do not
  * say that it is the same stream (hipStreamPerThread is one value for all
- * threads, and that of a destroyed stream is given out again).
- * Nothing is put on another launch's stream: its owner may be capturing on it
- * in another thread, or have queued more work since. */
+ * threads, and that of a destroyed stream is given out again). */
 constexpr int MAX_DEVICES = 64;
 std::mutex turn_mu;
 struct {
     bool any, foreign; /* foreign: on a caller's stream */
     hipStream_t last;
-    hipEvent_t ev; /* after the last launch; created with the device's first plan */
+    hipEvent_t ev; /* behind the last launch; created with the device's first plan */
 } turn[MAX_DEVICES];
 
 template <int S, bool MIXED, int NS, bool SINGLE>
@@ -674,8 +682,11 @@ std::mutex &bp_resident_mutex() { return turn_mu; }
 int bp_resident_turn(int device, hipStream_t stream)
 {
     const auto &t = turn[device];
-    if (t.any && (t.foreign || t.last != stream))
+    if (t.any && (t.foreign || t.last != stream)) {
+        if (!t.foreign)
+            HIP_TRY(hipEventRecord(t.ev, t.last));
         HIP_TRY(hipStreamWaitEvent(stream, t.ev, 0));
+    }
     return 0;
 }
 
@@ -685,7 +696,8 @@ int bp_resident_turn_taken(int device, hipStream_t stream, bool foreign)
     t.any = true;
     t.foreign = foreign;
     t.last = stream;
-    HIP_TRY(hipEventRecord(t.ev, stream));
+    if (foreign)
+        HIP_TRY(hipEventRecord(t.ev, stream));
     return 0;
 }
 

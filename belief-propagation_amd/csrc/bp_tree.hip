@@ -641,9 +641,12 @@ extern "C" int bp_tree(bp_dev *d)
     hipGraphExec_t &exec = d->tree->graph[a_index(d)];
     if (!exec) {
         hipGraph_t graph;
-        HIP_TRY(hipStreamBeginCapture(d->stream, hipStreamCaptureModeThreadLocal));
-        enqueue(d, d->tree, true);
-        HIP_TRY(hipStreamEndCapture(d->stream, &graph));
+        {
+            std::lock_guard<std::mutex> lock(bp_resident_mutex());
+            HIP_TRY(hipStreamBeginCapture(d->stream, hipStreamCaptureModeThreadLocal));
+            enqueue(d, d->tree, true);
+            HIP_TRY(hipStreamEndCapture(d->stream, &graph));
+        }
         hipError_t e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
         (void)hipGraphDestroy(graph);
         if (e != hipSuccess) {

@@ -90,6 +90,7 @@ def test_uploads_beside_a_capture(run, what):
 
 
 def child_uploads_beside_a_capture(fake, what):
+    import time
     from concurrent.futures import ThreadPoolExecutor
 
     B, lib = fake.B, fake.lib
@@ -113,9 +114,16 @@ def child_uploads_beside_a_capture(fake, what):
 
     a = fake.device(3000)
     a.init()
+    runs = []
+
+    def meanwhile():
+        runs.append(thread.submit(other))
+        time.sleep(0.3)
+
     with ThreadPoolExecutor(1) as thread:
-        fake.when("capture", lambda: thread.submit(other).result(timeout=60))
+        fake.when("capture", meanwhile)
         a.iterate(2)
+        runs[0].result(timeout=30)
     assert len(fake.calls("stream")) == 2 and not fake.calls("memcpy", "memset", "devicesync")
 
 
@@ -127,6 +135,7 @@ def test_a_run_keeps_off_a_stream_in_capture(run, captures):
 
 
 def child_a_run_keeps_off_a_stream_in_capture(fake, captures):
+    import time
     from concurrent.futures import ThreadPoolExecutor
 
     a, b = fake.device(3000), fake.device(5000)
@@ -134,16 +143,22 @@ def child_a_run_keeps_off_a_stream_in_capture(fake, captures):
     b.init()
     a.iterate(9)
     fake.clear()
-    with ThreadPoolExecutor(1) as other:
-        fake.when("capture", lambda: other.submit(b.iterate, 9).result(timeout=30))
+    runs = []
+
+    def meanwhile():
+        runs.append(thread.submit(b.iterate, 9))
+        time.sleep(0.3)
+
+    with ThreadPoolExecutor(1) as thread:
+        fake.when("capture", meanwhile)
         a.iterate(2) if captures == "iterate" else a.tree()
-    begin, end = (fake.log().index(x[0]) for x in (fake.calls("begincapture"), fake.calls("endcapture")))
-    inside = fake.log()[begin:end]
+        runs[0].result(timeout=30)
     own = fake.calls("begincapture")[0][1]
-    # b's run went to its own stream, after a's run, and left a's stream alone
-    assert [x for x in inside if x[0] == "launch" and x[1] != own and "captured" not in x]
-    assert [x for x in inside if x[0] == "wait" and x[1] != own]
-    assert not [x for x in inside if x[0] == "record" and x[2] == own], inside
+    # b's run went to its own stream, behind a's run, and nothing that is not
+    # a's own got into the capture
+    assert [x for x in fake.calls("launch") if x[1] != own and "captured" not in x]
+    assert [x for x in fake.calls("wait") if x[1] != own]
+    assert not [x for x in fake.calls("record") if "captured" in x], fake.log()
 
 
 def test_equal_streams_of_two_callers(run):

@@ -64,8 +64,9 @@ int bp_batch_set_config(bp_batch *b, unsigned int slots_per_lane, unsigned int l
 int bp_batch_get_config(const bp_batch *b, unsigned int *slots_per_lane, unsigned int *lanes_per_slot,
                         unsigned int *queue_block);
 
-/* Times every candidate shape over `iterations` iterations and keeps the
- * fastest.  cache_path (nullable): a JSON file of earlier choices keyed by
+/* Times every candidate shape over `iterations` iterations with deltas and
+ * keeps the fastest (iterations without deltas rank the shapes the same to a
+ * few per cent).  cache_path (nullable): a JSON file of earlier choices keyed by
  * the device and the batch's sizes; a hit skips the timing, a miss adds an
  * entry. */
 int bp_batch_tune(bp_batch *b, unsigned int iterations, const char *cache_path);

@@ -19,7 +19,8 @@
  * Forward.  init_previous_edge + K iterations of the node-centric schedule
  * (bit-identical beliefs to bp_loopy_iterate on the same tables), keeping
  * the beliefs and combine buffers of every iteration where they take at
- * most 512 MB, and otherwise of every c-th.
+ * most 512 MB, whatever c is, and otherwise (or where that memory is not to be
+ * had) of every c-th.
  *
  * Backward.  Reverse-mode adjoint of the same recursion, in exact
  * arithmetic terms:
@@ -29,8 +30,11 @@
  * recomputed by the forward kernel, segment by segment.  Returns dL/dTABLE
  * for every parameter entry given dL/dbeliefs after iteration K.  Networks
  * whose tables, and their gradients, fit on the chip go through all
- * iterations in one launch, forward and backward; under stream capture each
- * iteration is a launch of its own.  The first call with a K and c allocates
+ * iterations in one launch, forward and backward; the backward then keeps a
+ * row per message edge and step, in up to 512 MB more.  A launch that was
+ * given up (include/bp_hip.h) is made up for on the device, and the handle
+ * runs a launch per iteration from then on.  Under stream capture each
+ * iteration is a launch of its own too.  The first call with a K and c allocates
  * and cannot be captured.  A captured graph uses what is stored for its K and
  * c: a call with another pair, or bp_diff_free, ends its use.
  *

@@ -102,10 +102,13 @@ int bp_loopy_init(bp_dev *d);
 
 /* n loopy iterations; deltas (nullable) receives the FP64 delta of each;
  * without it deltas are not formed.  A network that fits on the chip (up to
- * 2.1M message edges of 2 states, 262k of 8) runs them in one launch;
- * otherwise the launches are replayed from a cached HIP graph.  A launch
- * that was given up (its workgroups wait for each other at most a second) is
- * made up for by the handle's next call. */
+ * 2.03M message edges of 2 states, 1.01M of 3, 0.76M of 4, 0.25M of 5 to 8,
+ * less where nodes with many edges do not share out evenly) runs them in one
+ * launch; otherwise the launches are replayed from a cached HIP graph.  A
+ * launch that was given up (its workgroups wait for each other at most a
+ * second: other work kept part of the chip for longer, another process for
+ * one) is made up for by the handle's next call, and the handle runs a launch
+ * per iteration from then on. */
 int bp_loopy_iterate(bp_dev *d, unsigned int n, double *deltas);
 
 /* No counterpart in the reference.  For callers that cannot allocate device

@@ -503,7 +503,7 @@ extern "C" int bp_batch_upload(bp_batch *b, int device)
         return -1;
     }
     int ndev = 0;
-    if (hipGetDeviceCount(&ndev) != hipSuccess || ndev == 0) {
+    if (taken(hipGetDeviceCount(&ndev)) != hipSuccess || ndev == 0) {
         bp_set_error("no HIP device available: the belief-propagation kernels need an MI355X (gfx950)");
         return -1;
     }
@@ -831,7 +831,7 @@ extern "C" int bp_batch_iterate(bp_batch *b, unsigned int n, double *deltas)
         hipGraph_t graph = nullptr;
         HIP_TRY(hipStreamEndCapture(b->stream, &graph));
         hipGraphExec_t exec = nullptr;
-        hipError_t err = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
+        hipError_t err = taken(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
         (void)hipGraphDestroy(graph);
         if (err != hipSuccess) {
             bp_set_error("hipGraphInstantiate failed: %s", hipGetErrorString(err));

@@ -16,9 +16,19 @@
 
 extern "C" void bp_set_error(const char *fmt, ...);
 
+/* The result of a call whose failure the library reports in its own way: the
+ * runtime's record of it goes, which the check after the thread's next launch
+ * would report again. */
+inline hipError_t taken(hipError_t err)
+{
+    if (err != hipSuccess)
+        (void)hipGetLastError();
+    return err;
+}
+
 #define HIP_TRY(expr)                                                                        \
     do {                                                                                     \
-        hipError_t err_ = (expr);                                                            \
+        hipError_t err_ = taken(expr);                                                       \
         if (err_ != hipSuccess) {                                                            \
             bp_set_error("%s failed: %s (%s:%d)", #expr, hipGetErrorString(err_), __FILE__, \
                          __LINE__);                                                          \

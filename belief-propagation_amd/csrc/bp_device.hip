@@ -136,7 +136,7 @@ extern "C" void bp_free(bp_dev *d)
 extern "C" int bp_device_count(void)
 {
     int n = 0;
-    if (hipGetDeviceCount(&n) != hipSuccess)
+    if (taken(hipGetDeviceCount(&n)) != hipSuccess)
         return 0;
     return n;
 }
@@ -473,8 +473,9 @@ static float *stage_buf(bp_dev *d, size_t n)
             (void)hipHostFree(d->h_stage);
         d->h_stage = nullptr;
         d->h_stage_n = 0;
-        if (hipHostMalloc((void **)&d->h_stage, sizeof(bp_resident_status) + std::max<size_t>(n, 1) * sizeof(float),
-                          hipHostMallocDefault) != hipSuccess) {
+        if (taken(hipHostMalloc((void **)&d->h_stage,
+                                sizeof(bp_resident_status) + std::max<size_t>(n, 1) * sizeof(float),
+                                hipHostMallocDefault)) != hipSuccess) {
             d->h_stage = nullptr;
             bp_set_error("pinned staging buffer of %zu floats: allocation failed", n);
             return nullptr;
@@ -874,7 +875,7 @@ static int upload_impl(Graph_t g, int device, bp_dev **out, bool plan, bool grad
     if (check_graph(g))
         return -1;
     int ndev = 0;
-    if (hipGetDeviceCount(&ndev) != hipSuccess || ndev == 0) {
+    if (taken(hipGetDeviceCount(&ndev)) != hipSuccess || ndev == 0) {
         bp_set_error("no HIP device available: the belief-propagation kernels need an MI355X (gfx950)");
         return -1;
     }
@@ -891,7 +892,7 @@ static int upload_impl(Graph_t g, int device, bp_dev **out, bool plan, bool grad
         delete d;
         return -1;
     }
-    if (hipStreamCreateWithFlags(&d->stream, hipStreamNonBlocking) != hipSuccess) {
+    if (taken(hipStreamCreateWithFlags(&d->stream, hipStreamNonBlocking)) != hipSuccess) {
         bp_set_error("hipStreamCreate failed");
         delete d;
         return -1;
@@ -1035,7 +1036,7 @@ static int upload_impl(Graph_t g, int device, bp_dev **out, bool plan, bool grad
         at.add(d->Jp, nullptr, (size_t)E * S * S);
         at.add(d->slot_pool, nullptr, E);
     }
-    if (hipMalloc((void **)&d->memory, at.bytes) != hipSuccess) {
+    if (taken(hipMalloc((void **)&d->memory, at.bytes)) != hipSuccess) {
         bp_set_error("upload: no %zu bytes of device memory", at.bytes);
         d->memory = nullptr;
         bp_free(d);
@@ -1046,9 +1047,9 @@ static int upload_impl(Graph_t g, int device, bp_dev **out, bool plan, bool grad
     bool ok = head != nullptr;
     if (ok) {
         at.gather(head);
-        ok = hipMemcpyAsync(d->memory, head, copied, hipMemcpyHostToDevice, d->stream) == hipSuccess &&
-             hipMemsetAsync(d->memory + zero, 0, zeroed - zero, d->stream) == hipSuccess &&
-             hipStreamSynchronize(d->stream) == hipSuccess;
+        ok = taken(hipMemcpyAsync(d->memory, head, copied, hipMemcpyHostToDevice, d->stream)) == hipSuccess &&
+             taken(hipMemsetAsync(d->memory + zero, 0, zeroed - zero, d->stream)) == hipSuccess &&
+             taken(hipStreamSynchronize(d->stream)) == hipSuccess;
     }
     if (!ok) {
         bp_set_error("upload of the graph structure failed");
@@ -1063,7 +1064,6 @@ static int upload_impl(Graph_t g, int device, bp_dev **out, bool plan, bool grad
      * for that it runs them one launch each */
     if (bp_resident_plan(d, slot_src, gradients, prop.multiProcessorCount) != 0) {
         bp_resident_free(d);
-        (void)hipGetLastError();
         bp_clear_error();
     }
     /* the tree schedule needs levels; without them bp_tree() reports it */
@@ -1420,7 +1420,7 @@ static int iterate_launches(bp_dev *d, unsigned n, double *deltas)
                 HIP_TRY(hipStreamEndCapture(d->stream, &graph));
             }
             hipGraphExec_t exec;
-            hipError_t e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
+            hipError_t e = taken(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
             (void)hipGraphDestroy(graph);
             if (e != hipSuccess) {
                 bp_set_error("hipGraphInstantiate failed: %s", hipGetErrorString(e));
@@ -1470,7 +1470,7 @@ static int noalloc_scratch(int device, double **out)
     std::lock_guard<std::mutex> lock(noalloc_mu);
     if (!noalloc_ptr[device]) {
         void *p = nullptr;
-        hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
+        hipError_t e = taken(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
         if (e != hipSuccess || !p) {
             bp_set_error("bp_loopy_iterate_noalloc: hipGetSymbolAddress(scratch) on device %d failed: %s", device,
                          hipGetErrorString(e));
@@ -1897,7 +1897,7 @@ extern "C" int bp_download_states(bp_dev *d, float *out)
     HIP_TRY(hipEventSynchronize(d->slice_ev[0]));
     std::atomic<int> bad{0};
     bp_parallel(slices, [&](unsigned i) {
-        if (hipSetDevice(d->device) != hipSuccess || hipEventSynchronize(d->slice_ev[i]) != hipSuccess) {
+        if (taken(hipSetDevice(d->device)) != hipSuccess || taken(hipEventSynchronize(d->slice_ev[i])) != hipSuccess) {
             bad = 1;
             return;
         }
@@ -2136,27 +2136,28 @@ extern "C" void send_message(float *states, unsigned int offset, unsigned int ed
     for (unsigned j = 0; j < y; ++j)
         in[NJ + j] = states[offset + j];
     int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= SEND_MAX_DEVICES) {
+    if (taken(hipGetDevice(&dev)) != hipSuccess || dev < 0 || dev >= SEND_MAX_DEVICES) {
         bp_fail("send_message: no usable HIP device");
         return;
     }
     std::lock_guard<std::mutex> lock(g_send_mu);
     auto &st = g_send[dev];
     if (!st.buf) {
-        if (hipStreamCreateWithFlags(&st.stream, hipStreamNonBlocking) != hipSuccess ||
-            hipMalloc((void **)&st.buf, (NJ + 2 * MAX_STATES) * sizeof(float)) != hipSuccess) {
+        if (taken(hipStreamCreateWithFlags(&st.stream, hipStreamNonBlocking)) != hipSuccess ||
+            taken(hipMalloc((void **)&st.buf, (NJ + 2 * MAX_STATES) * sizeof(float))) != hipSuccess) {
             st.buf = nullptr;
             bp_fail("send_message: no usable HIP device");
             return;
         }
     }
-    bool ok = hipMemcpyAsync(st.buf, in, sizeof(in), hipMemcpyHostToDevice, st.stream) == hipSuccess;
+    bool ok = taken(hipMemcpyAsync(st.buf, in, sizeof(in), hipMemcpyHostToDevice, st.stream)) == hipSuccess;
     if (ok) {
         hipLaunchKernelGGL(k_send_one<MAX_STATES>, dim3(1), dim3(64), 0, st.stream, st.buf, st.buf + NJ, x, y,
                            st.buf + NJ + MAX_STATES);
         ok = hipGetLastError() == hipSuccess &&
-             hipMemcpyAsync(m, st.buf + NJ + MAX_STATES, sizeof(m), hipMemcpyDeviceToHost, st.stream) == hipSuccess &&
-             hipStreamSynchronize(st.stream) == hipSuccess;
+             taken(hipMemcpyAsync(m, st.buf + NJ + MAX_STATES, sizeof(m), hipMemcpyDeviceToHost, st.stream)) ==
+                 hipSuccess &&
+             taken(hipStreamSynchronize(st.stream)) == hipSuccess;
     }
     if (!ok) {
         bp_fail("send_message: the GPU send failed");

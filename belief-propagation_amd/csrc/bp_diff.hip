@@ -757,12 +757,12 @@ extern "C" int bp_diff_create(const bp_bn *bn, unsigned int num_param_defs, int 
         rc = diff_build(x, bn, num_param_defs, g);
         /* nodes without a parameter prior keep their initial beliefs */
         if (rc == 0 && x->V &&
-            hipMemcpyAsync(x->st0, x->d->states0, (size_t)x->V * x->SP * sizeof(float), hipMemcpyDeviceToDevice,
-                           x->d->stream) != hipSuccess) {
+            taken(hipMemcpyAsync(x->st0, x->d->states0, (size_t)x->V * x->SP * sizeof(float), hipMemcpyDeviceToDevice,
+                                 x->d->stream)) != hipSuccess) {
             bp_set_error("bp_diff_create: copying the initial beliefs failed");
             rc = -1;
         }
-        if (rc == 0 && hipStreamSynchronize(x->d->stream) != hipSuccess)
+        if (rc == 0 && taken(hipStreamSynchronize(x->d->stream)) != hipSuccess)
             rc = -1;
         if (rc == 0 && bp_resident_diff_fits(x->d, x->max_in) &&
             (dmalloc(&x->out_at, x->E) || bp_resident_diff_places(x->d, x->slot_pos, x->out_at)))
@@ -854,10 +854,9 @@ static int diff_storage(bp_diff *x, unsigned K, unsigned c)
     /* (without the memory for it the backward runs its launches) */
     if (c == 1 && x->out_at) {
         const size_t rows = ((size_t)K + 1) * bp_resident_diff_rows(x->d);
-        if (rows * sizeof(float) <= x->keep_bytes && hipMalloc((void **)&x->rows, rows * sizeof(float)) != hipSuccess) {
+        if (rows * sizeof(float) <= x->keep_bytes &&
+            taken(hipMalloc((void **)&x->rows, rows * sizeof(float))) != hipSuccess)
             x->rows = nullptr;
-            (void)hipGetLastError();
-        }
     }
     x->K = K;
     x->c = c;
@@ -891,7 +890,7 @@ static int capture_end(bp_diff *x, hipGraphExec_t *exec)
 {
     hipGraph_t graph = nullptr;
     HIP_TRY(hipStreamEndCapture(x->d->stream, &graph));
-    hipError_t err = hipGraphInstantiate(exec, graph, nullptr, nullptr, 0);
+    hipError_t err = taken(hipGraphInstantiate(exec, graph, nullptr, nullptr, 0));
     (void)hipGraphDestroy(graph);
     if (err != hipSuccess) {
         bp_set_error("hipGraphInstantiate failed: %s", hipGetErrorString(err));
@@ -926,8 +925,8 @@ static void enqueue_forward(bp_diff *x, hipStream_t st)
 static bool is_capturing(hipStream_t st)
 {
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    if (st && hipStreamIsCapturing(st, &capturing) != hipSuccess)
-        (void)hipGetLastError();
+    if (st)
+        (void)taken(hipStreamIsCapturing(st, &capturing));
     return capturing != hipStreamCaptureStatusNone;
 }
 
@@ -992,8 +991,7 @@ extern "C" int bp_diff_forward(bp_diff *x, unsigned int K, unsigned int c, float
     if (!stored && diff_storage(x, K, every)) {
         if (every == c)
             return -1;
-        (void)hipGetLastError(); /* not the memory for all of them */
-        bp_clear_error();
+        bp_clear_error(); /* not the memory for all of them */
         if (diff_storage(x, K, c))
             return -1;
     }

@@ -647,7 +647,7 @@ extern "C" int bp_tree(bp_dev *d)
             enqueue(d, d->tree, true);
             HIP_TRY(hipStreamEndCapture(d->stream, &graph));
         }
-        hipError_t e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
+        hipError_t e = taken(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
         (void)hipGraphDestroy(graph);
         if (e != hipSuccess) {
             exec = nullptr;
@@ -693,7 +693,7 @@ static void run_partial(Graph_t g, const char *who, int mode, unsigned level)
             return;
         }
     }
-    if (hipSetDevice(d->device) != hipSuccess) {
+    if (taken(hipSetDevice(d->device)) != hipSuccess) {
         bp_tree_plan_free(p);
         bp_fail("%s: hipSetDevice failed", who);
         return;
@@ -701,7 +701,7 @@ static void run_partial(Graph_t g, const char *who, int mode, unsigned level)
     enqueue(d, p, mode == 2);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess)
-        e = hipStreamSynchronize(d->stream);
+        e = taken(hipStreamSynchronize(d->stream));
     bp_tree_plan_free(p);
     if (e != hipSuccess) {
         bp_fail("%s: %s", who, hipGetErrorString(e));

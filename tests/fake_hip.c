@@ -20,6 +20,7 @@ static pthread_mutex_t mu = PTHREAD_MUTEX_INITIALIZER;
 static char log_text[LOG_BYTES];
 static size_t log_at, most_bytes = (size_t)-1;
 static unsigned long long heap_calls; /* operator new of the library and libstdc++ */
+static int fail_at = -1;
 static void (*on_capture)(void);
 static void (*on_launch)(void);
 
@@ -51,6 +52,7 @@ void fake_clear(void)
     heap_calls = 0;
     pthread_mutex_unlock(&mu);
 }
+void fake_fail_at(int n) { fail_at = n; } /* the n-th allocation from now on fails, 0: the next */
 void fake_most_bytes(size_t bytes) { most_bytes = bytes; } /* larger allocations fail from now on */
 void fake_on_capture(void (*f)(void)) { on_capture = f; }  /* called while a stream is in capture */
 void fake_on_launch(void (*f)(void)) { on_launch = f; }
@@ -66,14 +68,24 @@ void *_Znwm(size_t n) /* operator new */
 
 /* ---- memory --------------------------------------------------------------- */
 
+/* the last error of the calling thread, as the runtime keeps it */
+static __thread hipError_t last_error;
+
+static hipError_t allocate(void **p, size_t n)
+{
+    int fails = n > most_bytes;
+    if (fail_at >= 0)
+        fails |= fail_at-- == 0;
+    *p = fails ? NULL : aligned_alloc(256, (n + 511) / 256 * 256);
+    if (!*p)
+        return last_error = hipErrorOutOfMemory;
+    memset(*p, 0, n);
+    return hipSuccess;
+}
 hipError_t hipMalloc(void **p, size_t n)
 {
     note("malloc %zu\n", n);
-    *p = n > most_bytes ? NULL : aligned_alloc(256, (n + 511) / 256 * 256);
-    if (!*p)
-        return hipErrorOutOfMemory;
-    memset(*p, 0, n);
-    return hipSuccess;
+    return allocate(p, n);
 }
 hipError_t hipFree(void *p)
 {
@@ -85,8 +97,7 @@ hipError_t hipHostMalloc(void **p, size_t n, unsigned flags)
 {
     (void)flags;
     note("hostmalloc %zu\n", n);
-    *p = aligned_alloc(256, (n + 511) / 256 * 256);
-    return *p ? hipSuccess : hipErrorOutOfMemory;
+    return allocate(p, n);
 }
 hipError_t hipHostFree(void *p)
 {
@@ -155,8 +166,6 @@ hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600 *p, int d)
     return hipSuccess;
 }
 
-/* the last error of the calling thread, as the runtime keeps it */
-static __thread hipError_t last_error;
 hipError_t hipGetLastError(void)
 {
     hipError_t e = last_error;

@@ -282,5 +282,63 @@ def child_downloads_of_one_handle_from_two_threads(fake, what):
     assert seen[1] == 1 and len(fake.calls("launch")) == 2
 
 
+@pytest.mark.parametrize("what", ["device", "diff"])
+def test_an_error_is_reported_once(run, what):
+    """Each allocation of an upload fails in turn: the call says so or does
+    without the memory, and the calls after it do not say it again."""
+    run(what)
+
+
+def child_an_error_is_reported_once(fake, what):
+    B, lib = fake.B, fake.lib
+    bn = B.generate("c5" if what == "diff" else "c2", num_nodes=1500)
+    g = B.bn_to_graph(bn, levels=True)
+    healthy = B.Device(g)
+
+    def failing(f, n):
+        """f() with its n-th allocation failing; whether there was an n-th"""
+        fake.clear()
+        fake.so.fake_fail_at(n)
+        rc = f()
+        fake.so.fake_fail_at(-1)
+        failed = len(fake.calls("malloc", "hostmalloc")) > n
+        assert B.last_error() if rc else True
+        assert failed or rc == 0
+        healthy.init()
+        return rc, failed
+
+    n, failed = 0, True
+    while failed and what == "device":
+        h = C.c_void_p()
+        rc, failed = failing(lambda: lib.bp_upload(g, -1, C.byref(h)), n)
+        assert (rc == 0) == bool(h)
+        if h:  # (without the memory for resident runs or the tree)
+            assert lib.bp_loopy_init(h) == 0 and lib.bp_loopy_iterate(h, 9, None) == 0 and lib.bp_download(h, g) == 0
+            lib.bp_free(h)
+        n += 1
+    while failed and what == "diff":
+        x = C.c_void_p()
+        rc, failed = failing(lambda: lib.bp_diff_create(bn, 1500, 0, C.byref(x)), n)
+        assert (rc == 0) == bool(x)
+        if failed and x:
+            lib.bp_diff_free(x)
+        n += 1
+    if what == "diff":
+        created, n, failed = n, 0, True
+        info = (C.c_uint64 * 6)()
+        lib.bp_diff_info(x, info)
+        theta, out = (C.c_float * info[4])(), (C.c_float * (info[0] * info[3]))()
+        assert lib.bp_diff_set_log_params(x, theta, None) == 0
+        while failed:  # another K each time, so that each call allocates
+            rc, failed = failing(lambda: lib.bp_diff_forward(x, 5 + n, 2, out, None), n)
+            assert rc == 0 or lib.bp_diff_backward_log(x, out, theta, None) == -1
+            assert lib.bp_diff_forward(x, 5 + n, 2, out, None) == 0
+            assert lib.bp_diff_backward_log(x, out, theta, None) == 0
+            n += 1
+        lib.bp_diff_free(x)
+        n += created
+    assert n > 1
+
+
 if __name__ == "__main__":
     globals()["child_" + sys.argv[2]](Fake(sys.argv[1]), *sys.argv[3:])

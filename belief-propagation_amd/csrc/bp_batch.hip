@@ -169,7 +169,8 @@ struct bp_batch {
     std::vector<unsigned long long> node_row_off{0}, msg_row_off{0};
     double alg_bytes = 0.0;
     uint64_t distinct_floats = 0; /* a table and its transpose counted once */
-    bool uploaded = false;
+    bool begun = false;    /* an upload has begun: nothing more is added, and bp_batch_free releases device memory */
+    bool uploaded = false; /* ... and ended well */
 
     /* device */
     int device = 0;
@@ -217,7 +218,7 @@ extern "C" void bp_batch_free(bp_batch *b)
 {
     if (!b)
         return;
-    if (b->uploaded) {
+    if (b->begun) {
         (void)hipSetDevice(b->device);
         if (b->stream)
             (void)hipStreamSynchronize(b->stream);
@@ -290,7 +291,7 @@ extern "C" int bp_batch_add(bp_batch *b, Graph_t g, unsigned int *index)
         bp_set_error("bp_batch_add: NULL argument");
         return -1;
     }
-    if (b->uploaded) {
+    if (b->begun) {
         bp_set_error("bp_batch_add: the batch is already on the device");
         return -1;
     }
@@ -498,8 +499,8 @@ extern "C" int bp_batch_upload(bp_batch *b, int device)
         bp_set_error("bp_batch_upload: NULL argument");
         return -1;
     }
-    if (b->uploaded) {
-        bp_set_error("bp_batch_upload: already uploaded");
+    if (b->begun) {
+        bp_set_error(b->uploaded ? "bp_batch_upload: already uploaded" : "bp_batch_upload: an earlier upload failed");
         return -1;
     }
     int ndev = 0;
@@ -528,7 +529,7 @@ extern "C" int bp_batch_upload(bp_batch *b, int device)
     b->R = (b->S <= 4) ? 2 : 1;
     b->qblock = 0;
     HIP_TRY(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking));
-    b->uploaded = true; /* from here on bp_batch_free releases device memory */
+    b->begun = true;
 
     /* compact rows; floats of slack past the last row, which the kernels'
      * unpredicated row loads (up to 8 floats, or S) may read */
@@ -585,6 +586,7 @@ extern "C" int bp_batch_upload(bp_batch *b, int device)
     std::vector<unsigned char>().swap(b->slot_xy);
     std::vector<float>().swap(b->tabs);
     b->lookup.clear();
+    b->uploaded = true;
     return 0;
 }
 

@@ -340,5 +340,35 @@ def child_an_error_is_reported_once(fake, what):
     assert n > 1
 
 
+def test_a_batch_whose_upload_failed(run):
+    """Each allocation of the upload fails in turn: the batch is refused
+    everywhere, nothing is launched on it, and it can be freed."""
+    run()
+
+
+def child_a_batch_whose_upload_failed(fake):
+    B, lib = fake.B, fake.lib
+    bn = B.generate("c4net", num_nodes=300, states_hi=4)
+    g = B.bn_to_graph(bn)
+    n, failed = 0, True
+    while failed:
+        b = B.Batch()
+        b.add(g)
+        fake.clear()
+        fake.so.fake_fail_at(n)
+        rc = lib.bp_batch_upload(b.h, -1)
+        fake.so.fake_fail_at(-1)
+        failed = len(fake.calls("malloc", "hostmalloc")) > n
+        assert rc == (-1 if failed else 0)
+        fake.clear()
+        uses = [lib.bp_batch_init(b.h), lib.bp_batch_iterate(b.h, 3, None), lib.bp_batch_download(b.h, 0, g),
+                lib.bp_batch_sync(b.h), lib.bp_batch_set_config(b.h, 1, 1, 0), lib.bp_batch_tune(b.h, 1, None)]
+        assert set(uses) == {rc} and bool(fake.calls("launch")) == (rc == 0)
+        assert lib.bp_batch_upload(b.h, -1) == -1 and lib.bp_batch_add(b.h, g, None) == -1
+        b.free()
+        n += 1
+    assert n > 10
+
+
 if __name__ == "__main__":
     globals()["child_" + sys.argv[2]](Fake(sys.argv[1]), *sys.argv[3:])

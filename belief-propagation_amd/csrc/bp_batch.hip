@@ -790,6 +790,7 @@ static int ensure_deltas(bp_batch *b, unsigned n)
     if (b->d_deltas)
         HIP_TRY(hipFree(b->d_deltas));
     b->d_deltas = nullptr;
+    b->deltas_cap = 0;
     batch_clear_graphs(b); /* captured graphs hold the old address */
     if (dmalloc(&b->d_deltas, need))
         return -1;

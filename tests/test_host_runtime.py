@@ -370,5 +370,26 @@ def child_a_batch_whose_upload_failed(fake):
     assert n > 10
 
 
+def test_deltas_that_found_no_memory(run):
+    """A batch's deltas: a call that finds no memory for them fails, and a
+    smaller one after it has memory of its own."""
+    run()
+
+
+def child_deltas_that_found_no_memory(fake):
+    B, lib = fake.B, fake.lib
+    bn = B.generate("c4net", num_nodes=300, states_hi=4)
+    b = B.Batch()
+    b.add(B.bn_to_graph(bn))
+    b.upload()
+    b.init()
+    b.iterate(10, want_deltas=True)
+    fake.so.fake_fail_at(0)
+    assert lib.bp_batch_iterate(b.h, 20, (C.c_double * 20)()) == -1
+    fake.clear()
+    b.iterate(10, want_deltas=True)
+    assert len(fake.calls("malloc")) == 1
+
+
 if __name__ == "__main__":
     globals()["child_" + sys.argv[2]](Fake(sys.argv[1]), *sys.argv[3:])
